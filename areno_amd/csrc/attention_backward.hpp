@@ -1,6 +1,6 @@
 // Arguments shared by the backward kernels of the causal varlen / dense attention ops (attention_backward.hip: the
 // vector-ALU kernels for every head dim and dtype; attention_backward_mfma.hip: matrix-core kernels for 16-bit
-// inputs at head dims 64 and 128).
+// inputs at head dims 64, 128, 192 and 256).
 #pragma once
 
 #include <stdint.h>

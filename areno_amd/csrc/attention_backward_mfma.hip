@@ -1,5 +1,5 @@
-// Backward of the causal varlen / dense attention ops on the matrix cores (gfx950): 16-bit inputs, head dims 64 and
-// 128.  Same contract as the vector-ALU kernels of attention_backward.hip (fp32 dQ, dK, dV from dO, Q, K, V and the
+// Backward of the causal varlen / dense attention ops on the matrix cores (gfx950): 16-bit inputs, head dims 64,
+// 128, 192 and 256.  Same contract as the vector-ALU kernels of attention_backward.hip (fp32 dQ, dK, dV from dO, Q, K, V and the
 // saved output; areno/accel/csrc/attention.cu:244-524 in the reference), same two launches, no atomics:
 //
 //   dq kernel    a workgroup owns 64 or 128 packed query rows of one q head (four waves of 16 or 32 rows) and streams
@@ -69,7 +69,7 @@ template <int D>
 struct BmTile {
   static constexpr int RS = D * 2 + 16;
   static constexpr int kChunksPerRow = D * 2 / 16;
-  static constexpr int kChunks = kBmTile * kChunksPerRow / kBmThreads;  // per thread: 1 (D = 64) or 2 (D = 128)
+  static constexpr int kChunks = kBmTile * kChunksPerRow / kBmThreads;  // per thread: 1 (D = 64) to 4 (D = 256)
   static_assert(kBmTile * kChunksPerRow % kBmThreads == 0, "tile chunks");
   static __device__ __forceinline__ int chunk_pos(int r, int c) { return r * RS + (c << 4); }
 };
@@ -664,17 +664,24 @@ DkvLaunch dkv_launch() {
   }
   return DkvLaunch{fn, L::kLdsBytes, L::kThreads, KR};
 }
+// Head dims 192 and 256 have one shape: the sums and operands of 16 key rows take all registers of two waves per SIMD,
+// and six or eight waves behind one stream of tiles stage two chunks of a tensor per thread and step (four waves:
+// four chunks, which the registers have no room for).
 template <int KIND, int D>
 DkvLaunch dkv_launch(int parts) {
-  if (parts == 4) return dkv_launch<KIND, D, 32, 4>();
-  return parts == 2 ? dkv_launch<KIND, D, 64, 2>() : dkv_launch<KIND, D, 64, 1>();
+  if constexpr (D > 128) return dkv_launch<KIND, D, D == 256 ? 128 : 96, 1>();
+  if constexpr (D <= 128) {
+    if (parts == 4) return dkv_launch<KIND, D, 32, 4>();
+    if (parts == 2) return dkv_launch<KIND, D, 64, 2>();
+    return dkv_launch<KIND, D, 64, 1>();
+  }
 }
 
 }  // namespace
 
 int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
   if (p.dtype != ARENO_DT_BF16 && p.dtype != ARENO_DT_F16) return ARENO_ERR_UNSUPPORTED;
-  if (p.head_dim != 64 && p.head_dim != 128) return ARENO_ERR_UNSUPPORTED;
+  if (p.head_dim != 64 && p.head_dim != 128 && p.head_dim != 192 && p.head_dim != 256) return ARENO_ERR_UNSUPPORTED;
   if (p.q_heads > 65535 || p.kv_heads > 65535) return ARENO_ERR_UNSUPPORTED;
   const int64_t q_blocks = (p.q_tokens + kBmRows - 1) / kBmRows, k_blocks = (p.k_tokens + kBmRows - 1) / kBmRows;
   if (q_blocks * p.q_heads > 0x7fffffffLL || k_blocks * p.kv_heads > 0x7fffffffLL) return ARENO_ERR_UNSUPPORTED;
@@ -713,6 +720,13 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
     if (strcmp(e, "32") == 0) dq_cb = 2;
     if (strcmp(e, "16") == 0) dq_cb = 1;
   }
+  // Head dims 192 and 256 (the sliding-window layers of wide heads) have one shape of either kernel.  2 400 tokens in
+  // four sequences, 16 / 8 heads of 256, window 512, bf16: 323 us for both launches against 7 470 us on the
+  // vector-ALU kernels, which recompute every product on 16 lanes' dot products.
+  if (p.head_dim > 128) {
+    dkv_parts = 1;
+    dq_cb = 1;
+  }
   const int64_t dq_blocks = (p.q_tokens + kBmRows * dq_cb - 1) / (kBmRows * dq_cb);
   bm_fn dq;
   DkvLaunch dkv;
@@ -720,6 +734,12 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
     dq = dq_cb == 2 ? (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 64, 2> : bwd_mfma_dq_kernel<KV_F16, 64, 2>)
                     : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 64, 1> : bwd_mfma_dq_kernel<KV_F16, 64, 1>);
     dkv = bf16 ? dkv_launch<KV_BF16, 64>(dkv_parts) : dkv_launch<KV_F16, 64>(dkv_parts);
+  } else if (p.head_dim == 192) {
+    dq = bf16 ? bwd_mfma_dq_kernel<KV_BF16, 192, 1> : bwd_mfma_dq_kernel<KV_F16, 192, 1>;
+    dkv = bf16 ? dkv_launch<KV_BF16, 192>(1) : dkv_launch<KV_F16, 192>(1);
+  } else if (p.head_dim == 256) {
+    dq = bf16 ? bwd_mfma_dq_kernel<KV_BF16, 256, 1> : bwd_mfma_dq_kernel<KV_F16, 256, 1>;
+    dkv = bf16 ? dkv_launch<KV_BF16, 256>(1) : dkv_launch<KV_F16, 256>(1);
   } else {
     dq = dq_cb == 2 ? (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 128, 2> : bwd_mfma_dq_kernel<KV_F16, 128, 2>)
                     : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 128, 1> : bwd_mfma_dq_kernel<KV_F16, 128, 1>);

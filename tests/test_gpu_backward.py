@@ -81,6 +81,25 @@ def test_varlen_backward_long_sequences_on_the_matrix_core_kernels(dtype, hq, hk
         _close(got, ref, REL[dtype], f"{name} {dtype} {hq}/{hkv} d={d} window={window_left}")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d,window_left", [(4, 2, 256, None), (6, 2, 256, 70), (3, 3, 192, None), (4, 1, 192, 97), (2, 1, 256, 0)])
+@pytest.mark.parametrize("lens", [[300, 1, 0, 130, 5, 95, 97, 161], [127], [129, 31], [1]])
+def test_varlen_backward_of_wide_heads_on_the_matrix_core_kernels(dtype, hq, hkv, d, window_left, lens):
+    """Head dims 192 and 256: sequences longer than the dkv kernel's blocks (96 and 128 packed keys), blocks that hold
+    several sequences, lengths one off a block and a tile, windows shorter and longer than a block.  The bar is the
+    file's."""
+    g = torch.Generator().manual_seed(hq * 31 + d + len(lens))
+    t = sum(lens)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
+    q, k, v, go = (torch.randn(t, h, d, generator=g).to(dtype) for h in (hq, hkv, hkv, hq))
+    qd, kd, vd = (x.to(DEV).requires_grad_(True) for x in (q, k, v))
+    ops.areno_varlen_causal_attention(qd, kd, vd, cu.to(DEV), window_left=window_left).backward(go.to(DEV))
+    qf, kf, vf = (x.float().requires_grad_(True) for x in (q, k, v))
+    ar.ref_varlen(qf, kf, vf, cu, ar.window_left_arg(window_left), d**-0.5).backward(go.float())
+    for got, ref, name in ((qd.grad, qf.grad, "dq"), (kd.grad, kf.grad, "dk"), (vd.grad, vf.grad, "dv")):
+        _close(got, ref, REL[dtype], f"{name} {dtype} {hq}/{hkv} d={d} window={window_left}")
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("query_start,window_left", [(0, None), (7, None), (3, 5)])
 def test_dense_backward(dtype, query_start, window_left):
