@@ -1,0 +1,397 @@
+// Causal attention over packed new tokens (the varlen op's forward; areno/accel/csrc/attention.cu:145-242 in the
+// reference) on the matrix cores: 16-bit inputs, head dims 64, 128, 192 and 256.
+//
+// A workgroup of four waves computes one query block of one kv head -- 128 rows, row r being (token r / fold, q head
+// r % fold) as in prefill_mfma.hip -- from its first visible key to its last.  No block is cut, so nothing is left
+// to merge; the blocks of a launch are taken longest first (find_block), and two workgroups share a compute unit
+// (four at head dim 64), so one's waits and softmax fall into the other's products.  Per step of 64 keys (32 at the wide
+// heads) a wave, which owns 32 of the rows:
+//   * passes one barrier and asks for the next step's K and V tiles, which the memory pipe writes into LDS by itself
+//     (two buffers; mfma32_tiles.hpp);
+//   * S^T = K . Q^T on 32 x 32 x 16 products, Q in registers; a lane holds half of the keys of one query row;
+//   * the softmax of prefill_mfma.hip (the lazily raised reference), one lane swap where a row's halves meet;
+//   * O^T += V^T . P^T with the probabilities as they lie.
+// Measured against the kernel of prefill_mfma.hip and its merge, which this replaces for packed K / V (bf16, us):
+// 32 prompts of 33 .. 512 tokens, 28 / 4 heads of 128: 127 -> 66; 2 x 2 048: 166 -> 77; 4 x 4 096, 32 / 8 heads:
+// 725 -> 557 (987 TFLOP/s); 300 tokens alone, 8 / 2 heads: 42 -> 12; 4 x 300 .. 1 000, 16 / 8 heads of 256, window 512:
+// 88 -> 35; 16 x 20 .. 600, 16 heads of 64, fp16: 50 -> 19.  What it does not spend any more: a ~10 us fill and drain
+// per query block with nothing beside it, the partials of cut blocks (up to 67 MB written and read), a third of the
+// loop's vector instructions (staging, half the lane swaps).  Bound at length by the matrix cores and the LDS
+// reads behind them (an operand read per product), at short lengths by a block's chain of steps.
+#include "mfma32_tiles.hpp"
+
+namespace areno {
+namespace {
+
+constexpr int kVmWaves = 4;
+constexpr int kVmThreads = kVmWaves * kWave;
+constexpr int kVmRows = 32 * kVmWaves;  // query rows of a workgroup
+constexpr int kVmMaxSeqs = 1024;
+
+struct VarlenMfmaParams {
+  const void* q;
+  const void* k;
+  const void* v;
+  void* out;
+  float* lse;  // [tokens][q_heads], log2 domain, or nullptr
+  const int32_t* cu_seqlens;
+  int32_t num_seqs;
+  int32_t q_heads;
+  int32_t kv_heads;
+  int32_t group;
+  int32_t head_parts;    // workgroups of a block per kv head: up to 16 of its q heads each
+  int32_t fold;          // row r of a block is (token r / fold, q head r % fold of the part)
+  int32_t fold_magic;    // ceil(2^16 / fold)
+  int32_t block_tokens;  // kVmRows / fold
+  int32_t window_left;
+  float scale_log2e;
+};
+
+// What the i-th workgroup of a head computes: query block `j` of sequence `seq`.  Blocks are taken by their place in
+// their sequence, the last ones first over all sequences: a block's keys grow with its place, and a launch ends soonest
+// when the longest blocks start first.  With nb[s] blocks in sequence s, F(j) = sum over s of max(0, nb[s] - j) blocks
+// lie at place j or behind it; the i-th has the largest j with i < F(j).  Every lane holds the sequences lane,
+// lane + 64, ... and a bisection over j costs a wave-wide sum per step.
+struct BlockAt {
+  int seq, j;
+};
+__device__ __forceinline__ int wave_sum_int(int x) {
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m, kWave);
+  return x;
+}
+__device__ __forceinline__ int wave_max_int(int x) {
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) x = max(x, __shfl_xor(x, m, kWave));
+  return x;
+}
+__device__ __forceinline__ int blocks_of(const int32_t* cu, int s, int num_seqs, int tq) {
+  if (s >= num_seqs) return 0;
+  return (cu[s + 1] - cu[s] + tq - 1) / tq;
+}
+template <typename Blocks>
+__device__ __forceinline__ bool find_block(Blocks blocks, int rounds, int i, BlockAt& at) {
+  const int lane = threadIdx.x & (kWave - 1);
+  int most = 0;
+  for (int r = 0; r < rounds; ++r) most = max(most, blocks(r));
+  most = wave_max_int(most);
+  auto behind = [&](int j) {
+    int n = 0;
+    for (int r = 0; r < rounds; ++r) n += max(0, blocks(r) - j);
+    return uniform(wave_sum_int(n));
+  };
+  if (i >= behind(0)) return false;
+  int lo = 0, hi = most;  // F(lo) > i, F(hi) = 0
+  while (lo + 1 < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (behind(mid) > i) {
+      lo = mid;
+    } else {
+      hi = mid;
+    }
+  }
+  int nth = i - behind(lo + 1);  // among the sequences with more than lo blocks, in order
+  for (int r = 0; r < rounds; ++r) {
+    const uint64_t has = __builtin_amdgcn_ballot_w64(blocks(r) > lo);
+    const int n = __builtin_popcountll(has);
+    if (nth < n) {
+      const bool mine = (has >> lane & 1) != 0 &&
+                        __builtin_popcountll(has & ((uint64_t{1} << lane) - 1)) == nth;
+      at.seq = 64 * r + uniform(__builtin_ctzll(__builtin_amdgcn_ballot_w64(mine)));
+      at.j = lo;
+      return true;
+    }
+    nth -= n;
+  }
+  return false;
+}
+
+extern __shared__ __attribute__((aligned(1024))) char vm_lds[];
+constexpr int kSchedMatrix = 0x8, kSchedLdsRead = 0x100;  // instruction classes of sched_group_barrier
+
+template <int D>
+struct VmShape {
+  static constexpr int kTile = D <= 128 ? 64 : 32;  // keys per step
+  using Tile = LdsTile<D, kTile, kVmWaves>;
+  static constexpr int kBuffer = 2 * Tile::kBytes;  // K, V
+  static constexpr int kLdsBytes = 2 * kBuffer;
+};
+
+template <int KIND, int D>
+__global__ __launch_bounds__(kVmThreads, 2) void varlen_mfma_kernel(VarlenMfmaParams p) {
+  using S = VmShape<D>;
+  using T = typename S::Tile;
+  using M = Mfma32<KIND>;
+  using V8 = typename M::vec8;
+  constexpr int TK = S::kTile;
+  constexpr int KT = TK / 32;   // 32-key score tiles per step
+  constexpr int NKS = D / 16;   // contraction steps of a score tile
+  constexpr int NB = D / 32;    // 32-element blocks of the head
+  constexpr int NF = T::kFetches;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = uniform(tid >> 6);
+  const int l32 = lane & 31, h = lane >> 5;
+  const int vheads = p.kv_heads * p.head_parts;
+  const int vhead = static_cast<int>(blockIdx.x % static_cast<unsigned>(vheads));
+  const int kvh = p.head_parts > 1 ? vhead / p.head_parts : vhead;
+  const int head0 = kvh * p.group + 16 * (vhead - kvh * p.head_parts);
+  const int group_here = min(16, (kvh + 1) * p.group - head0);
+  const int tq = p.block_tokens;
+
+  BlockAt at;
+  {
+    const int i = static_cast<int>(blockIdx.x / static_cast<unsigned>(vheads));
+    bool found;
+    if (p.num_seqs <= kWave) {
+      const int nb = blocks_of(p.cu_seqlens, lane, p.num_seqs, tq);
+      found = find_block([&](int) { return nb; }, 1, i, at);
+    } else {
+      found = find_block([&](int r) { return blocks_of(p.cu_seqlens, 64 * r + lane, p.num_seqs, tq); },
+                         (p.num_seqs + kWave - 1) / kWave, i, at);
+    }
+    if (!found) return;  // (the grid covers the most blocks the token count allows; the same for the whole workgroup)
+  }
+  const int seq = uniform(at.seq);
+  const int q_begin = uniform(p.cu_seqlens[seq]);
+  const int n_new = uniform(p.cu_seqlens[seq + 1]) - q_begin;
+  const int tok0 = uniform(at.j) * tq;
+  const int tok_cnt = min(tq, n_new - tok0);
+
+  // ---- this lane's query row -------------------------------------------------------------------------------------
+  auto token_of_row = [&](int r) { return (r * p.fold_magic) >> 16; };
+  const int r = 32 * wave + l32;
+  const int t_row = token_of_row(r);
+  const int hh = r - t_row * p.fold;
+  const bool live = t_row < tok_cnt && hh < group_here;
+  const int q_pos = live ? tok0 + t_row : -1;
+  const int64_t row_elem = (static_cast<int64_t>(q_begin + tok0 + t_row) * p.q_heads + head0 + hh) * D;
+  V8 qop[NKS];
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks) {
+    uint4_t w = {0u, 0u, 0u, 0u};
+    if (live) w = load16(p.q, (row_elem + 16 * ks + 8 * h) * 2);
+    qop[ks] = __builtin_bit_cast(V8, w);
+  }
+  const bool wave_live = 32 * wave < tok_cnt * p.fold;
+  const int wave_qmin = tok0 + token_of_row(32 * wave);
+  const int wave_qmax = tok0 + min(tok_cnt - 1, token_of_row(32 * wave + 31));
+
+  // ---- the stream of key tiles -----------------------------------------------------------------------------------
+  const int key_hi = tok0 + tok_cnt - 1;  // the last key any row of the block sees
+  const int key_lo = p.window_left >= 0 ? max(0, tok0 - p.window_left) : 0;
+  const int ta = key_lo / TK, tb = key_hi / TK;
+  const int64_t stride = static_cast<int64_t>(p.kv_heads) * D * 2;
+  const int64_t head_base = (static_cast<int64_t>(q_begin) * p.kv_heads + kvh) * (D * 2);
+  const char* const k_base = static_cast<const char*>(p.k) + head_base;
+  const char* const v_base = static_cast<const char*>(p.v) + head_base;
+  const uint32_t lds0 = lds_address(vm_lds);
+  int fetch_row[NF];
+  uint32_t fetch_chunk[NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    const int slot = (wave * NF + f) * 64 + lane;
+    fetch_row[f] = slot / T::kChunksPerRow;
+    fetch_chunk[f] = static_cast<uint32_t>((slot % T::kChunksPerRow) ^ T::twist(fetch_row[f])) * 16u;
+  }
+  auto fetch = [&](int t, int buf) {
+    const int rows = key_hi + 1 - t * TK;  // rows of the tile that exist; the ones behind repeat the last
+    const char* kb = k_base + static_cast<int64_t>(t) * TK * stride;
+    const char* vb = v_base + static_cast<int64_t>(t) * TK * stride;
+    const uint32_t dst = lds0 + static_cast<uint32_t>(buf * S::kBuffer + wave * (NF * 1024));
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const uint32_t off = static_cast<uint32_t>(min(fetch_row[f], rows - 1)) * static_cast<uint32_t>(stride) + fetch_chunk[f];
+      fetch_to_lds(kb, off, dst + f * 1024);
+      fetch_to_lds(vb, off, dst + T::kBytes + f * 1024);
+    }
+  };
+
+  float16_t acc[NB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) acc[nb] = zero16();
+  float m_run = kNegInf, l_lane = 0.0f;
+
+  uint32_t at_rows = T::rows_base(l32, h), at_columns = T::columns_base(lane);
+  auto step = [&](int t, int buf) {
+    // (wide heads: the 32 addresses of a step are worked out where they are used, instead of being kept in registers
+    // that the sums need)
+    if constexpr (D > 128) asm volatile("" : "+v"(at_rows), "+v"(at_columns));
+    fetched_barrier();  // tile t (asked for a step ago) is there, and every wave has left tile t - 1
+    if (t < tb) fetch(t + 1, buf ^ 1);
+    const int k0 = t * TK;
+    if (!wave_live || k0 > wave_qmax) return;
+    if (p.window_left >= 0 && k0 + TK - 1 < wave_qmin - p.window_left) return;
+    const char* kt_lds = vm_lds + buf * S::kBuffer;
+    char* vt_lds = vm_lds + buf * S::kBuffer + T::kBytes;
+    float16_t s[KT];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) s[kt] = zero16();
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) s[kt] = M::mfma(tile_rows<KIND, T>(kt_lds, at_rows, 32 * kt, ks), qop[ks], s[kt]);
+    }
+    // four operand reads ahead of the products (two where registers are short): left alone the compiler waits for
+    // every pair of reads right behind it (4 x 4 096 tokens, 32 / 8 heads of 128: 577 -> 557 us)
+    constexpr int kAhead = D <= 128 ? 4 : 2;
+    __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, kAhead, 0);
+#pragma unroll
+    for (int x = 0; x < NKS * KT - kAhead; ++x) {
+      __builtin_amdgcn_sched_group_barrier(kSchedMatrix, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(kSchedMatrix, kAhead, 0);
+    if (k0 + TK - 1 > wave_qmin || (p.window_left >= 0 && k0 < wave_qmax - p.window_left)) {
+      const int hi = q_pos - k0 - 4 * h;
+      const int lo = p.window_left >= 0 ? hi - p.window_left : -0x40000000;
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int key = 32 * kt + 8 * (i >> 2) + (i & 3);
+          s[kt][i] = key <= hi && key >= lo ? s[kt][i] : kNegInf;
+        }
+      }
+    }
+    // online softmax as in prefill_mfma.hip: the reference value is raised only when a tile exceeds it by 2^8
+    constexpr float kLazy = 8.0f;
+    float mt = max3_f32(s[0][0], s[0][1], s[0][2]);
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+#pragma unroll
+      for (int i = kt == 0 ? 3 : 0; i < 16; i += 2) mt = max3_f32(mt, s[kt][i], s[kt][i + 1 < 16 ? i + 1 : i]);
+    }
+    if (__builtin_amdgcn_ballot_w64(mt * p.scale_log2e > m_run + kLazy) != 0) {
+      uint32_t a = __builtin_bit_cast(uint32_t, mt), b = a;
+      swap_rows32(a, b);
+      mt = max_f32(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+      const float m_new = max_f32(m_run, mt * p.scale_log2e);
+      const float m_ref = m_new == kNegInf ? 0.0f : m_new;
+      const float alpha = settled(fast_exp2(m_run - m_ref));
+      m_run = m_new;
+      scale_in_place(l_lane, alpha);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          float x = acc[nb][i];
+          scale_in_place(x, alpha);
+          acc[nb][i] = x;
+        }
+      }
+    }
+    const float m_safe = m_run == kNegInf ? 0.0f : m_run;
+    V8 pop[2 * KT];
+#pragma unroll
+    for (int b = 0; b < 2 * KT; ++b) {
+      uint32_t w[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = 8 * (b & 1) + 2 * j;
+        w[j] = pack_pair<KIND>(fast_exp2(__builtin_fmaf(s[b >> 1][i], p.scale_log2e, -m_safe)),
+                               fast_exp2(__builtin_fmaf(s[b >> 1][i + 1], p.scale_log2e, -m_safe)));
+        l_lane = M::add_pair(w[j], l_lane);  // sums the probabilities as rounded for the product
+      }
+      pop[b] = __builtin_bit_cast(V8, uint4_t{w[0], w[1], w[2], w[3]});
+    }
+#pragma unroll
+    for (int b = 0; b < 2 * KT; ++b) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) acc[nb] = M::mfma(tile_columns<KIND, T>(vt_lds, at_columns, 16 * b, nb), pop[b], acc[nb]);
+    }
+  };
+
+  fetch(ta, 0);
+  // (the query rows are waited for here: left to their first use inside the loop, that wait would cover every step's
+  // fetches as well)
+#pragma unroll
+  for (int ks = 0; ks < NKS; ++ks) {
+    uint4_t w = __builtin_bit_cast(uint4_t, qop[ks]);
+    asm volatile("" : "+v"(w));
+    qop[ks] = __builtin_bit_cast(V8, w);
+  }
+  for (int t = ta; t <= tb; t += 2) {
+    step(t, 0);
+    if (t + 1 <= tb) step(t + 1, 1);
+  }
+
+  if (!live) return;
+  uint32_t a = __builtin_bit_cast(uint32_t, l_lane), b = a;
+  swap_rows32(a, b);
+  const float l_tot = __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+  const float inv = 1.0f / l_tot;
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const uint2_t w = {pack_pair<KIND>(acc[nb][4 * c] * inv, acc[nb][4 * c + 1] * inv),
+                         pack_pair<KIND>(acc[nb][4 * c + 2] * inv, acc[nb][4 * c + 3] * inv)};
+      *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + (row_elem + 32 * nb + 8 * c + 4 * h) * 2) = w;
+    }
+  }
+  if (p.lse != nullptr && h == 0)
+    p.lse[static_cast<int64_t>(q_begin + tok0 + t_row) * p.q_heads + head0 + hh] = m_run + __builtin_log2f(l_tot);
+}
+
+typedef void (*vm_fn)(VarlenMfmaParams);
+struct VmLaunch {
+  vm_fn fn;
+  int lds_bytes;
+};
+template <int KIND>
+VmLaunch vm_lookup(int head_dim) {
+  switch (head_dim) {
+    case 64: return {varlen_mfma_kernel<KIND, 64>, VmShape<64>::kLdsBytes};
+    case 128: return {varlen_mfma_kernel<KIND, 128>, VmShape<128>::kLdsBytes};
+    case 192: return {varlen_mfma_kernel<KIND, 192>, VmShape<192>::kLdsBytes};
+    case 256: return {varlen_mfma_kernel<KIND, 256>, VmShape<256>::kLdsBytes};
+    default: return {nullptr, 0};
+  }
+}
+
+}  // namespace
+
+// ARENO_ERR_UNSUPPORTED: not a launch this kernel serves
+int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, float* lse, int32_t dtype, int64_t tokens,
+                       int32_t q_heads, int32_t kv_heads, int32_t head_dim, const int32_t* cu_seqlens, int32_t num_seqs,
+                       int32_t window_left, float softmax_scale, void* stream) {
+  const char* op = "areno_hip_varlen_attention";
+  if (dtype != ARENO_DT_BF16 && dtype != ARENO_DT_F16) return ARENO_ERR_UNSUPPORTED;
+  if (!(softmax_scale > 0.0f) || num_seqs > kVmMaxSeqs || tokens > 0x3fffffff) return ARENO_ERR_UNSUPPORTED;
+  const VmLaunch l = dtype == ARENO_DT_BF16 ? vm_lookup<KV_BF16>(head_dim) : vm_lookup<KV_F16>(head_dim);
+  if (l.fn == nullptr) return ARENO_ERR_UNSUPPORTED;
+  for (const void* ptr : {q, k, v, static_cast<const void*>(out)}) {
+    if (reinterpret_cast<uintptr_t>(ptr) % 16 != 0) return ARENO_ERR_UNSUPPORTED;
+  }
+  const int group = q_heads / kv_heads;
+  const int head_parts = (group + 15) / 16;
+  const int64_t vheads = static_cast<int64_t>(kv_heads) * head_parts;
+  // offsets inside a key tile are 32 bits wide
+  if (static_cast<int64_t>(kv_heads) * head_dim * 2 * 64 > 0x7fffffffLL) return ARENO_ERR_UNSUPPORTED;
+  VarlenMfmaParams p;
+  p.q = q;
+  p.k = k;
+  p.v = v;
+  p.out = out;
+  p.lse = lse;
+  p.cu_seqlens = cu_seqlens;
+  p.num_seqs = num_seqs;
+  p.q_heads = q_heads;
+  p.kv_heads = kv_heads;
+  p.group = group;
+  p.head_parts = head_parts;
+  p.fold = head_parts > 1 ? 16 : group;
+  p.fold_magic = (65536 + p.fold - 1) / p.fold;
+  p.block_tokens = kVmRows / p.fold;
+  p.window_left = window_left;
+  p.scale_log2e = softmax_scale * kLog2e;
+  const int64_t blocks = (tokens / p.block_tokens + num_seqs) * vheads;
+  if (blocks > 0x7fffffffLL) return ARENO_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(l.fn, dim3(static_cast<unsigned>(blocks)), dim3(kVmThreads), l.lds_bytes,
+                     static_cast<hipStream_t>(stream), p);
+  return check_launch(op);
+}
+
+}  // namespace areno

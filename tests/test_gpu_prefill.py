@@ -322,3 +322,21 @@ def test_varlen_error_behaviour():
         ops.areno_varlen_causal_attention(q, k[:-1], v, cu)
     with pytest.raises(ValueError, match="divisible by kv heads"):
         ops.areno_varlen_causal_attention(q[:, :3], k, v, cu)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d,window_left", [
+    (28, 4, 128, None), (7, 1, 128, 63), (4, 4, 64, None), (3, 1, 64, 64), (20, 1, 128, None), (4, 2, 256, None),
+    (6, 6, 192, 31), (8, 1, 256, 33),
+])  # fmt: skip
+@pytest.mark.parametrize("lens", [
+    [1], [18, 19], [127, 128, 129], [63, 0, 64, 65, 1, 300], [3] * 70, [0] * 64 + [40, 0, 200], [5, 1, 0] * 50,
+])  # fmt: skip
+def test_varlen_query_blocks_and_key_tiles(dtype, hq, hkv, d, window_left, lens):
+    """Packed attention at the edges of its query blocks (128 rows: 128 tokens of one head, 18 of seven, 8 of sixteen),
+    of its key tiles (64 keys, 32 at the wide heads) and of its block list (up to 64 sequences in one lane each, more
+    in rounds; empty ones between).  Tolerance: that of the file's other 16-bit outputs against the fp32 oracle."""
+    q, k, v, cu = _packed(lens, hq, hkv, d, dtype, seed=d + len(lens))
+    out = ops.areno_varlen_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV), window_left=window_left)
+    want = ar.ref_varlen(q, k, v, cu, ar.window_left_arg(window_left), d**-0.5)
+    assert_close(out, want, *tolerances("bf16"), what=f"varlen {hq}/{hkv} d={d} window={window_left} lens={lens[:6]}")
