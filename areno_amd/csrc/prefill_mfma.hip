@@ -82,6 +82,16 @@ constexpr int kMaxPrefillSeqs = 1024;
 constexpr int kPrefillTargetWgs = 2048 / kPrefillWaves;  // eight resident waves on each of the 256 CUs
 constexpr int kMaxPrefillUnits = 512;   // per kv head
 
+// What a unit leaves for the merge: its last item, when that starts in the unit and is not finished there.
+struct CutItem {
+  int32_t first_slot;  // of its partials, the others are at slot 2u of the units behind; -1: nothing to merge
+  int32_t total;       // tile steps of the launch
+  int32_t step_end;    // the item's steps end in front of this one
+  int32_t token0;      // its first query token's row of q / out
+  int32_t tokens;
+  int32_t unused[3];
+};
+
 struct PrefillParams {
   const void* q;
   void* out;
@@ -94,6 +104,7 @@ struct PrefillParams {
   const int32_t* context_lens;
   float* part_ml;   // [2 * units][kv_heads * head_parts][rows_per_wg][2]
   float* part_acc;  // [2 * units][kv_heads * head_parts][rows_per_wg][head_dim]
+  CutItem* cuts;    // [units]
   int32_t num_seqs;
   int32_t q_heads;
   int32_t kv_heads;
@@ -118,24 +129,24 @@ struct PrefillParams {
   float scale_log2e;
 };
 
-// Exclusive prefix sum of tile steps per sequence into s_cum[0 .. num_seqs] (all threads take part).
+// Exclusive prefix sum of tile steps per sequence into s_cum[0 .. num_seqs] (all threads take part).  A launch seldom
+// has more sequences than the workgroup has threads, and the loops stay rolled: this runs once per workgroup, on code
+// that has to be fetched first (4 sequences of up to 64 new and 4 k cached tokens, 7 q heads per kv head: the kernel
+// 26.7 -> 25.6 us against a copy of the closed forms per sequence of a thread).
 __device__ __forceinline__ void prefix_tile_steps(const PrefillParams& p, int tq, int* s_cum, int* s_wave_tot) {
-  constexpr int SPT = kMaxPrefillSeqs / kPrefillThreads;
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = tid >> 6;
-  int steps[SPT];
+  const int per_thread = (p.num_seqs + kPrefillThreads - 1) / kPrefillThreads;
+  const int first = per_thread * tid, last = min(first + per_thread, p.num_seqs);
   int local = 0;
-#pragma unroll
-  for (int i = 0; i < SPT; ++i) {
-    const int s = SPT * tid + i;
-    steps[i] = 0;
-    if (s < p.num_seqs) {
-      const int n_new = p.cu_seqlens_q[s + 1] - p.cu_seqlens_q[s];
-      const int ctx = p.context_lens != nullptr ? p.context_lens[s] : 0;
-      steps[i] = sequence_steps(n_new, ctx, tq, p.window_left);
-    }
-    local += steps[i];
+#pragma unroll 1
+  for (int s = first; s < last; ++s) {
+    const int n_new = p.cu_seqlens_q[s + 1] - p.cu_seqlens_q[s];
+    const int ctx = p.context_lens != nullptr ? p.context_lens[s] : 0;
+    const int steps = sequence_steps(n_new, ctx, tq, p.window_left);
+    s_cum[s] = steps;
+    local += steps;
   }
   int incl = local;
 #pragma unroll
@@ -147,14 +158,13 @@ __device__ __forceinline__ void prefix_tile_steps(const PrefillParams& p, int tq
   __syncthreads();
   int excl = incl - local;
   for (int w2 = 0; w2 < wave; ++w2) excl += s_wave_tot[w2];
-#pragma unroll
-  for (int i = 0; i < SPT; ++i) {
-    const int s = SPT * tid + i;
-    if (s <= p.num_seqs) s_cum[s] = excl;
-    excl += steps[i];
+#pragma unroll 1
+  for (int s = first; s < last; ++s) {
+    const int steps = s_cum[s];
+    s_cum[s] = excl;
+    excl += steps;
   }
-  // the entry behind the last thread's sequences has no owner of its own: it is the total when the list is full
-  if (tid == kPrefillThreads - 1 && SPT * (tid + 1) <= p.num_seqs) s_cum[SPT * (tid + 1)] = excl;
+  if (last == p.num_seqs && (first < last || tid == 0)) s_cum[p.num_seqs] = excl;
   __syncthreads();
 }
 
@@ -196,7 +206,9 @@ __device__ __forceinline__ StepPos locate_step(const PrefillParams& p, const int
 }
 
 __device__ __forceinline__ int unit_start_step(int total, int u, int units) {
-  return static_cast<int>(static_cast<long long>(total) * u / units);
+  // floor(total * u / units) without a 64-bit division (some hundred instructions): units <= 512, u <= units
+  const uint32_t n = static_cast<uint32_t>(total), d = static_cast<uint32_t>(units), q = n / d;
+  return static_cast<int>(q * static_cast<uint32_t>(u) + (n - q * d) * static_cast<uint32_t>(u) / d);
 }
 
 // 16 codes of an 8-bit cache row (one 16-byte chunk) -> 16 fp16 values times the row's scale, as two 16-byte groups.
@@ -259,6 +271,7 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
   __shared__ __attribute__((aligned(16))) char s_v[2][TK * RSV];
   __shared__ int s_cum[kMaxPrefillSeqs + 1];
   __shared__ int s_wave_tot[kPrefillWaves];
+  __shared__ StepPos s_first;
   // score parts of a split head: [wave][tg][j][lane]
   __shared__ float s_part[DS > 1 ? kPrefillWaves : 1][2][4][DS > 1 ? kWave : 1];
 
@@ -283,7 +296,10 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
   const int total = s_cum[p.num_seqs];
   const int x_begin = unit_start_step(total, unit, p.units);
   const int x_end = unit_start_step(total, unit + 1, p.units);
-  if (x_begin >= x_end) return;  // same for the whole workgroup
+  if (x_begin >= x_end) {  // same for the whole workgroup
+    if (vhead == 0 && tid == 0) p.cuts[unit].first_slot = -1;
+    return;
+  }
 
   const bool q_is_operand_type = (OPK == KV_BF16 && p.q_dtype == ARENO_DT_BF16) ||
                                  (OPK == KV_F16 && p.q_dtype == ARENO_DT_F16);
@@ -313,7 +329,23 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
     }
   };
 
-  StepPos pos = locate_step(p, s_cum, tq, x_begin);
+  // One walk finds two places: the last wave looks up the unit's last step, for the merge, and the others its first,
+  // which they hand to the last wave through LDS.
+  const bool looks_at_end = wave == kPrefillWaves - 1;
+  StepPos pos = locate_step(p, s_cum, tq, looks_at_end ? x_end - 1 : x_begin);
+  if (looks_at_end && vhead == 0 && lane == 0) {
+    const BlockTiles item = block_tiles(pos.n_new, pos.ctx, pos.j, tq, p.window_left);
+    CutItem cut;
+    cut.step_end = pos.item_x0 + item.count();
+    cut.first_slot = cut.step_end > x_end && pos.item_x0 >= x_begin ? 2 * unit + (pos.item_x0 > x_begin ? 1 : 0) : -1;
+    cut.total = total;
+    cut.token0 = pos.q_begin + item.tok0;
+    cut.tokens = item.cnt;
+    p.cuts[unit] = cut;
+  }
+  if (tid == 0) s_first = pos;
+  __syncthreads();
+  if (looks_at_end) pos = s_first;
 
   // What the staging steps ask block ids for: the item whose tiles are being fetched.  It is switched to the next
   // item before the current item's output is stored (see the end of the item loop).
@@ -855,132 +887,116 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
   }
 }
 
-// Merge of the items cut by unit borders.  Workgroup (u, kv head) looks at the last item of unit u: if that item
-// starts in unit u and runs on into later units, it combines the partials of all units the item touches (slot
-// 2u' for a unit where the item comes first, 2u' + 1 where it comes last after other items), normalises and
+// Merge of the items cut by unit borders.  Workgroup (u, kv head) takes the last item of unit u, if that item starts
+// in unit u and runs on into later units: it combines the partials of all units the item touches, normalises and
 // writes the item's rows.
-constexpr int kMergeInFlight = 8;  // 16-byte chunks of each partial a thread of prefill_merge_kernel takes
+//
+// What the item is, unit u has left in `cuts`: finding it again from the sequences' lengths, as every workgroup did,
+// is a walk through more code than there is work (28 / 4 heads of 128: 42 -> 22 us for the follow-ups of
+// 4 sequences, up to 64 tokens on 4 k cached ones, about 11 pieces per item; 32 / 8 heads, 16 chunks of up to 512 tokens on
+// 16 k cached ones: 30 -> 15 us).  Bound by latency and by how many compute
+// units pull: a workgroup is a chain of round trips to partials that other XCDs wrote.  So an item's rows are spread
+// over many small workgroups (blockIdx.z; each thread has kMergeChunks 16-byte chunks of every partial), and
+// kMergeBatch partials are asked for before the first of them is used.
+constexpr int kMergeThreads = 256;
+constexpr int kMergeChunks = 2;
+constexpr int kMergeBatch = 4;
 
-__global__ __launch_bounds__(kPrefillThreads) void prefill_merge_kernel(PrefillParams p) {
-  __shared__ int s_cum[kMaxPrefillSeqs + 1];
-  __shared__ int s_wave_tot[kPrefillWaves];
+__global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(PrefillParams p) {
   const int tid = threadIdx.x;
   const int unit = blockIdx.x;
+  const CutItem cut = p.cuts[unit];
+  if (cut.first_slot < 0) return;
   const int vhead = blockIdx.y;
   const int kvh = p.head_parts > 1 ? vhead / p.head_parts : vhead;
   const int head0 = kvh * p.group + 16 * (vhead - kvh * p.head_parts);
   const int group_here = min(16, (kvh + 1) * p.group - head0);
   const int vheads = p.kv_heads * p.head_parts;
   const int kRowsPerWg = p.rows_per_wg;
-  const int tq = p.block_tokens;
   const int d = p.head_dim;
-  prefix_tile_steps(p, tq, s_cum, s_wave_tot);
-  const int total = s_cum[p.num_seqs];
-  const int x_begin = unit_start_step(total, unit, p.units);
-  const int x_end = unit_start_step(total, unit + 1, p.units);
-  if (x_begin >= x_end) return;
-  const StepPos pos = locate_step(p, s_cum, tq, x_end - 1);
-  const BlockTiles item = block_tiles(pos.n_new, pos.ctx, pos.j, tq, p.window_left);
-  const int item_x1 = pos.item_x0 + item.count();
-  if (item_x1 <= x_end || pos.item_x0 < x_begin) return;  // not cut here, or merged by the unit where it starts
-  // last unit that owns a step of the item: the largest u with unit_start_step(u) <= item_x1 - 1
-  int u_hi = static_cast<int>((static_cast<long long>(item_x1) * p.units - 1) / total);
-  if (u_hi > p.units - 1) u_hi = p.units - 1;
-  while (unit_start_step(total, u_hi, p.units) > item_x1 - 1) --u_hi;
-  while (u_hi + 1 < p.units && unit_start_step(total, u_hi + 1, p.units) <= item_x1 - 1) ++u_hi;
 
-  const int q_begin = pos.q_begin;
   // The partials of a slot are one contiguous block of rows x head_dim floats, walked as a flat array of 16-byte
-  // chunks, consecutive threads on consecutive chunks (a thread per row part left three quarters of every fetched
-  // line to a later instruction).  The kernel is a chain of dependent round trips on one workgroup per CU, so the
-  // chain is kept short: a workgroup takes kInFlight chunks per thread of every partial (blockIdx.z picks which; the
-  // launcher sizes the grid), the partials are combined in one pass with a running maximum, and the fetches of the
-  // next partial are issued before the current one is used.  (One workgroup per cut item walking all chunks in two
-  // passes took 32 us for the ~500 partials of a launch, 2.1 TB/s.)  The (m, l) pair of a chunk's row is the same
-  // for the lanes of the row and comes out of the cache.
+  // chunks, consecutive threads on consecutive chunks.  Rows behind the item's last token are not read.
   const int chunks_per_row = d >> 2;
-  const int total_chunks = kRowsPerWg * chunks_per_row;
+  const int total_chunks = min(kRowsPerWg, cut.tokens * p.fold) * chunks_per_row;
   const float inv_chunks_per_row = 1.0f / static_cast<float>(chunks_per_row);
-  const int base = blockIdx.z * kMergeInFlight * kPrefillThreads + tid;
+  const int base = blockIdx.z * kMergeChunks * kMergeThreads + tid;
   if (base >= total_chunks) return;
-  {
-    constexpr int kInFlight = kMergeInFlight;
-    int row[kInFlight];
-    bool live[kInFlight];
-    float m[kInFlight], lsum[kInFlight];
-    float4_t o[kInFlight];
+  int chunk[kMergeChunks], row[kMergeChunks];
+  float m[kMergeChunks], lsum[kMergeChunks];
+  float4_t o[kMergeChunks];
 #pragma unroll
-    for (int k = 0; k < kInFlight; ++k) {
-      const int idx = min(base + k * kPrefillThreads, total_chunks - 1);
-      // idx / chunks_per_row: the product with the rounded reciprocal is exact here (idx + 0.5 is at least half a
-      // chunk away from a multiple of chunks_per_row, and idx < 2^16)
-      row[k] = static_cast<int>((static_cast<float>(idx) + 0.5f) * inv_chunks_per_row);
-      const int t = (row[k] * p.fold_magic) >> 16;
-      const int hh = row[k] - t * p.fold;
-      live[k] = base + k * kPrefillThreads < total_chunks && t < item.cnt && hh < group_here;
-      m[k] = kNegInf;
-      lsum[k] = 0.0f;
-      o[k] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    struct Fetched {
-      float4_t a[kInFlight];
-      float2_t v[kInFlight];
-    };
-    auto next_unit = [&](int u) {  // the next unit from u on that owns steps, or u_hi + 1
-      while (u <= u_hi && unit_start_step(total, u, p.units) == unit_start_step(total, u + 1, p.units)) ++u;
-      return u;
-    };
-    auto fetch = [&](Fetched& f, int u) {
-      const int slot = 2 * u + ((u == unit && pos.item_x0 > x_begin) ? 1 : 0);
-      const int64_t slot_row0 = (static_cast<int64_t>(slot) * vheads + vhead) * kRowsPerWg;
-      const float* ml = p.part_ml + slot_row0 * 2;
-      const float4_t* acc = reinterpret_cast<const float4_t*>(p.part_acc + slot_row0 * d);
+  for (int k = 0; k < kMergeChunks; ++k) {
+    chunk[k] = min(base + k * kMergeThreads, total_chunks - 1);
+    // chunk / chunks_per_row: the product with the rounded reciprocal is exact here (chunk + 0.5 is at least half a
+    // chunk away from a multiple of chunks_per_row, and chunk < 2^16)
+    row[k] = static_cast<int>((static_cast<float>(chunk[k]) + 0.5f) * inv_chunks_per_row);
+    m[k] = kNegInf;
+    lsum[k] = 0.0f;
+    o[k] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  int u = unit, slot = cut.first_slot;
+  bool more = true;
+  while (more) {
+    // the next partials: one of every unit that owns steps of the item (units without steps wrote none)
+    int count = 0;
+    float4_t a[kMergeBatch][kMergeChunks];
+    float2_t v[kMergeBatch][kMergeChunks];
 #pragma unroll
-      for (int k = 0; k < kInFlight; ++k) {
-        f.a[k] = acc[min(base + k * kPrefillThreads, total_chunks - 1)];
-        f.v[k] = *reinterpret_cast<const float2_t*>(ml + 2 * row[k]);
+    for (int i = 0; i < kMergeBatch; ++i) {
+      if (more) {
+        const int64_t slot_row0 = (static_cast<int64_t>(slot) * vheads + vhead) * kRowsPerWg;
+        const float* ml = p.part_ml + slot_row0 * 2;
+        const float4_t* acc = reinterpret_cast<const float4_t*>(p.part_acc + slot_row0 * d);
+#pragma unroll
+        for (int k = 0; k < kMergeChunks; ++k) {
+          a[i][k] = acc[chunk[k]];
+          v[i][k] = *reinterpret_cast<const float2_t*>(ml + 2 * row[k]);
+        }
+        count = i + 1;
+        int at = unit_start_step(cut.total, u + 1, p.units);
+        for (++u; u < p.units; ++u) {
+          const int next = unit_start_step(cut.total, u + 1, p.units);
+          if (next > at) break;
+          at = next;
+        }
+        slot = 2 * u;
+        more = u < p.units && at < cut.step_end;
       }
-    };
-    Fetched cur, nxt;
-    int u = next_unit(unit);  // (unit itself owns steps: checked above)
-    fetch(cur, u);
-    for (;;) {
-      const int u2 = next_unit(u + 1);
-      if (u2 <= u_hi) fetch(nxt, u2);
+    }
 #pragma unroll
-      for (int k = 0; k < kInFlight; ++k) {
-        if (cur.v[k][1] == 0.0f) continue;  // a partial without visible keys contributes nothing
-        const float m_new = fmaxf(m[k], cur.v[k][0]);
+    for (int i = 0; i < kMergeBatch; ++i) {
+      if (i >= count) continue;
+#pragma unroll
+      for (int k = 0; k < kMergeChunks; ++k) {
+        if (v[i][k][1] == 0.0f) continue;  // a partial without visible keys contributes nothing
+        const float m_new = fmaxf(m[k], v[i][k][0]);
         const float keep = fast_exp2(m[k] - m_new);  // 0 for the first partial (m = -inf)
-        const float w = fast_exp2(cur.v[k][0] - m_new);
-        lsum[k] = lsum[k] * keep + w * cur.v[k][1];
+        const float w = fast_exp2(v[i][k][0] - m_new);
+        lsum[k] = lsum[k] * keep + w * v[i][k][1];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) o[k][j] = o[k][j] * keep + w * cur.a[k][j];
+        for (int j = 0; j < 4; ++j) o[k][j] = o[k][j] * keep + w * a[i][k][j];
         m[k] = m_new;
       }
-      if (u2 > u_hi) break;
-      cur = nxt;
-      u = u2;
     }
+  }
 #pragma unroll
-    for (int k = 0; k < kInFlight; ++k) {
-      if (!live[k]) continue;
-      const int idx = base + k * kPrefillThreads;
-      const int t = (row[k] * p.fold_magic) >> 16;
-      const int hh = row[k] - t * p.fold;
-      const float inv = 1.0f / lsum[k];
-      const int64_t out_elem = (static_cast<int64_t>(q_begin + item.tok0 + t) * p.q_heads + head0 + hh) * d +
-                               4 * (idx - row[k] * chunks_per_row);
-      uint32_t lo, hi;
-      if (p.q_dtype == ARENO_DT_BF16) {
-        lo = float_to_bf16_bits(o[k][0] * inv) | (float_to_bf16_bits(o[k][1] * inv) << 16);
-        hi = float_to_bf16_bits(o[k][2] * inv) | (float_to_bf16_bits(o[k][3] * inv) << 16);
-      } else {
-        lo = float_to_f16_bits(o[k][0] * inv) | (float_to_f16_bits(o[k][1] * inv) << 16);
-        hi = float_to_f16_bits(o[k][2] * inv) | (float_to_f16_bits(o[k][3] * inv) << 16);
-      }
-      *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + out_elem * 2) = uint2_t{lo, hi};
+  for (int k = 0; k < kMergeChunks; ++k) {
+    const int t = (row[k] * p.fold_magic) >> 16;
+    const int hh = row[k] - t * p.fold;
+    if (base + k * kMergeThreads >= total_chunks || t >= cut.tokens || hh >= group_here) continue;
+    const float inv = 1.0f / lsum[k];
+    const int64_t out_elem = (static_cast<int64_t>(cut.token0 + t) * p.q_heads + head0 + hh) * d +
+                             4 * (chunk[k] - row[k] * chunks_per_row);
+    uint32_t lo, hi;
+    if (p.q_dtype == ARENO_DT_BF16) {
+      lo = float_to_bf16_bits(o[k][0] * inv) | (float_to_bf16_bits(o[k][1] * inv) << 16);
+      hi = float_to_bf16_bits(o[k][2] * inv) | (float_to_bf16_bits(o[k][3] * inv) << 16);
+    } else {
+      lo = float_to_f16_bits(o[k][0] * inv) | (float_to_f16_bits(o[k][1] * inv) << 16);
+      hi = float_to_f16_bits(o[k][2] * inv) | (float_to_f16_bits(o[k][3] * inv) << 16);
     }
+    *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + out_elem * 2) = uint2_t{lo, hi};
   }
 }
 
@@ -1062,7 +1078,7 @@ size_t prefill_ml_bytes(int units, int kv_heads) {
 size_t prefill_mfma_workspace_bytes(int32_t kv_heads, int32_t head_dim) {
   if (kv_heads <= 0 || head_dim <= 0) return 0;
   const int units = prefill_units(kv_heads);
-  return prefill_ml_bytes(units, kv_heads) +
+  return kMaxPrefillUnits * sizeof(CutItem) + prefill_ml_bytes(units, kv_heads) +
          static_cast<size_t>(2) * units * kv_heads * prefill_rows_per_wg(head_dim) * head_dim * sizeof(float);
 }
 
@@ -1153,13 +1169,15 @@ int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out
   p.units = prefill_units(vheads);
   p.rows_per_wg = rows_per_wg;
   p.scale_log2e = softmax_scale * kLog2e;
-  p.part_ml = static_cast<float*>(workspace);
-  p.part_acc = reinterpret_cast<float*>(static_cast<char*>(workspace) + prefill_ml_bytes(p.units, vheads));
+  p.cuts = static_cast<CutItem*>(workspace);
+  char* const partials = static_cast<char*>(workspace) + kMaxPrefillUnits * sizeof(CutItem);
+  p.part_ml = reinterpret_cast<float*>(partials);
+  p.part_acc = reinterpret_cast<float*>(partials + prefill_ml_bytes(p.units, vheads));
   const dim3 grid(p.units, vheads);
   hipLaunchKernelGGL(fn, grid, dim3(kPrefillThreads), 0, static_cast<hipStream_t>(stream), p);
   if (int rc = check_launch(op)) return rc;
-  const int merge_parts = (rows_per_wg * (cache->head_dim / 4) + kMergeInFlight * kPrefillThreads - 1) / (kMergeInFlight * kPrefillThreads);
-  hipLaunchKernelGGL(prefill_merge_kernel, dim3(p.units, vheads, merge_parts), dim3(kPrefillThreads), 0,
+  const int merge_parts = (rows_per_wg * (cache->head_dim / 4) + kMergeChunks * kMergeThreads - 1) / (kMergeChunks * kMergeThreads);
+  hipLaunchKernelGGL(prefill_merge_kernel, dim3(p.units, vheads, merge_parts), dim3(kMergeThreads), 0,
                      static_cast<hipStream_t>(stream), p);
   return check_launch(op);
 }
