@@ -18,7 +18,7 @@ struct BwdParams {
   void* grad_q;  // gradients in fp32, or in the inputs' 16-bit type (grad_dtype)
   void* grad_k;
   void* grad_v;
-  float* row_stats;  // [q_tokens * q_heads][2]: log2-domain log-sum-exp of the scaled scores, dO . O
+  float* row_stats;  // [q_tokens * q_heads][2]: log2-domain log-sum-exp of the scaled scores, dO . O (matrix cores: -(dO . O))
   const int32_t* cu_q;
   const int32_t* cu_k;
   const int32_t* ctx;  // may be nullptr: 0

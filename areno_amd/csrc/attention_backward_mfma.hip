@@ -115,6 +115,11 @@ __device__ __forceinline__ float operand_element(uint32_t word, int hi) {
 // CB = blocks of 16 query rows a wave owns: 1 (a workgroup of four waves owns 64 packed rows) or 2 (128 rows).  With
 // two, every operand read from the LDS tile serves two products (the tile's K and V rows in the first pair, K^T in
 // the second), at twice the registers for the rows' operands and sums.
+// Bound by what a wave issues and waits for between its products (825 of 2 500 TFLOP/s at length), so a tile has one
+// barrier (two LDS buffers), a row's softmax reference mostly stays where it is (no lane swaps, no rescaling), and
+// dP - dO . O comes out of the product, which starts at -(dO . O); the dkv kernel's does too.  Forward and backward,
+// before -> after: 2 x 2 048 tokens, 28 / 4 heads of 128, bf16: 435 -> 427 us; 4 x 4 096, 32 / 8 heads: 3 006 -> 2 913 us;
+// ragged 16 x 20 .. 600, 16 heads of 64, fp16, and heads of 256 (whose buffers do not fit twice): within the noise.
 template <int KIND, int D, int CB>
 __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p) {
   using Ops = MfmaOps<KIND>;
@@ -123,8 +128,10 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
   constexpr int NS = D / 32, NB = D / 16;
   constexpr int kRows = kBmRows * CB;  // packed rows of the workgroup
   constexpr int kWaveRows = 16 * CB;
-  __shared__ __attribute__((aligned(16))) char s_k[kBmTile * T::RS];
-  __shared__ __attribute__((aligned(16))) char s_v[kBmTile * T::RS];
+  // two buffers per tensor and one barrier a tile, where they fit the 64 KB of a plain launch (all but head dim 256)
+  constexpr int kBuffers = 4 * kBmTile * T::RS <= 64 * 1024 ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) char k_lds[kBuffers * kBmTile * T::RS];
+  __shared__ __attribute__((aligned(16))) char v_lds[kBuffers * kBmTile * T::RS];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -214,20 +221,18 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
           vreg[i] = load16(p.v, off);
         }
       };
-      auto publish = [&]() {
+      auto publish = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < T::kChunks; ++i) {
           const int c = tid + kBmThreads * i;
           const int r = c / T::kChunksPerRow, col = c % T::kChunksPerRow;
-          *reinterpret_cast<uint4_t*>(s_k + T::chunk_pos(r, col)) = kreg[i];
-          *reinterpret_cast<uint4_t*>(s_v + T::chunk_pos(r, col)) = vreg[i];
+          *reinterpret_cast<uint4_t*>(k_lds + buf * (kBmTile * T::RS) + T::chunk_pos(r, col)) = kreg[i];
+          *reinterpret_cast<uint4_t*>(v_lds + buf * (kBmTile * T::RS) + T::chunk_pos(r, col)) = vreg[i];
         }
       };
-      fetch(t0);
-      __syncthreads();  // the tiles' previous readers (an earlier sequence of this block) are done
-      publish();
-      __syncthreads();
-      for (int t = t0; t <= t1; ++t) {
+      auto step = [&](int t, int buf) {
+        char* const s_k = k_lds + buf * (kBmTile * T::RS);
+        char* const s_v = v_lds + buf * (kBmTile * T::RS);
         if (t < t1) fetch(t + 1);
         if (wave_live) {
           float sc[CB][2][4], dp[CB][2][4];
@@ -236,7 +241,10 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
             for (int tg = 0; tg < 2; ++tg) {
               float4_t c1[CB], c2[CB];
 #pragma unroll
-              for (int cb = 0; cb < CB; ++cb) c1[cb] = c2[cb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+              for (int cb = 0; cb < CB; ++cb) {
+                c1[cb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                c2[cb] = float4_t{-delta[cb], -delta[cb], -delta[cb], -delta[cb]};  // dP comes out less dO . O
+              }
 #pragma unroll
               for (int sl = 0; sl < NS; ++sl) {
                 const V8 k_rows = tile_row_operand<KIND, T, D>(s_k, tg, sl, lr, lk);
@@ -273,46 +281,46 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
           } else {
             first_products(std::true_type{});
           }
+          // The reference of a row is raised only when a score of the wave exceeds its row's by more than 2^kLazy: most
+          // tiles then take no lane swaps and no rescaling.  bf16 has room for probabilities up to 2^8 in dS; fp16 may
+          // not (dS is packed with them), so there the reference follows every new maximum as it is.
+          constexpr float kLazy = KIND == KV_BF16 ? 8.0f : 0.0f;
           V8 dsop[CB];
-          bool moved = false;
-          float alpha[CB];
 #pragma unroll
           for (int cb = 0; cb < CB; ++cb) {
-            float mt = sc[cb][0][0];
+            float mt = max3_f32(sc[cb][0][0], sc[cb][0][1], sc[cb][0][2]);
+            mt = max3_f32(mt, sc[cb][0][3], sc[cb][1][0]);
+            mt = max3_f32(mt, sc[cb][1][1], sc[cb][1][2]);
+            mt = max_f32(mt, sc[cb][1][3]);
+            if (__builtin_amdgcn_ballot_w64(mt * p.scale_log2e > m_run[cb] + kLazy) != 0) {
+              const float m_new = max_f32(m_run[cb], rows_max(mt) * p.scale_log2e);  // (the scale is positive)
+              const float m_ref = m_new == kBmNegInf ? 0.0f : m_new;
+              const float alpha = settled(fast_exp2(m_run[cb] - m_ref));  // 0 while the row has seen no key
+              m_run[cb] = m_new;
+              scale_in_place(l_lane[cb], alpha);
 #pragma unroll
-            for (int tg = 0; tg < 2; ++tg) {
+              for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
-              for (int j = 0; j < 4; ++j) mt = fmaxf(mt, sc[cb][tg][j]);
+                for (int j = 0; j < 4; ++j) {
+                  float x = acc[cb][nb][j];
+                  scale_in_place(x, alpha);
+                  acc[cb][nb][j] = x;
+                }
+              }
             }
-            mt = rows_max(mt);
-            const float m_new = fmaxf(m_run[cb], mt * p.scale_log2e);  // (the scale is positive)
-            const float m_ref = m_new == kBmNegInf ? 0.0f : m_new;
-            alpha[cb] = fast_exp2(m_run[cb] - m_ref);  // 0 while the row has seen no key
-            m_run[cb] = m_new;
-            float ds[2][4], psum = 0.0f;
+            const float m_ref = m_run[cb] == kBmNegInf ? 0.0f : m_run[cb];
+            float ds[2][4];
 #pragma unroll
             for (int tg = 0; tg < 2; ++tg) {
 #pragma unroll
               for (int j = 0; j < 4; ++j) {
                 // (exp2(-inf) = 0: masked keys)
                 const float pe = fast_exp2(__builtin_fmaf(sc[cb][tg][j], p.scale_log2e, -m_ref));
-                psum += pe;
-                ds[tg][j] = pe * (dp[cb][tg][j] - delta[cb]);
+                l_lane[cb] += pe;
+                ds[tg][j] = pe * dp[cb][tg][j];
               }
             }
-            l_lane[cb] = l_lane[cb] * alpha[cb] + psum;
             dsop[cb] = streamed_operand<KIND>(ds);
-            moved = moved || __builtin_amdgcn_ballot_w64(alpha[cb] != 1.0f) != 0;
-          }
-          if (moved) {  // (after the first tiles a new maximum is rare)
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb) {
-#pragma unroll
-              for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[cb][nb][j] *= alpha[cb];
-              }
-            }
           }
 #pragma unroll
           for (int nb = 0; nb < NB; ++nb) {
@@ -321,13 +329,22 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
             for (int cb = 0; cb < CB; ++cb) acc[cb][nb] = Ops::mfma(k_cols, dsop[cb], acc[cb][nb]);
           }
         }
-        __syncthreads();  // every wave has read tile t
-        if (t < t1) publish();
+        if constexpr (kBuffers == 1) __syncthreads();  // every wave has read tile t
+        // (with two buffers: tile t - 1, which lay where t + 1 goes, was read in front of the last barrier)
+        if (t < t1) publish(kBuffers == 2 ? buf ^ 1 : 0);
         __syncthreads();
+      };
+      fetch(t0);
+      __syncthreads();  // the tiles' previous readers (an earlier sequence of this block) are done
+      publish(0);
+      __syncthreads();
+      for (int t = t0; t <= t1; t += 2) {
+        step(t, 0);
+        if (t + 1 <= t1) step(t + 1, kBuffers - 1);
       }
     }
 
-    // dQ = scale / l * sum_k p_k (dP_k - dO . O) K_k; the row's log-sum-exp (log2 domain) and dO . O for the dkv kernel
+    // dQ = scale / l * sum_k p_k (dP_k - dO . O) K_k; the row's log-sum-exp (log2 domain) and -(dO . O) for the dkv kernel
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
       const float l_tot = rows_sum(l_lane[cb]);
@@ -342,7 +359,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
           float* st = p.row_stats + (row[cb] * p.q_heads + h) * 2;
           // a row without visible keys gets a reference no score reaches: its probabilities come out as zeros
           st[0] = l_tot > 0.0f ? m_run[cb] + __builtin_log2f(l_tot) : __builtin_huge_valf();
-          st[1] = delta[cb];
+          st[1] = -delta[cb];
         }
       }
     }
@@ -531,8 +548,8 @@ __global__ __launch_bounds__((DkvShape<D, KR, P>::kThreads), (DkvShape<D, KR, P>
             const float4_t st01 = *reinterpret_cast<const float4_t*>(s_stat(buf) + 2 * (16 * tg + 4 * lk));
             const float4_t st23 = *reinterpret_cast<const float4_t*>(s_stat(buf) + 2 * (16 * tg + 4 * lk + 2));
             const float lse[4] = {st01[0], st01[2], st23[0], st23[2]};
-            const float dlt[4] = {st01[1], st01[3], st23[1], st23[3]};
-            float4_t c1 = {0.0f, 0.0f, 0.0f, 0.0f}, c2 = c1;
+            float4_t c1 = {0.0f, 0.0f, 0.0f, 0.0f};
+            float4_t c2 = {st01[1], st01[3], st23[1], st23[3]};  // -(dO . O): dP comes out less it
 #pragma unroll
             for (int sl = 0; sl < NS; ++sl) {
               c1 = Ops::mfma(tile_row_operand<KIND, T, D>(s_q(buf), tg, sl, lr, lk), kop[sl], c1);
@@ -550,7 +567,7 @@ __global__ __launch_bounds__((DkvShape<D, KR, P>::kThreads), (DkvShape<D, KR, P>
               // (a query without visible keys has +inf as its log-sum-exp: exp2(-inf) = 0 either way)
               const float pe = fast_exp2(x);
               pr[tg][j] = pe;
-              ds[tg][j] = pe * (c2[j] - dlt[j]);
+              ds[tg][j] = pe * c2[j];
             }
           }
         };
