@@ -35,6 +35,7 @@
 #include "attention_backward.hpp"
 #include "backward_order.hpp"
 #include "decode_mfma_kernels.hpp"
+#include "mfma32_tiles.hpp"
 
 namespace areno {
 namespace {
@@ -112,22 +113,18 @@ __device__ __forceinline__ float operand_element(uint32_t word, int hi) {
 }
 
 // ---- dQ (and the rows' statistics) ------------------------------------------------------------------------------------
-// CB = blocks of 16 query rows a wave owns: 1 (a workgroup of four waves owns 64 packed rows) or 2 (128 rows).  With
-// two, every operand read from the LDS tile serves two products (the tile's K and V rows in the first pair, K^T in
-// the second), at twice the registers for the rows' operands and sums.
-// Bound by what a wave issues and waits for between its products (825 of 2 500 TFLOP/s at length), so a tile has one
-// barrier (two LDS buffers), a row's softmax reference mostly stays where it is (no lane swaps, no rescaling), and
-// dP - dO . O comes out of the product, which starts at -(dO . O); the dkv kernel's does too.  Forward and backward,
-// before -> after: 2 x 2 048 tokens, 28 / 4 heads of 128, bf16: 435 -> 427 us; 4 x 4 096, 32 / 8 heads: 3 006 -> 2 913 us;
-// ragged 16 x 20 .. 600, 16 heads of 64, fp16, and heads of 256 (whose buffers do not fit twice): within the noise.
-template <int KIND, int D, int CB>
+// Bound by what a wave issues and waits for between its products, so a tile has one barrier (two LDS buffers), a
+// row's softmax reference mostly stays where it is (no lane swaps, no rescaling), and dP - dO . O comes out of the
+// product, which starts at -(dO . O); the dkv kernel's does too (forward and backward of 2 x 2 048 tokens, 28 / 4 heads of
+// 128, bf16: 435 -> 427 us; heads of 256, whose buffers do not fit twice: within the noise).
+template <int KIND, int D>
 __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p) {
   using Ops = MfmaOps<KIND>;
   using V8 = typename Ops::vec8;
   using T = BmTile<D>;
   constexpr int NS = D / 32, NB = D / 16;
-  constexpr int kRows = kBmRows * CB;  // packed rows of the workgroup
-  constexpr int kWaveRows = 16 * CB;
+  constexpr int kRows = kBmRows;  // packed rows of the workgroup
+  constexpr int kWaveRows = 16;
   // two buffers per tensor and one barrier a tile, where they fit the 64 KB of a plain launch (all but head dim 256)
   constexpr int kBuffers = 4 * kBmTile * T::RS <= 64 * 1024 ? 2 : 1;
   __shared__ __attribute__((aligned(16))) char k_lds[kBuffers * kBmTile * T::RS];
@@ -144,9 +141,8 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
   const int64_t r0 = block_in_cost_order(blockIdx.x / static_cast<unsigned>(p.q_heads), q_blocks, p.num_seqs, true) * kRows;
   const int64_t block_end = r0 + kRows < p.q_tokens ? r0 + kRows : p.q_tokens;
   const int64_t wave_row0 = r0 + kWaveRows * wave;
-  int64_t row[CB];  // this lane's query rows (columns of the products)
-#pragma unroll
-  for (int cb = 0; cb < CB; ++cb) row[cb] = wave_row0 + 16 * cb + lr;
+  int64_t row;  // this lane's query rows (columns of the products)
+  row = wave_row0 + lr;
 
   for (int s = seq_of_row(p.cu_q, p.num_seqs, r0); s < p.num_seqs; ++s) {
     const int64_t sq0 = p.cu_q[s], sq1 = p.cu_q[s + 1];
@@ -156,17 +152,14 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
     const int ctx = p.ctx != nullptr ? p.ctx[s] : 0;
     const int64_t k_base = p.cu_k[s];
     const int n_k = p.cu_k[s + 1] - p.cu_k[s];
-    bool live[CB];
-    int pos[CB];
+    bool live;
+    int pos;
     bool wave_live = false, wave_full = true;
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      live[cb] = row[cb] >= q_lo && row[cb] < q_hi;
-      pos[cb] = live[cb] ? ctx + static_cast<int>(row[cb] - sq0) : -1;
-      const uint64_t live_lanes = __builtin_amdgcn_ballot_w64(live[cb]);
-      wave_live = wave_live || live_lanes != 0;
-      wave_full = wave_full && live_lanes == ~0ull;
-    }
+    live = row >= q_lo && row < q_hi;
+    pos = live ? ctx + static_cast<int>(row - sq0) : -1;
+    const uint64_t live_lanes = __builtin_amdgcn_ballot_w64(live);
+    wave_live = wave_live || live_lanes != 0;
+    wave_full = wave_full && live_lanes == ~0ull;
     // (the positions of the wave's query rows, when all of them belong to this sequence)
     const int wave_pos_lo = ctx + static_cast<int>(wave_row0 - sq0), wave_pos_hi = wave_pos_lo + kWaveRows - 1;
     const int pos_min = ctx + static_cast<int>(q_lo - sq0), pos_max = ctx + static_cast<int>(q_hi - 1 - sq0);
@@ -174,38 +167,35 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
     const int key_hi = pos_max < n_k - 1 ? pos_max : n_k - 1;
 
     // this lane's parts of its rows of Q and dO (B operands), and dO . O
-    int64_t row_elem[CB];
-    V8 qop[CB][NS], gop[CB][NS];
-    float delta[CB];
-    float4_t acc[CB][NB];
-    float m_run[CB], l_lane[CB];
+    int64_t row_elem;
+    V8 qop[NS], gop[NS];
+    float delta;
+    float4_t acc[NB];
+    float m_run, l_lane;
+    row_elem = (row * p.q_heads + h) * D;
+    float d = 0.0f;
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      row_elem[cb] = (row[cb] * p.q_heads + h) * D;
-      float d = 0.0f;
-#pragma unroll
-      for (int sl = 0; sl < NS; ++sl) {
-        uint4_t qw = {0u, 0u, 0u, 0u}, gw = qw, ow = qw;
-        if (live[cb]) {
-          const int64_t off = (row_elem[cb] + (D / 4) * lk + 8 * sl) * 2;
-          qw = load16(p.q, off);
-          gw = load16(p.grad_out, off);
-          ow = load16(p.out, off);
-        }
-        qop[cb][sl] = __builtin_bit_cast(V8, qw);
-        gop[cb][sl] = __builtin_bit_cast(V8, gw);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          d += operand_element<KIND>(gw[j], 0) * operand_element<KIND>(ow[j], 0) +
-               operand_element<KIND>(gw[j], 1) * operand_element<KIND>(ow[j], 1);
-        }
+    for (int sl = 0; sl < NS; ++sl) {
+      uint4_t qw = {0u, 0u, 0u, 0u}, gw = qw, ow = qw;
+      if (live) {
+        const int64_t off = (row_elem + (D / 4) * lk + 8 * sl) * 2;
+        qw = load16(p.q, off);
+        gw = load16(p.grad_out, off);
+        ow = load16(p.out, off);
       }
-      delta[cb] = rows_sum(d);
+      qop[sl] = __builtin_bit_cast(V8, qw);
+      gop[sl] = __builtin_bit_cast(V8, gw);
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) acc[cb][nb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-      m_run[cb] = kBmNegInf;
-      l_lane[cb] = 0.0f;
+      for (int j = 0; j < 4; ++j) {
+        d += operand_element<KIND>(gw[j], 0) * operand_element<KIND>(ow[j], 0) +
+             operand_element<KIND>(gw[j], 1) * operand_element<KIND>(ow[j], 1);
+      }
     }
+    delta = rows_sum(d);
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[nb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    m_run = kBmNegInf;
+    l_lane = 0.0f;
 
     if (key_hi >= key_lo) {  // (the same for the whole workgroup)
       const int t0 = key_lo / kBmTile, t1 = key_hi / kBmTile;
@@ -235,39 +225,30 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
         char* const s_v = v_lds + buf * (kBmTile * T::RS);
         if (t < t1) fetch(t + 1);
         if (wave_live) {
-          float sc[CB][2][4], dp[CB][2][4];
+          float sc[2][4], dp[2][4];
           auto first_products = [&](auto masked) {
 #pragma unroll
             for (int tg = 0; tg < 2; ++tg) {
-              float4_t c1[CB], c2[CB];
-#pragma unroll
-              for (int cb = 0; cb < CB; ++cb) {
-                c1[cb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                c2[cb] = float4_t{-delta[cb], -delta[cb], -delta[cb], -delta[cb]};  // dP comes out less dO . O
-              }
+              float4_t c1, c2;
+              c1 = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+              c2 = float4_t{-delta, -delta, -delta, -delta};  // dP comes out less dO . O
 #pragma unroll
               for (int sl = 0; sl < NS; ++sl) {
                 const V8 k_rows = tile_row_operand<KIND, T, D>(s_k, tg, sl, lr, lk);
                 const V8 v_rows = tile_row_operand<KIND, T, D>(s_v, tg, sl, lr, lk);
-#pragma unroll
-                for (int cb = 0; cb < CB; ++cb) {
-                  c1[cb] = Ops::mfma(k_rows, qop[cb][sl], c1[cb]);
-                  c2[cb] = Ops::mfma(v_rows, gop[cb][sl], c2[cb]);
-                }
+                c1 = Ops::mfma(k_rows, qop[sl], c1);
+                c2 = Ops::mfma(v_rows, gop[sl], c2);
               }
 #pragma unroll
-              for (int cb = 0; cb < CB; ++cb) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                  sc[cb][tg][j] = c1[cb][j];  // (the softmax scale goes in with the reference, below)
-                  if constexpr (decltype(masked)::value) {
-                    const int key = kBmTile * t + 16 * tg + 4 * lk + j;
-                    const bool ok =
-                        key <= pos[cb] && key < n_k && (p.window_left < 0 || key >= pos[cb] - p.window_left);
-                    sc[cb][tg][j] = ok ? sc[cb][tg][j] : kBmNegInf;
-                  }
-                  dp[cb][tg][j] = c2[cb][j];
+              for (int j = 0; j < 4; ++j) {
+                sc[tg][j] = c1[j];  // (the softmax scale goes in with the reference, below)
+                if constexpr (decltype(masked)::value) {
+                  const int key = kBmTile * t + 16 * tg + 4 * lk + j;
+                  const bool ok =
+                      key <= pos && key < n_k && (p.window_left < 0 || key >= pos - p.window_left);
+                  sc[tg][j] = ok ? sc[tg][j] : kBmNegInf;
                 }
+                dp[tg][j] = c2[j];
               }
             }
           };
@@ -285,48 +266,44 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
           // tiles then take no lane swaps and no rescaling.  bf16 has room for probabilities up to 2^8 in dS; fp16 may
           // not (dS is packed with them), so there the reference follows every new maximum as it is.
           constexpr float kLazy = KIND == KV_BF16 ? 8.0f : 0.0f;
-          V8 dsop[CB];
+          V8 dsop;
+          float mt = max3_f32(sc[0][0], sc[0][1], sc[0][2]);
+          mt = max3_f32(mt, sc[0][3], sc[1][0]);
+          mt = max3_f32(mt, sc[1][1], sc[1][2]);
+          mt = max_f32(mt, sc[1][3]);
+          if (__builtin_amdgcn_ballot_w64(mt * p.scale_log2e > m_run + kLazy) != 0) {
+            const float m_new = max_f32(m_run, rows_max(mt) * p.scale_log2e);  // (the scale is positive)
+            const float m_ref = m_new == kBmNegInf ? 0.0f : m_new;
+            const float alpha = settled(fast_exp2(m_run - m_ref));  // 0 while the row has seen no key
+            m_run = m_new;
+            scale_in_place(l_lane, alpha);
 #pragma unroll
-          for (int cb = 0; cb < CB; ++cb) {
-            float mt = max3_f32(sc[cb][0][0], sc[cb][0][1], sc[cb][0][2]);
-            mt = max3_f32(mt, sc[cb][0][3], sc[cb][1][0]);
-            mt = max3_f32(mt, sc[cb][1][1], sc[cb][1][2]);
-            mt = max_f32(mt, sc[cb][1][3]);
-            if (__builtin_amdgcn_ballot_w64(mt * p.scale_log2e > m_run[cb] + kLazy) != 0) {
-              const float m_new = max_f32(m_run[cb], rows_max(mt) * p.scale_log2e);  // (the scale is positive)
-              const float m_ref = m_new == kBmNegInf ? 0.0f : m_new;
-              const float alpha = settled(fast_exp2(m_run[cb] - m_ref));  // 0 while the row has seen no key
-              m_run[cb] = m_new;
-              scale_in_place(l_lane[cb], alpha);
-#pragma unroll
-              for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                  float x = acc[cb][nb][j];
-                  scale_in_place(x, alpha);
-                  acc[cb][nb][j] = x;
-                }
-              }
-            }
-            const float m_ref = m_run[cb] == kBmNegInf ? 0.0f : m_run[cb];
-            float ds[2][4];
-#pragma unroll
-            for (int tg = 0; tg < 2; ++tg) {
+            for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
               for (int j = 0; j < 4; ++j) {
-                // (exp2(-inf) = 0: masked keys)
-                const float pe = fast_exp2(__builtin_fmaf(sc[cb][tg][j], p.scale_log2e, -m_ref));
-                l_lane[cb] += pe;
-                ds[tg][j] = pe * dp[cb][tg][j];
+                float x = acc[nb][j];
+                scale_in_place(x, alpha);
+                acc[nb][j] = x;
               }
             }
-            dsop[cb] = streamed_operand<KIND>(ds);
           }
+          const float m_ref = m_run == kBmNegInf ? 0.0f : m_run;
+          float ds[2][4];
+#pragma unroll
+          for (int tg = 0; tg < 2; ++tg) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              // (exp2(-inf) = 0: masked keys)
+              const float pe = fast_exp2(__builtin_fmaf(sc[tg][j], p.scale_log2e, -m_ref));
+              l_lane += pe;
+              ds[tg][j] = pe * dp[tg][j];
+            }
+          }
+          dsop = streamed_operand<KIND>(ds);
 #pragma unroll
           for (int nb = 0; nb < NB; ++nb) {
             const V8 k_cols = tile_transposed_operand<KIND, T>(s_k, nb, lr, lk);
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb) acc[cb][nb] = Ops::mfma(k_cols, dsop[cb], acc[cb][nb]);
+            acc[nb] = Ops::mfma(k_cols, dsop, acc[nb]);
           }
         }
         if constexpr (kBuffers == 1) __syncthreads();  // every wave has read tile t
@@ -345,22 +322,229 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
     }
 
     // dQ = scale / l * sum_k p_k (dP_k - dO . O) K_k; the row's log-sum-exp (log2 domain) and -(dO . O) for the dkv kernel
+    const float l_tot = rows_sum(l_lane);
+    if (live) {
+      const float f = l_tot > 0.0f ? p.scale / l_tot : 0.0f;
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      const float l_tot = rows_sum(l_lane[cb]);
-      if (live[cb]) {
-        const float f = l_tot > 0.0f ? p.scale / l_tot : 0.0f;
+      for (int nb = 0; nb < NB; ++nb) {
+        store_grad4(p.grad_q, row_elem + 4 * lk + 16 * nb, acc[nb][0] * f, acc[nb][1] * f,
+                    acc[nb][2] * f, acc[nb][3] * f, p.grad_dtype);
+      }
+      if (lk == 0) {
+        float* st = p.row_stats + (row * p.q_heads + h) * 2;
+        // a row without visible keys gets a reference no score reaches: its probabilities come out as zeros
+        st[0] = l_tot > 0.0f ? m_run + __builtin_log2f(l_tot) : __builtin_huge_valf();
+        st[1] = -delta;
+      }
+    }
+  }
+}
+
+// The same with 32 query rows per wave, 128 per workgroup, on 32 x 32 x 16 products, for launches that fill the chip with
+// such workgroups: an operand read from LDS serves a product of twice the size, the K and V tiles are fetched straight
+// into LDS (mfma32_tiles.hpp).  Bound by the matrix cores and the LDS reads behind them.  Against a 16 x 16 form of as
+// many rows, which spilled 84 registers: the backward of 4 x 4 096 tokens, 32 / 8 heads of 128, bf16: 2 646 -> 2 283 us.
+template <int KIND, int D>
+__global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams p) {
+  using M = Mfma32<KIND>;
+  using V8 = typename M::vec8;
+  using T = LdsTile<D, kBmTile, kBmWaves>;
+  constexpr int NKS = D / 16, NB = D / 32, NF = T::kFetches;
+  constexpr int kRows = 32 * kBmWaves;
+  constexpr int kBuffer = 2 * T::kBytes;  // K, V
+  __shared__ __attribute__((aligned(1024))) char lds[2 * kBuffer];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = uniform(tid >> 6);
+  const int l32 = lane & 31, half = lane >> 5;
+  const int h = static_cast<int>(blockIdx.x % static_cast<unsigned>(p.q_heads));
+  const int kvh = h / (p.q_heads / p.kv_heads);
+  const int64_t q_blocks = (p.q_tokens + kRows - 1) / kRows;
+  const int block = uniform(static_cast<int>(
+      block_in_cost_order(blockIdx.x / static_cast<unsigned>(p.q_heads), q_blocks, p.num_seqs, true)));
+  const int64_t r0 = static_cast<int64_t>(block) * kRows;
+  const int64_t block_end = r0 + kRows < p.q_tokens ? r0 + kRows : p.q_tokens;
+  const int64_t wave_row0 = r0 + 32 * wave;
+  const int64_t row = wave_row0 + l32;  // this lane's query row (a column of the products)
+  const uint32_t at_rows = T::rows_base(l32, half), at_columns = T::columns_base(lane);
+  const uint32_t lds0 = lds_address(lds);
+  const uint32_t stride = static_cast<uint32_t>(p.kv_heads) * (D * 2);
+  int fetch_row[NF];
+  uint32_t fetch_chunk[NF];
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          store_grad4(p.grad_q, row_elem[cb] + 4 * lk + 16 * nb, acc[cb][nb][0] * f, acc[cb][nb][1] * f,
-                      acc[cb][nb][2] * f, acc[cb][nb][3] * f, p.grad_dtype);
+  for (int f = 0; f < NF; ++f) {
+    const int slot = (wave * NF + f) * 64 + lane;
+    fetch_row[f] = slot / T::kChunksPerRow;
+    fetch_chunk[f] = static_cast<uint32_t>((slot % T::kChunksPerRow) ^ T::twist(fetch_row[f])) * 16u;
+  }
+
+  for (int s = uniform(seq_of_row(p.cu_q, p.num_seqs, r0)); s < p.num_seqs; ++s) {
+    const int64_t sq0 = uniform(p.cu_q[s]), sq1 = uniform(p.cu_q[s + 1]);
+    if (sq0 >= block_end) break;
+    const int64_t q_lo = sq0 > r0 ? sq0 : r0, q_hi = sq1 < block_end ? sq1 : block_end;
+    if (q_lo >= q_hi) continue;
+    const int ctx = p.ctx != nullptr ? uniform(p.ctx[s]) : 0;
+    const int64_t k_first = uniform(p.cu_k[s]);
+    const int n_k = uniform(p.cu_k[s + 1]) - static_cast<int>(k_first);
+    const bool live = row >= q_lo && row < q_hi;
+    const int pos = live ? ctx + static_cast<int>(row - sq0) : -1;
+    const uint64_t live_lanes = __builtin_amdgcn_ballot_w64(live);
+    const bool wave_live = live_lanes != 0, wave_full = live_lanes == ~0ull;
+    const int wave_pos_lo = ctx + static_cast<int>(wave_row0 - sq0), wave_pos_hi = wave_pos_lo + 31;
+    const int pos_min = ctx + static_cast<int>(q_lo - sq0), pos_max = ctx + static_cast<int>(q_hi - 1 - sq0);
+    const int key_lo = p.window_left >= 0 ? (pos_min - p.window_left > 0 ? pos_min - p.window_left : 0) : 0;
+    const int key_hi = pos_max < n_k - 1 ? pos_max : n_k - 1;
+
+    // this lane's parts of its row of Q and dO (B operands), and dO . O
+    const int64_t row_elem = (row * p.q_heads + h) * D;
+    V8 qop[NKS], gop[NKS];
+    float delta = 0.0f;
+    uint4_t qw[NKS], gw[NKS], ow[NKS];
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) qw[ks] = gw[ks] = ow[ks] = uint4_t{0u, 0u, 0u, 0u};
+    if (live) {
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) {
+        const int64_t off = (row_elem + 16 * ks + 8 * half) * 2;
+        qw[ks] = load16(p.q, off);
+        gw[ks] = load16(p.grad_out, off);
+        ow[ks] = load16(p.out, off);
+      }
+    }
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      // (waited for here: left to their first use inside the loop, that wait would cover every tile's fetches as well)
+      asm volatile("" : "+v"(qw[ks]), "+v"(gw[ks]));
+      qop[ks] = __builtin_bit_cast(V8, qw[ks]);
+      gop[ks] = __builtin_bit_cast(V8, gw[ks]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        delta += operand_element<KIND>(gw[ks][j], 0) * operand_element<KIND>(ow[ks][j], 0) +
+                 operand_element<KIND>(gw[ks][j], 1) * operand_element<KIND>(ow[ks][j], 1);
+      }
+    }
+    auto both_halves = [](float x, auto op) {
+      uint32_t a = __builtin_bit_cast(uint32_t, x), b = a;
+      swap_rows32(a, b);
+      return op(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+    };
+    auto sum = [](float a, float b) { return a + b; };
+    delta = both_halves(delta, sum);
+    float16_t acc[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[nb] = zero16();
+    float m_run = kBmNegInf, l_lane = 0.0f;
+
+    if (key_hi >= key_lo) {  // (the same for the whole workgroup)
+      const int t0 = key_lo / kBmTile, t1 = key_hi / kBmTile;
+      const int64_t head_base = (k_first * p.kv_heads + kvh) * (D * 2);
+      auto fetch = [&](int t, int buf) {
+        const int rows = n_k - t * kBmTile;  // rows of the tile that exist; the ones behind repeat the last
+        const int64_t tile_base = head_base + static_cast<int64_t>(t) * kBmTile * stride;
+        const char* kb = static_cast<const char*>(p.k) + tile_base;
+        const char* vb = static_cast<const char*>(p.v) + tile_base;
+        const uint32_t dst = lds0 + static_cast<uint32_t>(buf * kBuffer + wave * (NF * 1024));
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          const uint32_t off = static_cast<uint32_t>(min(fetch_row[f], rows - 1)) * stride + fetch_chunk[f];
+          fetch_to_lds(kb, off, dst + f * 1024);
+          fetch_to_lds(vb, off, dst + T::kBytes + f * 1024);
         }
-        if (lk == 0) {
-          float* st = p.row_stats + (row[cb] * p.q_heads + h) * 2;
-          // a row without visible keys gets a reference no score reaches: its probabilities come out as zeros
-          st[0] = l_tot > 0.0f ? m_run[cb] + __builtin_log2f(l_tot) : __builtin_huge_valf();
-          st[1] = -delta[cb];
+      };
+      auto step = [&](int t, int buf) {
+        fetched_barrier();  // tile t (asked for a step ago) is there, and every wave has left tile t - 1
+        if (t < t1) fetch(t + 1, buf ^ 1);
+        if (!wave_live) return;
+        const int key_first = kBmTile * t, key_last = key_first + kBmTile - 1;
+        if (wave_full && key_first > wave_pos_hi) return;
+        char* const k_lds = lds + buf * kBuffer;
+        const char* const v_lds = k_lds + T::kBytes;
+        float16_t sc = zero16(), dp;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dp[i] = -delta;
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+          sc = M::mfma(tile_rows<KIND, T>(k_lds, at_rows, 0, ks), qop[ks], sc);
+          dp = M::mfma(tile_rows<KIND, T>(v_lds, at_rows, 0, ks), gop[ks], dp);
         }
+        const bool plain = wave_full && key_last < n_k && key_last <= wave_pos_lo &&
+                           (p.window_left < 0 || key_first >= wave_pos_hi - p.window_left);
+        if (!plain) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int key = key_first + 8 * (i >> 2) + 4 * half + (i & 3);
+            const bool ok = key <= pos && key < n_k && (p.window_left < 0 || key >= pos - p.window_left);
+            sc[i] = ok ? sc[i] : kBmNegInf;
+          }
+        }
+        constexpr float kLazy = KIND == KV_BF16 ? 8.0f : 0.0f;  // (as above)
+        float mt = sc[0];
+#pragma unroll
+        for (int i = 1; i < 15; i += 2) mt = max3_f32(mt, sc[i], sc[i + 1]);
+        mt = max_f32(mt, sc[15]);
+        if (__builtin_amdgcn_ballot_w64(mt * p.scale_log2e > m_run + kLazy) != 0) {
+          mt = both_halves(mt, [](float a, float b) { return max_f32(a, b); });
+          const float m_new = max_f32(m_run, mt * p.scale_log2e);  // (the scale is positive)
+          const float m_ref = m_new == kBmNegInf ? 0.0f : m_new;
+          const float alpha = settled(fast_exp2(m_run - m_ref));  // 0 while the row has seen no key
+          m_run = m_new;
+          scale_in_place(l_lane, alpha);
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              float x = acc[nb][i];
+              scale_in_place(x, alpha);
+              acc[nb][i] = x;
+            }
+          }
+        }
+        const float m_ref = m_run == kBmNegInf ? 0.0f : m_run;
+        V8 dsop[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          uint32_t w[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int i = 8 * b + 2 * j;
+            const float p0 = fast_exp2(__builtin_fmaf(sc[i], p.scale_log2e, -m_ref));
+            const float p1 = fast_exp2(__builtin_fmaf(sc[i + 1], p.scale_log2e, -m_ref));
+            l_lane += p0 + p1;
+            w[j] = pack_pair<KIND>(p0 * dp[i], p1 * dp[i + 1]);
+          }
+          dsop[b] = __builtin_bit_cast(V8, uint4_t{w[0], w[1], w[2], w[3]});
+        }
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb)
+            acc[nb] = M::mfma(tile_columns<KIND, T>(k_lds, at_columns, 16 * b, nb), dsop[b], acc[nb]);
+        }
+      };
+      fetched_barrier();  // the tiles' previous readers (an earlier sequence of this block) are done
+      fetch(t0, 0);
+      for (int t = t0; t <= t1; t += 2) {
+        step(t, 0);
+        if (t + 1 <= t1) step(t + 1, 1);
+      }
+    }
+
+    const float l_tot = both_halves(l_lane, sum);
+    if (live) {
+      const float f = l_tot > 0.0f ? p.scale / l_tot : 0.0f;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          store_grad4(p.grad_q, row_elem + 32 * nb + 8 * c + 4 * half, acc[nb][4 * c] * f, acc[nb][4 * c + 1] * f,
+                      acc[nb][4 * c + 2] * f, acc[nb][4 * c + 3] * f, p.grad_dtype);
+        }
+      }
+      if (half == 0) {
+        float* st = p.row_stats + (row * p.q_heads + h) * 2;
+        st[0] = l_tot > 0.0f ? m_run + __builtin_log2f(l_tot) : __builtin_huge_valf();
+        st[1] = -delta;
       }
     }
   }
@@ -727,39 +911,41 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
     if (strcmp(e, "2") == 0) dkv_parts = 2;
     if (strcmp(e, "4") == 0) dkv_parts = 4;
   }
-  // The dq kernel with 32 rows per wave at head dim 128 once the launch has 8 workgroups of 64 rows per compute unit:
-  // half the LDS reads per product (4 x 4 096 tokens, 32 / 8 heads: both launches 2 970 -> 2 760 us; 4 x 2 048
-  // tokens, 28 / 4 heads: 834 -> 807 us), but half the workgroups and two waves per SIMD instead of three, which
-  // costs small launches (8 x 512 tokens: +4 %) and head dim 64 (four waves per SIMD down to two: +5 %).
+  // The dq kernel with 32 rows per wave once the launch has 6 workgroups of 64 rows per compute unit at head dim 128, 8
+  // at head dim 64.  The backward, 16 -> 32 rows, us: D = 128: 4 x 4 096 tokens, 32 / 8 heads (32 per unit) 2 646 ->
+  // 2 283; 1 x 4 096, 28 / 4 heads (7) 639 -> 561; 8 x 512, 28 / 4 heads (7) 133 -> 130; 4 x 600, 32 / 8 heads (4.6)
+  // 161 -> 163; 1 x 1 024, 8 / 2 heads (0.5) 94 -> 105.  D = 64: 4 x 4 096, 32 / 8 heads (32) 1 357 -> 1 240; 2 x 4 096,
+  // 16 heads (8) 365 -> 342; 8 x 512, 28 / 4 heads (7) 72 -> 75; 16 x 310, 16 heads (4.8) 62 -> 69.  Small launches
+  // want the more and shorter workgroups.
   // ARENO_BACKWARD_DQ_ROWS=16|32 (read at every launch) fixes the choice, for tests and timing.
-  int dq_cb = p.head_dim == 128 && q_blocks * p.q_heads >= 8 * kBmComputeUnits ? 2 : 1;
+  int dq_rows = q_blocks * p.q_heads >= (p.head_dim == 128 ? 6 : 8) * kBmComputeUnits ? 32 : 16;
   if (const char* e = getenv("ARENO_BACKWARD_DQ_ROWS")) {
-    if (strcmp(e, "32") == 0) dq_cb = 2;
-    if (strcmp(e, "16") == 0) dq_cb = 1;
+    if (strcmp(e, "32") == 0) dq_rows = 32;
+    if (strcmp(e, "16") == 0) dq_rows = 16;
   }
   // Head dims 192 and 256 (the sliding-window layers of wide heads) have one shape of either kernel.  2 400 tokens in
   // four sequences, 16 / 8 heads of 256, window 512, bf16: 323 us for both launches against 7 470 us on the
   // vector-ALU kernels, which recompute every product on 16 lanes' dot products.
   if (p.head_dim > 128) {
     dkv_parts = 1;
-    dq_cb = 1;
+    dq_rows = 16;
   }
-  const int64_t dq_blocks = (p.q_tokens + kBmRows * dq_cb - 1) / (kBmRows * dq_cb);
+  const int64_t dq_blocks = (p.q_tokens + kBmWaves * dq_rows - 1) / (kBmWaves * dq_rows);
   bm_fn dq;
   DkvLaunch dkv;
   if (p.head_dim == 64) {
-    dq = dq_cb == 2 ? (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 64, 2> : bwd_mfma_dq_kernel<KV_F16, 64, 2>)
-                    : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 64, 1> : bwd_mfma_dq_kernel<KV_F16, 64, 1>);
+    dq = dq_rows == 32 ? (bf16 ? bwd_mfma32_dq_kernel<KV_BF16, 64> : bwd_mfma32_dq_kernel<KV_F16, 64>)
+                    : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 64> : bwd_mfma_dq_kernel<KV_F16, 64>);
     dkv = bf16 ? dkv_launch<KV_BF16, 64>(dkv_parts) : dkv_launch<KV_F16, 64>(dkv_parts);
   } else if (p.head_dim == 192) {
-    dq = bf16 ? bwd_mfma_dq_kernel<KV_BF16, 192, 1> : bwd_mfma_dq_kernel<KV_F16, 192, 1>;
+    dq = bf16 ? bwd_mfma_dq_kernel<KV_BF16, 192> : bwd_mfma_dq_kernel<KV_F16, 192>;
     dkv = bf16 ? dkv_launch<KV_BF16, 192>(1) : dkv_launch<KV_F16, 192>(1);
   } else if (p.head_dim == 256) {
-    dq = bf16 ? bwd_mfma_dq_kernel<KV_BF16, 256, 1> : bwd_mfma_dq_kernel<KV_F16, 256, 1>;
+    dq = bf16 ? bwd_mfma_dq_kernel<KV_BF16, 256> : bwd_mfma_dq_kernel<KV_F16, 256>;
     dkv = bf16 ? dkv_launch<KV_BF16, 256>(1) : dkv_launch<KV_F16, 256>(1);
   } else {
-    dq = dq_cb == 2 ? (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 128, 2> : bwd_mfma_dq_kernel<KV_F16, 128, 2>)
-                    : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 128, 1> : bwd_mfma_dq_kernel<KV_F16, 128, 1>);
+    dq = dq_rows == 32 ? (bf16 ? bwd_mfma32_dq_kernel<KV_BF16, 128> : bwd_mfma32_dq_kernel<KV_F16, 128>)
+                    : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 128> : bwd_mfma_dq_kernel<KV_F16, 128>);
     dkv = bf16 ? dkv_launch<KV_BF16, 128>(dkv_parts) : dkv_launch<KV_F16, 128>(dkv_parts);
   }
   const char* op = "areno_hip_attention_backward";
