@@ -883,6 +883,9 @@ DkvLaunch dkv_launch(int parts) {
 int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
   if (p.dtype != ARENO_DT_BF16 && p.dtype != ARENO_DT_F16) return ARENO_ERR_UNSUPPORTED;
   if (p.head_dim != 64 && p.head_dim != 128 && p.head_dim != 192 && p.head_dim != 256) return ARENO_ERR_UNSUPPORTED;
+  // the kernels mask raw scores and take row maxima before scaling: any other scale is for the vector-ALU kernels, as in
+  // the forward (launch_prefill_mfma)
+  if (!(p.scale_log2e > 0.0f)) return ARENO_ERR_UNSUPPORTED;
   if (p.q_heads > 65535 || p.kv_heads > 65535) return ARENO_ERR_UNSUPPORTED;
   const int64_t q_blocks = (p.q_tokens + kBmRows - 1) / kBmRows, k_blocks = (p.k_tokens + kBmRows - 1) / kBmRows;
   if (q_blocks * p.q_heads > 0x7fffffffLL || k_blocks * p.kv_heads > 0x7fffffffLL) return ARENO_ERR_UNSUPPORTED;

@@ -125,6 +125,25 @@ def test_varlen_backward_where_the_softmax_reference_moves(dtype, hq, hkv, d, dq
         _close(got, ref, REL[dtype], f"{name} {dtype} d={d} falling={falling}")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("scale", [0.0, -0.05])
+@pytest.mark.parametrize("d", [64, 128, 192, 256])
+def test_varlen_backward_with_a_scale_that_is_not_positive(dtype, scale, d):
+    """The op takes any softmax scale: 0 (every visible key weighs the same) and negative ones (a row's maximum is
+    that of its negated products).  Masked keys count for nothing either way.  The bar is the file's."""
+    g = torch.Generator().manual_seed(d)
+    lens = [130, 0, 33]
+    t = sum(lens)
+    cu = torch.tensor([0, 130, 130, 163], dtype=torch.int32)
+    q, k, v, go = (torch.randn(t, h, d, generator=g).to(dtype) for h in (4, 2, 2, 4))
+    qd, kd, vd = (x.to(DEV).requires_grad_(True) for x in (q, k, v))
+    ops.areno_varlen_causal_attention(qd, kd, vd, cu.to(DEV), softmax_scale=scale).backward(go.to(DEV))
+    qf, kf, vf = (x.float().requires_grad_(True) for x in (q, k, v))
+    ar.ref_varlen(qf, kf, vf, cu, -1, scale).backward(go.float())
+    for got, ref, name in ((qd.grad, qf.grad, "dq"), (kd.grad, kf.grad, "dk"), (vd.grad, vf.grad, "dv")):
+        _close(got, ref, REL[dtype], f"{name} {dtype} d={d} scale={scale}")
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("query_start,window_left", [(0, None), (7, None), (3, 5)])
 def test_dense_backward(dtype, query_start, window_left):
