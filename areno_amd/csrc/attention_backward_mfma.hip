@@ -60,6 +60,11 @@ __device__ __forceinline__ int seq_of_row(const int32_t* cu, int num_seqs, int64
   return lo;
 }
 
+// a query row in front of the first sequence or behind the last (the end of a padded pack): no keys, a gradient of zeros
+__device__ __forceinline__ bool row_of_no_sequence(const BwdParams& p, int64_t row) {
+  return row < p.q_tokens && (row >= p.cu_q[p.num_seqs] || row < p.cu_q[0]);
+}
+
 // A tile of 32 rows x D 16-bit elements in LDS, row stride D * 2 + 16 bytes: the row operands (16 lanes read the same
 // 16-byte chunk of 16 rows) meet every bank once, the transposed ones (32 lanes read 32 bytes of 8 consecutive rows)
 // meet every bank twice.  (A layout without any bank conflict -- rows back to back, the chunks of a row permuted by
@@ -338,6 +343,11 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
       }
     }
   }
+  if (row_of_no_sequence(p, row)) {
+    const int64_t row_elem = (row * p.q_heads + h) * D;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) store_grad4(p.grad_q, row_elem + 4 * lk + 16 * nb, 0.0f, 0.0f, 0.0f, 0.0f, p.grad_dtype);
+  }
 }
 
 // The same with 32 query rows per wave, 128 per workgroup, on 32 x 32 x 16 products, for launches that fill the chip with
@@ -547,6 +557,11 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
         st[1] = -delta;
       }
     }
+  }
+  if (row_of_no_sequence(p, row)) {
+    const int64_t row_elem = (row * p.q_heads + h) * D;
+#pragma unroll
+    for (int c = 0; c < D / 8; ++c) store_grad4(p.grad_q, row_elem + 8 * c + 4 * half, 0.0f, 0.0f, 0.0f, 0.0f, p.grad_dtype);
   }
 }
 

@@ -7,10 +7,13 @@ relative to the largest gradient of the tensor: 3e-2 for bf16, 1e-2 for fp16 (on
 format's rounding at that magnitude, plus the rounding of the saved output that both this build and the reference
 use for dO . O), 1e-4 for fp32."""
 
+import ctypes
+
 import pytest
 import torch
 
 from areno_amd.accel import attention as ops
+from areno_amd.accel import cabi
 from oracle import attention_ref as ar
 from tests.gpu_util import DEV
 
@@ -142,6 +145,38 @@ def test_varlen_backward_with_a_scale_that_is_not_positive(dtype, scale, d):
     ar.ref_varlen(qf, kf, vf, cu, -1, scale).backward(go.float())
     for got, ref, name in ((qd.grad, qf.grad, "dq"), (kd.grad, kf.grad, "dk"), (vd.grad, vf.grad, "dv")):
         _close(got, ref, REL[dtype], f"{name} {dtype} d={d} scale={scale}")
+
+
+def _c_backward(go, q, k, v, out, cu, grad_dtype, scale):
+    """The C entry on gradient buffers full of NaN: what it leaves unwritten shows."""
+    t, hq, d = q.shape
+    grads = [torch.full(x.shape, float("nan"), dtype=grad_dtype, device=DEV) for x in (q, k, v)]
+    workspace = torch.empty(t * hq * 8, dtype=torch.uint8, device=DEV)
+    ptr = lambda x: ctypes.c_void_p(x.data_ptr())  # noqa: E731
+    status = cabi.lib().areno_hip_attention_backward_typed(
+        *map(ptr, (go, q, k, v, out, *grads)), cabi.dtype_code(grads[0]), cabi.dtype_code(q), ctypes.c_int64(t),
+        ctypes.c_int64(k.shape[0]), hq, k.shape[1], d, ptr(cu), None, None, cu.numel() - 1, -1, ctypes.c_float(scale),
+        ptr(workspace), ctypes.c_size_t(workspace.numel()), ctypes.c_void_p(cabi.current_stream_ptr()))  # fmt: skip
+    cabi.check(status, "areno_hip_attention_backward_typed")
+    return grads
+
+
+@pytest.mark.parametrize("d,dq_rows", [(64, "16"), (64, "32"), (128, "16"), (128, "32"), (192, "16"), (256, "16"), (96, "16")])
+@pytest.mark.parametrize("dtype,grad_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("behind", [1, 70, 300])
+def test_gradients_of_rows_behind_the_last_sequence_are_zeros(d, dq_rows, dtype, grad_dtype, behind, monkeypatch):
+    """A padded pack: its rows behind the last sequence get zeros, the others the gradients that they have without the
+    padding, bit for bit (every row has one owner, which does the same for it)."""
+    monkeypatch.setenv("ARENO_BACKWARD_DQ_ROWS", dq_rows)
+    g = torch.Generator().manual_seed(d + behind)
+    t, hq, hkv = 163, 4, 2
+    padded = [torch.randn(t + behind, h, d, generator=g).to(dtype).to(DEV) for h in (hq, hq, hkv, hkv, hq)]
+    plain = [x[:t].contiguous() for x in padded]
+    cu = torch.tensor([0, 130, 130, 163], dtype=torch.int32, device=DEV)
+    for got, want in zip(_c_backward(*padded, cu, grad_dtype, d**-0.5), _c_backward(*plain, cu, grad_dtype, d**-0.5)):
+        assert torch.isfinite(want).all()
+        assert torch.equal(got[:t], want)
+        assert (got[t:] == 0).all()
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
