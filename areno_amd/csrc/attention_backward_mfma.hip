@@ -111,6 +111,59 @@ __device__ __forceinline__ typename MfmaOps<KIND>::vec8 streamed_operand(const f
   return __builtin_bit_cast(V8, uint4_t{pack_pair<KIND>(x[0][0], x[0][1]), pack_pair<KIND>(x[0][2], x[0][3]),
                                         pack_pair<KIND>(x[1][0], x[1][1]), pack_pair<KIND>(x[1][2], x[1][3])});
 }
+// The same without rounding, for the wide heads (whose 16-bit inputs had fp32 kernels until these took them, and lose
+// nothing by it): the eight values as three bf16 operands that add up to them.  A bf16 holds eight significant bits
+// with fp32's exponents, so the upper half of a value's word, that of the rest and what is left then are the value's 24.
+__device__ __forceinline__ void split_weights(const float (&x)[2][4], bf16x8_t (&part)[3]) {
+  uint32_t w[3][4];
+#pragma unroll
+  for (int pair = 0; pair < 4; ++pair) {
+    float a = x[pair >> 1][2 * (pair & 1)], b = x[pair >> 1][2 * (pair & 1) + 1];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
+      w[i][pair] = __builtin_amdgcn_perm(ub, ua, 0x07060302u);  // the upper halves, a's in the low one
+      a -= __builtin_bit_cast(float, ua & 0xffff0000u);  // exact
+      b -= __builtin_bit_cast(float, ub & 0xffff0000u);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i) part[i] = __builtin_bit_cast(bf16x8_t, uint4_t{w[i][0], w[i][1], w[i][2], w[i][3]});
+}
+// c + columns . the values that `part` adds up to.  An fp16 operand has 11 significant bits and goes in as the two
+// bf16 that hold them (the product of its rest with the weights' last part, 2^-25 of the whole, is left out).  A tile's
+// products are summed by themselves, the small ones first, so the running sum rounds once per tile.
+// Relative error of dV against 64 bits (four sequences of 300 .. 1 000 tokens, 16 / 8 heads of 256, window 512, fp32 out):
+// rounded weights 1.6e-3 (bf16) and 2.0e-4 (fp16), these 2.7e-7 and 2.8e-7, the fp32 kernels 2.8e-7 and 3.1e-7; all
+// products straight into the running sum 4.5e-7 and 5.5e-7.  The price, forward and backward: bf16 343 -> 403 us (365
+// without the sum of its own), fp16 350 -> 601 us; the fp32 kernels take 7 500.
+template <int KIND>
+__device__ __forceinline__ float4_t split_product(typename MfmaOps<KIND>::vec8 columns, const bf16x8_t (&part)[3], float4_t c) {
+  using Ops = MfmaOps<KV_BF16>;
+  float4_t tile = {0.0f, 0.0f, 0.0f, 0.0f};
+  if constexpr (KIND == KV_BF16) {
+#pragma unroll
+    for (int i = 2; i >= 0; --i) tile = Ops::mfma(columns, part[i], tile);
+  } else {
+    uint32_t hi[4], lo[4];
+#pragma unroll
+    for (int pair = 0; pair < 4; ++pair) {
+      const float a = static_cast<float>(columns[2 * pair]), b = static_cast<float>(columns[2 * pair + 1]);
+      const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
+      hi[pair] = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
+      const float ra = a - __builtin_bit_cast(float, ua & 0xffff0000u), rb = b - __builtin_bit_cast(float, ub & 0xffff0000u);
+      lo[pair] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, rb), __builtin_bit_cast(uint32_t, ra), 0x07060302u);
+    }
+    const bf16x8_t h = __builtin_bit_cast(bf16x8_t, uint4_t{hi[0], hi[1], hi[2], hi[3]});
+    const bf16x8_t l = __builtin_bit_cast(bf16x8_t, uint4_t{lo[0], lo[1], lo[2], lo[3]});
+    tile = Ops::mfma(l, part[1], tile);
+    tile = Ops::mfma(h, part[2], tile);
+    tile = Ops::mfma(l, part[0], tile);
+    tile = Ops::mfma(h, part[1], tile);
+    tile = Ops::mfma(h, part[0], tile);
+  }
+  return c + tile;
+}
 template <int KIND>
 __device__ __forceinline__ float operand_element(uint32_t word, int hi) {
   const uint32_t bits = hi ? word >> 16 : word & 0xffffu;
@@ -128,6 +181,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
   using V8 = typename Ops::vec8;
   using T = BmTile<D>;
   constexpr int NS = D / 32, NB = D / 16;
+  constexpr bool kSplit = D > 128;
   constexpr int kRows = kBmRows;  // packed rows of the workgroup
   constexpr int kWaveRows = 16;
   // two buffers per tensor and one barrier a tile, where they fit the 64 KB of a plain launch (all but head dim 256)
@@ -270,8 +324,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
           // The reference of a row is raised only when a score of the wave exceeds its row's by more than 2^kLazy: most
           // tiles then take no lane swaps and no rescaling.  bf16 has room for probabilities up to 2^8 in dS; fp16 may
           // not (dS is packed with them), so there the reference follows every new maximum as it is.
-          constexpr float kLazy = KIND == KV_BF16 ? 8.0f : 0.0f;
-          V8 dsop;
+          constexpr float kLazy = KIND == KV_BF16 || kSplit ? 8.0f : 0.0f;
           float mt = max3_f32(sc[0][0], sc[0][1], sc[0][2]);
           mt = max3_f32(mt, sc[0][3], sc[1][0]);
           mt = max3_f32(mt, sc[1][1], sc[1][2]);
@@ -304,11 +357,17 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
               ds[tg][j] = pe * dp[tg][j];
             }
           }
-          dsop = streamed_operand<KIND>(ds);
+          if constexpr (kSplit) {
+            bf16x8_t dsop[3];
+            split_weights(ds, dsop);
 #pragma unroll
-          for (int nb = 0; nb < NB; ++nb) {
-            const V8 k_cols = tile_transposed_operand<KIND, T>(s_k, nb, lr, lk);
-            acc[nb] = Ops::mfma(k_cols, dsop, acc[nb]);
+            for (int nb = 0; nb < NB; ++nb)
+              acc[nb] = split_product<KIND>(tile_transposed_operand<KIND, T>(s_k, nb, lr, lk), dsop, acc[nb]);
+          } else {
+            const V8 dsop = streamed_operand<KIND>(ds);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+              acc[nb] = Ops::mfma(tile_transposed_operand<KIND, T>(s_k, nb, lr, lk), dsop, acc[nb]);
           }
         }
         if constexpr (kBuffers == 1) __syncthreads();  // every wave has read tile t
@@ -785,12 +844,24 @@ __global__ __launch_bounds__((DkvShape<D, KR, P>::kThreads), (DkvShape<D, KR, P>
         if (step + 1 < steps) publish(next, buf ^ 1);
         fetch(next);
         if (compute) {
-          const V8 pop = streamed_operand<KIND>(pr);
-          const V8 dsop = streamed_operand<KIND>(ds);
+          if constexpr (D > 128) {
+            bf16x8_t w[3];
+            split_weights(pr, w);
 #pragma unroll
-          for (int nb = 0; nb < NB; ++nb) {
-            acc_v[nb] = Ops::mfma(tile_transposed_operand<KIND, T>(s_g(buf), nb, lr, lk), pop, acc_v[nb]);
-            acc_k[nb] = Ops::mfma(tile_transposed_operand<KIND, T>(s_q(buf), nb, lr, lk), dsop, acc_k[nb]);
+            for (int nb = 0; nb < NB; ++nb)
+              acc_v[nb] = split_product<KIND>(tile_transposed_operand<KIND, T>(s_g(buf), nb, lr, lk), w, acc_v[nb]);
+            split_weights(ds, w);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb)
+              acc_k[nb] = split_product<KIND>(tile_transposed_operand<KIND, T>(s_q(buf), nb, lr, lk), w, acc_k[nb]);
+          } else {
+            const V8 pop = streamed_operand<KIND>(pr);
+            const V8 dsop = streamed_operand<KIND>(ds);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+              acc_v[nb] = Ops::mfma(tile_transposed_operand<KIND, T>(s_g(buf), nb, lr, lk), pop, acc_v[nb]);
+              acc_k[nb] = Ops::mfma(tile_transposed_operand<KIND, T>(s_q(buf), nb, lr, lk), dsop, acc_k[nb]);
+            }
           }
         }
         __syncthreads();  // every wave has read this step's tile, the next one is in place
@@ -941,9 +1012,9 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
     if (strcmp(e, "32") == 0) dq_rows = 32;
     if (strcmp(e, "16") == 0) dq_rows = 16;
   }
-  // Head dims 192 and 256 (the sliding-window layers of wide heads) have one shape of either kernel.  2 400 tokens in
-  // four sequences, 16 / 8 heads of 256, window 512, bf16: 323 us for both launches against 7 470 us on the
-  // vector-ALU kernels, which recompute every product on 16 lanes' dot products.
+  // Head dims 192 and 256 (the sliding-window layers of wide heads) have one shape of either kernel.  2 717 tokens in
+  // four sequences, 16 / 8 heads of 256, window 512, bf16, forward and backward: 403 us (weights kept in 32 bits, see
+  // split_weights) against 7 500 us on the vector-ALU kernels, which recompute every product on 16 lanes' dot products.
   if (p.head_dim > 128) {
     dkv_parts = 1;
     dq_rows = 16;

@@ -147,7 +147,7 @@ def test_varlen_backward_with_a_scale_that_is_not_positive(dtype, scale, d):
         _close(got, ref, REL[dtype], f"{name} {dtype} d={d} scale={scale}")
 
 
-def _c_backward(go, q, k, v, out, cu, grad_dtype, scale):
+def _c_backward(go, q, k, v, out, cu, grad_dtype, scale, window_left=-1):
     """The C entry on gradient buffers full of NaN: what it leaves unwritten shows."""
     t, hq, d = q.shape
     grads = [torch.full(x.shape, float("nan"), dtype=grad_dtype, device=DEV) for x in (q, k, v)]
@@ -155,7 +155,7 @@ def _c_backward(go, q, k, v, out, cu, grad_dtype, scale):
     ptr = lambda x: ctypes.c_void_p(x.data_ptr())  # noqa: E731
     status = cabi.lib().areno_hip_attention_backward_typed(
         *map(ptr, (go, q, k, v, out, *grads)), cabi.dtype_code(grads[0]), cabi.dtype_code(q), ctypes.c_int64(t),
-        ctypes.c_int64(k.shape[0]), hq, k.shape[1], d, ptr(cu), None, None, cu.numel() - 1, -1, ctypes.c_float(scale),
+        ctypes.c_int64(k.shape[0]), hq, k.shape[1], d, ptr(cu), None, None, cu.numel() - 1, window_left, ctypes.c_float(scale),
         ptr(workspace), ctypes.c_size_t(workspace.numel()), ctypes.c_void_p(cabi.current_stream_ptr()))  # fmt: skip
     cabi.check(status, "areno_hip_attention_backward_typed")
     return grads
@@ -177,6 +177,45 @@ def test_gradients_of_rows_behind_the_last_sequence_are_zeros(d, dq_rows, dtype,
         assert torch.isfinite(want).all()
         assert torch.equal(got[:t], want)
         assert (got[t:] == 0).all()
+
+
+def _gradients_in_64_bits(go, q, k, v, out, lens, window_left, scale):
+    """dQ, dK, dV of the packed op from the output that the forward saved (whose rounding is not the backward's)."""
+    go, q, k, v, out = (x.double().cpu() for x in (go, q, k, v, out))
+    grads = [torch.zeros_like(x) for x in (q, k, v)]
+    group, at = q.shape[1] // k.shape[1], 0
+    for n in lens:
+        rows, i = slice(at, at + n), torch.arange(n)
+        at += n
+        seen = (i[None] <= i[:, None]) & (i[None] >= i[:, None] - (n if window_left is None else window_left))
+        for h in range(q.shape[1]):
+            qh, kh, vh, gh = q[rows, h], k[rows, h // group], v[rows, h // group], go[rows, h]
+            prob = torch.softmax((scale * qh @ kh.T).masked_fill(~seen, float("-inf")), -1)
+            ds = prob * (gh @ vh.T - (gh * out[rows, h]).sum(-1, keepdim=True))
+            grads[0][rows, h] = scale * ds @ kh
+            grads[1][rows, h // group] += scale * ds.T @ qh
+            grads[2][rows, h // group] += prob.T @ gh
+    return grads
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d,window_left", [(4, 2, 256, None), (3, 3, 192, 70), (4, 1, 192, None), (2, 1, 256, 40), (2, 1, 200, None)])
+@pytest.mark.parametrize("size", [1.0, 2.0**-12, 2.0**12])
+def test_wide_heads_keep_their_weights_in_32_bits(dtype, hq, hkv, d, window_left, size):
+    """Head dims above 128 with gradients in fp32: probabilities and dS are not rounded to 16 bits on the way (2e-4 and
+    more would show), nor limited to fp16's range (a loss scaled up or down).  The bar, in the 2-norm: a score of up
+    to 2^4 in the exponent and its sum over 256 products put 2^4 * 2^-24 * a few on every weight, 4e-6."""
+    g = torch.Generator().manual_seed(d + hq)
+    lens = [300, 1, 0, 131]
+    t = sum(lens)
+    cu = torch.tensor([0, 300, 301, 301, 432], dtype=torch.int32, device=DEV)
+    q, k, v, go = (torch.randn(t, h, d, generator=g).to(dtype).to(DEV) for h in (hq, hkv, hkv, hq))
+    go = go * size
+    out = ops.areno_varlen_causal_attention(q, k, v, cu, window_left=window_left)
+    got = _c_backward(go, q, k, v, out, cu, torch.float32, d**-0.5, -1 if window_left is None else window_left)
+    for x, want, name in zip(got, _gradients_in_64_bits(go, q, k, v, out, lens, window_left, d**-0.5), ("dq", "dk", "dv")):
+        err = ((x.cpu().double() - want).norm() / want.norm()).item()
+        assert err <= 4e-6, f"{name} {dtype} d={d} window={window_left} size={size}: {err:.3g}"
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
