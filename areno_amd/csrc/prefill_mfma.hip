@@ -1082,6 +1082,11 @@ size_t prefill_mfma_workspace_bytes(int32_t kv_heads, int32_t head_dim) {
          static_cast<size_t>(2) * units * kv_heads * prefill_rows_per_wg(head_dim) * head_dim * sizeof(float);
 }
 
+// Defined in varlen_mfma.hip: packed K/V, one workgroup per query block.
+int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, int32_t dtype, int64_t tokens,
+                       int32_t q_heads, int32_t kv_heads, int32_t head_dim, const int32_t* cu_seqlens, int32_t num_seqs,
+                       int32_t window_left, float softmax_scale, void* stream);
+
 // block_table == nullptr selects packed K/V: cache->k / cache->v then point at (tokens, kv_heads, D) tensors and
 // context_lens may be nullptr (no cached context).
 int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out, int32_t q_dtype, int64_t tokens,
@@ -1139,6 +1144,11 @@ int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out
   if (workspace == nullptr || workspace_bytes < need || reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
     return fail(ARENO_ERR_WORKSPACE, "%s: workspace of %zu bytes (16-byte aligned) required, got %zu", op, need,
                 workspace_bytes);
+  if (block_table == nullptr && context_lens == nullptr) {
+    const int rc = launch_varlen_mfma(q, cache->k, cache->v, out, q_dtype, tokens, q_heads, cache->kv_heads, cache->head_dim,
+                                      cu_seqlens_q, num_seqs, window_left, softmax_scale, stream);
+    if (rc != ARENO_ERR_UNSUPPORTED) return rc;
+  }
 
   PrefillParams p;
   p.q = q;

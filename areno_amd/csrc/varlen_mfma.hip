@@ -26,14 +26,12 @@ namespace {
 constexpr int kVmWaves = 4;
 constexpr int kVmThreads = kVmWaves * kWave;
 constexpr int kVmRows = 32 * kVmWaves;  // query rows of a workgroup
-constexpr int kVmMaxSeqs = 1024;
 
 struct VarlenMfmaParams {
   const void* q;
   const void* k;
   const void* v;
   void* out;
-  float* lse;  // [tokens][q_heads], log2 domain, or nullptr
   const int32_t* cu_seqlens;
   int32_t num_seqs;
   int32_t q_heads;
@@ -331,8 +329,6 @@ __global__ __launch_bounds__(kVmThreads, 2) void varlen_mfma_kernel(VarlenMfmaPa
       *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + (row_elem + 32 * nb + 8 * c + 4 * h) * 2) = w;
     }
   }
-  if (p.lse != nullptr && h == 0)
-    p.lse[static_cast<int64_t>(q_begin + tok0 + t_row) * p.q_heads + head0 + hh] = m_run + __builtin_log2f(l_tot);
 }
 
 typedef void (*vm_fn)(VarlenMfmaParams);
@@ -353,18 +349,15 @@ VmLaunch vm_lookup(int head_dim) {
 
 }  // namespace
 
-// ARENO_ERR_UNSUPPORTED: not a launch this kernel serves
-int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, float* lse, int32_t dtype, int64_t tokens,
+// Called by launch_prefill_mfma behind its checks (types, scale, sizes, alignment, workspace), so that a packed call is
+// taken or refused, by the matrix cores or the generic kernel, as it is there.  ARENO_ERR_UNSUPPORTED: a launch for
+// the kernel of prefill_mfma.hip.
+int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, int32_t dtype, int64_t tokens,
                        int32_t q_heads, int32_t kv_heads, int32_t head_dim, const int32_t* cu_seqlens, int32_t num_seqs,
                        int32_t window_left, float softmax_scale, void* stream) {
   const char* op = "areno_hip_varlen_attention";
-  if (dtype != ARENO_DT_BF16 && dtype != ARENO_DT_F16) return ARENO_ERR_UNSUPPORTED;
-  if (!(softmax_scale > 0.0f) || num_seqs > kVmMaxSeqs || tokens > 0x3fffffff) return ARENO_ERR_UNSUPPORTED;
   const VmLaunch l = dtype == ARENO_DT_BF16 ? vm_lookup<KV_BF16>(head_dim) : vm_lookup<KV_F16>(head_dim);
   if (l.fn == nullptr) return ARENO_ERR_UNSUPPORTED;
-  for (const void* ptr : {q, k, v, static_cast<const void*>(out)}) {
-    if (reinterpret_cast<uintptr_t>(ptr) % 16 != 0) return ARENO_ERR_UNSUPPORTED;
-  }
   const int group = q_heads / kv_heads;
   const int head_parts = (group + 15) / 16;
   const int64_t vheads = static_cast<int64_t>(kv_heads) * head_parts;
@@ -375,7 +368,6 @@ int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, f
   p.k = k;
   p.v = v;
   p.out = out;
-  p.lse = lse;
   p.cu_seqlens = cu_seqlens;
   p.num_seqs = num_seqs;
   p.q_heads = q_heads;
@@ -388,7 +380,7 @@ int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, f
   p.window_left = window_left;
   p.scale_log2e = softmax_scale * kLog2e;
   const int64_t blocks = (tokens / p.block_tokens + num_seqs) * vheads;
-  if (blocks > 0x7fffffffLL) return ARENO_ERR_UNSUPPORTED;
+  if (blocks * kVmThreads > 0xffffffffLL) return ARENO_ERR_UNSUPPORTED;  // (a launch counts its work items in 32 bits)
   hipLaunchKernelGGL(l.fn, dim3(static_cast<unsigned>(blocks)), dim3(kVmThreads), l.lds_bytes,
                      static_cast<hipStream_t>(stream), p);
   return check_launch(op);

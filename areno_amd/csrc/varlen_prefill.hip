@@ -149,10 +149,6 @@ int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out
                         const int32_t* cu_seqlens_q, const int32_t* context_lens, int32_t window_left,
                         float softmax_scale, void* workspace, size_t workspace_bytes, void* stream);
 size_t prefill_mfma_workspace_bytes(int32_t kv_heads, int32_t head_dim);
-// Defined in varlen_mfma.hip: packed K/V, one workgroup per query block; ARENO_ERR_UNSUPPORTED as above.
-int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, float* lse, int32_t dtype, int64_t tokens,
-                       int32_t q_heads, int32_t kv_heads, int32_t head_dim, const int32_t* cu_seqlens, int32_t num_seqs,
-                       int32_t window_left, float softmax_scale, void* stream);
 
 }  // namespace areno
 
@@ -176,11 +172,6 @@ extern "C" int areno_hip_varlen_attention(const void* q, const void* k, const vo
     return fail(ARENO_ERR_UNSUPPORTED, "%s: dtype must be f32, f16 or bf16", op);
   if (head_dim > kMaxPerLane * kWave) return fail(ARENO_ERR_UNSUPPORTED, "%s: head_dim %d > 512", op, head_dim);
   if (tokens == 0) return ARENO_OK;
-  {
-    const int rc = launch_varlen_mfma(q, k, v, out, nullptr, dtype, tokens, q_heads, kv_heads, head_dim, cu_seqlens,
-                                      num_seqs, window_left, softmax_scale, stream);
-    if (rc != ARENO_ERR_UNSUPPORTED) return rc;
-  }
   {
     // packed K/V described as a one-block "cache" for the MFMA kernel (it addresses rows directly in this mode)
     areno_paged_cache packed = {};

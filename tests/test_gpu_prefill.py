@@ -6,6 +6,7 @@ import torch
 
 from areno_amd import workloads
 from areno_amd.accel import attention as ops
+from areno_amd.accel import cabi
 from oracle import attention_ref as ar
 from tests.gpu_util import DEV, assert_close, compact_pages, dequant_cpu, gpu_quantize, tolerances
 
@@ -340,3 +341,32 @@ def test_varlen_query_blocks_and_key_tiles(dtype, hq, hkv, d, window_left, lens)
     out = ops.areno_varlen_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV), window_left=window_left)
     want = ar.ref_varlen(q, k, v, cu, ar.window_left_arg(window_left), d**-0.5)
     assert_close(out, want, *tolerances("bf16"), what=f"varlen {hq}/{hkv} d={d} window={window_left} lens={lens[:6]}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d", [(129, 1, 64), (320, 2, 128), (136, 1, 256)])
+def test_packed_calls_of_the_generic_kernel_stay_there(dtype, hq, hkv, d):
+    """More than 128 q heads per kv head have no matrix-core launch: such calls are computed in fp32 like fp32 inputs,
+    and rounded once, bit for bit."""
+    q, k, v, cu = _packed([40, 0, 1, 90], hq, hkv, d, dtype, seed=hq)
+    q, k, v, cu = (x.to(DEV) for x in (q, k, v, cu))
+    want = ops.areno_varlen_causal_attention(q.float(), k.float(), v.float(), cu).to(dtype)
+    assert torch.equal(ops.areno_varlen_causal_attention(q, k, v, cu), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128, 192, 256, 512])
+def test_packed_calls_without_their_workspace_are_refused(dtype, d):
+    """The C entry's contract: 16-bit inputs come with the workspace that areno_hip_prefill_workspace_bytes names."""
+    q, k, v, cu = (x.to(DEV) for x in _packed([40, 9], 4, 2, d, dtype, seed=d))
+    out = torch.full_like(q, float("nan"))
+    need = cabi.prefill_workspace_bytes(2, d)
+    workspace = torch.empty(need, dtype=torch.uint8, device=DEV)
+    for ptr, size in ((None, need), (workspace.data_ptr(), need - 1), (workspace.data_ptr(), need)):
+        status = cabi.lib().areno_hip_varlen_attention(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), cabi.dtype_code(q), q.shape[0], 4, 2, d,
+            cu.data_ptr(), 2, -1, d**-0.5, ptr, size, cabi.current_stream_ptr())  # fmt: skip
+        torch.cuda.synchronize()
+        served = ptr is not None and size == need
+        assert (status == 0) == served
+        assert torch.isfinite(out).all() if served else torch.isnan(out).all()
