@@ -3,7 +3,7 @@
 //
 // A workgroup of four waves computes one query block of one kv head -- 128 rows, row r being (token r / fold, q head
 // r % fold) as in prefill_mfma.hip -- from its first visible key to its last.  No block is cut, so nothing is left
-// to merge; the blocks of a launch are taken longest first (find_block), and two workgroups share a compute unit
+// to merge; the blocks of a launch are taken longest first (varlen_blocks.hpp), and two workgroups share a compute unit
 // (four at head dim 64), so one's waits and softmax fall into the other's products.  Per step of 64 keys (32 at the wide
 // heads) a wave, which owns 32 of the rows:
 //   * passes one barrier and asks for the next step's K and V tiles, which the memory pipe writes into LDS by itself
@@ -18,7 +18,10 @@
 // per query block with nothing beside it, the partials of cut blocks (up to 67 MB written and read), a third of the
 // loop's vector instructions (staging, half the lane swaps).  Bound at length by the matrix cores and the LDS
 // reads behind them (an operand read per product), at short lengths by a block's chain of steps.
+#include <type_traits>
+
 #include "mfma32_tiles.hpp"
+#include "varlen_blocks.hpp"
 
 namespace areno {
 namespace {
@@ -41,67 +44,77 @@ struct VarlenMfmaParams {
   int32_t fold;          // row r of a block is (token r / fold, q head r % fold of the part)
   int32_t fold_magic;    // ceil(2^16 / fold)
   int32_t block_tokens;  // kVmRows / fold
+  BlockDivision block_division;
   int32_t window_left;
   float scale_log2e;
 };
 
-// What the i-th workgroup of a head computes: query block `j` of sequence `seq`.  Blocks are taken by their place in
-// their sequence, the last ones first over all sequences: a block's keys grow with its place, and a launch ends soonest
-// when the longest blocks start first.  With nb[s] blocks in sequence s, F(j) = sum over s of max(0, nb[s] - j) blocks
-// lie at place j or behind it; the i-th has the largest j with i < F(j).  Every lane holds the sequences lane,
-// lane + 64, ... and a bisection over j costs a wave-wide sum per step.
-struct BlockAt {
-  int seq, j;
-};
-__device__ __forceinline__ int wave_sum_int(int x) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m, kWave);
-  return x;
-}
-__device__ __forceinline__ int wave_max_int(int x) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) x = max(x, __shfl_xor(x, m, kWave));
-  return x;
-}
-__device__ __forceinline__ int blocks_of(const int32_t* cu, int s, int num_seqs, int tq) {
-  if (s >= num_seqs) return 0;
-  return (cu[s + 1] - cu[s] + tq - 1) / tq;
-}
-template <typename Blocks>
-__device__ __forceinline__ bool find_block(Blocks blocks, int rounds, int i, BlockAt& at) {
-  const int lane = threadIdx.x & (kWave - 1);
-  int most = 0;
-  for (int r = 0; r < rounds; ++r) most = max(most, blocks(r));
-  most = wave_max_int(most);
-  auto behind = [&](int j) {
-    int n = 0;
-    for (int r = 0; r < rounds; ++r) n += max(0, blocks(r) - j);
-    return uniform(wave_sum_int(n));
+// Whole-wave reductions of integers, by the steps of wave_max_fast
+template <typename Op>
+__device__ __forceinline__ int wave_reduce(int x, Op op) {
+  auto lanes = [](int v, auto ctrl) {
+    return __builtin_bit_cast(int, dpp_lanes<decltype(ctrl)::value>(__builtin_bit_cast(float, v)));
   };
-  if (i >= behind(0)) return false;
-  int lo = 0, hi = most;  // F(lo) > i, F(hi) = 0
-  while (lo + 1 < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (behind(mid) > i) {
-      lo = mid;
-    } else {
-      hi = mid;
-    }
+  x = op(x, lanes(x, std::integral_constant<int, kDppQuadSwap1>{}));
+  x = op(x, lanes(x, std::integral_constant<int, kDppQuadSwap2>{}));
+  x = op(x, lanes(x, std::integral_constant<int, kDppRowHalfMirror>{}));
+  x = op(x, lanes(x, std::integral_constant<int, kDppRowMirror>{}));
+  uint32_t a = static_cast<uint32_t>(x), b = a;
+  swap_rows16(a, b);
+  x = op(static_cast<int>(a), static_cast<int>(b));
+  a = b = static_cast<uint32_t>(x);
+  swap_rows32(a, b);
+  return uniform(op(static_cast<int>(a), static_cast<int>(b)));
+}
+
+// What the i-th workgroup of a head computes (block_place); false: nothing.  A lane
+// holds the blocks of sequences lane, lane + 64, ... in registers: a step of the bisection is a sum over the wave.
+// (Read again from cu_seqlens at every step, 1 024 sequences of 24 tokens, 28 / 4 heads, took 355 us instead of 159, and
+// a prefix sum by the whole workgroup, as in prefill_mfma.hip, 154.)
+struct BlockAt {
+  int j, q_begin, n_new;  // block j of the sequence whose n_new tokens start at q_begin
+};
+template <int ROUNDS>
+__device__ __forceinline__ bool find_block(const VarlenMfmaParams& p, int i, BlockAt& at) {
+  const int lane = threadIdx.x & (kWave - 1);
+  int begin[ROUNDS], tokens[ROUNDS], blocks[ROUNDS], most = 0;
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    const int s = 64 * r + lane;
+    begin[r] = p.cu_seqlens[min(s, p.num_seqs)];
+    tokens[r] = max(p.cu_seqlens[min(s + 1, p.num_seqs)] - begin[r], 0);
   }
-  int nth = i - behind(lo + 1);  // among the sequences with more than lo blocks, in order
-  for (int r = 0; r < rounds; ++r) {
-    const uint64_t has = __builtin_amdgcn_ballot_w64(blocks(r) > lo);
-    const int n = __builtin_popcountll(has);
-    if (nth < n) {
-      const bool mine = (has >> lane & 1) != 0 &&
-                        __builtin_popcountll(has & ((uint64_t{1} << lane) - 1)) == nth;
-      at.seq = 64 * r + uniform(__builtin_ctzll(__builtin_amdgcn_ballot_w64(mine)));
-      at.j = lo;
-      return true;
-    }
-    nth -= n;
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    blocks[r] = p.block_division(tokens[r] + p.block_tokens - 1);
+    most = max(most, blocks[r]);
   }
-  return false;
+  BlockPlace place;
+  const bool found = block_place(
+      i, wave_reduce(most, [](int a, int b) { return max(a, b); }),
+      [&](int j) {
+        int n = 0;
+#pragma unroll
+        for (int r = 0; r < ROUNDS; ++r) n += max(0, blocks[r] - j);
+        return wave_reduce(n, [](int a, int b) { return a + b; });
+      },
+      place);
+  if (!found) return false;
+  at.j = place.j;
+  int nth = place.nth;
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    const uint64_t has = __builtin_amdgcn_ballot_w64(blocks[r] > place.j);
+    const bool mine = (has >> lane & 1) != 0 && __builtin_popcountll(has & ((uint64_t{1} << lane) - 1)) == nth;
+    const uint64_t chosen = __builtin_amdgcn_ballot_w64(mine);
+    if (chosen != 0) {
+      const int from = __builtin_ctzll(chosen);
+      at.q_begin = __builtin_amdgcn_readlane(begin[r], from);
+      at.n_new = __builtin_amdgcn_readlane(tokens[r], from);
+    }
+    nth -= __builtin_popcountll(has);  // (below zero behind the chosen one: no lane has that rank)
+  }
+  return true;
 }
 
 extern __shared__ __attribute__((aligned(1024))) char vm_lds[];
@@ -145,18 +158,16 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
   {
     const int i = static_cast<int>(blockIdx.x / static_cast<unsigned>(vheads));
     bool found;
-    if (p.num_seqs <= kWave) {
-      const int nb = blocks_of(p.cu_seqlens, lane, p.num_seqs, tq);
-      found = find_block([&](int) { return nb; }, 1, i, at);
+    if (p.num_seqs <= 64) {
+      found = find_block<1>(p, i, at);
+    } else if (p.num_seqs <= 256) {
+      found = find_block<4>(p, i, at);
     } else {
-      found = find_block([&](int r) { return blocks_of(p.cu_seqlens, 64 * r + lane, p.num_seqs, tq); },
-                         (p.num_seqs + kWave - 1) / kWave, i, at);
+      found = find_block<16>(p, i, at);
     }
     if (!found) return;  // (the grid covers the most blocks the token count allows; the same for the whole workgroup)
   }
-  const int seq = uniform(at.seq);
-  const int q_begin = uniform(p.cu_seqlens[seq]);
-  const int n_new = uniform(p.cu_seqlens[seq + 1]) - q_begin;
+  const int q_begin = uniform(at.q_begin), n_new = uniform(at.n_new);
   const int tok0 = uniform(at.j) * tq;
   const int tok_cnt = min(tq, n_new - tok0);
 
@@ -383,6 +394,7 @@ int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, i
   p.fold = head_parts > 1 ? 16 : group;
   p.fold_magic = (65536 + p.fold - 1) / p.fold;
   p.block_tokens = kVmRows / p.fold;
+  p.block_division = block_division(p.block_tokens);
   p.window_left = window_left;
   p.scale_log2e = softmax_scale * kLog2e;
   const int64_t blocks = (tokens / p.block_tokens + num_seqs) * vheads;
