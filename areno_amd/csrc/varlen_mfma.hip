@@ -364,6 +364,28 @@ VmLaunch vm_lookup(int head_dim) {
   }
 }
 
+// Few heads over long sequences: such a launch has fewer blocks than the chip has places for, and lasts as long as its
+// longest block, one chain of steps over all its keys.  The kernel of prefill_mfma.hip, which cuts the blocks' steps
+// into equal shares and merges them, is the faster one there, us (shares, this kernel; q / kv heads):
+//   64 wide:  6 144 tokens, 1/1: 60, 76;  8 192, 2/1: 66, 101;  4 096, 3/3: 46, 52;  12 288, 4/4: 150, 153
+//             4 096, 1/1: 65, 52;  32 768, 2/1: 430, 420;  32 768, 3/3: 610, 525;  8 192, 5/1: 144, 103
+//   128 wide: 6 144, 1/1: 72, 101;  16 384, 1/1: 127, 263;  8 192, 2/1: 96, 136;  4 096, 3/3: 62, 70;  12 288, 4/4: 217, 223
+//             4 096, 1/1: 78, 69;  4 096, 4/1: 80, 70;  32 768, 3/3: 880, 791;  8 192, 5/1: 217, 146
+//   192 wide: 4 096, 1/1: 62, 101;  16 384, 2/1: 379, 381;  8 192, 3/3: 173, 198;  12 288, 3/3: 309, 300;  2 048, 1/1: 74, 55
+//   256 wide: 2 048, 2/1: 63, 77;  16 384, 1/1: 246, 542;  12 288, 3/3: 366, 418;  12 288, 4/4: 471, 453;  2 048, 5/1: 116, 78
+//   with a window: 16 384, 1/1, 256 wide, window 8 192: 206, 285;  128 wide, 4 096: 89, 77;  2/1, 256 wide, 8 192: 368, 290
+// The lengths are not known on the host: they are taken to be about equal (two of 8 192, 1/1: 100, 134; four: 134, 139).
+bool equal_shares_are_faster(int64_t tokens, int32_t num_seqs, int32_t q_heads, int32_t group, int32_t head_dim, int32_t window_left) {
+  if (static_cast<int64_t>(q_heads) * num_seqs > (group == 1 ? 4 : 3)) return false;  // chains side by side
+  const int64_t mean = tokens / num_seqs;
+  // a block sees half a sequence on the average, or all of a shorter window
+  const bool cut = window_left >= 0 && window_left + int64_t{1} < mean;
+  const int64_t length = cut ? (window_left + int64_t{1}) / 2 : mean;
+  const int64_t blocks = (cut ? 2 : 1) * tokens * q_heads / kVmRows;
+  if (head_dim <= 128) return length >= 4096 && blocks >= 48 && blocks <= 384;
+  return head_dim == 192 ? length >= 4096 && blocks <= 256 : length >= 2048 && blocks <= 320;
+}
+
 }  // namespace
 
 // Called by launch_prefill_mfma behind its checks (types, scale, sizes, alignment, workspace), so that a packed call is
@@ -376,6 +398,7 @@ int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, i
   const VmLaunch l = dtype == ARENO_DT_BF16 ? vm_lookup<KV_BF16>(head_dim) : vm_lookup<KV_F16>(head_dim);
   if (l.fn == nullptr) return ARENO_ERR_UNSUPPORTED;
   const int group = q_heads / kv_heads;
+  if (equal_shares_are_faster(tokens, num_seqs, q_heads, group, head_dim, window_left)) return ARENO_ERR_UNSUPPORTED;
   const int head_parts = (group + 15) / 16;
   const int64_t vheads = static_cast<int64_t>(kv_heads) * head_parts;
   // offsets inside a key tile are 32 bits wide

@@ -370,3 +370,18 @@ def test_packed_calls_without_their_workspace_are_refused(dtype, d):
         served = ptr is not None and size == need
         assert (status == 0) == served
         assert torch.isfinite(out).all() if served else torch.isnan(out).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens,hq,hkv,d,window_left", [
+    ([6143], 1, 1, 128, None), ([6145], 1, 1, 128, None), ([4099], 3, 3, 64, None), ([4100, 4095], 2, 2, 64, None),
+    ([4097], 2, 1, 192, None), ([2047], 2, 1, 256, None), ([2049], 2, 1, 256, None), ([4500], 1, 1, 256, 4100),
+    ([8300, 40], 1, 1, 64, None),
+])  # fmt: skip
+def test_packed_calls_of_few_heads_and_long_sequences(dtype, lens, hq, hkv, d, window_left):
+    """Launches on either side of the rule that gives few heads over long sequences to the kernel that cuts blocks into
+    equal shares.  Tolerance as in the file's other 16-bit outputs against the fp32 oracle."""
+    q, k, v, cu = _packed(lens, hq, hkv, d, dtype, seed=sum(lens))
+    out = ops.areno_varlen_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV), window_left=window_left)
+    want = ar.ref_varlen(q, k, v, cu, ar.window_left_arg(window_left), d**-0.5)
+    assert_close(out, want, *tolerances("bf16"), what=f"varlen {hq}/{hkv} d={d} window={window_left} lens={lens}")
