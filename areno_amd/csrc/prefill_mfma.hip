@@ -105,6 +105,7 @@ struct PrefillParams {
   float* part_ml;   // [2 * units][kv_heads * head_parts][rows_per_wg][2]
   float* part_acc;  // [2 * units][kv_heads * head_parts][rows_per_wg][head_dim]
   CutItem* cuts;    // [units]
+  int32_t tokens;
   int32_t num_seqs;
   int32_t q_heads;
   int32_t kv_heads;
@@ -906,6 +907,15 @@ __global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(PrefillPar
   const int tid = threadIdx.x;
   const int unit = blockIdx.x;
   const CutItem cut = p.cuts[unit];
+  const int end = p.cu_seqlens_q[p.num_seqs];
+  if (end < p.tokens) {  // rows behind the last sequence, the end of a padded pack, become zeros
+    const int64_t words = static_cast<int64_t>(p.tokens) * p.q_heads * (p.head_dim / 4);
+    const int64_t wgs = static_cast<int64_t>(gridDim.x) * gridDim.y * gridDim.z;
+    const int64_t wg = (static_cast<int64_t>(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + unit;
+    for (int64_t w = static_cast<int64_t>(end) * p.q_heads * (p.head_dim / 4) + wg * kMergeThreads + tid; w < words;
+         w += wgs * kMergeThreads)
+      *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + w * 8) = uint2_t{0u, 0u};
+  }
   if (cut.first_slot < 0) return;
   const int vhead = blockIdx.y;
   const int kvh = p.head_parts > 1 ? vhead / p.head_parts : vhead;
@@ -1160,6 +1170,7 @@ int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out
   p.block_table = block_table;
   p.cu_seqlens_q = cu_seqlens_q;
   p.context_lens = context_lens;
+  p.tokens = static_cast<int32_t>(tokens);
   p.num_seqs = num_seqs;
   p.q_heads = q_heads;
   p.kv_heads = cache->kv_heads;

@@ -16,9 +16,14 @@ namespace areno {
 struct BlockPlace {
   int j, nth;
 };
+// False: workgroup i is the nth that has no block.
 template <typename Behind>
 ARENO_HD bool block_place(int i, int most, Behind behind, BlockPlace& at) {
-  if (i >= behind(0)) return false;
+  const int all = behind(0);
+  if (i >= all) {
+    at.nth = i - all;
+    return false;
+  }
   int lo = 0, hi = most, behind_hi = 0;  // behind(lo) > i >= behind(hi)
   while (lo + 1 < hi) {
     const int mid = (lo + hi) >> 1, n = behind(mid);

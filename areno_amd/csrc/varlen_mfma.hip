@@ -36,6 +36,7 @@ struct VarlenMfmaParams {
   const void* v;
   void* out;
   const int32_t* cu_seqlens;
+  int32_t tokens;
   int32_t num_seqs;
   int32_t q_heads;
   int32_t kv_heads;
@@ -73,6 +74,7 @@ __device__ __forceinline__ int wave_reduce(int x, Op op) {
 // a prefix sum by the whole workgroup, as in prefill_mfma.hip, 154.)
 struct BlockAt {
   int j, q_begin, n_new;  // block j of the sequence whose n_new tokens start at q_begin
+  int idle;               // of a workgroup without a block: its place among those
 };
 template <int ROUNDS>
 __device__ __forceinline__ bool find_block(const VarlenMfmaParams& p, int i, BlockAt& at) {
@@ -99,7 +101,10 @@ __device__ __forceinline__ bool find_block(const VarlenMfmaParams& p, int i, Blo
         return wave_reduce(n, [](int a, int b) { return a + b; });
       },
       place);
-  if (!found) return false;
+  if (!found) {
+    at.idle = place.nth;
+    return false;
+  }
   at.j = place.j;
   int nth = place.nth;
 #pragma unroll
@@ -165,7 +170,20 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
     } else {
       found = find_block<16>(p, i, at);
     }
-    if (!found) return;  // (the grid covers the most blocks the token count allows; the same for the whole workgroup)
+    if (!found) {
+      // (the same for the whole workgroup; the grid covers the most blocks the token count allows and one more).  Rows
+      // behind the last sequence -- the end of a padded pack -- become zeros, over the workgroups that have no block
+      const int end = p.cu_seqlens[p.num_seqs], rest = p.tokens - end;
+      if (rest <= 0) return;
+      const int idle = static_cast<int>(gridDim.x / static_cast<unsigned>(vheads)) - i + at.idle;  // so many
+      const int per_token = group_here * (D / 4);
+      const int64_t words = static_cast<int64_t>(rest) * per_token;
+      for (int64_t w = at.idle * kVmThreads + tid; w < words; w += static_cast<int64_t>(idle) * kVmThreads) {
+        const int64_t elem = ((end + w / per_token) * p.q_heads + head0) * D + 4 * (w % per_token);
+        *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + elem * 2) = uint2_t{0u, 0u};
+      }
+      return;
+    }
   }
   const int q_begin = uniform(at.q_begin), n_new = uniform(at.n_new);
   const int tok0 = uniform(at.j) * tq;
@@ -409,6 +427,7 @@ int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, i
   p.v = v;
   p.out = out;
   p.cu_seqlens = cu_seqlens;
+  p.tokens = static_cast<int32_t>(tokens);
   p.num_seqs = num_seqs;
   p.q_heads = q_heads;
   p.kv_heads = kv_heads;
@@ -420,7 +439,7 @@ int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, i
   p.block_division = block_division(p.block_tokens);
   p.window_left = window_left;
   p.scale_log2e = softmax_scale * kLog2e;
-  const int64_t blocks = (tokens / p.block_tokens + num_seqs) * vheads;
+  const int64_t blocks = (tokens / p.block_tokens + num_seqs + 1) * vheads;
   if (blocks * kVmThreads > 0xffffffffLL) return ARENO_ERR_UNSUPPORTED;  // (a launch counts its work items in 32 bits)
   hipLaunchKernelGGL(l.fn, dim3(static_cast<unsigned>(blocks)), dim3(kVmThreads), l.lds_bytes,
                      static_cast<hipStream_t>(stream), p);

@@ -29,15 +29,15 @@ extern "C" int varlen_blocks_check(const int* lens, int num_seqs, int block, cha
   std::vector<std::vector<int>> seen(num_seqs);
   for (int s = 0; s < num_seqs; ++s) seen[s].assign(nb[s], 0);
   int last = most;
-  const int grid = tokens / block + num_seqs;
-  if (grid < all) {
+  const int grid = tokens / block + num_seqs + 1;
+  if (grid <= all) {
     snprintf(msg, msg_len, "grid of %d for %d blocks", grid, all);
     return 1;
   }
   for (int i = 0; i < grid; ++i) {
     areno::BlockPlace at;
     const bool found = areno::block_place(i, most, behind, at);
-    if (found != (i < all)) {
+    if (found != (i < all) || (!found && at.nth != i - all)) {
       snprintf(msg, msg_len, "workgroup %d of %d blocks: found %d", i, all, found);
       return 1;
     }

@@ -385,3 +385,42 @@ def test_packed_calls_of_few_heads_and_long_sequences(dtype, lens, hq, hkv, d, w
     out = ops.areno_varlen_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV), window_left=window_left)
     want = ar.ref_varlen(q, k, v, cu, ar.window_left_arg(window_left), d**-0.5)
     assert_close(out, want, *tolerances("bf16"), what=f"varlen {hq}/{hkv} d={d} window={window_left} lens={lens}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("lens,hq,hkv,d", [
+    ([5, 0, 130], 7, 1, 64), ([128, 127], 6, 6, 128), ([1], 4, 2, 128), ([60], 4, 4, 192), ([40, 33], 20, 1, 256),
+    ([90, 7], 4, 2, 512), ([30], 4, 2, 96), ([2] * 70, 28, 4, 128), ([0, 0], 3, 1, 64), ([2100], 2, 1, 256),
+])  # fmt: skip
+@pytest.mark.parametrize("behind", [1, 37, 1500])
+def test_rows_behind_the_last_sequence_are_zeros(dtype, lens, hq, hkv, d, behind):
+    """A padded pack (``cu_seqlens[-1]`` below the tokens): the output's last rows are written, as zeros, whatever their
+    inputs hold, and the others are what they are without the padding."""
+    q, k, v, cu = (x.to(DEV) for x in _packed(lens, hq, hkv, d, dtype, seed=d))
+    want = ops.areno_varlen_causal_attention(q, k, v, cu) if sum(lens) else q
+    pads = [torch.full((behind, *x.shape[1:]), float("nan"), dtype=dtype, device=DEV) for x in (q, k, v)]
+    q, k, v = (torch.cat(pair) for pair in zip((q, k, v), pads))
+    out = torch.full_like(q, float("nan"))
+    workspace = torch.empty(cabi.prefill_workspace_bytes(hkv, d), dtype=torch.uint8, device=DEV)
+    cabi.check(cabi.lib().areno_hip_varlen_attention(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), cabi.dtype_code(q), q.shape[0], hq, hkv, d,
+        cu.data_ptr(), len(lens), -1, d**-0.5, workspace.data_ptr(), workspace.numel(), cabi.current_stream_ptr()), "varlen")  # fmt: skip
+    assert (out[sum(lens) :] == 0).all()
+    if sum(lens):
+        assert_close(out[: sum(lens)], want.cpu().float(), *tolerances("bf16"), what="rows in front of the padding")
+
+
+@pytest.mark.parametrize("kv", ["bf16", "int8"])
+@pytest.mark.parametrize("d,page", [(128, 16), (256, 24), (512, 16), (96, 16)])
+@pytest.mark.parametrize("behind", [1, 600])
+def test_paged_rows_behind_the_last_sequence_are_zeros(kv, d, page, behind):
+    new, ctx = torch.tensor([3, 150, 0, 33]), torch.tensor([900, 0, 77, 31])
+    w = workloads.make_prefill_workload("padded", seed=d, new_lens=new, ctx_lens=ctx, hq=8, hkv=2, d=d, bs=page, kv=kv,
+                                        device=DEV, quantize_fn=gpu_quantize)  # fmt: skip
+    q = torch.cat([w.q, torch.full((behind, *w.q.shape[1:]), float("nan"), dtype=w.q.dtype, device=DEV)])
+    out = torch.full_like(q, float("nan"))
+    workspace = torch.empty(cabi.prefill_workspace_bytes(2, d), dtype=torch.uint8, device=DEV)
+    cache = cabi.describe_cache(w.k_cache, w.v_cache, w.k_scale, w.v_scale)
+    cabi.check(cabi.paged_varlen_prefill(cache, q, out, w.block_table, w.cu_seqlens_q, w.context_lens, workspace), "prefill")
+    assert (out[w.q.shape[0] :] == 0).all()
+    assert_close(out[: w.q.shape[0]], _run_prefill(w).cpu().float(), *tolerances(kv), what="rows in front of the padding")
