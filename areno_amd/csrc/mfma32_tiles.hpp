@@ -77,10 +77,11 @@ struct LdsTile {
 };
 
 // One wave instruction that moves 64 chunks of 16 bytes from memory into LDS: lane l's chunk, at base + offset,
-// lands at lds + 16 l.  Asm, so that the compiler does not wait for it at the next LDS read: the caller waits
-// (fetched_barrier) before anything is read and leaves none in flight at the kernel's end.
+// lands at lds + 16 l (in m0: an operand, so that the compiler knows).  Asm, so that the compiler does not wait for it at
+// the next LDS read: the caller waits (fetched_barrier) before anything is read and leaves none in flight at the
+// kernel's end.
 __device__ __forceinline__ void fetch_to_lds(const char* base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(offset), "s"(base) : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "{m0}"(lds) : "memory");
 }
 // The wave's fetches have landed and its LDS reads are in registers; then every wave's have: the tiles asked for may be
 // read and the tiles read so far may be fetched over.
