@@ -130,11 +130,12 @@ struct PrefillParams {
   float scale_log2e;
 };
 
-// Exclusive prefix sum of tile steps per sequence into s_cum[0 .. num_seqs] (all threads take part).  A launch seldom
+// Exclusive prefix sum of tile steps per sequence into s_cum[0 .. num_seqs] (all threads take part), and where the last
+// sequence ends.  A launch seldom
 // has more sequences than the workgroup has threads, and the loops stay rolled: this runs once per workgroup, on code
 // that has to be fetched first (4 sequences of up to 64 new and 4 k cached tokens, 7 q heads per kv head: the kernel
 // 26.7 -> 25.6 us against a copy of the closed forms per sequence of a thread).
-__device__ __forceinline__ void prefix_tile_steps(const PrefillParams& p, int tq, int* s_cum, int* s_wave_tot) {
+__device__ __forceinline__ void prefix_tile_steps(const PrefillParams& p, int tq, int* s_cum, int* s_wave_tot, int* s_end) {
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = tid >> 6;
@@ -143,10 +144,12 @@ __device__ __forceinline__ void prefix_tile_steps(const PrefillParams& p, int tq
   int local = 0;
 #pragma unroll 1
   for (int s = first; s < last; ++s) {
-    const int n_new = p.cu_seqlens_q[s + 1] - p.cu_seqlens_q[s];
+    const int end = p.cu_seqlens_q[s + 1];
+    const int n_new = end - p.cu_seqlens_q[s];
     const int ctx = p.context_lens != nullptr ? p.context_lens[s] : 0;
     const int steps = sequence_steps(n_new, ctx, tq, p.window_left);
     s_cum[s] = steps;
+    if (s + 1 == p.num_seqs) *s_end = end;
     local += steps;
   }
   int incl = local;
@@ -272,6 +275,7 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
   __shared__ __attribute__((aligned(16))) char s_v[2][TK * RSV];
   __shared__ int s_cum[kMaxPrefillSeqs + 1];
   __shared__ int s_wave_tot[kPrefillWaves];
+  __shared__ int s_end;
   __shared__ StepPos s_first;
   // score parts of a split head: [wave][tg][j][lane]
   __shared__ float s_part[DS > 1 ? kPrefillWaves : 1][2][4][DS > 1 ? kWave : 1];
@@ -293,7 +297,15 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
   const int unit = blockIdx.x;
   const int tq = p.block_tokens;  // query tokens per item
 
-  prefix_tile_steps(p, tq, s_cum, s_wave_tot);
+  prefix_tile_steps(p, tq, s_cum, s_wave_tot, &s_end);
+  if (s_end < p.tokens) {
+    // rows behind the last sequence, the end of a padded pack, become zeros.  (Here, where the sequences' ends have been
+    // read; a read of its own cost the merge 0.4 us.)
+    const int64_t words_per_row = static_cast<int64_t>(p.q_heads) * (D / 4), words = p.tokens * words_per_row;
+    const int64_t wg = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x, wgs = static_cast<int64_t>(gridDim.x) * gridDim.y;
+    for (int64_t w = s_end * words_per_row + wg * kPrefillThreads + tid; w < words; w += wgs * kPrefillThreads)
+      *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + w * 8) = uint2_t{0u, 0u};
+  }
   const int total = s_cum[p.num_seqs];
   const int x_begin = unit_start_step(total, unit, p.units);
   const int x_end = unit_start_step(total, unit + 1, p.units);
@@ -907,15 +919,6 @@ __global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(PrefillPar
   const int tid = threadIdx.x;
   const int unit = blockIdx.x;
   const CutItem cut = p.cuts[unit];
-  const int end = p.cu_seqlens_q[p.num_seqs];
-  if (end < p.tokens) {  // rows behind the last sequence, the end of a padded pack, become zeros
-    const int64_t words = static_cast<int64_t>(p.tokens) * p.q_heads * (p.head_dim / 4);
-    const int64_t wgs = static_cast<int64_t>(gridDim.x) * gridDim.y * gridDim.z;
-    const int64_t wg = (static_cast<int64_t>(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + unit;
-    for (int64_t w = static_cast<int64_t>(end) * p.q_heads * (p.head_dim / 4) + wg * kMergeThreads + tid; w < words;
-         w += wgs * kMergeThreads)
-      *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + w * 8) = uint2_t{0u, 0u};
-  }
   if (cut.first_slot < 0) return;
   const int vhead = blockIdx.y;
   const int kvh = p.head_parts > 1 ? vhead / p.head_parts : vhead;
