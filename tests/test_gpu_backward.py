@@ -104,11 +104,11 @@ def test_varlen_backward_of_wide_heads_on_the_matrix_core_kernels(dtype, hq, hkv
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("hq,hkv,d,dq_rows", [(4, 2, 64, "16"), (4, 2, 128, "16"), (4, 2, 128, "32"), (2, 1, 256, "16")])
+@pytest.mark.parametrize("hq,hkv,d,dq_rows", [(4, 2, 64, "16"), (4, 2, 64, "32"), (4, 2, 128, "16"), (4, 2, 128, "32"), (3, 3, 192, "16"), (2, 1, 256, "16")])
 @pytest.mark.parametrize("falling", [False, True])
 def test_varlen_backward_where_the_softmax_reference_moves(dtype, hq, hkv, d, dq_rows, falling, monkeypatch):
     """Keys whose scores grow along the sequence (spread 0.2 to 8: by more than 2^8 within a row, several times, and by
-    less in other tiles) or fall, over an odd number of tiles and a single one: the dq kernel's lazily raised
+    less in other tiles) or fall along it, over an odd number of tiles and a single one: the dq kernel's lazily raised
     reference.  The bar is the file's: the gradients' largest values come from single keys, whose probabilities and
     products round as everywhere."""
     monkeypatch.setenv("ARENO_BACKWARD_DQ_ROWS", dq_rows)
@@ -116,9 +116,10 @@ def test_varlen_backward_where_the_softmax_reference_moves(dtype, hq, hkv, d, dq
     lens = [321, 30, 0, 65]
     t = sum(lens)
     cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
-    ramp = torch.cat([torch.linspace(0.2, 8.0, n) for n in lens])[:, None, None]
+    first, last = (8.0, 0.2) if falling else (0.2, 8.0)
+    ramp = torch.cat([torch.linspace(first, last, n) for n in lens])[:, None, None]
     q, k, v, go = (torch.randn(t, h, d, generator=g) for h in (hq, hkv, hkv, hq))
-    k = k * (ramp.flip(0) if falling else ramp)
+    k = k * ramp
     q, k, v, go = (x.to(dtype) for x in (q, k, v, go))
     qd, kd, vd = (x.to(DEV).requires_grad_(True) for x in (q, k, v))
     ops.areno_varlen_causal_attention(qd, kd, vd, cu.to(DEV)).backward(go.to(DEV))
