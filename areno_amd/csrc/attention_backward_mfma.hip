@@ -60,11 +60,6 @@ __device__ __forceinline__ int seq_of_row(const int32_t* cu, int num_seqs, int64
   return lo;
 }
 
-// a query row in front of the first sequence or behind the last (the end of a padded pack): no keys, a gradient of zeros
-__device__ __forceinline__ bool row_of_no_sequence(const BwdParams& p, int64_t row) {
-  return row < p.q_tokens && (row >= p.cu_q[p.num_seqs] || row < p.cu_q[0]);
-}
-
 // A tile of 32 rows x D 16-bit elements in LDS, row stride D * 2 + 16 bytes: the row operands (16 lanes read the same
 // 16-byte chunk of 16 rows) meet every bank once, the transposed ones (32 lanes read 32 bytes of 8 consecutive rows)
 // meet every bank twice.  (A layout without any bank conflict -- rows back to back, the chunks of a row permuted by
@@ -203,8 +198,10 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
   int64_t row;  // this lane's query rows (columns of the products)
   row = wave_row0 + lr;
 
+  int64_t covered = 0;  // the rows in front of it belong to sequences
   for (int s = seq_of_row(p.cu_q, p.num_seqs, r0); s < p.num_seqs; ++s) {
     const int64_t sq0 = p.cu_q[s], sq1 = p.cu_q[s + 1];
+    covered = sq0 >= block_end ? block_end : sq1;
     if (sq0 >= block_end) break;
     const int64_t q_lo = sq0 > r0 ? sq0 : r0, q_hi = sq1 < block_end ? sq1 : block_end;
     if (q_lo >= q_hi) continue;
@@ -402,7 +399,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
       }
     }
   }
-  if (row_of_no_sequence(p, row)) {
+  if (row >= covered && row < p.q_tokens) {  // behind the last sequence, the end of a padded pack
     const int64_t row_elem = (row * p.q_heads + h) * D;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) store_grad4(p.grad_q, row_elem + 4 * lk + 16 * nb, 0.0f, 0.0f, 0.0f, 0.0f, p.grad_dtype);
@@ -448,8 +445,10 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
     fetch_chunk[f] = static_cast<uint32_t>((slot % T::kChunksPerRow) ^ T::twist(fetch_row[f])) * 16u;
   }
 
+  int64_t covered = 0;  // the rows in front of it belong to sequences
   for (int s = uniform(seq_of_row(p.cu_q, p.num_seqs, r0)); s < p.num_seqs; ++s) {
     const int64_t sq0 = uniform(p.cu_q[s]), sq1 = uniform(p.cu_q[s + 1]);
+    covered = sq0 >= block_end ? block_end : sq1;
     if (sq0 >= block_end) break;
     const int64_t q_lo = sq0 > r0 ? sq0 : r0, q_hi = sq1 < block_end ? sq1 : block_end;
     if (q_lo >= q_hi) continue;
@@ -617,7 +616,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
       }
     }
   }
-  if (row_of_no_sequence(p, row)) {
+  if (row >= covered && row < p.q_tokens) {  // behind the last sequence, the end of a padded pack
     const int64_t row_elem = (row * p.q_heads + h) * D;
 #pragma unroll
     for (int c = 0; c < D / 8; ++c) store_grad4(p.grad_q, row_elem + 8 * c + 4 * half, 0.0f, 0.0f, 0.0f, 0.0f, p.grad_dtype);
