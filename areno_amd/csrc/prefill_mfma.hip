@@ -89,7 +89,8 @@ struct CutItem {
   int32_t step_end;    // the item's steps end in front of this one
   int32_t token0;      // its first query token's row of q / out
   int32_t tokens;
-  int32_t unused[3];
+  int32_t end;  // where the last sequence ends (also in units without anything to merge)
+  int32_t unused[2];
 };
 
 struct PrefillParams {
@@ -298,19 +299,14 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
   const int tq = p.block_tokens;  // query tokens per item
 
   prefix_tile_steps(p, tq, s_cum, s_wave_tot, &s_end);
-  if (s_end < p.tokens) {
-    // rows behind the last sequence, the end of a padded pack, become zeros.  (Here, where the sequences' ends have been
-    // read; a read of its own cost the merge 0.4 us.)
-    const int64_t words_per_row = static_cast<int64_t>(p.q_heads) * (D / 4), words = p.tokens * words_per_row;
-    const int64_t wg = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x, wgs = static_cast<int64_t>(gridDim.x) * gridDim.y;
-    for (int64_t w = s_end * words_per_row + wg * kPrefillThreads + tid; w < words; w += wgs * kPrefillThreads)
-      *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + w * 8) = uint2_t{0u, 0u};
-  }
   const int total = s_cum[p.num_seqs];
   const int x_begin = unit_start_step(total, unit, p.units);
   const int x_end = unit_start_step(total, unit + 1, p.units);
   if (x_begin >= x_end) {  // same for the whole workgroup
-    if (vhead == 0 && tid == 0) p.cuts[unit].first_slot = -1;
+    if (vhead == 0 && tid == 0) {
+      p.cuts[unit].first_slot = -1;
+      p.cuts[unit].end = s_end;
+    }
     return;
   }
 
@@ -354,11 +350,16 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
     cut.total = total;
     cut.token0 = pos.q_begin + item.tok0;
     cut.tokens = item.cnt;
+    cut.end = s_end;
     p.cuts[unit] = cut;
   }
   if (tid == 0) s_first = pos;
   __syncthreads();
   if (looks_at_end) pos = s_first;
+  // (the same in every lane, and told so where vector registers are short: 1 024 sequences of 3 tokens, 16 heads of 512,
+  // 619 -> 593 us; at the other head dims the scalar registers it takes are missed more, by up to 4 %)
+  if constexpr (D > 256)
+    pos = {uniform(pos.seq), uniform(pos.j), uniform(pos.tile), uniform(pos.n_new), uniform(pos.ctx), uniform(pos.q_begin), uniform(pos.item_x0)};
 
   // What the staging steps ask block ids for: the item whose tiles are being fetched.  It is switched to the next
   // item before the current item's output is stored (see the end of the item loop).
@@ -919,6 +920,13 @@ __global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(PrefillPar
   const int tid = threadIdx.x;
   const int unit = blockIdx.x;
   const CutItem cut = p.cuts[unit];
+  if (cut.end < p.tokens) {  // rows behind the last sequence, the end of a padded pack, become zeros
+    const int64_t words_per_row = static_cast<int64_t>(p.q_heads) * (p.head_dim / 4), words = p.tokens * words_per_row;
+    const int64_t wgs = static_cast<int64_t>(gridDim.x) * gridDim.y * gridDim.z;
+    const int64_t wg = (static_cast<int64_t>(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + unit;
+    for (int64_t w = cut.end * words_per_row + wg * kMergeThreads + tid; w < words; w += wgs * kMergeThreads)
+      *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + w * 8) = uint2_t{0u, 0u};
+  }
   if (cut.first_slot < 0) return;
   const int vhead = blockIdx.y;
   const int kvh = p.head_parts > 1 ? vhead / p.head_parts : vhead;
