@@ -6,10 +6,10 @@
 //                the keys its rows may see in tiles of 32 through LDS.  Per tile, with the keys as the rows of the products (the
 //                layout of the forward kernel):  S^T = K . Q^T  and  dP^T = V . dO^T  (two products per 16 keys and 32
 //                elements of the head), the online softmax of the forward on S^T, dS^T = P^T * (dP^T - dO . O), and
-//                dQ^T += K^T . dS^T  with the lane's own dS^T values as the B operand and K^T read transposed from the
-//                same LDS tile.  A row's softmax reference moves as in the forward (the accumulator is rescaled), so
+//                dQ^T += K^T . dS^T  with the lane's own dS^T values as the B operand (rounded to the inputs' type; at
+//                the wide heads not rounded, split_weights) and K^T read transposed from the same LDS tile.  A row's softmax reference moves as in the forward (the accumulator is rescaled), so
 //                one pass over the keys gives dQ, the row's log-sum-exp and dO . O (left in the workspace).
-//   dkv kernel   a workgroup owns 64 or 32 packed key rows of one kv head (16 per wave) and streams, for every q head
+//   dkv kernel   a workgroup owns 32 to 128 packed key rows of one kv head (16 per wave) and streams, for every q head
 //                of the group, the query rows that may see them in tiles of 32 (Q and dO tiles in LDS, the rows'
 //                statistics next to them):  S = Q . K^T,  dP = dO . V^T,  P = exp2(S - lse),  dS = P * (dP - dO . O),
 //                dV^T += dO^T . P  and  dK^T += Q^T . dS.  Every gradient element has one owner; in a small launch
@@ -169,7 +169,7 @@ __device__ __forceinline__ float operand_element(uint32_t word, int hi) {
 // Bound by what a wave issues and waits for between its products, so a tile has one barrier (two LDS buffers), a
 // row's softmax reference mostly stays where it is (no lane swaps, no rescaling), and dP - dO . O comes out of the
 // product, which starts at -(dO . O); the dkv kernel's does too (forward and backward of 2 x 2 048 tokens, 28 / 4 heads of
-// 128, bf16: 435 -> 427 us; heads of 256, whose buffers do not fit twice: within the noise).
+// 128, bf16: 435 -> 427 us; heads of 256, which have one buffer and two barriers: within the noise).
 template <int KIND, int D>
 __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p) {
   using Ops = MfmaOps<KIND>;
@@ -179,7 +179,8 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
   constexpr bool kSplit = D > 128;
   constexpr int kRows = kBmRows;  // packed rows of the workgroup
   constexpr int kWaveRows = 16;
-  // two buffers per tensor and one barrier a tile, where they fit the 64 KB of a plain launch (all but head dim 256)
+  // two buffers per tensor and one barrier a tile, where they fit the 64 KB of a plain launch: all but head dim 256,
+  // whose padded rows make 66 KB of them (the unpadded tiles of mfma32_tiles.hpp would make 64; not built for this kernel)
   constexpr int kBuffers = 4 * kBmTile * T::RS <= 64 * 1024 ? 2 : 1;
   __shared__ __attribute__((aligned(16))) char k_lds[kBuffers * kBmTile * T::RS];
   __shared__ __attribute__((aligned(16))) char v_lds[kBuffers * kBmTile * T::RS];
@@ -198,10 +199,9 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
   int64_t row;  // this lane's query rows (columns of the products)
   row = wave_row0 + lr;
 
-  int64_t covered = 0;  // the rows in front of it belong to sequences
+  int covered = 0;  // (where the sequences seen so far end)
   for (int s = seq_of_row(p.cu_q, p.num_seqs, r0); s < p.num_seqs; ++s) {
-    const int64_t sq0 = p.cu_q[s], sq1 = p.cu_q[s + 1];
-    covered = sq0 >= block_end ? block_end : sq1;
+    const int64_t sq0 = p.cu_q[s], sq1 = covered = p.cu_q[s + 1];
     if (sq0 >= block_end) break;
     const int64_t q_lo = sq0 > r0 ? sq0 : r0, q_hi = sq1 < block_end ? sq1 : block_end;
     if (q_lo >= q_hi) continue;
@@ -409,7 +409,8 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
 // The same with 32 query rows per wave, 128 per workgroup, on 32 x 32 x 16 products, for launches that fill the chip with
 // such workgroups: an operand read from LDS serves a product of twice the size, the K and V tiles are fetched straight
 // into LDS (mfma32_tiles.hpp).  Bound by the matrix cores and the LDS reads behind them.  Against a 16 x 16 form of as
-// many rows, which spilled 84 registers: the backward of 4 x 4 096 tokens, 32 / 8 heads of 128, bf16: 2 646 -> 2 283 us.
+// many rows: the backward of 4 x 4 096 tokens, 32 / 8 heads of 128, bf16: 2 646 -> 2 283 us.  (That form spilled 84 registers;
+// this one spills 26 at head dim 128, once per sequence of a block and not in the tile loop.)
 template <int KIND, int D>
 __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams p) {
   using M = Mfma32<KIND>;
@@ -445,10 +446,9 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
     fetch_chunk[f] = static_cast<uint32_t>((slot % T::kChunksPerRow) ^ T::twist(fetch_row[f])) * 16u;
   }
 
-  int64_t covered = 0;  // the rows in front of it belong to sequences
+  int covered = 0;  // (where the sequences seen so far end)
   for (int s = uniform(seq_of_row(p.cu_q, p.num_seqs, r0)); s < p.num_seqs; ++s) {
-    const int64_t sq0 = uniform(p.cu_q[s]), sq1 = uniform(p.cu_q[s + 1]);
-    covered = sq0 >= block_end ? block_end : sq1;
+    const int64_t sq0 = uniform(p.cu_q[s]), sq1 = covered = uniform(p.cu_q[s + 1]);
     if (sq0 >= block_end) break;
     const int64_t q_lo = sq0 > r0 ? sq0 : r0, q_hi = sq1 < block_end ? sq1 : block_end;
     if (q_lo >= q_hi) continue;
@@ -624,7 +624,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
 }
 
 // ---- dK, dV -------------------------------------------------------------------------------------------------------------
-// A workgroup owns a block of KR packed key rows of one kv head, or two of them one after the other: block i and
+// A workgroup owns a block of KR (32, 64, or 96 and 128 at the wide heads) packed key rows of one kv head, or two of them one after the other: block i and
 // block blocks - 1 - i.  A key block early in its sequence is seen by all later queries and one late in it by few.
 // A launch of many workgroups per compute unit evens that out by starting the expensive blocks first
 // (block_in_cost_order); in a launch of about one workgroup per unit nothing comes after the expensive block to
@@ -634,7 +634,8 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
 // step of the stream of query tiles (tiles and statistics of its own in LDS); the sums of parts 1 .. P - 1 go to
 // part 0 through LDS at the end of a block, in a fixed order.  More parts shorten the chain of steps a block is:
 // (KR, P) = (64, 1) four waves, two workgroups per compute unit, for launches that fill the units several times;
-// (64, 2) and (32, 4) eight waves, for launches of about one workgroup per unit.
+// (64, 2) and (32, 4) eight waves, for launches of about one workgroup per unit; (96, 1) and (128, 1) six and eight waves
+// at head dims 192 and 256.
 template <int D, int KR, int P>
 struct DkvShape {
   static constexpr int kKeyWaves = KR / 16;
@@ -951,8 +952,9 @@ DkvLaunch dkv_launch() {
   return DkvLaunch{fn, L::kLdsBytes, L::kThreads, KR};
 }
 // Head dims 192 and 256 have one shape: the sums and operands of 16 key rows take all registers of two waves per SIMD,
-// and six or eight waves behind one stream of tiles stage two chunks of a tensor per thread and step (four waves:
-// four chunks, which the registers have no room for).
+// and six or eight waves behind one stream of tiles stage two chunks of a tensor per thread and step (with four waves it
+// would be four chunks, twice the staging registers).  At 256 the kernel still keeps some of its staging in scratch, a
+// dozen loads and half as many stores in every two steps of the tile loop; at 192 a few registers, outside it.
 template <int KIND, int D>
 DkvLaunch dkv_launch(int parts) {
   if constexpr (D > 128) return dkv_launch<KIND, D, D == 256 ? 128 : 96, 1>();
@@ -1000,13 +1002,19 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
     if (strcmp(e, "4") == 0) dkv_parts = 4;
   }
   // The dq kernel with 32 rows per wave once the launch has 6 workgroups of 64 rows per compute unit at head dim 128, 8
-  // at head dim 64.  The backward, 16 -> 32 rows, us: D = 128: 4 x 4 096 tokens, 32 / 8 heads (32 per unit) 2 646 ->
-  // 2 283; 1 x 4 096, 28 / 4 heads (7) 639 -> 561; 8 x 512, 28 / 4 heads (7) 133 -> 130; 4 x 600, 32 / 8 heads (4.6)
-  // 161 -> 163; 1 x 1 024, 8 / 2 heads (0.5) 94 -> 105.  D = 64: 4 x 4 096, 32 / 8 heads (32) 1 357 -> 1 240; 2 x 4 096,
-  // 16 heads (8) 365 -> 342; 8 x 512, 28 / 4 heads (7) 72 -> 75; 16 x 310, 16 heads (4.8) 62 -> 69.  Small launches
-  // want the more and shorter workgroups.
+  // at head dim 64, and the sequences are long enough (512 and 1 024 tokens on the average).  The backward, 16 -> 32 rows,
+  // us: D = 128: 4 x 4 096 tokens, 32 / 8 heads (32 per unit) 2 646 -> 2 283; 1 x 4 096, 28 / 4 heads (7) 639 -> 561;
+  // 64 x 512 (56) 946 -> 896; 8 x 512 (7) 135 -> 132; 4 x 600, 32 / 8 heads (4.6) 161 -> 163; 1 x 1 024, 8 / 2 heads (0.5)
+  // 94 -> 105.  D = 64: 4 x 4 096, 32 / 8 heads (32) 1 357 -> 1 240; 2 x 4 096, 16 heads (8) 365 -> 342; 32 x 1 024, 28 / 4
+  // (56) 776 -> 737; 16 x 310, 16 heads (4.8) 62 -> 69.  Small launches want the more and shorter workgroups, and a block
+  // of many short sequences, which it takes one after the other, is a longer chain in the larger block: 28 / 4 heads of
+  // 128, 512 x 8 tokens (7) 187 -> 253, 64 x 64 70 -> 80, 256 x 128 (56) 553 -> 570, 16 x 256 (7) 119 -> 119; of 64,
+  // 1 024 x 8 (14) 158 -> 272, 256 x 128 (56) 265 -> 294, 64 x 512 482 -> 478, 16 x 512 (14) 136 -> 139.
   // ARENO_BACKWARD_DQ_ROWS=16|32 (read at every launch) fixes the choice, for tests and timing.
-  int dq_rows = q_blocks * p.q_heads >= (p.head_dim == 128 ? 6 : 8) * kBmComputeUnits ? 32 : 16;
+  const int64_t mean_length = p.q_tokens / (p.num_seqs > 0 ? p.num_seqs : 1);
+  int dq_rows = q_blocks * p.q_heads >= (p.head_dim == 128 ? 6 : 8) * kBmComputeUnits && mean_length >= (p.head_dim == 128 ? 512 : 1024)
+                    ? 32
+                    : 16;
   if (const char* e = getenv("ARENO_BACKWARD_DQ_ROWS")) {
     if (strcmp(e, "32") == 0) dq_rows = 32;
     if (strcmp(e, "16") == 0) dq_rows = 16;
