@@ -29,6 +29,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -965,6 +966,36 @@ DkvLaunch dkv_launch(int parts) {
   }
 }
 
+// Whether the vector-ALU kernels take a launch of wide heads in less time.  A matrix-core workgroup goes through the
+// sequences of its block one after the other, at least one tile each (the dkv kernel for every q head of the group);
+// the vector-ALU kernels have a wave per row and do not care.  For sequences of 64 tokens and more the matrix cores
+// win by up to 30 times, for many single tokens they lose by as much; in between both are estimated, in us, from what
+// 624 launches took (head dims 192 and 256, both types, 1 .. 512 sequences of 1 .. 64 tokens, six head ratios: the one
+// taken is at most 8 % slower than the other).  vector ALU, matrix cores, in us: 64 sequences of 1 token, 32 / 1 heads
+// of 256, bf16: 82, 9 035; 512 x 4 tokens, 8 / 1 heads of 192, fp16: 346, 914; 8 x 32, 16 / 1 of 256, bf16: 286, 316; 64 x 16,
+// 16 heads of 256, bf16: 834, 121; 1 token, 8 / 1 heads of 256, fp16: 54, 70, bf16: 51, 51; 300 tokens: 801, 441.
+bool vector_alu_is_faster(const BwdParams& p, int key_rows) {
+  const bool d256 = p.head_dim == 256, fp16 = p.dtype == ARENO_DT_F16;
+  auto ceil_div = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  // (lengths are taken to be about equal; a window of w shows w + 1 keys to a query)
+  const int64_t seqs = p.num_seqs, group = p.q_heads / p.kv_heads;
+  const int64_t queries = std::max<int64_t>(p.q_tokens / seqs, 1), keys = std::max<int64_t>(p.k_tokens / seqs, 1);
+  const int64_t reach = p.window_left >= 0 ? p.window_left + int64_t{1} : INT32_MAX;
+  // matrix cores: sequences in a block, tiles of each, rounds of workgroups; us per step of the dkv and the dq kernel
+  const int64_t dkv_steps = std::min(seqs, std::max<int64_t>(key_rows / keys, 1)) * ceil_div(std::min(queries, reach + key_rows), kBmTile) * group *
+                            ceil_div(ceil_div(p.k_tokens, key_rows) * p.kv_heads, kBmComputeUnits);
+  const int64_t dq_steps = std::min(seqs, std::max<int64_t>(kBmRows / queries, 1)) * ceil_div(std::min(keys, reach + kBmRows), kBmTile) *
+                           ceil_div(ceil_div(p.q_tokens, kBmRows) * p.q_heads, 2 * kBmComputeUnits);
+  const double dkv_us = d256 ? (fp16 ? 6.6 : 4.2) : (fp16 ? 4.1 : 2.7), dq_us = d256 ? (fp16 ? 8.0 : 6.9) : (fp16 ? 5.4 : 4.9);
+  const double matrix_cores = 8 + dkv_us * dkv_steps + dq_us * dq_steps;
+  // vector ALU: all rows' work, or one row's chain, 16 keys or pairs at a time
+  const double seen = static_cast<double>(std::min(keys, reach)), pairs = static_cast<double>(std::min(queries, reach) * group);
+  const double work = (d256 ? 0.0245 : 0.0182) * (static_cast<double>(p.q_tokens * p.q_heads) * std::max(1.0, seen / 24) +
+                                                  static_cast<double>(p.k_tokens * p.kv_heads) * std::max(1.0, pairs / 48));
+  const double chain = d256 ? 43 + 4.6 * pairs / 16 + 5.0 * seen / 16 : 33 + 3.0 * pairs / 16 + 3.5 * seen / 16;
+  return std::max(work, chain) < matrix_cores;
+}
+
 }  // namespace
 
 int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
@@ -1022,7 +1053,9 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
   // Head dims 192 and 256 (the sliding-window layers of wide heads) have one shape of either kernel.  2 717 tokens in
   // four sequences, 16 / 8 heads of 256, window 512, bf16, forward and backward: 403 us (weights kept in 32 bits, see
   // split_weights) against 7 500 us on the vector-ALU kernels, which recompute every product on 16 lanes' dot products.
+  // (Not for many very short sequences, unless a switch fixes the shapes.)
   if (p.head_dim > 128) {
+    if (getenv("ARENO_BACKWARD_DQ_ROWS") == nullptr && vector_alu_is_faster(p, p.head_dim == 256 ? 128 : 96)) return ARENO_ERR_UNSUPPORTED;
     dkv_parts = 1;
     dq_rows = 16;
   }

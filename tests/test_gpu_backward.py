@@ -87,10 +87,11 @@ def test_varlen_backward_long_sequences_on_the_matrix_core_kernels(dtype, hq, hk
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("hq,hkv,d,window_left", [(4, 2, 256, None), (6, 2, 256, 70), (3, 3, 192, None), (4, 1, 192, 97), (2, 1, 256, 0)])
 @pytest.mark.parametrize("lens", [[300, 1, 0, 130, 5, 95, 97, 161], [127], [129, 31], [1]])
-def test_varlen_backward_of_wide_heads_on_the_matrix_core_kernels(dtype, hq, hkv, d, window_left, lens):
+def test_varlen_backward_of_wide_heads_on_the_matrix_core_kernels(dtype, hq, hkv, d, window_left, lens, monkeypatch):
     """Head dims 192 and 256: sequences longer than the dkv kernel's blocks (96 and 128 packed keys), blocks that hold
     several sequences, lengths one off a block and a tile, windows shorter and longer than a block.  The bar is the
     file's."""
+    monkeypatch.setenv("ARENO_BACKWARD_DQ_ROWS", "16")  # (and not the kernels that a launch's estimate may prefer)
     g = torch.Generator().manual_seed(hq * 31 + d + len(lens))
     t = sum(lens)
     cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
@@ -180,6 +181,24 @@ def test_gradients_of_rows_behind_the_last_sequence_are_zeros(d, dq_rows, dtype,
         assert (got[t:] == 0).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d", [(32, 1, 256), (8, 1, 192), (4, 4, 256), (16, 4, 192)])
+@pytest.mark.parametrize("lens", [[1], [1] * 64, [2, 0, 1] * 100, [4] * 200, [8] * 30, [16] * 8, [32] * 4, [1] * 30 + [200]])
+def test_many_short_sequences_of_wide_heads(dtype, hq, hkv, d, lens):
+    """Launches on either side of the estimate that sends short sequences of wide heads to the vector-ALU kernels.  The
+    bar is the file's."""
+    g = torch.Generator().manual_seed(d + hq)
+    t = sum(lens)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
+    q, k, v, go = (torch.randn(t, h, d, generator=g).to(dtype) for h in (hq, hkv, hkv, hq))
+    qd, kd, vd = (x.to(DEV).requires_grad_(True) for x in (q, k, v))
+    ops.areno_varlen_causal_attention(qd, kd, vd, cu.to(DEV)).backward(go.to(DEV))
+    qf, kf, vf = (x.float().requires_grad_(True) for x in (q, k, v))
+    ar.ref_varlen(qf, kf, vf, cu, -1, d**-0.5).backward(go.float())
+    for got, ref, name in ((qd.grad, qf.grad, "dq"), (kd.grad, kf.grad, "dk"), (vd.grad, vf.grad, "dv")):
+        _close(got, ref, REL[dtype], f"{name} {dtype} {hq}/{hkv} d={d} lens={lens[:3]}")
+
+
 def _gradients_in_64_bits(go, q, k, v, out, lens, window_left, scale):
     """dQ, dK, dV of the packed op from the output that the forward saved (whose rounding is not the backward's)."""
     go, q, k, v, out = (x.double().cpu() for x in (go, q, k, v, out))
@@ -202,10 +221,13 @@ def _gradients_in_64_bits(go, q, k, v, out, lens, window_left, scale):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("hq,hkv,d,window_left", [(4, 2, 256, None), (3, 3, 192, 70), (4, 1, 192, None), (2, 1, 256, 40), (2, 1, 200, None)])
 @pytest.mark.parametrize("size", [1.0, 2.0**-12, 2.0**12])
-def test_wide_heads_keep_their_weights_in_32_bits(dtype, hq, hkv, d, window_left, size):
+@pytest.mark.parametrize("fixed", [True, False])
+def test_wide_heads_keep_their_weights_in_32_bits(dtype, hq, hkv, d, window_left, size, fixed, monkeypatch):
     """Head dims above 128 with gradients in fp32: probabilities and dS are not rounded to 16 bits on the way (2e-4 and
     more would show), nor limited to fp16's range (a loss scaled up or down).  The bar, in the 2-norm: a score of up
     to 2^4 in the exponent and its sum over 256 products put 2^4 * 2^-24 * a few on every weight, 4e-6."""
+    if fixed:  # on the matrix cores
+        monkeypatch.setenv("ARENO_BACKWARD_DQ_ROWS", "16")
     g = torch.Generator().manual_seed(d + hq)
     lens = [300, 1, 0, 131]
     t = sum(lens)
