@@ -227,7 +227,9 @@ int areno_hip_paged_decode_planned(const areno_paged_cache* cache, const void* q
  * cu_seqlens[s] sees keys [max(cu_seqlens[s], t - window_left), t] (all of [cu_seqlens[s], t] when window_left < 0).
  *   q, out  device [tokens, q_heads, head_dim];  k, v  device [tokens, kv_heads, head_dim];  all `dtype`
  *   cu_seqlens  device [num_seqs + 1] int32
- *   workspace   device, at least areno_hip_prefill_workspace_bytes(kv_heads, head_dim) bytes (may be NULL for F32)
+ *   workspace   device, at least areno_hip_prefill_workspace_bytes(kv_heads, head_dim) bytes (may be NULL for F32): the
+ *               launch's sizes decide whether it is used, and no 16-bit call is taken without it
+ * Rows of out behind the last sequence (cu_seqlens[num_seqs] < tokens) become zeros.
  */
 int areno_hip_varlen_attention(const void* q, const void* k, const void* v, void* out, int32_t dtype, int64_t tokens,
                                int32_t q_heads, int32_t kv_heads, int32_t head_dim, const int32_t* cu_seqlens,
@@ -244,6 +246,7 @@ int areno_hip_varlen_attention(const void* q, const void* k, const void* v, void
  *   cu_seqlens_q  device [num_seqs + 1] int32;  context_lens device [num_seqs] int32
  *   block_table   device [num_seqs, max_blocks] int32
  *   workspace     device, at least areno_hip_prefill_workspace_bytes(cache->kv_heads, cache->head_dim) bytes
+ * Rows of out behind the last sequence become zeros.
  */
 int areno_hip_paged_varlen_prefill(const areno_paged_cache* cache, const void* q, void* out, int32_t q_dtype,
                                    int64_t tokens, int32_t q_heads, int32_t num_seqs, const int32_t* block_table,
@@ -407,8 +410,9 @@ int areno_hip_block_tables_prefill_slots(const areno_block_tables* tables, const
  *   cu_seqlens_q      device [num_seqs + 1] int32;  cu_seqlens_k  the same for the keys, NULL = cu_seqlens_q (varlen op)
  *   context_lens      device [num_seqs] int32 position of each sequence's first query, NULL = 0 (dense op: query_start)
  *   workspace         areno_hip_attention_backward_workspace_bytes(q_tokens, q_heads) bytes: per-row log-sum-exp and dO . O
- * head_dim a multiple of 8 up to 256 (F16 / BF16 at 64, 128, 192 and 256: matrix-core kernels).  Two launches; deterministic
- * (no atomics).
+ * head_dim a multiple of 8 up to 256 (F16 / BF16 at 64, 128, 192 and 256 with a positive scale: matrix-core kernels; at 64
+ * and 128 these round the probabilities and dS to the inputs' type, everywhere else they stay fp32).  Any softmax scale.
+ * Gradients of rows behind the last sequence are zeros.  Two launches; deterministic (no atomics).
  */
 size_t areno_hip_attention_backward_workspace_bytes(int64_t q_tokens, int32_t q_heads);
 int areno_hip_attention_backward(const void* grad_out, const void* q, const void* k, const void* v, const void* out,
