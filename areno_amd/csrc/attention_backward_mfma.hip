@@ -108,57 +108,70 @@ __device__ __forceinline__ typename MfmaOps<KIND>::vec8 streamed_operand(const f
                                         pack_pair<KIND>(x[1][0], x[1][1]), pack_pair<KIND>(x[1][2], x[1][3])});
 }
 // The same without rounding, for the wide heads (whose 16-bit inputs had fp32 kernels until these took them, and lose
-// nothing by it): the eight values as three bf16 operands that add up to them.  A bf16 holds eight significant bits
-// with fp32's exponents, so the upper half of a value's word, that of the rest and what is left then are the value's 24.
-__device__ __forceinline__ void split_weights(const float (&x)[2][4], bf16x8_t (&part)[3]) {
+// nothing by it): the eight values as three operands that add up to them, times a power of two in fp16.
+// bf16 holds eight significant bits with fp32's exponents: the upper half of a value's word, that of the rest and what is
+// left then are its 24.  fp16 holds eleven in a narrow range: the values of a column (the four lane groups) are first
+// scaled together, so that the largest comes to lie in [2^14, 2^15); what three parts leave is 2^-40 of it and less.
+template <int KIND>
+struct SplitWeights {
+  typename MfmaOps<KIND>::vec8 part[3];
+  float unscale;
+};
+template <int KIND>
+__device__ __forceinline__ SplitWeights<KIND> split_weights(const float (&x)[2][4]) {
+  SplitWeights<KIND> s;
+  float scale = 1.0f;
+  if constexpr (KIND == KV_F16) {
+    float most = max_f32(__builtin_fabsf(x[0][0]), __builtin_fabsf(x[0][1]));
+    most = max3_f32(most, __builtin_fabsf(x[0][2]), __builtin_fabsf(x[0][3]));
+    most = max3_f32(most, __builtin_fabsf(x[1][0]), __builtin_fabsf(x[1][1]));
+    most = rows_max(max3_f32(most, __builtin_fabsf(x[1][2]), __builtin_fabsf(x[1][3])));
+    // exponent field of the scale: 2^14 over the largest value's power of two (at most 2^126, for its inverse)
+    const uint32_t field = min(268u - (__builtin_bit_cast(uint32_t, most) >> 23), 253u);
+    scale = __builtin_bit_cast(float, field << 23);
+    s.unscale = __builtin_bit_cast(float, (254u - field) << 23);
+  }
   uint32_t w[3][4];
 #pragma unroll
   for (int pair = 0; pair < 4; ++pair) {
     float a = x[pair >> 1][2 * (pair & 1)], b = x[pair >> 1][2 * (pair & 1) + 1];
+    if constexpr (KIND == KV_F16) {
+      a *= scale;
+      b *= scale;
+    }
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
-      w[i][pair] = __builtin_amdgcn_perm(ub, ua, 0x07060302u);  // the upper halves, a's in the low one
-      a -= __builtin_bit_cast(float, ua & 0xffff0000u);  // exact
-      b -= __builtin_bit_cast(float, ub & 0xffff0000u);
+    for (int i = 0; i < 3; ++i) {  // (the subtractions are exact)
+      if constexpr (KIND == KV_F16) {
+        const auto h = __builtin_amdgcn_cvt_pkrtz(a, b);
+        w[i][pair] = __builtin_bit_cast(uint32_t, h);
+        a -= static_cast<float>(h[0]);
+        b -= static_cast<float>(h[1]);
+      } else {
+        const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
+        w[i][pair] = __builtin_amdgcn_perm(ub, ua, 0x07060302u);  // the upper halves, a's in the low one
+        a -= __builtin_bit_cast(float, ua & 0xffff0000u);
+        b -= __builtin_bit_cast(float, ub & 0xffff0000u);
+      }
     }
   }
 #pragma unroll
-  for (int i = 0; i < 3; ++i) part[i] = __builtin_bit_cast(bf16x8_t, uint4_t{w[i][0], w[i][1], w[i][2], w[i][3]});
+  for (int i = 0; i < 3; ++i) s.part[i] = __builtin_bit_cast(typename MfmaOps<KIND>::vec8, uint4_t{w[i][0], w[i][1], w[i][2], w[i][3]});
+  return s;
 }
-// c + columns . the values that `part` adds up to.  An fp16 operand has 11 significant bits and goes in as the two
-// bf16 that hold them (the product of its rest with the weights' last part, 2^-25 of the whole, is left out).  A tile's
-// products are summed by themselves, the small ones first, so the running sum rounds once per tile.
+// c + columns . the values that the parts add up to.  A tile's products are summed by themselves, the small ones first,
+// so the running sum rounds once per tile.
 // Relative error of dV against 64 bits (four sequences of 300 .. 1 000 tokens, 16 / 8 heads of 256, window 512, fp32 out):
 // rounded weights 1.6e-3 (bf16) and 2.0e-4 (fp16), these 2.7e-7 and 2.8e-7, the fp32 kernels 2.8e-7 and 3.1e-7; all
-// products straight into the running sum 4.5e-7 and 5.5e-7.  The price, forward and backward: bf16 343 -> 403 us (365
-// without the sum of its own), fp16 350 -> 601 us; the fp32 kernels take 7 500.
+// products straight into the running sum 4.5e-7 (bf16).  The price, forward and backward: bf16 343 -> 403 us (365
+// without the sum of its own), fp16 350 -> 414 us; the fp32 kernels take 7 500.
 template <int KIND>
-__device__ __forceinline__ float4_t split_product(typename MfmaOps<KIND>::vec8 columns, const bf16x8_t (&part)[3], float4_t c) {
-  using Ops = MfmaOps<KV_BF16>;
+__device__ __forceinline__ float4_t split_product(typename MfmaOps<KIND>::vec8 columns, const SplitWeights<KIND>& s, float4_t c) {
   float4_t tile = {0.0f, 0.0f, 0.0f, 0.0f};
-  if constexpr (KIND == KV_BF16) {
 #pragma unroll
-    for (int i = 2; i >= 0; --i) tile = Ops::mfma(columns, part[i], tile);
-  } else {
-    uint32_t hi[4], lo[4];
-#pragma unroll
-    for (int pair = 0; pair < 4; ++pair) {
-      const float a = static_cast<float>(columns[2 * pair]), b = static_cast<float>(columns[2 * pair + 1]);
-      const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
-      hi[pair] = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
-      const float ra = a - __builtin_bit_cast(float, ua & 0xffff0000u), rb = b - __builtin_bit_cast(float, ub & 0xffff0000u);
-      lo[pair] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, rb), __builtin_bit_cast(uint32_t, ra), 0x07060302u);
-    }
-    const bf16x8_t h = __builtin_bit_cast(bf16x8_t, uint4_t{hi[0], hi[1], hi[2], hi[3]});
-    const bf16x8_t l = __builtin_bit_cast(bf16x8_t, uint4_t{lo[0], lo[1], lo[2], lo[3]});
-    tile = Ops::mfma(l, part[1], tile);
-    tile = Ops::mfma(h, part[2], tile);
-    tile = Ops::mfma(l, part[0], tile);
-    tile = Ops::mfma(h, part[1], tile);
-    tile = Ops::mfma(h, part[0], tile);
-  }
-  return c + tile;
+  for (int i = 2; i >= 0; --i) tile = MfmaOps<KIND>::mfma(columns, s.part[i], tile);
+  // (on whole vectors: element by element the compiler moves the sums around, 183 copies in the dq kernel at 256)
+  if constexpr (KIND == KV_BF16) return c + tile;
+  return __builtin_elementwise_fma(tile, float4_t{s.unscale, s.unscale, s.unscale, s.unscale}, c);
 }
 template <int KIND>
 __device__ __forceinline__ float operand_element(uint32_t word, int hi) {
@@ -356,8 +369,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
             }
           }
           if constexpr (kSplit) {
-            bf16x8_t dsop[3];
-            split_weights(ds, dsop);
+            const SplitWeights<KIND> dsop = split_weights<KIND>(ds);
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb)
               acc[nb] = split_product<KIND>(tile_transposed_operand<KIND, T>(s_k, nb, lr, lk), dsop, acc[nb]);
@@ -846,12 +858,11 @@ __global__ __launch_bounds__((DkvShape<D, KR, P>::kThreads), (DkvShape<D, KR, P>
         fetch(next);
         if (compute) {
           if constexpr (D > 128) {
-            bf16x8_t w[3];
-            split_weights(pr, w);
+            SplitWeights<KIND> w = split_weights<KIND>(pr);
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb)
               acc_v[nb] = split_product<KIND>(tile_transposed_operand<KIND, T>(s_g(buf), nb, lr, lk), w, acc_v[nb]);
-            split_weights(ds, w);
+            w = split_weights<KIND>(ds);
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb)
               acc_k[nb] = split_product<KIND>(tile_transposed_operand<KIND, T>(s_q(buf), nb, lr, lk), w, acc_k[nb]);
@@ -972,10 +983,10 @@ DkvLaunch dkv_launch(int parts) {
 // win by up to 30 times, for many single tokens they lose by as much; in between both are estimated, in us, from what
 // 624 launches took (head dims 192 and 256, both types, 1 .. 512 sequences of 1 .. 64 tokens, six head ratios: the one
 // taken is at most 8 % slower than the other).  vector ALU, matrix cores, in us: 64 sequences of 1 token, 32 / 1 heads
-// of 256, bf16: 82, 9 035; 512 x 4 tokens, 8 / 1 heads of 192, fp16: 346, 914; 8 x 32, 16 / 1 of 256, bf16: 286, 316; 64 x 16,
-// 16 heads of 256, bf16: 834, 121; 1 token, 8 / 1 heads of 256, fp16: 54, 70, bf16: 51, 51; 300 tokens: 801, 441.
+// of 256, bf16: 82, 9 035; 512 x 4 tokens, 8 / 1 heads of 192, fp16: 346, 638; 8 x 32, 16 / 1 of 256, bf16: 286, 316; 64 x 16,
+// 16 heads of 256, bf16: 834, 121; 1 token, 8 / 1 heads of 256, fp16: 54, 51; 300 tokens, bf16: 801, 441.
 bool vector_alu_is_faster(const BwdParams& p, int key_rows) {
-  const bool d256 = p.head_dim == 256, fp16 = p.dtype == ARENO_DT_F16;
+  const bool d256 = p.head_dim == 256;
   auto ceil_div = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   // (lengths are taken to be about equal; a window of w shows w + 1 keys to a query)
   const int64_t seqs = p.num_seqs, group = p.q_heads / p.kv_heads;
@@ -986,7 +997,7 @@ bool vector_alu_is_faster(const BwdParams& p, int key_rows) {
                             ceil_div(ceil_div(p.k_tokens, key_rows) * p.kv_heads, kBmComputeUnits);
   const int64_t dq_steps = std::min(seqs, std::max<int64_t>(kBmRows / queries, 1)) * ceil_div(std::min(keys, reach + kBmRows), kBmTile) *
                            ceil_div(ceil_div(p.q_tokens, kBmRows) * p.q_heads, 2 * kBmComputeUnits);
-  const double dkv_us = d256 ? (fp16 ? 6.6 : 4.2) : (fp16 ? 4.1 : 2.7), dq_us = d256 ? (fp16 ? 8.0 : 6.9) : (fp16 ? 5.4 : 4.9);
+  const double dkv_us = d256 ? 4.2 : 2.7, dq_us = d256 ? 6.8 : 4.8;
   const double matrix_cores = 8 + dkv_us * dkv_steps + dq_us * dq_steps;
   // vector ALU: all rows' work, or one row's chain, 16 keys or pairs at a time
   const double seen = static_cast<double>(std::min(keys, reach)), pairs = static_cast<double>(std::min(queries, reach) * group);
