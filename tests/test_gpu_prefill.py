@@ -429,3 +429,17 @@ def test_paged_rows_behind_the_last_sequence_are_zeros(kv, d, page, behind):
     cabi.check(cabi.paged_varlen_prefill(cache, q, out, w.block_table, w.cu_seqlens_q, w.context_lens, workspace), "prefill")
     assert (out[w.q.shape[0] :] == 0).all()
     assert_close(out[: w.q.shape[0]], _run_prefill(w).cpu().float(), *tolerances(kv), what="rows in front of the padding")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d", [(7, 1, 128), (2, 2, 64), (3, 1, 192)])
+@pytest.mark.parametrize("lens", [
+    [2] * 256, [2] * 257, [1] * 1000 + [150] * 24, [7, 0] * 512, [0] * 1023 + [300], [40] + [0, 3] * 300, [1] * 1025,
+])  # fmt: skip
+def test_varlen_of_many_sequences(dtype, hq, hkv, d, lens):
+    """Up to 256 and up to 1 024 sequences have their block counts in four and sixteen registers per lane; more take the
+    generic kernel.  Tolerance as in the file's other 16-bit outputs against the fp32 oracle."""
+    q, k, v, cu = _packed(lens, hq, hkv, d, dtype, seed=len(lens))
+    out = ops.areno_varlen_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV))
+    want = ar.ref_varlen(q, k, v, cu, -1, d**-0.5)
+    assert_close(out, want, *tolerances("bf16"), what=f"varlen of {len(lens)} sequences {hq}/{hkv} d={d}")
