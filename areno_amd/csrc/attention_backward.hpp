@@ -5,7 +5,12 @@
 
 #include <stdint.h>
 
+#include <atomic>
+
 #include "areno_hip.h"
+#if defined(__HIPCC__)
+#include <hip/hip_runtime.h>
+#endif
 
 namespace areno {
 
@@ -18,7 +23,7 @@ struct BwdParams {
   void* grad_q;  // gradients in fp32, or in the inputs' 16-bit type (grad_dtype)
   void* grad_k;
   void* grad_v;
-  float* row_stats;  // [q_tokens * q_heads][2]: log2-domain log-sum-exp of the scaled scores, dO . O (matrix cores: -(dO . O))
+  float* row_stats;  // [q_tokens * q_heads][2] (matrix cores: by head, then row): log2-domain log-sum-exp of the scaled scores, dO . O (matrix cores: -(dO . O))
   const int32_t* cu_q;
   const int32_t* cu_k;
   const int32_t* ctx;  // may be nullptr: 0
@@ -59,6 +64,45 @@ __device__ inline __attribute__((always_inline)) void store_grad4(void* base, in
     *reinterpret_cast<f16x4*>(static_cast<_Float16*>(base) + i) = __builtin_convertvector(v, f16x4);
   }
 }
+// the last sequence that starts at or in front of `row` (the one that holds it, when the row exists)
+__device__ inline __attribute__((always_inline)) int seq_of_row(const int32_t* cu, int num_seqs, int64_t row) {
+  int lo = 0, hi = num_seqs;
+  while (lo + 1 < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (static_cast<int64_t>(cu[mid]) <= row) {
+      lo = mid;
+    } else {
+      hi = mid;
+    }
+  }
+  return lo;
+}
+
+// a dkv kernel with its launch shape
+typedef void (*bwd_fn)(BwdParams);
+struct DkvLaunch {
+  bwd_fn fn;  // nullptr: its LDS size was refused
+  int lds_bytes, threads, key_rows;
+};
+// more than 64 KB of LDS has to be allowed once per device; one bit per device (the attribute belongs to the device's copy)
+template <int BYTES>
+bool allow_lds(bwd_fn fn, std::atomic<uint64_t>& allowed_on) {
+  if constexpr (BYTES > 64 * 1024) {
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return false;
+    if ((allowed_on.load(std::memory_order_acquire) >> device & 1) == 0) {
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, BYTES) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+      }
+      allowed_on.fetch_or(uint64_t{1} << device, std::memory_order_release);
+    }
+  }
+  return true;
+}
+// the kernels on 32 x 32 x 16 products (attention_backward_dkv.hip), head dims 64 and 128, 16-bit types; `groups`: workgroups
+// of a kv head
+DkvLaunch dkv32_launch(const BwdParams& p, int64_t* groups);
 #endif
 
 // Matrix-core backward (attention_backward_mfma.hip): launches both kernels on `stream` and returns ARENO_OK, or

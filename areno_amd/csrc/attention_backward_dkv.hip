@@ -1,0 +1,461 @@
+// dK and dV of the causal varlen / dense attention ops on 32 x 32 x 16 matrix products (gfx950): 16-bit inputs, head dims
+// 64 and 128.  The second launch of attention_backward_mfma.hip, for sequences long enough to fill its tiles; reads the
+// rows' statistics that the dq kernel left.  The reference: areno/accel/csrc/attention.cu:244-524.
+//
+// A wave owns 32 packed key rows of one kv head: K and V of them as B operands and both sums in registers.  It goes
+// through the query rows that may see them, for every q head of the group, in tiles of 32 that the memory pipe puts into
+// LDS:  S = Q . K^T,  dP = dO . V^T - dO . O,  P = exp2(S - lse),  dS = P * dP,  dV^T += dO^T . P,  dK^T += Q^T . dS.  A
+// C tile of the first two is the B operand of the last two as it lies (mfma32_tiles.hpp).
+//
+// A workgroup is four waves: KW waves own neighbouring keys and share a stream of tiles, and P such parts own the same keys
+// and take every P-th tile of the stream each; the sums of parts 1 .. P - 1 go to part 0 through LDS at the end, in a fixed
+// order.  (4, 1) for large launches, two workgroups per compute unit; (2, 2); (1, 4) for small ones, whose time is that of
+// their longest block: there a wave has its tiles for itself, no barrier, and 512 registers.  In a (1, 4) launch of about
+// one workgroup per compute unit it takes block i and then block `blocks - 1 - i`: their costs add up to the same.
+//
+// Bound: (4, 1) by the matrix cores (54 % of the cycles, at the clock that they then leave, 1.66 GHz) and LDS; (1, 4) by
+// what one wave issues, 350 instructions and 34 products of 32 cycles in 2 500.  Where the time was: 16 x 16 x 32 products
+// read an operand of 1 KB each where these read one per two; the compiler waited for every operand right behind its read;
+// the spilled addresses of a step (a scratch load waits for all the fetches in front of it).  Forward and backward, us:
+// 4 x 4 096 tokens, 32 / 8 heads of 128, bf16: 2 904 -> 2 429 (the kernel 1 600 -> 1 000); 2 x 2 048, 28 / 4 heads: 393 -> 340
+// (245 -> 145).
+#include <stdlib.h>
+#include <string.h>
+
+#include <algorithm>
+#include <atomic>
+
+#include "attention_backward.hpp"
+#include "backward_order.hpp"
+#include "mfma32_tiles.hpp"
+
+namespace areno {
+namespace {
+
+constexpr int kDkvTile = 32;  // query rows per step
+constexpr float kDkvNegInf = -__builtin_huge_valf();
+
+template <int D, int KW, int P>
+struct Dkv32Shape {
+  using Tile = LdsTile<D, kDkvTile, KW>;
+  static constexpr int kWaves = KW * P;
+  static constexpr int kThreads = kWaves * kWave;
+  static constexpr int kKeys = 32 * KW;                        // key rows of a block
+  static constexpr int kStat = kDkvTile * 2 * 4;               // the rows' statistics
+  static constexpr int kBuffer = 2 * Tile::kBytes + kStat;     // Q, dO
+  static constexpr int kPart = 2 * kBuffer;
+  static constexpr int kSums = (P - 1) * KW * D * 32 * 2 * 4;  // what parts 1 .. P - 1 hand to part 0
+  static constexpr int kLdsBytes = P * kPart > kSums ? P * kPart : kSums;
+};
+extern __shared__ __attribute__((aligned(1024))) char dkv32_lds[];
+
+// The lane's number, worked out where it is needed (the sums leave no register to keep it in).
+__device__ __forceinline__ int lane_now() {
+  int x;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(x));
+  return x;
+}
+
+// x as an A operand whose row sums are x: three bf16 parts (24 bits) in the first elements of lane half 0, and zeros
+__device__ __forceinline__ bf16x8_t three_parts(float x, int half) {
+  uint32_t w[2], u = half == 0 ? __builtin_bit_cast(uint32_t, x) : 0u;
+  const float rest = __builtin_bit_cast(float, u) - __builtin_bit_cast(float, u & 0xffff0000u);  // (exact)
+  const uint32_t v = __builtin_bit_cast(uint32_t, rest);
+  const float last = rest - __builtin_bit_cast(float, v & 0xffff0000u);
+  w[0] = __builtin_amdgcn_perm(v, u, 0x07060302u);  // the upper halves, u's in the low one
+  w[1] = __builtin_bit_cast(uint32_t, last) >> 16;
+  return __builtin_bit_cast(bf16x8_t, uint4_t{w[0], w[1], 0u, 0u});
+}
+
+template <int KIND, int D, int KW, int P, int OCC>
+__global__ __launch_bounds__((Dkv32Shape<D, KW, P>::kThreads)) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void bwd_mfma32_dkv_kernel(BwdParams p) {
+  using M = Mfma32<KIND>;
+  using Start = Mfma32<KV_BF16>;
+  using V8 = typename M::vec8;
+  using L = Dkv32Shape<D, KW, P>;
+  using T = typename L::Tile;
+  constexpr int NKS = D / 16, NB = D / 32, NF = T::kFetches;
+  constexpr bool kTight = D > 64 && OCC > 1;  // sums, K and V and the scores leave 32 registers for all the rest
+
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave_of_block = uniform(tid >> 6);
+  const int part = wave_of_block / KW, wave = wave_of_block % KW;
+  const int l32 = lane & 31, half = lane >> 5;
+  const int kvh = static_cast<int>(blockIdx.x % static_cast<unsigned>(p.kv_heads));
+  const int group = p.q_heads / p.kv_heads;
+  const int k_blocks = static_cast<int>((p.k_tokens + L::kKeys - 1) / L::kKeys);
+  const int wg = static_cast<int>(blockIdx.x / static_cast<unsigned>(p.kv_heads));
+  // (launched with a workgroup per pair of blocks, or with one per block: then in cost order, one block each)
+  const bool paired = gridDim.x / static_cast<unsigned>(p.kv_heads) < static_cast<unsigned>(k_blocks);
+  const int first_block = paired ? wg : uniform(static_cast<int>(block_in_cost_order(wg, k_blocks, p.num_seqs, false)));
+
+  // (with the part's place: a multiple of 256, which the reads' exclusive-ors leave alone)
+  static_assert(L::kPart % 256 == 0, "the parts' places");
+  uint32_t at_rows = T::rows_base(l32, half) + part * L::kPart, at_columns = T::columns_base(lane) + part * L::kPart;
+  const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, uint4_t{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
+  const float unscale = __builtin_bit_cast(float, uniform(__builtin_bit_cast(int, 1.0f / p.scale_log2e)));  // (the scale is positive)
+  const uint32_t lds0 = lds_address(dkv32_lds) + part * L::kPart;
+  const uint32_t stride = static_cast<uint32_t>(p.q_heads) * (D * 2);
+  // Fetch f of a wave fills kFetchRows rows; the chunk a lane fetches is the one that belongs where its bytes land.  A wave
+  // that fetches whole tiles keeps its offsets, others work out their few anew.
+  constexpr int kFetchRows = 64 / T::kChunksPerRow;
+  auto fetch_row = [&](int f, int lane) { return kFetchRows * (NF * wave + f) + lane / T::kChunksPerRow; };
+  auto fetch_offset = [&](int f, int lane) {
+    const int r = fetch_row(f, lane);
+    return static_cast<uint32_t>(r) * stride + static_cast<uint32_t>((lane % T::kChunksPerRow) ^ T::twist(r)) * 16u;
+  };
+  uint32_t kept_offset[NF];
+  if constexpr (KW == 1) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) kept_offset[f] = fetch_offset(f, lane);
+  }
+
+  for (int turn = 0; turn < 2; ++turn) {
+    const int block = turn == 0 ? first_block : k_blocks - 1 - first_block;
+    // (no second block without pairs, and none for the middle one of an odd number of blocks)
+    if (turn == 1 && (!paired || block <= first_block)) break;
+    const int64_t r0 = static_cast<int64_t>(block) * L::kKeys;
+    const int64_t block_end = r0 + L::kKeys < p.k_tokens ? r0 + L::kKeys : p.k_tokens;
+    const int64_t row = r0 + 32 * wave + l32;  // this lane's key row (a column of the products)
+    const bool row_exists = row < p.k_tokens;
+    const int64_t row_elem = (row * p.kv_heads + kvh) * D;
+    V8 kop[NKS], vop[NKS];
+    {
+      uint4_t kw[NKS], vw[NKS];
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) kw[ks] = vw[ks] = uint4_t{0u, 0u, 0u, 0u};
+      if (row_exists) {
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+          const int64_t off = (row_elem + 16 * ks + 8 * half) * 2;
+          kw[ks] = load16(p.k, off);
+          vw[ks] = load16(p.v, off);
+        }
+      }
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) {
+        // (waited for here: left to their first use inside the loop, that wait would cover every tile's fetches as well)
+        asm volatile("" : "+v"(kw[ks]), "+v"(vw[ks]));
+        kop[ks] = __builtin_bit_cast(V8, kw[ks]);
+        vop[ks] = __builtin_bit_cast(V8, vw[ks]);
+      }
+    }
+    float16_t acc_k[NB], acc_v[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc_k[nb] = acc_v[nb] = zero16();
+
+    int s = uniform(seq_of_row(p.cu_k, p.num_seqs, r0));
+    for (int64_t sk0 = uniform(p.cu_k[s]), sk1; s < p.num_seqs && sk0 < block_end; ++s, sk0 = sk1) {
+      // (asked for together)
+      const int k_end = p.cu_k[s + 1], q_begin = p.cu_q[s], q_end = p.cu_q[s + 1], before = p.ctx != nullptr ? p.ctx[s] : 0;
+      sk1 = uniform(k_end);
+      const int64_t k_lo = sk0 > r0 ? sk0 : r0, k_hi = sk1 < block_end ? sk1 : block_end;
+      if (k_lo >= k_hi) continue;
+      const int ctx = uniform(before);
+      const int64_t q_first = uniform(q_begin);
+      const int n_q = uniform(q_end) - static_cast<int>(q_first);
+      const bool live = row >= k_lo && row < k_hi;
+      const uint64_t live_lanes = __builtin_amdgcn_ballot_w64(live);
+      const bool wave_live = live_lanes != 0, wave_full = live_lanes == ~0ull;
+      const int wave_key_lo = static_cast<int>(r0 + 32 * wave - sk0), wave_key_hi = wave_key_lo + 31;
+      // queries i (position ctx + i) that see one of the block's keys: key <= ctx + i <= key + window
+      const int key_min = static_cast<int>(k_lo - sk0), key_max = static_cast<int>(k_hi - 1 - sk0);
+      const int i_lo = key_min - ctx > 0 ? key_min - ctx : 0;
+      int i_hi = n_q - 1;
+      if (p.window_left >= 0 && key_max + p.window_left - ctx < i_hi) i_hi = key_max + p.window_left - ctx;
+      if (i_hi < i_lo) continue;  // (the same for the whole workgroup)
+      const int t0 = i_lo / kDkvTile, t1 = i_hi / kDkvTile;
+      const int tiles = t1 - t0 + 1;
+      // the stream: tiles of every q head of the group, head by head; this part takes steps part, part + P, ...
+      const int stream_steps = tiles * group;
+      const int steps = (stream_steps - part + P - 1) / P;  // this part's
+      const int rounds = (stream_steps + P - 1) / P;        // the longest part's: every part keeps the barriers of all
+      // the step whose tile is fetched next: its tile, where its rows of Q (and, a fixed way off, of dO) and statistics lie
+      const int64_t tile_bytes = static_cast<int64_t>(kDkvTile) * stride;
+      const int64_t head_bytes = D * 2 - tiles * tile_bytes, head_stats = (p.q_tokens - static_cast<int64_t>(tiles) * kDkvTile) * 8;
+      const int64_t to_grad = static_cast<const char*>(p.grad_out) - static_cast<const char*>(p.q);
+      int tile = t0 + part, ahead = tile;
+      const char* q_ahead = static_cast<const char*>(p.q) + q_first * stride + kvh * group * (D * 2) + tile * tile_bytes;
+      const char* stat_ahead = reinterpret_cast<const char*>(p.row_stats) + ((kvh * group) * p.q_tokens + q_first + tile * kDkvTile) * 8;
+      auto to_next_heads = [&] {
+        while (ahead > t1) {
+          ahead -= tiles;
+          q_ahead += head_bytes;
+          stat_ahead += head_stats;
+        }
+      };
+      to_next_heads();
+      while (tile > t1) tile -= tiles;
+      // tiles this wave computes on (the first to the last that one of its keys is seen from), and those without a mask
+      int seen_lo = 0, seen_hi = t1, plain_lo = max(wave_key_hi - ctx + kDkvTile - 1, 0) / kDkvTile, plain_hi = n_q / kDkvTile - 1;
+      if constexpr (KW > 1) {
+        seen_lo = max(wave_key_lo - ctx, 0) / kDkvTile;
+        if (p.window_left >= 0) seen_hi = wave_key_hi + p.window_left - ctx < 0 ? -1 : (wave_key_hi + p.window_left - ctx) / kDkvTile;
+        if (!wave_live) seen_hi = -1;
+      }
+      if (p.window_left >= 0) {
+        const int reach = wave_key_lo + p.window_left - ctx - (kDkvTile - 1);
+        plain_hi = reach < 0 ? -1 : min(plain_hi, reach / kDkvTile);
+      }
+      if (!wave_full) plain_hi = -1;
+      auto fetch = [&](int buf) {
+        const int last = min(n_q - ahead * kDkvTile, kDkvTile) - 1;  // rows behind the sequence's last repeat it
+        const char* const qb = q_ahead;
+        const char* const gb = q_ahead + to_grad;
+        const char* const sb = stat_ahead;
+        const uint32_t dst = lds0 + static_cast<uint32_t>(buf * L::kBuffer + wave * (NF * 1024));
+        const int lane = lane_now();
+        if (last == kDkvTile - 1) {
+#pragma unroll
+          for (int f = 0; f < NF; ++f) {
+            const uint32_t off = KW == 1 ? kept_offset[f] : fetch_offset(f, lane);
+            fetch_to_lds(qb, off, dst + f * 1024);
+            fetch_to_lds(gb, off, dst + T::kBytes + f * 1024);
+          }
+        } else {
+#pragma unroll
+          for (int f = 0; f < NF; ++f) {
+            const uint32_t back = static_cast<uint32_t>(max(fetch_row(f, lane) - last, 0)) * stride;
+            const uint32_t off = (KW == 1 ? kept_offset[f] : fetch_offset(f, lane)) - back;
+            fetch_to_lds(qb, off, dst + f * 1024);
+            fetch_to_lds(gb, off, dst + T::kBytes + f * 1024);
+          }
+        }
+        if (wave == 0) {
+          fetch_words_to_lds(sb, static_cast<uint32_t>(min(lane >> 1, last)) * 8u + (lane & 1) * 4u,
+                             lds0 + static_cast<uint32_t>(buf * L::kBuffer + 2 * T::kBytes));
+        }
+        ahead += P;
+        q_ahead += P * tile_bytes;
+        stat_ahead += P * kDkvTile * 8;
+        to_next_heads();
+      };
+      auto step = [&](int i, int buf) {
+        // the step's tile (asked for a step ago) is there, and every wave of the part has left the one before
+        if constexpr (KW == 1) {
+          fetched();
+        } else {
+          fetched_barrier();
+        }
+        if (i + 1 < steps) fetch(buf ^ 1);
+        if (KW > 1 && i >= steps) return;
+        const int t = tile;
+        tile += P;
+        while (tile > t1) tile -= tiles;
+        if (KW > 1 && (t < seen_lo || t > seen_hi)) return;
+        // (where registers are short the addresses of a step are worked out where they are used)
+        if constexpr (OCC > 1) asm volatile("" : "+v"(at_rows), "+v"(at_columns));
+        char* const q_lds = dkv32_lds + buf * L::kBuffer;
+        char* const g_lds = q_lds + T::kBytes;
+        // The products' operands come out of LDS in one stream, each read kAhead products in front of its own (left
+        // alone the compiler reads one, waits for it and reads the next): rows of Q and of dO, columns of dO and of Q.
+        constexpr int kAhead = kTight ? 2 : 8;
+        auto read = [&](int x) {
+          if (x < NKS) return tile_rows<KIND, T>(q_lds, at_rows, 0, x);
+          if (x < 2 * NKS) return tile_rows<KIND, T>(g_lds, at_rows, 0, x - NKS);
+          const int y = x - 2 * NKS;
+          if (y < 2 * NB) return tile_columns<KIND, T>(g_lds, at_columns, 16 * (y / NB), y % NB);
+          return tile_columns<KIND, T>(q_lds, at_columns, 16 * (y / NB - 2), y % NB);
+        };
+        constexpr int kReads = 2 * NKS + 4 * NB;
+        V8 operand[kAhead];
+        // The statistics go into the products as one more contraction step, so that a lane reads those of one row
+        // instead of sixteen: what is added to S and dP, -lse / scale and -(dO . O), in three bf16 parts times ones.
+        const float2_t stat = *reinterpret_cast<const float2_t*>(q_lds + 2 * T::kBytes + part * L::kPart + 8 * (lane_now() & 31));
+#pragma unroll
+        for (int x = 0; x < kAhead; ++x) operand[x] = read(x);
+        float16_t sc = zero16();
+#pragma unroll
+        for (int x = 0; x < NKS; ++x) {
+          __builtin_amdgcn_sched_barrier(0);
+          sc = M::mfma(operand[x % kAhead], kop[x], sc);
+          operand[x % kAhead] = read(x + kAhead);
+        }
+        sc = Start::mfma(three_parts(max_f32(stat[0] * -unscale, -3e38f), half), ones, sc);
+        if (t < plain_lo || t > plain_hi) {
+          const int lane = lane_now();
+          const int base = kDkvTile * t + 4 * (lane >> 5);  // queries base + 8 c + j
+          const int key = wave_key_lo + (lane & 31);        // this lane's key position in the sequence
+          const int first = key - ctx - base;
+          int last = n_q - 1;
+          if (p.window_left >= 0) last = min(last, key - ctx + p.window_left);
+          last = live ? last - base : -1;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const int q = 8 * (e >> 2) + (e & 3);
+            sc[e] = q >= first && q <= last ? sc[e] : kDkvNegInf;
+          }
+        }
+        float16_t dp = zero16();
+        V8 pop[2], dsop[2];
+        uint32_t w[8], dw[8];
+        // (a query without visible keys has +inf as its log-sum-exp: exp2 of what comes of it is 0)
+#pragma unroll
+        for (int x = 0; x < NKS; ++x) {
+          __builtin_amdgcn_sched_barrier(0);
+          dp = M::mfma(operand[(NKS + x) % kAhead], vop[x], dp);
+          operand[(NKS + x) % kAhead] = read(NKS + x + kAhead);
+          if constexpr (!kTight) {  // the exponentials between the products of dP
+#pragma unroll
+            for (int e = 16 / NKS * x; e < 16 / NKS * (x + 1); e += 2) {
+              sc[e] = fast_exp2(sc[e] * p.scale_log2e);
+              sc[e + 1] = fast_exp2(sc[e + 1] * p.scale_log2e);
+              w[e / 2] = pack_pair<KIND>(sc[e], sc[e + 1]);
+            }
+          }
+        }
+        dp = Start::mfma(three_parts(stat[1], half), ones, dp);
+        if constexpr (kTight) {  // (P and dS at once, so that packed ones take the registers of those they come from)
+#pragma unroll
+          for (int e = 0; e < 16; e += 2) {
+            __builtin_amdgcn_sched_barrier(0);
+            const float p0 = fast_exp2(sc[e] * p.scale_log2e), p1 = fast_exp2(sc[e + 1] * p.scale_log2e);
+            w[e / 2] = pack_pair<KIND>(p0, p1);
+            dw[e / 2] = pack_pair<KIND>(p0 * dp[e], p1 * dp[e + 1]);
+          }
+        }
+#pragma unroll
+        for (int b = 0; b < 2; ++b) pop[b] = __builtin_bit_cast(V8, uint4_t{w[4 * b], w[4 * b + 1], w[4 * b + 2], w[4 * b + 3]});
+#pragma unroll
+        for (int x = 0; x < 2 * NB; ++x) {
+          constexpr int kFrom = 2 * NKS;
+          __builtin_amdgcn_sched_barrier(0);
+          acc_v[x % NB] = M::mfma(operand[(kFrom + x) % kAhead], pop[x / NB], acc_v[x % NB]);
+          if (kFrom + x + kAhead < kReads) operand[(kFrom + x) % kAhead] = read(kFrom + x + kAhead);
+          if constexpr (!kTight) {  // dS between the products of dV
+#pragma unroll
+            for (int e = 8 / NB * x; e < 8 / NB * (x + 1); e += 2) dw[e / 2] = pack_pair<KIND>(sc[e] * dp[e], sc[e + 1] * dp[e + 1]);
+          }
+        }
+#pragma unroll
+        for (int b = 0; b < 2; ++b) dsop[b] = __builtin_bit_cast(V8, uint4_t{dw[4 * b], dw[4 * b + 1], dw[4 * b + 2], dw[4 * b + 3]});
+#pragma unroll
+        for (int x = 0; x < 2 * NB; ++x) {
+          constexpr int kFrom = 2 * NKS + 2 * NB;
+          __builtin_amdgcn_sched_barrier(0);
+          acc_k[x % NB] = M::mfma(operand[(kFrom + x) % kAhead], dsop[x / NB], acc_k[x % NB]);
+          if (kFrom + x + kAhead < kReads) operand[(kFrom + x) % kAhead] = read(kFrom + x + kAhead);
+        }
+      };
+      // the tiles' previous readers (an earlier sequence of this block, the sums of the block before) are done
+      fetched_barrier();
+      if (steps > 0) fetch(0);
+      const int turns = KW == 1 ? steps : rounds;
+      for (int i = 0; i < turns; i += 2) {
+        step(i, 0);
+        if (i + 1 < turns) step(i + 1, 1);
+      }
+    }
+
+    if constexpr (P > 1) {
+      // the other parts' sums to part 0, in a fixed order: a float4 per lane at a time, lanes next to each other
+      float4_t* const sums = reinterpret_cast<float4_t*>(dkv32_lds) + wave * kWave + lane_now();
+      constexpr int kStep = KW * kWave, kFours = 8 * NB;  // (per part)
+      __syncthreads();  // the tiles' last readers are done
+      if (part > 0) {
+        float4_t* const mine = sums + (part - 1) * (kFours * kStep);
+#pragma unroll
+        for (int x = 0; x < 4 * NB; ++x) {
+          const int nb = x >> 2, c = 4 * (x & 3);
+          mine[x * kStep] = float4_t{acc_k[nb][c], acc_k[nb][c + 1], acc_k[nb][c + 2], acc_k[nb][c + 3]};
+          mine[(4 * NB + x) * kStep] = float4_t{acc_v[nb][c], acc_v[nb][c + 1], acc_v[nb][c + 2], acc_v[nb][c + 3]};
+        }
+      }
+      __syncthreads();
+      if (part == 0) {
+#pragma unroll
+        for (int other = 0; other < P - 1; ++other) {
+          const float4_t* const theirs = sums + other * (kFours * kStep);
+#pragma unroll
+          for (int x = 0; x < 4 * NB; ++x) {
+            const float4_t dk = theirs[x * kStep], dv = theirs[(4 * NB + x) * kStep];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              acc_k[x >> 2][4 * (x & 3) + j] += dk[j];
+              acc_v[x >> 2][4 * (x & 3) + j] += dv[j];
+            }
+          }
+        }
+      }
+    }
+
+    // every gradient element is written, also the zeros of keys no query sees
+    const int lane_ = lane_now();
+    const int64_t out_row = r0 + 32 * wave + (lane_ & 31);
+    if (part == 0 && out_row < p.k_tokens) {
+      const int64_t out_elem = (out_row * p.kv_heads + kvh) * D + 4 * (lane_ >> 5);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int64_t at_elem = out_elem + 32 * nb + 8 * c;
+          store_grad4(p.grad_k, at_elem, acc_k[nb][4 * c] * p.scale, acc_k[nb][4 * c + 1] * p.scale, acc_k[nb][4 * c + 2] * p.scale,
+                      acc_k[nb][4 * c + 3] * p.scale, p.grad_dtype);
+          store_grad4(p.grad_v, at_elem, acc_v[nb][4 * c], acc_v[nb][4 * c + 1], acc_v[nb][4 * c + 2], acc_v[nb][4 * c + 3], p.grad_dtype);
+        }
+      }
+    }
+  }
+}
+
+template <int KIND, int D, int KW, int P, int OCC>
+DkvLaunch launch_of() {
+  using L = Dkv32Shape<D, KW, P>;
+  const bwd_fn fn = bwd_mfma32_dkv_kernel<KIND, D, KW, P, OCC>;
+  static std::atomic<uint64_t> allowed_on{0};
+  if (!allow_lds<L::kLdsBytes>(fn, allowed_on)) return DkvLaunch{nullptr, 0, 0, 0};
+  return DkvLaunch{fn, L::kLdsBytes, L::kThreads, L::kKeys};
+}
+template <int KIND, int D>
+DkvLaunch launch_of(int parts) {
+  if (parts == 4) return launch_of<KIND, D, 1, 4, 1>();
+  if (parts == 2) return launch_of<KIND, D, 2, 2, 2>();
+  return launch_of<KIND, D, 4, 1, 2>();
+}
+
+constexpr int64_t kComputeUnits = 256;
+
+}  // namespace
+
+// The shape, from the launch's size (blocks of 32 keys of a kv head) and what a block's stream is for sequences of the mean
+// length: `per_seq` steps for a sequence, `steps` for all that a block holds.  Four parts want streams that keep all four
+// busy for longer than handing their sums over takes, and pay until their workgroups, one per compute unit, come round a
+// second or third time; one part wants the chip filled twice with blocks of 128 keys.  The backward in us, in one part, two,
+// four (what the 16-row kernels took): D = 128, 28 / 4 heads: 2 x 2 048 tokens (512 blocks) 565, 397, 261 (310); 4 x 2 048
+// (1 024) 679, 569, 524 (573); 6 x 2 048 (1 536) 842, 745, 792 (891); 8 x 2 048 (2 048) 1 006, 963, 1 053 (1 154); 16 x 256 (512)
+// 126, 113, 95 (119); 48 x 256 (1 536) 239, 262, 276 (262); 4 x 4 096, 32 / 8 (4 096) 1 977, 2 056, 2 214 (2 248); 8 / 8 heads, 32 x 128
+// (1 024) 36.0, 37.6, 59 (35.5).  D = 64: 2 x 2 048, 32 / 8 (1 024) 266, 186, 182 (213); 3 x 4 096, 28 / 4 (1 536) 958, 723, 773 (994);
+// 16 / 16 heads: 8 x 128 (512) 22.1, 20.4, 24.6 (21.1); 16 x 310 (2 480) 66, 69, 102 (65).
+DkvLaunch dkv32_launch(const BwdParams& p, int64_t* groups) {
+  const int64_t blocks = (p.k_tokens + 31) / 32, workgroups = blocks * p.kv_heads;
+  const int64_t seqs = std::max<int64_t>(p.num_seqs, 1), mean = std::max<int64_t>(p.q_tokens / seqs, 1), group = p.q_heads / p.kv_heads;
+  const int64_t chain = mean / kDkvTile * group, per_seq = std::max(chain, group);
+  const int64_t steps = mean < 32 ? per_seq * std::min(seqs, 32 / mean) : per_seq;
+  int parts = 1;
+  if (workgroups <= (chain >= 128 ? 1152 : 640) && per_seq >= 4 && steps >= 16) {
+    parts = 4;
+  } else if (workgroups <= (chain >= 64 ? 2304 : chain < 8 ? (mean < 32 ? 1280 : 768) : p.head_dim == 64 ? 2048 : 1280)) {
+    parts = 2;
+  }
+  // Pairs of blocks where every one of them then has a compute unit (two share one at head dim 64) and single blocks would not
+  const int64_t units = (p.head_dim == 64 ? 2 : 1) * kComputeUnits;
+  bool pairs = workgroups > units && (blocks + 1) / 2 * p.kv_heads <= units;
+  // ARENO_BACKWARD_PARTS=1|2|4 (read at every launch; 4 in pairs) fixes the choice: the same dK and dV up to the order of
+  // the last sums, so this is for tests of the kernels a launch of the test's size would not take, and for timing
+  if (const char* e = getenv("ARENO_BACKWARD_PARTS")) {
+    if (strcmp(e, "1") == 0) parts = 1;
+    if (strcmp(e, "2") == 0) parts = 2;
+    if (strcmp(e, "4") == 0 && workgroups <= 0x7fffffffLL) parts = 4, pairs = true;
+  }
+  DkvLaunch launch;
+  if (p.head_dim == 64) {
+    launch = p.dtype == ARENO_DT_BF16 ? launch_of<KV_BF16, 64>(parts) : launch_of<KV_F16, 64>(parts);
+  } else {
+    launch = p.dtype == ARENO_DT_BF16 ? launch_of<KV_BF16, 128>(parts) : launch_of<KV_F16, 128>(parts);
+  }
+  *groups = parts < 4 ? (p.k_tokens + launch.key_rows - 1) / std::max(launch.key_rows, 1) : pairs ? (blocks + 1) / 2 : blocks;
+  return launch;
+}
+
+}  // namespace areno

@@ -9,13 +9,12 @@
 //                dQ^T += K^T . dS^T  with the lane's own dS^T values as the B operand (rounded to the inputs' type; at
 //                the wide heads not rounded, split_weights) and K^T read transposed from the same LDS tile.  A row's softmax reference moves as in the forward (the accumulator is rescaled), so
 //                one pass over the keys gives dQ, the row's log-sum-exp and dO . O (left in the workspace).
-//   dkv kernel   a workgroup owns 32 to 128 packed key rows of one kv head (16 per wave) and streams, for every q head
+//   dkv kernel   (head dims 192 and 256 here, 64 and 128 in attention_backward_dkv.hip) a workgroup owns 96 or 128 packed key
+//                rows of one kv head (16 per wave) and streams, for every q head
 //                of the group, the query rows that may see them in tiles of 32 (Q and dO tiles in LDS, the rows'
 //                statistics next to them):  S = Q . K^T,  dP = dO . V^T,  P = exp2(S - lse),  dS = P * (dP - dO . O),
-//                dV^T += dO^T . P  and  dK^T += Q^T . dS.  Every gradient element has one owner; in a small launch
-//                the stream of tiles is split over two or four sets of waves whose sums are added in a fixed order.
-// Both launches take their blocks in an order (or in pairs) that lets their workgroups end together: see
-// block_in_cost_order and the dkv kernel.
+//                dV^T += dO^T . P  and  dK^T += Q^T . dS.  Every gradient element has one owner.
+// Both launches take their blocks in an order that lets their workgroups end together: see block_in_cost_order.
 //
 // The streamed index of a tile (keys in the dq kernel, queries in the dkv kernel) is the contraction index of the
 // second pair of products; a 16 x 16 product leaves element 4 g + j of that index in lane group g, which is exactly
@@ -46,20 +45,6 @@ constexpr int kBmThreads = kBmWaves * kWave;
 constexpr int kBmRows = 16 * kBmWaves;  // packed rows a workgroup owns
 constexpr int kBmTile = 32;             // streamed rows per step
 constexpr float kBmNegInf = -__builtin_huge_valf();
-
-// the last sequence that starts at or in front of `row` (the one that holds it, when the row exists)
-__device__ __forceinline__ int seq_of_row(const int32_t* cu, int num_seqs, int64_t row) {
-  int lo = 0, hi = num_seqs;
-  while (lo + 1 < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (static_cast<int64_t>(cu[mid]) <= row) {
-      lo = mid;
-    } else {
-      hi = mid;
-    }
-  }
-  return lo;
-}
 
 // A tile of 32 rows x D 16-bit elements in LDS, row stride D * 2 + 16 bytes: the row operands (16 lanes read the same
 // 16-byte chunk of 16 rows) meet every bank once, the transposed ones (32 lanes read 32 bytes of 8 consecutive rows)
@@ -405,7 +390,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
                     acc[nb][2] * f, acc[nb][3] * f, p.grad_dtype);
       }
       if (lk == 0) {
-        float* st = p.row_stats + (row * p.q_heads + h) * 2;
+        float* st = p.row_stats + (h * p.q_tokens + row) * 2;
         // a row without visible keys gets a reference no score reaches: its probabilities come out as zeros
         st[0] = l_tot > 0.0f ? m_run + __builtin_log2f(l_tot) : __builtin_huge_valf();
         st[1] = -delta;
@@ -623,7 +608,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
         }
       }
       if (half == 0) {
-        float* st = p.row_stats + (row * p.q_heads + h) * 2;
+        float* st = p.row_stats + (h * p.q_tokens + row) * 2;
         st[0] = l_tot > 0.0f ? m_run + __builtin_log2f(l_tot) : __builtin_huge_valf();
         st[1] = -delta;
       }
@@ -637,50 +622,37 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
 }
 
 // ---- dK, dV -------------------------------------------------------------------------------------------------------------
-// A workgroup owns a block of KR (32, 64, or 96 and 128 at the wide heads) packed key rows of one kv head, or two of them one after the other: block i and
-// block blocks - 1 - i.  A key block early in its sequence is seen by all later queries and one late in it by few.
-// A launch of many workgroups per compute unit evens that out by starting the expensive blocks first
-// (block_in_cost_order); in a launch of about one workgroup per unit nothing comes after the expensive block to
-// fill the gap, and there the pairs help: for sequences of about equal length the costs of such a pair add up to
-// the same for every i, so the workgroups end together.  (The launcher says which by the size of the grid.)
-// The workgroup has P parts of KR / 16 waves.  Every part owns all KR key rows (16 per wave) and takes every P-th
-// step of the stream of query tiles (tiles and statistics of its own in LDS); the sums of parts 1 .. P - 1 go to
-// part 0 through LDS at the end of a block, in a fixed order.  More parts shorten the chain of steps a block is:
-// (KR, P) = (64, 1) four waves, two workgroups per compute unit, for launches that fill the units several times;
-// (64, 2) and (32, 4) eight waves, for launches of about one workgroup per unit; (96, 1) and (128, 1) six and eight waves
-// at head dims 192 and 256.
-template <int D, int KR, int P>
+// Head dims 192 and 256 (attention_backward_dkv.hip has 64 and 128).  A workgroup owns a block of KR (96, 128) packed key
+// rows of one kv head, 16 per wave, and streams the query rows that may see them, for every q head of the group.  A key
+// block early in its sequence is seen by all later queries and one late in it by few: the expensive blocks start first
+// (block_in_cost_order).
+template <int D, int KR>
 struct DkvShape {
   static constexpr int kKeyWaves = KR / 16;
-  static constexpr int kPartThreads = kKeyWaves * kWave;
-  static constexpr int kThreads = kPartThreads * P;
+  static constexpr int kThreads = kKeyWaves * kWave;
   static constexpr int RS = BmTile<D>::RS;
   static constexpr int kChunksPerRow = BmTile<D>::kChunksPerRow;
-  static constexpr int kChunks = kBmTile * kChunksPerRow / kPartThreads;  // 16-byte chunks of a tile per thread of a part
-  static_assert(kBmTile * kChunksPerRow % kPartThreads == 0, "tile chunks");
+  static constexpr int kChunks = kBmTile * kChunksPerRow / kThreads;  // 16-byte chunks of a tile per thread
+  static_assert(kBmTile * kChunksPerRow % kThreads == 0, "tile chunks");
   static constexpr int kTile = kBmTile * RS;
   static constexpr int kStat = kBmTile * 2 * 4;
-  // per part and buffer: a Q tile, a dO tile, the rows' statistics
+  // per buffer: a Q tile, a dO tile, the rows' statistics
   static constexpr int kBuffer = 2 * kTile + kStat;
-  static constexpr int kStream = P * 2 * kBuffer;
-  static constexpr int kSums = (P - 1) * kPartThreads * (D / 16) * 2 * 16;  // a float4 per lane, block of 16 and tensor
-  static constexpr int kLdsBytes = kStream > kSums ? kStream : kSums;
+  static constexpr int kLdsBytes = 2 * kBuffer;
 };
 extern __shared__ __attribute__((aligned(16))) char bm_dkv_lds[];
 
-template <int KIND, int D, int KR, int P>
-__global__ __launch_bounds__((DkvShape<D, KR, P>::kThreads), (DkvShape<D, KR, P>::kThreads == 256 ? 2 : 1)) void bwd_mfma_dkv_kernel(
+template <int KIND, int D, int KR>
+__global__ __launch_bounds__((DkvShape<D, KR>::kThreads), 1) void bwd_mfma_dkv_kernel(
     BwdParams p) {
   using Ops = MfmaOps<KIND>;
   using V8 = typename Ops::vec8;
   using T = BmTile<D>;
-  using L = DkvShape<D, KR, P>;
+  using L = DkvShape<D, KR>;
   constexpr int NS = D / 32, NB = D / 16;
 
-  // (the same for a wave, and told so: the part's steps, cursors and loop counts then live in scalar registers)
-  const int part = P > 1 ? uniform(static_cast<int>(threadIdx.x) / L::kPartThreads) : 0;
-  const int tid = P > 1 ? static_cast<int>(threadIdx.x) % L::kPartThreads : static_cast<int>(threadIdx.x);  // in the part
-  char* const lds = bm_dkv_lds + part * (2 * L::kBuffer);
+  const int tid = threadIdx.x;
+  char* const lds = bm_dkv_lds;
   auto s_q = [&](int buf) { return lds + buf * L::kBuffer; };
   auto s_g = [&](int buf) { return lds + buf * L::kBuffer + L::kTile; };
   auto s_stat = [&](int buf) { return reinterpret_cast<float*>(lds + buf * L::kBuffer + 2 * L::kTile); };  // [row][2]
@@ -692,14 +664,8 @@ __global__ __launch_bounds__((DkvShape<D, KR, P>::kThreads), (DkvShape<D, KR, P>
   const int group = p.q_heads / p.kv_heads;
   const int64_t k_blocks = (p.k_tokens + KR - 1) / KR;
   const int64_t wg = blockIdx.x / static_cast<unsigned>(p.kv_heads);
-  // (launched with a workgroup per pair of blocks, or with one per block: then in cost order, one block each)
-  const bool paired = gridDim.x / static_cast<unsigned>(p.kv_heads) < k_blocks;
-  const int64_t first_block = paired ? wg : block_in_cost_order(wg, k_blocks, p.num_seqs, false);
-
-  for (int half = 0; half < 2; ++half) {
-    const int64_t block = half == 0 ? first_block : k_blocks - 1 - first_block;
-    // (no second block without pairs, and none for the middle one of an odd number of blocks)
-    if (half == 1 && (!paired || block <= first_block)) break;
+  const int64_t block = block_in_cost_order(wg, k_blocks, p.num_seqs, false);
+  {
     const int64_t r0 = block * KR;
     const int64_t block_end = r0 + KR < p.k_tokens ? r0 + KR : p.k_tokens;
     const int64_t row = r0 + 16 * wave + lr;  // this lane's key row (a column of the products)
@@ -745,26 +711,19 @@ __global__ __launch_bounds__((DkvShape<D, KR, P>::kThreads), (DkvShape<D, KR, P>
       if (i_hi < i_lo) continue;  // (the same for the whole workgroup)
       const int t0 = i_lo / kBmTile, t1 = i_hi / kBmTile;
       const int tiles = t1 - t0 + 1;
-      // the stream: tiles of every q head of the group, head by head; this part takes steps part, part + P, ...
-      const int stream_steps = tiles * group;
-      const int steps = (stream_steps - part + P - 1) / P;  // this part's
-      const int rounds = (stream_steps + P - 1) / P;        // the longest part's: every part keeps the barriers of all
-      // (head, tile) of a step of the stream, counted up by P steps at a time
+      // the stream: tiles of every q head of the group, head by head
+      const int steps = tiles * group;
+      // (head, tile) of a step of the stream
       struct Cursor {
         int head, tile;
       };
       auto advance = [&](Cursor& c) {
-        c.tile += P;
-        while (c.tile > t1) {
-          c.tile -= tiles;
+        if (++c.tile > t1) {
+          c.tile = t0;
           ++c.head;
         }
       };
-      Cursor first = {kvh * group, t0 + part};
-      while (first.tile > t1) {
-        first.tile -= tiles;
-        ++first.head;
-      }
+      const Cursor first = {kvh * group, t0};
 
       // Two register sets hold the tiles of the next two steps while they are in flight; a step computes on one of
       // the two LDS buffers, moves the next step's tile into the other one and asks for the tile two steps further on.
@@ -782,7 +741,7 @@ __global__ __launch_bounds__((DkvShape<D, KR, P>::kThreads), (DkvShape<D, KR, P>
         advance(fetch_at);
 #pragma unroll
         for (int i = 0; i < L::kChunks; ++i) {
-          const int c = tid + L::kPartThreads * i;
+          const int c = tid + L::kThreads * i;
           const int r = c / T::kChunksPerRow, col = c % T::kChunksPerRow;
           const int qi = kBmTile * t + r < n_q ? kBmTile * t + r : n_q - 1;  // rows past the end repeat the last query
           const int64_t off = ((q_base + qi) * p.q_heads + hq) * (D * 2) + col * 16;
@@ -791,13 +750,13 @@ __global__ __launch_bounds__((DkvShape<D, KR, P>::kThreads), (DkvShape<D, KR, P>
         }
         if (tid < kBmTile) {
           const int qi = kBmTile * t + tid < n_q ? kBmTile * t + tid : n_q - 1;
-          st.stat = *reinterpret_cast<const float2_t*>(p.row_stats + ((q_base + qi) * p.q_heads + hq) * 2);
+          st.stat = *reinterpret_cast<const float2_t*>(p.row_stats + (hq * p.q_tokens + q_base + qi) * 2);
         }
       };
       auto publish = [&](const Staged& st, int buf) {
 #pragma unroll
         for (int i = 0; i < L::kChunks; ++i) {
-          const int c = tid + L::kPartThreads * i;
+          const int c = tid + L::kThreads * i;
           const int r = c / T::kChunksPerRow, col = c % T::kChunksPerRow;
           *reinterpret_cast<uint4_t*>(s_q(buf) + T::chunk_pos(r, col)) = st.q[i];
           *reinterpret_cast<uint4_t*>(s_g(buf) + T::chunk_pos(r, col)) = st.g[i];
@@ -810,7 +769,7 @@ __global__ __launch_bounds__((DkvShape<D, KR, P>::kThreads), (DkvShape<D, KR, P>
       auto step_on = [&](int step, int buf, Staged& next) {
         const int t = at.tile;
         advance(at);
-        const bool compute = wave_live && step < steps;
+        const bool compute = wave_live;
         float pr[2][4], ds[2][4];
         auto first_products = [&](auto masked) {
 #pragma unroll
@@ -878,52 +837,20 @@ __global__ __launch_bounds__((DkvShape<D, KR, P>::kThreads), (DkvShape<D, KR, P>
         }
         __syncthreads();  // every wave has read this step's tile, the next one is in place
       };
-      // (every wave has passed a barrier behind the last use of the buffers: an earlier sequence's last step, or the
-      // hand-over of the block before)
+      // (every wave has passed a barrier behind the last use of the buffers: an earlier sequence's last step)
       fetch(set_a);
       fetch(set_b);
-      if (steps > 0) publish(set_a, 0);
+      publish(set_a, 0);
       fetch(set_a);
       __syncthreads();
-      for (int step = 0; step < rounds; step += 2) {
+      for (int step = 0; step < steps; step += 2) {
         step_on(step, 0, set_b);
-        if (step + 1 < rounds) step_on(step + 1, 1, set_a);
+        if (step + 1 < steps) step_on(step + 1, 1, set_a);
       }
-    }
-
-    if constexpr (P > 1) {
-      // the other parts' sums to part 0: a float4 per lane, block of 16 and tensor, lanes next to each other
-      // (the tiles' last readers have passed a barrier, or no step ran at all)
-      float4_t* sums = reinterpret_cast<float4_t*>(bm_dkv_lds);
-      if (part > 0) {
-        float4_t* mine = sums + (part - 1) * (2 * NB * L::kPartThreads);
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          mine[(2 * nb) * L::kPartThreads + tid] = acc_k[nb];
-          mine[(2 * nb + 1) * L::kPartThreads + tid] = acc_v[nb];
-        }
-      }
-      __syncthreads();
-      if (part == 0) {
-#pragma unroll
-        for (int other = 1; other < P; ++other) {
-          const float4_t* theirs = sums + (other - 1) * (2 * NB * L::kPartThreads);
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb) {
-            const float4_t dk = theirs[(2 * nb) * L::kPartThreads + tid], dv = theirs[(2 * nb + 1) * L::kPartThreads + tid];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              acc_k[nb][j] += dk[j];
-              acc_v[nb][j] += dv[j];
-            }
-          }
-        }
-      }
-      __syncthreads();  // the sums are read: the second block's tiles may overwrite them
     }
 
     // every gradient element is written, also the zeros of keys no query sees
-    if (part == 0 && row_exists) {
+    if (row_exists) {
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
         const int64_t at_elem = row_elem + 4 * lk + 16 * nb;
@@ -935,46 +862,20 @@ __global__ __launch_bounds__((DkvShape<D, KR, P>::kThreads), (DkvShape<D, KR, P>
   }
 }
 
-typedef void (*bm_fn)(BwdParams);
 constexpr int64_t kBmComputeUnits = 256;
 
-// the dkv kernel of a (type, head dim, key rows per block, parts) with its launch shape; more than 64 KB of LDS has
-// to be allowed once per device
-struct DkvLaunch {
-  bm_fn fn;
-  int lds_bytes, threads, key_rows;
-};
-template <int KIND, int D, int KR, int P>
-DkvLaunch dkv_launch() {
-  using L = DkvShape<D, KR, P>;
-  const bm_fn fn = bwd_mfma_dkv_kernel<KIND, D, KR, P>;
-  if constexpr (L::kLdsBytes > 64 * 1024) {
-    static std::atomic<uint64_t> allowed_on{0};  // one bit per device (the attribute belongs to the device's copy)
-    int device = 0;
-    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return DkvLaunch{nullptr, 0, 0, 0};
-    if ((allowed_on.load(std::memory_order_acquire) >> device & 1) == 0) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              L::kLdsBytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return DkvLaunch{nullptr, 0, 0, 0};
-      }
-      allowed_on.fetch_or(uint64_t{1} << device, std::memory_order_release);
-    }
-  }
-  return DkvLaunch{fn, L::kLdsBytes, L::kThreads, KR};
-}
 // Head dims 192 and 256 have one shape: the sums and operands of 16 key rows take all registers of two waves per SIMD,
 // and six or eight waves behind one stream of tiles stage two chunks of a tensor per thread and step (with four waves it
 // would be four chunks, twice the staging registers).  At 256 the kernel still keeps some of its staging in scratch, a
 // dozen loads and half as many stores in every two steps of the tile loop; at 192 a few registers, outside it.
 template <int KIND, int D>
-DkvLaunch dkv_launch(int parts) {
-  if constexpr (D > 128) return dkv_launch<KIND, D, D == 256 ? 128 : 96, 1>();
-  if constexpr (D <= 128) {
-    if (parts == 4) return dkv_launch<KIND, D, 32, 4>();
-    if (parts == 2) return dkv_launch<KIND, D, 64, 2>();
-    return dkv_launch<KIND, D, 64, 1>();
-  }
+DkvLaunch dkv_launch() {
+  constexpr int KR = D == 256 ? 128 : 96;
+  using L = DkvShape<D, KR>;
+  const bwd_fn fn = bwd_mfma_dkv_kernel<KIND, D, KR>;
+  static std::atomic<uint64_t> allowed_on{0};
+  if (!allow_lds<L::kLdsBytes>(fn, allowed_on)) return DkvLaunch{nullptr, 0, 0, 0};
+  return DkvLaunch{fn, L::kLdsBytes, L::kThreads, KR};
 }
 
 // Whether the vector-ALU kernels take a launch of wide heads in less time.  A matrix-core workgroup goes through the
@@ -1015,34 +916,12 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
   // the kernels mask raw scores and take row maxima before scaling: any other scale is for the vector-ALU kernels, as in
   // the forward (launch_prefill_mfma)
   if (!(p.scale_log2e > 0.0f)) return ARENO_ERR_UNSUPPORTED;
+  // (the dkv kernels up to head dim 128 divide a row's log-sum-exp by the scale: 128 / 1e-36 has to stay a number)
+  if (p.head_dim <= 128 && p.scale_log2e < 1e-36f) return ARENO_ERR_UNSUPPORTED;
   if (p.q_heads > 65535 || p.kv_heads > 65535) return ARENO_ERR_UNSUPPORTED;
   const int64_t q_blocks = (p.q_tokens + kBmRows - 1) / kBmRows, k_blocks = (p.k_tokens + kBmRows - 1) / kBmRows;
   if (q_blocks * p.q_heads > 0x7fffffffLL || k_blocks * p.kv_heads > 0x7fffffffLL) return ARENO_ERR_UNSUPPORTED;
   const bool bf16 = p.dtype == ARENO_DT_BF16;
-  // The dkv kernel's shape by the size of the launch.  About one workgroup per compute unit: pairs of blocks of 32
-  // key rows, eight waves in four parts (2 x 2 048 tokens, 28 / 4 heads: 527 -> 463 us for both launches; one
-  // sequence of 4 096: 975 -> 814 us).  Up to 4 per unit at head dim 128 and 2 at head dim 64: a block of 64 rows
-  // each, in cost order, eight waves in two parts (2 to 20 % faster than one part; above that the two are equal at
-  // 128, and at 64 a two-part workgroup fills a unit's registers alone where four one-part ones fit: 2.3 x slower at
-  // 8 per unit).  Else one part.  Chains too short to matter stay in one part: more parts want about 64 steps in
-  // the longest chain, estimated from the mean sequence length.
-  const int64_t blocks64 = (p.k_tokens + 63) / 64 * p.kv_heads, pairs32 = ((p.k_tokens + 31) / 32 + 1) / 2 * p.kv_heads;
-  const int64_t longest_chain = p.q_tokens / (p.num_seqs > 0 ? p.num_seqs : 1) / kBmTile * (p.q_heads / p.kv_heads);
-  int dkv_parts = 1;
-  if (longest_chain >= 64) {
-    if (pairs32 <= kBmComputeUnits * 5 / 4) {
-      dkv_parts = 4;
-    } else if (blocks64 <= (p.head_dim == 128 ? 4 : 2) * kBmComputeUnits) {
-      dkv_parts = 2;
-    }
-  }
-  // ARENO_BACKWARD_PARTS=1|2|4 (read at every launch) fixes the choice: the same dK and dV up to the order of the
-  // last sums, so this is for tests of the kernels a launch of the test's size would not take, and for timing
-  if (const char* e = getenv("ARENO_BACKWARD_PARTS")) {
-    if (strcmp(e, "1") == 0) dkv_parts = 1;
-    if (strcmp(e, "2") == 0) dkv_parts = 2;
-    if (strcmp(e, "4") == 0) dkv_parts = 4;
-  }
   // The dq kernel with 32 rows per wave once the launch has 6 workgroups of 64 rows per compute unit at head dim 128, 8
   // at head dim 64, and the sequences are long enough (512 and 1 024 tokens on the average).  The backward, 16 -> 32 rows,
   // us: D = 128: 4 x 4 096 tokens, 32 / 8 heads (32 per unit) 2 646 -> 2 283; 1 x 4 096, 28 / 4 heads (7) 639 -> 561;
@@ -1067,26 +946,26 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
   // (Not for many very short sequences, unless a switch fixes the shapes.)
   if (p.head_dim > 128) {
     if (getenv("ARENO_BACKWARD_DQ_ROWS") == nullptr && vector_alu_is_faster(p, p.head_dim == 256 ? 128 : 96)) return ARENO_ERR_UNSUPPORTED;
-    dkv_parts = 1;
     dq_rows = 16;
   }
   const int64_t dq_blocks = (p.q_tokens + kBmWaves * dq_rows - 1) / (kBmWaves * dq_rows);
-  bm_fn dq;
+  bwd_fn dq;
   DkvLaunch dkv;
+  int64_t dkv_groups = 0;  // workgroups of a kv head
   if (p.head_dim == 64) {
     dq = dq_rows == 32 ? (bf16 ? bwd_mfma32_dq_kernel<KV_BF16, 64> : bwd_mfma32_dq_kernel<KV_F16, 64>)
-                    : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 64> : bwd_mfma_dq_kernel<KV_F16, 64>);
-    dkv = bf16 ? dkv_launch<KV_BF16, 64>(dkv_parts) : dkv_launch<KV_F16, 64>(dkv_parts);
+                       : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 64> : bwd_mfma_dq_kernel<KV_F16, 64>);
+    dkv = dkv32_launch(p, &dkv_groups);
   } else if (p.head_dim == 192) {
     dq = bf16 ? bwd_mfma_dq_kernel<KV_BF16, 192> : bwd_mfma_dq_kernel<KV_F16, 192>;
-    dkv = bf16 ? dkv_launch<KV_BF16, 192>(1) : dkv_launch<KV_F16, 192>(1);
+    dkv = bf16 ? dkv_launch<KV_BF16, 192>() : dkv_launch<KV_F16, 192>();
   } else if (p.head_dim == 256) {
     dq = bf16 ? bwd_mfma_dq_kernel<KV_BF16, 256> : bwd_mfma_dq_kernel<KV_F16, 256>;
-    dkv = bf16 ? dkv_launch<KV_BF16, 256>(1) : dkv_launch<KV_F16, 256>(1);
+    dkv = bf16 ? dkv_launch<KV_BF16, 256>() : dkv_launch<KV_F16, 256>();
   } else {
     dq = dq_rows == 32 ? (bf16 ? bwd_mfma32_dq_kernel<KV_BF16, 128> : bwd_mfma32_dq_kernel<KV_F16, 128>)
-                    : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 128> : bwd_mfma_dq_kernel<KV_F16, 128>);
-    dkv = bf16 ? dkv_launch<KV_BF16, 128>(dkv_parts) : dkv_launch<KV_F16, 128>(dkv_parts);
+                       : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 128> : bwd_mfma_dq_kernel<KV_F16, 128>);
+    dkv = dkv32_launch(p, &dkv_groups);
   }
   const char* op = "areno_hip_attention_backward";
   if (dkv.fn == nullptr) return fail(ARENO_ERR_LAUNCH, "%s: the dkv kernel's LDS size was refused", op);
@@ -1096,9 +975,8 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
     if (int rc = check_launch(op)) return rc;
   }
   if (k_blocks > 0) {
-    const int64_t blocks = (p.k_tokens + dkv.key_rows - 1) / dkv.key_rows;
-    const int64_t groups = dkv_parts == 4 ? (blocks + 1) / 2 : blocks;  // (pairs with four parts, see above)
-    hipLaunchKernelGGL(dkv.fn, dim3(static_cast<unsigned>(groups * p.kv_heads)), dim3(dkv.threads), dkv.lds_bytes, s, p);
+    if (dkv_groups == 0) dkv_groups = (p.k_tokens + dkv.key_rows - 1) / dkv.key_rows;
+    hipLaunchKernelGGL(dkv.fn, dim3(static_cast<unsigned>(dkv_groups * p.kv_heads)), dim3(dkv.threads), dkv.lds_bytes, s, p);
     if (int rc = check_launch(op)) return rc;
   }
   return ARENO_OK;

@@ -83,6 +83,12 @@ struct LdsTile {
 __device__ __forceinline__ void fetch_to_lds(const char* base, uint32_t offset, uint32_t lds) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "{m0}"(lds) : "memory");
 }
+// the same for 64 words of 4 bytes
+__device__ __forceinline__ void fetch_words_to_lds(const char* base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(offset), "s"(base), "{m0}"(lds) : "memory");
+}
+// The wave's fetches have landed and its LDS reads are in registers (what a wave waits for that shares its tiles with none).
+__device__ __forceinline__ void fetched() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : : : "memory"); }
 // The wave's fetches have landed and its LDS reads are in registers; then every wave's have: the tiles asked for may be
 // read and the tiles read so far may be fetched over.
 __device__ __forceinline__ void fetched_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory"); }

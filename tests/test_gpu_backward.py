@@ -241,6 +241,29 @@ def test_wide_heads_keep_their_weights_in_32_bits(dtype, hq, hkv, d, window_left
         assert err <= 4e-6, f"{name} {dtype} d={d} window={window_left} size={size}: {err:.3g}"
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("parts", ["1", "2", "4", None])
+@pytest.mark.parametrize("hq,hkv,d,window_left", [(4, 1, 128, None), (2, 2, 128, 33), (8, 2, 64, None), (3, 3, 64, 31)])
+@pytest.mark.parametrize("lens,scale", [([31, 33, 32, 97, 128, 129], 0.1), ([1], 0.1), ([161, 0, 1, 2, 95], 2.0), ([64, 65, 63], 1e-3), ([33], 1e-37)])
+def test_key_gradients_where_blocks_and_tiles_end(dtype, parts, hq, hkv, d, window_left, lens, scale, monkeypatch):
+    """The dkv kernel of head dims 64 and 128 in each of its shapes and as the launch's size picks them: sequences one off
+    its blocks (32, 64, 128 keys) and tiles, windows one off a tile, rows' statistics divided by small and large scales (the
+    smallest leaves the matrix cores).  The bar, in the 2-norm: P and dS are rounded to the inputs' type, by half a unit
+    in the last place at most; one unit."""
+    if parts is not None:
+        monkeypatch.setenv("ARENO_BACKWARD_PARTS", parts)
+    g = torch.Generator().manual_seed(d + len(lens))
+    t = sum(lens)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=DEV)
+    q, k, v, go = (torch.randn(t, h, d, generator=g).to(dtype).to(DEV) for h in (hq, hkv, hkv, hq))
+    out = ops.areno_varlen_causal_attention(q, k, v, cu, window_left=window_left, softmax_scale=scale)
+    got = _c_backward(go, q, k, v, out, cu, torch.float32, scale, -1 if window_left is None else window_left)
+    unit = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    for x, want, name in zip(got, _gradients_in_64_bits(go, q, k, v, out, lens, window_left, scale), ("dq", "dk", "dv")):
+        err = (x.cpu().double() - want).norm().item()
+        assert err <= unit * max(want.norm().item(), scale), f"{name} {dtype} {hq}/{hkv} d={d} lens={lens}: {err / want.norm().item():.3g}"
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("query_start,window_left", [(0, None), (7, None), (3, 5)])
 def test_dense_backward(dtype, query_start, window_left):
