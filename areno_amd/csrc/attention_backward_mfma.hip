@@ -404,11 +404,12 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
   }
 }
 
-// The same with 32 query rows per wave, 128 per workgroup, on 32 x 32 x 16 products, for launches that fill the chip with
-// such workgroups: an operand read from LDS serves a product of twice the size, the K and V tiles are fetched straight
-// into LDS (mfma32_tiles.hpp).  Bound by the matrix cores and the LDS reads behind them.  Against a 16 x 16 form of as
-// many rows: the backward of 4 x 4 096 tokens, 32 / 8 heads of 128, bf16: 2 646 -> 2 283 us.  (That form spilled 84 registers;
-// this one spills 26 at head dim 128, once per sequence of a block and not in the tile loop.)
+// The same with 32 query rows per wave, 128 per workgroup, on 32 x 32 x 16 products, for long sequences: an operand read
+// from LDS serves a product of twice the size, the K and V tiles are fetched straight into LDS (mfma32_tiles.hpp), an
+// operand is read four products in front of its own and the exponentials go between the products of dP.  Bound by the
+// matrix cores (56 % of the cycles at the clock that they then leave, 1.4 to 2 GHz) and the vector ALU.  Forward and
+// backward of 4 x 4 096 tokens, 32 / 8 heads of 128, bf16: 2 429 -> 2 375 us with the operands read ahead.  (Registers spill
+// at head dim 128 once per sequence of a block, not in the tile loop.)
 template <int KIND, int D>
 __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams p) {
   using M = Mfma32<KIND>;
@@ -525,23 +526,34 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
         const int key_first = kBmTile * t, key_last = key_first + kBmTile - 1;
         if (wave_full && key_first > wave_pos_hi) return;
         char* const k_lds = lds + buf * kBuffer;
-        const char* const v_lds = k_lds + T::kBytes;
+        char* const v_lds = k_lds + T::kBytes;
+        // the products' operands in one stream, each read kAhead products in front of its own (as in the dkv kernel):
+        // rows of K and of V, columns of K
+        auto read = [&](int x) {
+          if (x < NKS) return tile_rows<KIND, T>(k_lds, at_rows, 0, x);
+          if (x < 2 * NKS) return tile_rows<KIND, T>(v_lds, at_rows, 0, x - NKS);
+          return tile_columns<KIND, T>(k_lds, at_columns, 16 * ((x - 2 * NKS) / NB), (x - 2 * NKS) % NB);
+        };
+        constexpr int kAhead = 4, kReads = 2 * NKS + 2 * NB;
+        V8 operand[kAhead];
+#pragma unroll
+        for (int x = 0; x < kAhead; ++x) operand[x] = read(x);
         float16_t sc = zero16(), dp;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) dp[i] = -delta;
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-          sc = M::mfma(tile_rows<KIND, T>(k_lds, at_rows, 0, ks), qop[ks], sc);
-          dp = M::mfma(tile_rows<KIND, T>(v_lds, at_rows, 0, ks), gop[ks], dp);
+        for (int x = 0; x < NKS; ++x) {
+          __builtin_amdgcn_sched_barrier(0);
+          sc = M::mfma(operand[x % kAhead], qop[x], sc);
+          operand[x % kAhead] = read(x + kAhead);
         }
         const bool plain = wave_full && key_last < n_k && key_last <= wave_pos_lo &&
                            (p.window_left < 0 || key_first >= wave_pos_hi - p.window_left);
         if (!plain) {
+          const int base = key_first + 4 * half;  // keys base + 8 c + j
+          const int last = min(pos, n_k - 1) - base, first = p.window_left < 0 ? -base : pos - p.window_left - base;
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
-            const int key = key_first + 8 * (i >> 2) + 4 * half + (i & 3);
-            const bool ok = key <= pos && key < n_k && (p.window_left < 0 || key >= pos - p.window_left);
-            sc[i] = ok ? sc[i] : kBmNegInf;
+            const int key = 8 * (i >> 2) + (i & 3);
+            sc[i] = key >= first && key <= last ? sc[i] : kBmNegInf;
           }
         }
         constexpr float kLazy = KIND == KV_BF16 ? 8.0f : 0.0f;  // (as above)
@@ -567,6 +579,21 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
           }
         }
         const float m_ref = m_run == kBmNegInf ? 0.0f : m_run;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dp[i] = -delta;
+#pragma unroll
+        for (int x = 0; x < NKS; ++x) {
+          __builtin_amdgcn_sched_barrier(0);
+          dp = M::mfma(operand[(NKS + x) % kAhead], gop[x], dp);
+          operand[(NKS + x) % kAhead] = read(NKS + x + kAhead);
+          // the exponentials between the products of dP
+#pragma unroll
+          for (int i = 16 / NKS * x; i < 16 / NKS * (x + 1); ++i) {
+            sc[i] = fast_exp2(__builtin_fmaf(sc[i], p.scale_log2e, -m_ref));
+            l_lane += sc[i];
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
         V8 dsop[2];
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
@@ -574,18 +601,15 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const int i = 8 * b + 2 * j;
-            const float p0 = fast_exp2(__builtin_fmaf(sc[i], p.scale_log2e, -m_ref));
-            const float p1 = fast_exp2(__builtin_fmaf(sc[i + 1], p.scale_log2e, -m_ref));
-            l_lane += p0 + p1;
-            w[j] = pack_pair<KIND>(p0 * dp[i], p1 * dp[i + 1]);
+            w[j] = pack_pair<KIND>(sc[i] * dp[i], sc[i + 1] * dp[i + 1]);
           }
           dsop[b] = __builtin_bit_cast(V8, uint4_t{w[0], w[1], w[2], w[3]});
         }
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb)
-            acc[nb] = M::mfma(tile_columns<KIND, T>(k_lds, at_columns, 16 * b, nb), dsop[b], acc[nb]);
+        for (int x = 0; x < 2 * NB; ++x) {
+          acc[x % NB] = M::mfma(operand[(2 * NKS + x) % kAhead], dsop[x / NB], acc[x % NB]);
+          if (2 * NKS + x + kAhead < kReads) operand[(2 * NKS + x) % kAhead] = read(2 * NKS + x + kAhead);
+          __builtin_amdgcn_sched_barrier(0);
         }
       };
       fetched_barrier();  // the tiles' previous readers (an earlier sequence of this block) are done
@@ -922,20 +946,16 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
   const int64_t q_blocks = (p.q_tokens + kBmRows - 1) / kBmRows, k_blocks = (p.k_tokens + kBmRows - 1) / kBmRows;
   if (q_blocks * p.q_heads > 0x7fffffffLL || k_blocks * p.kv_heads > 0x7fffffffLL) return ARENO_ERR_UNSUPPORTED;
   const bool bf16 = p.dtype == ARENO_DT_BF16;
-  // The dq kernel with 32 rows per wave once the launch has 6 workgroups of 64 rows per compute unit at head dim 128, 8
-  // at head dim 64, and the sequences are long enough (512 and 1 024 tokens on the average).  The backward, 16 -> 32 rows,
-  // us: D = 128: 4 x 4 096 tokens, 32 / 8 heads (32 per unit) 2 646 -> 2 283; 1 x 4 096, 28 / 4 heads (7) 639 -> 561;
-  // 64 x 512 (56) 946 -> 896; 8 x 512 (7) 135 -> 132; 4 x 600, 32 / 8 heads (4.6) 161 -> 163; 1 x 1 024, 8 / 2 heads (0.5)
-  // 94 -> 105.  D = 64: 4 x 4 096, 32 / 8 heads (32) 1 357 -> 1 240; 2 x 4 096, 16 heads (8) 365 -> 342; 32 x 1 024, 28 / 4
-  // (56) 776 -> 737; 16 x 310, 16 heads (4.8) 62 -> 69.  Small launches want the more and shorter workgroups, and a block
-  // of many short sequences, which it takes one after the other, is a longer chain in the larger block: 28 / 4 heads of
-  // 128, 512 x 8 tokens (7) 187 -> 253, 64 x 64 70 -> 80, 256 x 128 (56) 553 -> 570, 16 x 256 (7) 119 -> 119; of 64,
-  // 1 024 x 8 (14) 158 -> 272, 256 x 128 (56) 265 -> 294, 64 x 512 482 -> 478, 16 x 512 (14) 136 -> 139.
+  // The dq kernel with 32 rows per wave over long sequences: 512 tokens on the average at head dim 128, 1 024 at head dim 64
+  // where the launch also has 4 workgroups of 64 rows per compute unit.  The backward with 16 and 32 rows, us: D = 128:
+  // 4 x 4 096 tokens, 32 / 8 heads (32 per unit) 2 183, 1 791; 2 x 2 048, 28 / 4 heads (7) 304, 264; 4 x 600, 32 / 8 (4.6) 140, 134;
+  // 1 x 2 048, 8 heads (1) 97, 93; 1 x 1 024, 8 / 2 heads (0.5) 78, 78; 16 x 256, 28 / 4 (7) 94, 95.  D = 64: 4 x 4 096, 32 / 8 (32) 1 144, 1 054;
+  // 6 x 1 024, 16 heads (6) 91, 87; 1 x 2 048, 28 / 4 (3.5) 125, 124; 1 x 2 048, 16 heads (2) 79, 81; 64 x 512, 28 / 4 (56) 418, 410; 12 x 512,
+  // 16 heads (6) 67.7, 68.6.  A block of many short sequences, which it takes one after the other, is a longer chain in
+  // the larger block: 28 / 4 heads of 128, 512 x 8 tokens (7) 162, 221; 256 x 128 (56) 497, 538; of 64, 256 x 128 (56) 248, 271.
   // ARENO_BACKWARD_DQ_ROWS=16|32 (read at every launch) fixes the choice, for tests and timing.
   const int64_t mean_length = p.q_tokens / (p.num_seqs > 0 ? p.num_seqs : 1);
-  int dq_rows = q_blocks * p.q_heads >= (p.head_dim == 128 ? 6 : 8) * kBmComputeUnits && mean_length >= (p.head_dim == 128 ? 512 : 1024)
-                    ? 32
-                    : 16;
+  int dq_rows = mean_length >= (p.head_dim == 128 ? 512 : 1024) && (p.head_dim == 128 || q_blocks * p.q_heads >= 4 * kBmComputeUnits) ? 32 : 16;
   if (const char* e = getenv("ARENO_BACKWARD_DQ_ROWS")) {
     if (strcmp(e, "32") == 0) dq_rows = 32;
     if (strcmp(e, "16") == 0) dq_rows = 16;
