@@ -78,11 +78,11 @@ __device__ inline __attribute__((always_inline)) int seq_of_row(const int32_t* c
   return lo;
 }
 
-// a dkv kernel with its launch shape
+// a kernel with its launch shape
 typedef void (*bwd_fn)(BwdParams);
-struct DkvLaunch {
+struct BwdLaunch {
   bwd_fn fn;  // nullptr: its LDS size was refused
-  int lds_bytes, threads, key_rows;
+  int lds_bytes, threads, rows;  // (rows of a block)
 };
 // more than 64 KB of LDS has to be allowed once per device; one bit per device (the attribute belongs to the device's copy)
 template <int BYTES>
@@ -102,7 +102,15 @@ bool allow_lds(bwd_fn fn, std::atomic<uint64_t>& allowed_on) {
 }
 // the kernels on 32 x 32 x 16 products (attention_backward_dkv.hip), head dims 64 and 128, 16-bit types; `groups`: workgroups
 // of a kv head
-DkvLaunch dkv32_launch(const BwdParams& p, int64_t* groups);
+BwdLaunch dkv32_launch(const BwdParams& p, int64_t* groups);
+// head dims 192 and 256 (attention_backward_wide.hip): the dkv kernel over blocks of 64 keys, or of 32 with its stream in two
+// parts while these do not fill the chip twice and a sequence has a step for either part
+inline int dkv32_wide_parts(const BwdParams& p) {
+  const int64_t mean = p.num_seqs > 0 ? p.q_tokens / p.num_seqs : 0;
+  return (p.k_tokens + 31) / 32 * p.kv_heads <= 512 && (mean > 32 || p.q_heads > p.kv_heads) ? 2 : 1;
+}
+BwdLaunch dq32_wide_launch(const BwdParams& p);
+BwdLaunch dkv32_wide_launch(const BwdParams& p, int64_t* groups);
 #endif
 
 // Matrix-core backward (attention_backward_mfma.hip): launches both kernels on `stream` and returns ARENO_OK, or

@@ -49,13 +49,6 @@ struct Dkv32Shape {
 };
 extern __shared__ __attribute__((aligned(1024))) char dkv32_lds[];
 
-// The lane's number, worked out where it is needed (the sums leave no register to keep it in).
-__device__ __forceinline__ int lane_now() {
-  int x;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(x));
-  return x;
-}
-
 // x as an A operand whose row sums are x: three bf16 parts (24 bits) in the first elements of lane half 0, and zeros
 __device__ __forceinline__ bf16x8_t three_parts(float x, int half) {
   uint32_t w[2], u = half == 0 ? __builtin_bit_cast(uint32_t, x) : 0u;
@@ -136,7 +129,11 @@ __global__ __launch_bounds__((Dkv32Shape<D, KW, P>::kThreads)) __attribute__((am
 #pragma unroll
       for (int ks = 0; ks < NKS; ++ks) {
         // (waited for here: left to their first use inside the loop, that wait would cover every tile's fetches as well)
-        asm volatile("" : "+v"(kw[ks]), "+v"(vw[ks]));
+        if constexpr (OCC == 1) {
+          asm volatile("" : "+a"(kw[ks]), "+a"(vw[ks]));  // (in accumulation registers, where the products read them as they are)
+        } else {
+          asm volatile("" : "+v"(kw[ks]), "+v"(vw[ks]));
+        }
         kop[ks] = __builtin_bit_cast(V8, kw[ks]);
         vop[ks] = __builtin_bit_cast(V8, vw[ks]);
       }
@@ -218,8 +215,8 @@ __global__ __launch_bounds__((Dkv32Shape<D, KW, P>::kThreads)) __attribute__((am
           for (int f = 0; f < NF; ++f) {
             const uint32_t back = static_cast<uint32_t>(max(fetch_row(f, lane) - last, 0)) * stride;
             const uint32_t off = (KW == 1 ? kept_offset[f] : fetch_offset(f, lane)) - back;
-            fetch_to_lds(qb, off, dst + f * 1024);
-            fetch_to_lds(gb, off, dst + T::kBytes + f * 1024);
+            fetch_end_to_lds(qb, off, dst + f * 1024);
+            fetch_end_to_lds(gb, off, dst + T::kBytes + f * 1024);
           }
         }
         if (wave == 0) {
@@ -400,15 +397,15 @@ __global__ __launch_bounds__((Dkv32Shape<D, KW, P>::kThreads)) __attribute__((am
 }
 
 template <int KIND, int D, int KW, int P, int OCC>
-DkvLaunch launch_of() {
+BwdLaunch launch_of() {
   using L = Dkv32Shape<D, KW, P>;
   const bwd_fn fn = bwd_mfma32_dkv_kernel<KIND, D, KW, P, OCC>;
   static std::atomic<uint64_t> allowed_on{0};
-  if (!allow_lds<L::kLdsBytes>(fn, allowed_on)) return DkvLaunch{nullptr, 0, 0, 0};
-  return DkvLaunch{fn, L::kLdsBytes, L::kThreads, L::kKeys};
+  if (!allow_lds<L::kLdsBytes>(fn, allowed_on)) return BwdLaunch{nullptr, 0, 0, 0};
+  return BwdLaunch{fn, L::kLdsBytes, L::kThreads, L::kKeys};
 }
 template <int KIND, int D>
-DkvLaunch launch_of(int parts) {
+BwdLaunch launch_of(int parts) {
   if (parts == 4) return launch_of<KIND, D, 1, 4, 1>();
   if (parts == 2) return launch_of<KIND, D, 2, 2, 2>();
   return launch_of<KIND, D, 4, 1, 2>();
@@ -427,7 +424,7 @@ constexpr int64_t kComputeUnits = 256;
 // 126, 113, 95 (119); 48 x 256 (1 536) 239, 262, 276 (262); 4 x 4 096, 32 / 8 (4 096) 1 977, 2 056, 2 214 (2 248); 8 / 8 heads, 32 x 128
 // (1 024) 36.0, 37.6, 59 (35.5).  D = 64: 2 x 2 048, 32 / 8 (1 024) 266, 186, 182 (213); 3 x 4 096, 28 / 4 (1 536) 958, 723, 773 (994);
 // 16 / 16 heads: 8 x 128 (512) 22.1, 20.4, 24.6 (21.1); 16 x 310 (2 480) 66, 69, 102 (65).
-DkvLaunch dkv32_launch(const BwdParams& p, int64_t* groups) {
+BwdLaunch dkv32_launch(const BwdParams& p, int64_t* groups) {
   const int64_t blocks = (p.k_tokens + 31) / 32, workgroups = blocks * p.kv_heads;
   const int64_t seqs = std::max<int64_t>(p.num_seqs, 1), mean = std::max<int64_t>(p.q_tokens / seqs, 1), group = p.q_heads / p.kv_heads;
   const int64_t chain = mean / kDkvTile * group, per_seq = std::max(chain, group);
@@ -448,13 +445,13 @@ DkvLaunch dkv32_launch(const BwdParams& p, int64_t* groups) {
     if (strcmp(e, "2") == 0) parts = 2;
     if (strcmp(e, "4") == 0 && workgroups <= 0x7fffffffLL) parts = 4, pairs = true;
   }
-  DkvLaunch launch;
+  BwdLaunch launch;
   if (p.head_dim == 64) {
     launch = p.dtype == ARENO_DT_BF16 ? launch_of<KV_BF16, 64>(parts) : launch_of<KV_F16, 64>(parts);
   } else {
     launch = p.dtype == ARENO_DT_BF16 ? launch_of<KV_BF16, 128>(parts) : launch_of<KV_F16, 128>(parts);
   }
-  *groups = parts < 4 ? (p.k_tokens + launch.key_rows - 1) / std::max(launch.key_rows, 1) : pairs ? (blocks + 1) / 2 : blocks;
+  *groups = parts < 4 ? (p.k_tokens + launch.rows - 1) / std::max(launch.rows, 1) : pairs ? (blocks + 1) / 2 : blocks;
   return launch;
 }
 

@@ -2,18 +2,18 @@
 // 128, 192 and 256.  Same contract as the vector-ALU kernels of attention_backward.hip (fp32 dQ, dK, dV from dO, Q, K, V and the
 // saved output; areno/accel/csrc/attention.cu:244-524 in the reference), same two launches, no atomics:
 //
-//   dq kernel    a workgroup owns 64 or 128 packed query rows of one q head (four waves of 16 or 32 rows) and streams
-//                the keys its rows may see in tiles of 32 through LDS.  Per tile, with the keys as the rows of the products (the
-//                layout of the forward kernel):  S^T = K . Q^T  and  dP^T = V . dO^T  (two products per 16 keys and 32
-//                elements of the head), the online softmax of the forward on S^T, dS^T = P^T * (dP^T - dO . O), and
-//                dQ^T += K^T . dS^T  with the lane's own dS^T values as the B operand (rounded to the inputs' type; at
-//                the wide heads not rounded, split_weights) and K^T read transposed from the same LDS tile.  A row's softmax reference moves as in the forward (the accumulator is rescaled), so
-//                one pass over the keys gives dQ, the row's log-sum-exp and dO . O (left in the workspace).
-//   dkv kernel   (head dims 192 and 256 here, 64 and 128 in attention_backward_dkv.hip) a workgroup owns 96 or 128 packed key
-//                rows of one kv head (16 per wave) and streams, for every q head
-//                of the group, the query rows that may see them in tiles of 32 (Q and dO tiles in LDS, the rows'
-//                statistics next to them):  S = Q . K^T,  dP = dO . V^T,  P = exp2(S - lse),  dS = P * (dP - dO . O),
-//                dV^T += dO^T . P  and  dK^T += Q^T . dS.  Every gradient element has one owner.
+//   dq kernel    (head dims 64 and 128 here) a workgroup owns 64 or 128 packed query rows of one q head (four waves of 16 or
+//                32 rows) and streams the keys its rows may see in tiles of 32 through LDS.  Per tile, with the keys as the
+//                rows of the products (the layout of the forward kernel):  S^T = K . Q^T  and  dP^T = V . dO^T,
+//                the online softmax of the forward on S^T, dS^T = P^T * (dP^T - dO . O), and
+//                dQ^T += K^T . dS^T  with the lane's own dS^T values as the B operand (rounded to the inputs' type) and K^T
+//                read transposed from the same LDS tile.  A row's softmax reference moves as in the forward (the
+//                accumulator is rescaled), so one pass over the keys gives dQ, the row's log-sum-exp and dO . O (left in
+//                the workspace).
+//   dkv kernel   (attention_backward_dkv.hip) a workgroup owns packed key rows of one kv head and streams, for every q head
+//                of the group, the query rows that may see them:  S = Q . K^T,  dP = dO . V^T,  P = exp2(S - lse),
+//                dS = P * (dP - dO . O),  dV^T += dO^T . P  and  dK^T += Q^T . dS.  Every gradient element has one owner.
+// Head dims 192 and 256 have both kernels in attention_backward_wide.hip.
 // Both launches take their blocks in an order that lets their workgroups end together: see block_in_cost_order.
 //
 // The streamed index of a tile (keys in the dq kernel, queries in the dkv kernel) is the contraction index of the
@@ -56,7 +56,7 @@ template <int D>
 struct BmTile {
   static constexpr int RS = D * 2 + 16;
   static constexpr int kChunksPerRow = D * 2 / 16;
-  static constexpr int kChunks = kBmTile * kChunksPerRow / kBmThreads;  // per thread: 1 (D = 64) to 4 (D = 256)
+  static constexpr int kChunks = kBmTile * kChunksPerRow / kBmThreads;  // per thread: 1 (D = 64) or 2 (D = 128)
   static_assert(kBmTile * kChunksPerRow % kBmThreads == 0, "tile chunks");
   static __device__ __forceinline__ int chunk_pos(int r, int c) { return r * RS + (c << 4); }
 };
@@ -92,72 +92,6 @@ __device__ __forceinline__ typename MfmaOps<KIND>::vec8 streamed_operand(const f
   return __builtin_bit_cast(V8, uint4_t{pack_pair<KIND>(x[0][0], x[0][1]), pack_pair<KIND>(x[0][2], x[0][3]),
                                         pack_pair<KIND>(x[1][0], x[1][1]), pack_pair<KIND>(x[1][2], x[1][3])});
 }
-// The same without rounding, for the wide heads (whose 16-bit inputs had fp32 kernels until these took them, and lose
-// nothing by it): the eight values as three operands that add up to them, times a power of two in fp16.
-// bf16 holds eight significant bits with fp32's exponents: the upper half of a value's word, that of the rest and what is
-// left then are its 24.  fp16 holds eleven in a narrow range: the values of a column (the four lane groups) are first
-// scaled together, so that the largest comes to lie in [2^14, 2^15); what three parts leave is 2^-40 of it and less.
-template <int KIND>
-struct SplitWeights {
-  typename MfmaOps<KIND>::vec8 part[3];
-  float unscale;
-};
-template <int KIND>
-__device__ __forceinline__ SplitWeights<KIND> split_weights(const float (&x)[2][4]) {
-  SplitWeights<KIND> s;
-  float scale = 1.0f;
-  if constexpr (KIND == KV_F16) {
-    float most = max_f32(__builtin_fabsf(x[0][0]), __builtin_fabsf(x[0][1]));
-    most = max3_f32(most, __builtin_fabsf(x[0][2]), __builtin_fabsf(x[0][3]));
-    most = max3_f32(most, __builtin_fabsf(x[1][0]), __builtin_fabsf(x[1][1]));
-    most = rows_max(max3_f32(most, __builtin_fabsf(x[1][2]), __builtin_fabsf(x[1][3])));
-    // exponent field of the scale: 2^14 over the largest value's power of two (at most 2^126, for its inverse)
-    const uint32_t field = min(268u - (__builtin_bit_cast(uint32_t, most) >> 23), 253u);
-    scale = __builtin_bit_cast(float, field << 23);
-    s.unscale = __builtin_bit_cast(float, (254u - field) << 23);
-  }
-  uint32_t w[3][4];
-#pragma unroll
-  for (int pair = 0; pair < 4; ++pair) {
-    float a = x[pair >> 1][2 * (pair & 1)], b = x[pair >> 1][2 * (pair & 1) + 1];
-    if constexpr (KIND == KV_F16) {
-      a *= scale;
-      b *= scale;
-    }
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {  // (the subtractions are exact)
-      if constexpr (KIND == KV_F16) {
-        const auto h = __builtin_amdgcn_cvt_pkrtz(a, b);
-        w[i][pair] = __builtin_bit_cast(uint32_t, h);
-        a -= static_cast<float>(h[0]);
-        b -= static_cast<float>(h[1]);
-      } else {
-        const uint32_t ua = __builtin_bit_cast(uint32_t, a), ub = __builtin_bit_cast(uint32_t, b);
-        w[i][pair] = __builtin_amdgcn_perm(ub, ua, 0x07060302u);  // the upper halves, a's in the low one
-        a -= __builtin_bit_cast(float, ua & 0xffff0000u);
-        b -= __builtin_bit_cast(float, ub & 0xffff0000u);
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 3; ++i) s.part[i] = __builtin_bit_cast(typename MfmaOps<KIND>::vec8, uint4_t{w[i][0], w[i][1], w[i][2], w[i][3]});
-  return s;
-}
-// c + columns . the values that the parts add up to.  A tile's products are summed by themselves, the small ones first,
-// so the running sum rounds once per tile.
-// Relative error of dV against 64 bits (four sequences of 300 .. 1 000 tokens, 16 / 8 heads of 256, window 512, fp32 out):
-// rounded weights 1.6e-3 (bf16) and 2.0e-4 (fp16), these 2.7e-7 and 2.8e-7, the fp32 kernels 2.8e-7 and 3.1e-7; all
-// products straight into the running sum 4.5e-7 (bf16).  The price, forward and backward: bf16 343 -> 403 us (365
-// without the sum of its own), fp16 350 -> 414 us; the fp32 kernels take 7 500.
-template <int KIND>
-__device__ __forceinline__ float4_t split_product(typename MfmaOps<KIND>::vec8 columns, const SplitWeights<KIND>& s, float4_t c) {
-  float4_t tile = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int i = 2; i >= 0; --i) tile = MfmaOps<KIND>::mfma(columns, s.part[i], tile);
-  // (on whole vectors: element by element the compiler moves the sums around, 183 copies in the dq kernel at 256)
-  if constexpr (KIND == KV_BF16) return c + tile;
-  return __builtin_elementwise_fma(tile, float4_t{s.unscale, s.unscale, s.unscale, s.unscale}, c);
-}
 template <int KIND>
 __device__ __forceinline__ float operand_element(uint32_t word, int hi) {
   const uint32_t bits = hi ? word >> 16 : word & 0xffffu;
@@ -168,21 +102,17 @@ __device__ __forceinline__ float operand_element(uint32_t word, int hi) {
 // Bound by what a wave issues and waits for between its products, so a tile has one barrier (two LDS buffers), a
 // row's softmax reference mostly stays where it is (no lane swaps, no rescaling), and dP - dO . O comes out of the
 // product, which starts at -(dO . O); the dkv kernel's does too (forward and backward of 2 x 2 048 tokens, 28 / 4 heads of
-// 128, bf16: 435 -> 427 us; heads of 256, which have one buffer and two barriers: within the noise).
+// 128, bf16: 435 -> 427 us).
 template <int KIND, int D>
 __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p) {
   using Ops = MfmaOps<KIND>;
   using V8 = typename Ops::vec8;
   using T = BmTile<D>;
   constexpr int NS = D / 32, NB = D / 16;
-  constexpr bool kSplit = D > 128;
   constexpr int kRows = kBmRows;  // packed rows of the workgroup
   constexpr int kWaveRows = 16;
-  // two buffers per tensor and one barrier a tile, where they fit the 64 KB of a plain launch: all but head dim 256,
-  // whose padded rows make 66 KB of them (the unpadded tiles of mfma32_tiles.hpp would make 64; not built for this kernel)
-  constexpr int kBuffers = 4 * kBmTile * T::RS <= 64 * 1024 ? 2 : 1;
-  __shared__ __attribute__((aligned(16))) char k_lds[kBuffers * kBmTile * T::RS];
-  __shared__ __attribute__((aligned(16))) char v_lds[kBuffers * kBmTile * T::RS];
+  __shared__ __attribute__((aligned(16))) char k_lds[2 * kBmTile * T::RS];
+  __shared__ __attribute__((aligned(16))) char v_lds[2 * kBmTile * T::RS];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -320,7 +250,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
           // The reference of a row is raised only when a score of the wave exceeds its row's by more than 2^kLazy: most
           // tiles then take no lane swaps and no rescaling.  bf16 has room for probabilities up to 2^8 in dS; fp16 may
           // not (dS is packed with them), so there the reference follows every new maximum as it is.
-          constexpr float kLazy = KIND == KV_BF16 || kSplit ? 8.0f : 0.0f;
+          constexpr float kLazy = KIND == KV_BF16 ? 8.0f : 0.0f;
           float mt = max3_f32(sc[0][0], sc[0][1], sc[0][2]);
           mt = max3_f32(mt, sc[0][3], sc[1][0]);
           mt = max3_f32(mt, sc[1][1], sc[1][2]);
@@ -353,21 +283,13 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
               ds[tg][j] = pe * dp[tg][j];
             }
           }
-          if constexpr (kSplit) {
-            const SplitWeights<KIND> dsop = split_weights<KIND>(ds);
+          const V8 dsop = streamed_operand<KIND>(ds);
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-              acc[nb] = split_product<KIND>(tile_transposed_operand<KIND, T>(s_k, nb, lr, lk), dsop, acc[nb]);
-          } else {
-            const V8 dsop = streamed_operand<KIND>(ds);
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-              acc[nb] = Ops::mfma(tile_transposed_operand<KIND, T>(s_k, nb, lr, lk), dsop, acc[nb]);
-          }
+          for (int nb = 0; nb < NB; ++nb)
+            acc[nb] = Ops::mfma(tile_transposed_operand<KIND, T>(s_k, nb, lr, lk), dsop, acc[nb]);
         }
-        if constexpr (kBuffers == 1) __syncthreads();  // every wave has read tile t
-        // (with two buffers: tile t - 1, which lay where t + 1 goes, was read in front of the last barrier)
-        if (t < t1) publish(kBuffers == 2 ? buf ^ 1 : 0);
+        // (tile t - 1, which lay where t + 1 goes, was read in front of the last barrier)
+        if (t < t1) publish(buf ^ 1);
         __syncthreads();
       };
       fetch(t0);
@@ -376,7 +298,7 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
       __syncthreads();
       for (int t = t0; t <= t1; t += 2) {
         step(t, 0);
-        if (t + 1 <= t1) step(t + 1, kBuffers - 1);
+        if (t + 1 <= t1) step(t + 1, 1);
       }
     }
 
@@ -645,291 +567,36 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
   }
 }
 
-// ---- dK, dV -------------------------------------------------------------------------------------------------------------
-// Head dims 192 and 256 (attention_backward_dkv.hip has 64 and 128).  A workgroup owns a block of KR (96, 128) packed key
-// rows of one kv head, 16 per wave, and streams the query rows that may see them, for every q head of the group.  A key
-// block early in its sequence is seen by all later queries and one late in it by few: the expensive blocks start first
-// (block_in_cost_order).
-template <int D, int KR>
-struct DkvShape {
-  static constexpr int kKeyWaves = KR / 16;
-  static constexpr int kThreads = kKeyWaves * kWave;
-  static constexpr int RS = BmTile<D>::RS;
-  static constexpr int kChunksPerRow = BmTile<D>::kChunksPerRow;
-  static constexpr int kChunks = kBmTile * kChunksPerRow / kThreads;  // 16-byte chunks of a tile per thread
-  static_assert(kBmTile * kChunksPerRow % kThreads == 0, "tile chunks");
-  static constexpr int kTile = kBmTile * RS;
-  static constexpr int kStat = kBmTile * 2 * 4;
-  // per buffer: a Q tile, a dO tile, the rows' statistics
-  static constexpr int kBuffer = 2 * kTile + kStat;
-  static constexpr int kLdsBytes = 2 * kBuffer;
-};
-extern __shared__ __attribute__((aligned(16))) char bm_dkv_lds[];
-
-template <int KIND, int D, int KR>
-__global__ __launch_bounds__((DkvShape<D, KR>::kThreads), 1) void bwd_mfma_dkv_kernel(
-    BwdParams p) {
-  using Ops = MfmaOps<KIND>;
-  using V8 = typename Ops::vec8;
-  using T = BmTile<D>;
-  using L = DkvShape<D, KR>;
-  constexpr int NS = D / 32, NB = D / 16;
-
-  const int tid = threadIdx.x;
-  char* const lds = bm_dkv_lds;
-  auto s_q = [&](int buf) { return lds + buf * L::kBuffer; };
-  auto s_g = [&](int buf) { return lds + buf * L::kBuffer + L::kTile; };
-  auto s_stat = [&](int buf) { return reinterpret_cast<float*>(lds + buf * L::kBuffer + 2 * L::kTile); };  // [row][2]
-
-  const int lane = tid & (kWave - 1);
-  const int wave = uniform(tid >> 6);
-  const int lr = lane & 15, lk = lane >> 4;
-  const int kvh = static_cast<int>(blockIdx.x % static_cast<unsigned>(p.kv_heads));
-  const int group = p.q_heads / p.kv_heads;
-  const int64_t k_blocks = (p.k_tokens + KR - 1) / KR;
-  const int64_t wg = blockIdx.x / static_cast<unsigned>(p.kv_heads);
-  const int64_t block = block_in_cost_order(wg, k_blocks, p.num_seqs, false);
-  {
-    const int64_t r0 = block * KR;
-    const int64_t block_end = r0 + KR < p.k_tokens ? r0 + KR : p.k_tokens;
-    const int64_t row = r0 + 16 * wave + lr;  // this lane's key row (a column of the products)
-    const bool row_exists = row < p.k_tokens;
-
-    // this lane's parts of its row of K and V (B operands)
-    const int64_t row_elem = (row * p.kv_heads + kvh) * D;
-    V8 kop[NS], vop[NS];
-#pragma unroll
-    for (int sl = 0; sl < NS; ++sl) {
-      uint4_t kw = {0u, 0u, 0u, 0u}, vw = kw;
-      if (row_exists) {
-        const int64_t off = (row_elem + (D / 4) * lk + 8 * sl) * 2;
-        kw = load16(p.k, off);
-        vw = load16(p.v, off);
-      }
-      kop[sl] = __builtin_bit_cast(V8, kw);
-      vop[sl] = __builtin_bit_cast(V8, vw);
-    }
-    float4_t acc_k[NB], acc_v[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) acc_k[nb] = acc_v[nb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-
-    for (int s = seq_of_row(p.cu_k, p.num_seqs, r0); s < p.num_seqs; ++s) {
-      const int64_t sk0 = p.cu_k[s], sk1 = p.cu_k[s + 1];
-      if (sk0 >= block_end) break;
-      const int64_t k_lo = sk0 > r0 ? sk0 : r0, k_hi = sk1 < block_end ? sk1 : block_end;
-      if (k_lo >= k_hi) continue;
-      const int ctx = p.ctx != nullptr ? p.ctx[s] : 0;
-      const int64_t q_base = p.cu_q[s];
-      const int n_q = p.cu_q[s + 1] - p.cu_q[s];
-      const bool live = row >= k_lo && row < k_hi;
-      const int key = live ? static_cast<int>(row - sk0) : -1;  // this lane's key position in the sequence
-      const uint64_t live_lanes = __builtin_amdgcn_ballot_w64(live);
-      const bool wave_live = live_lanes != 0, wave_full = live_lanes == ~0ull;
-      // (the wave's 16 key rows, when all of them belong to this sequence)
-      const int wave_key_lo = static_cast<int>(r0 + 16 * wave - sk0), wave_key_hi = wave_key_lo + 15;
-      // queries i (position ctx + i) that see one of the block's keys: key <= ctx + i <= key + window
-      const int key_min = static_cast<int>(k_lo - sk0), key_max = static_cast<int>(k_hi - 1 - sk0);
-      const int i_lo = key_min - ctx > 0 ? key_min - ctx : 0;
-      int i_hi = n_q - 1;
-      if (p.window_left >= 0 && key_max + p.window_left - ctx < i_hi) i_hi = key_max + p.window_left - ctx;
-      if (i_hi < i_lo) continue;  // (the same for the whole workgroup)
-      const int t0 = i_lo / kBmTile, t1 = i_hi / kBmTile;
-      const int tiles = t1 - t0 + 1;
-      // the stream: tiles of every q head of the group, head by head
-      const int steps = tiles * group;
-      // (head, tile) of a step of the stream
-      struct Cursor {
-        int head, tile;
-      };
-      auto advance = [&](Cursor& c) {
-        if (++c.tile > t1) {
-          c.tile = t0;
-          ++c.head;
-        }
-      };
-      const Cursor first = {kvh * group, t0};
-
-      // Two register sets hold the tiles of the next two steps while they are in flight; a step computes on one of
-      // the two LDS buffers, moves the next step's tile into the other one and asks for the tile two steps further on.
-      struct Staged {
-        uint4_t q[L::kChunks], g[L::kChunks];
-        float2_t stat;
-      };
-      Staged set_a, set_b;
-      Cursor fetch_at = first;
-      int fetched = 0;
-      auto fetch = [&](Staged& st) {
-        if (fetched >= steps) return;
-        ++fetched;
-        const int hq = fetch_at.head, t = fetch_at.tile;
-        advance(fetch_at);
-#pragma unroll
-        for (int i = 0; i < L::kChunks; ++i) {
-          const int c = tid + L::kThreads * i;
-          const int r = c / T::kChunksPerRow, col = c % T::kChunksPerRow;
-          const int qi = kBmTile * t + r < n_q ? kBmTile * t + r : n_q - 1;  // rows past the end repeat the last query
-          const int64_t off = ((q_base + qi) * p.q_heads + hq) * (D * 2) + col * 16;
-          st.q[i] = load16(p.q, off);
-          st.g[i] = load16(p.grad_out, off);
-        }
-        if (tid < kBmTile) {
-          const int qi = kBmTile * t + tid < n_q ? kBmTile * t + tid : n_q - 1;
-          st.stat = *reinterpret_cast<const float2_t*>(p.row_stats + (hq * p.q_tokens + q_base + qi) * 2);
-        }
-      };
-      auto publish = [&](const Staged& st, int buf) {
-#pragma unroll
-        for (int i = 0; i < L::kChunks; ++i) {
-          const int c = tid + L::kThreads * i;
-          const int r = c / T::kChunksPerRow, col = c % T::kChunksPerRow;
-          *reinterpret_cast<uint4_t*>(s_q(buf) + T::chunk_pos(r, col)) = st.q[i];
-          *reinterpret_cast<uint4_t*>(s_g(buf) + T::chunk_pos(r, col)) = st.g[i];
-        }
-        if (tid < kBmTile) *reinterpret_cast<float2_t*>(s_stat(buf) + 2 * tid) = st.stat;
-      };
-      Cursor at = first;  // the step being computed
-      // one step: the products of the tile in LDS buffer `buf`; between them the next step's tile goes from `next`
-      // into the other buffer and `next` is asked to fetch again
-      auto step_on = [&](int step, int buf, Staged& next) {
-        const int t = at.tile;
-        advance(at);
-        const bool compute = wave_live;
-        float pr[2][4], ds[2][4];
-        auto first_products = [&](auto masked) {
-#pragma unroll
-          for (int tg = 0; tg < 2; ++tg) {
-            // the statistics of the four query rows this lane gets from the products: rows 16 tg + 4 lk .. + 3
-            const float4_t st01 = *reinterpret_cast<const float4_t*>(s_stat(buf) + 2 * (16 * tg + 4 * lk));
-            const float4_t st23 = *reinterpret_cast<const float4_t*>(s_stat(buf) + 2 * (16 * tg + 4 * lk + 2));
-            const float lse[4] = {st01[0], st01[2], st23[0], st23[2]};
-            float4_t c1 = {0.0f, 0.0f, 0.0f, 0.0f};
-            float4_t c2 = {st01[1], st01[3], st23[1], st23[3]};  // -(dO . O): dP comes out less it
-#pragma unroll
-            for (int sl = 0; sl < NS; ++sl) {
-              c1 = Ops::mfma(tile_row_operand<KIND, T, D>(s_q(buf), tg, sl, lr, lk), kop[sl], c1);
-              c2 = Ops::mfma(tile_row_operand<KIND, T, D>(s_g(buf), tg, sl, lr, lk), vop[sl], c2);
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              float x = c1[j] * p.scale_log2e - lse[j];
-              if constexpr (decltype(masked)::value) {
-                const int qi = kBmTile * t + 16 * tg + 4 * lk + j;  // query of the sequence
-                const int pos = ctx + qi;
-                const bool ok = live && qi < n_q && key <= pos && (p.window_left < 0 || key >= pos - p.window_left);
-                x = ok ? x : kBmNegInf;
-              }
-              // (a query without visible keys has +inf as its log-sum-exp: exp2(-inf) = 0 either way)
-              const float pe = fast_exp2(x);
-              pr[tg][j] = pe;
-              ds[tg][j] = pe * c2[j];
-            }
-          }
-        };
-        if (compute) {
-          // most tiles lie below the diagonal and inside the window as a whole: every query of the tile sees every
-          // key of this wave, and nothing needs a mask
-          const int pos_lo = ctx + kBmTile * t, pos_hi = pos_lo + kBmTile - 1;
-          const bool plain = wave_full && kBmTile * t + kBmTile <= n_q && pos_lo >= wave_key_hi &&
-                             (p.window_left < 0 || pos_hi - p.window_left <= wave_key_lo);
-          if (plain) {
-            first_products(std::false_type{});
-          } else {
-            first_products(std::true_type{});
-          }
-        }
-        if (step + 1 < steps) publish(next, buf ^ 1);
-        fetch(next);
-        if (compute) {
-          if constexpr (D > 128) {
-            SplitWeights<KIND> w = split_weights<KIND>(pr);
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-              acc_v[nb] = split_product<KIND>(tile_transposed_operand<KIND, T>(s_g(buf), nb, lr, lk), w, acc_v[nb]);
-            w = split_weights<KIND>(ds);
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-              acc_k[nb] = split_product<KIND>(tile_transposed_operand<KIND, T>(s_q(buf), nb, lr, lk), w, acc_k[nb]);
-          } else {
-            const V8 pop = streamed_operand<KIND>(pr);
-            const V8 dsop = streamed_operand<KIND>(ds);
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-              acc_v[nb] = Ops::mfma(tile_transposed_operand<KIND, T>(s_g(buf), nb, lr, lk), pop, acc_v[nb]);
-              acc_k[nb] = Ops::mfma(tile_transposed_operand<KIND, T>(s_q(buf), nb, lr, lk), dsop, acc_k[nb]);
-            }
-          }
-        }
-        __syncthreads();  // every wave has read this step's tile, the next one is in place
-      };
-      // (every wave has passed a barrier behind the last use of the buffers: an earlier sequence's last step)
-      fetch(set_a);
-      fetch(set_b);
-      publish(set_a, 0);
-      fetch(set_a);
-      __syncthreads();
-      for (int step = 0; step < steps; step += 2) {
-        step_on(step, 0, set_b);
-        if (step + 1 < steps) step_on(step + 1, 1, set_a);
-      }
-    }
-
-    // every gradient element is written, also the zeros of keys no query sees
-    if (row_exists) {
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        const int64_t at_elem = row_elem + 4 * lk + 16 * nb;
-        store_grad4(p.grad_k, at_elem, acc_k[nb][0] * p.scale, acc_k[nb][1] * p.scale, acc_k[nb][2] * p.scale,
-                    acc_k[nb][3] * p.scale, p.grad_dtype);
-        store_grad4(p.grad_v, at_elem, acc_v[nb][0], acc_v[nb][1], acc_v[nb][2], acc_v[nb][3], p.grad_dtype);
-      }
-    }
-  }
-}
-
 constexpr int64_t kBmComputeUnits = 256;
-
-// Head dims 192 and 256 have one shape: the sums and operands of 16 key rows take all registers of two waves per SIMD,
-// and six or eight waves behind one stream of tiles stage two chunks of a tensor per thread and step (with four waves it
-// would be four chunks, twice the staging registers).  At 256 the kernel still keeps some of its staging in scratch, a
-// dozen loads and half as many stores in every two steps of the tile loop; at 192 a few registers, outside it.
-template <int KIND, int D>
-DkvLaunch dkv_launch() {
-  constexpr int KR = D == 256 ? 128 : 96;
-  using L = DkvShape<D, KR>;
-  const bwd_fn fn = bwd_mfma_dkv_kernel<KIND, D, KR>;
-  static std::atomic<uint64_t> allowed_on{0};
-  if (!allow_lds<L::kLdsBytes>(fn, allowed_on)) return DkvLaunch{nullptr, 0, 0, 0};
-  return DkvLaunch{fn, L::kLdsBytes, L::kThreads, KR};
-}
 
 // Whether the vector-ALU kernels take a launch of wide heads in less time.  A matrix-core workgroup goes through the
 // sequences of its block one after the other, at least one tile each (the dkv kernel for every q head of the group);
 // the vector-ALU kernels have a wave per row and do not care.  For sequences of 64 tokens and more the matrix cores
 // win by up to 30 times, for many single tokens they lose by as much; in between both are estimated, in us, from what
-// 624 launches took (head dims 192 and 256, both types, 1 .. 512 sequences of 1 .. 64 tokens, six head ratios: the one
-// taken is at most 8 % slower than the other).  vector ALU, matrix cores, in us: 64 sequences of 1 token, 32 / 1 heads
-// of 256, bf16: 82, 9 035; 512 x 4 tokens, 8 / 1 heads of 192, fp16: 346, 638; 8 x 32, 16 / 1 of 256, bf16: 286, 316; 64 x 16,
-// 16 heads of 256, bf16: 834, 121; 1 token, 8 / 1 heads of 256, fp16: 54, 51; 300 tokens, bf16: 801, 441.
-bool vector_alu_is_faster(const BwdParams& p, int key_rows) {
+// launches of 1 .. 300 sequences of 1 .. 64 tokens took (head dims 192 and 256, four head ratios; the matrix cores within 23 %
+// of 9 in 10).  vector ALU, matrix cores, in us, 16 / 8 heads of 256, bf16: 8 x 4 tokens 58, 96; 64 x 1 59, 467; 64 x 4 155, 145; 8 x 16
+// 86, 54; 300 x 2 383, 275.
+bool vector_alu_is_faster(const BwdParams& p) {
   const bool d256 = p.head_dim == 256;
   auto ceil_div = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   // (lengths are taken to be about equal; a window of w shows w + 1 keys to a query)
   const int64_t seqs = p.num_seqs, group = p.q_heads / p.kv_heads;
   const int64_t queries = std::max<int64_t>(p.q_tokens / seqs, 1), keys = std::max<int64_t>(p.k_tokens / seqs, 1);
   const int64_t reach = p.window_left >= 0 ? p.window_left + int64_t{1} : INT32_MAX;
-  // matrix cores: sequences in a block, tiles of each, rounds of workgroups; us per step of the dkv and the dq kernel
-  const int64_t dkv_steps = std::min(seqs, std::max<int64_t>(key_rows / keys, 1)) * ceil_div(std::min(queries, reach + key_rows), kBmTile) * group *
-                            ceil_div(ceil_div(p.k_tokens, key_rows) * p.kv_heads, kBmComputeUnits);
+  // matrix cores: sequences in a block, steps of each, rounds of workgroups
+  const int parts = dkv32_wide_parts(p);
+  const int64_t dkv_rows = 64 / parts, dkv_rounds = ceil_div(ceil_div(p.k_tokens, dkv_rows) * p.kv_heads, kBmComputeUnits);
+  const int64_t dkv_steps = std::min(seqs, std::max<int64_t>(dkv_rows / keys, 1)) *
+                            ceil_div(ceil_div(std::min(queries, reach + dkv_rows), kBmTile) * group, parts) * dkv_rounds;
   const int64_t dq_steps = std::min(seqs, std::max<int64_t>(kBmRows / queries, 1)) * ceil_div(std::min(keys, reach + kBmRows), kBmTile) *
                            ceil_div(ceil_div(p.q_tokens, kBmRows) * p.q_heads, 2 * kBmComputeUnits);
-  const double dkv_us = d256 ? 4.2 : 2.7, dq_us = d256 ? 6.8 : 4.8;
-  const double matrix_cores = 8 + dkv_us * dkv_steps + dq_us * dq_steps;
+  const double matrix_cores = d256 ? 21 * dkv_rounds + 2.8 * dkv_steps + 6.5 * dq_steps : 16.5 * dkv_rounds + 2.4 * dkv_steps + 4.4 * dq_steps;
   // vector ALU: all rows' work, or one row's chain, 16 keys or pairs at a time
   const double seen = static_cast<double>(std::min(keys, reach)), pairs = static_cast<double>(std::min(queries, reach) * group);
   const double work = (d256 ? 0.0245 : 0.0182) * (static_cast<double>(p.q_tokens * p.q_heads) * std::max(1.0, seen / 24) +
                                                   static_cast<double>(p.k_tokens * p.kv_heads) * std::max(1.0, pairs / 48));
   const double chain = d256 ? 43 + 4.6 * pairs / 16 + 5.0 * seen / 16 : 33 + 3.0 * pairs / 16 + 3.5 * seen / 16;
-  return std::max(work, chain) < matrix_cores;
+  return std::max(work, chain) * 1.1 < matrix_cores;
 }
 
 }  // namespace
@@ -960,42 +627,36 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
     if (strcmp(e, "32") == 0) dq_rows = 32;
     if (strcmp(e, "16") == 0) dq_rows = 16;
   }
-  // Head dims 192 and 256 (the sliding-window layers of wide heads) have one shape of either kernel.  2 717 tokens in
-  // four sequences, 16 / 8 heads of 256, window 512, bf16, forward and backward: 403 us (weights kept in 32 bits, see
-  // split_weights) against 7 500 us on the vector-ALU kernels, which recompute every product on 16 lanes' dot products.
-  // (Not for many very short sequences, unless a switch fixes the shapes.)
+  // (head dims 192 and 256: not for many very short sequences, unless a switch fixes the shapes)
   if (p.head_dim > 128) {
-    if (getenv("ARENO_BACKWARD_DQ_ROWS") == nullptr && vector_alu_is_faster(p, p.head_dim == 256 ? 128 : 96)) return ARENO_ERR_UNSUPPORTED;
-    dq_rows = 16;
+    if (getenv("ARENO_BACKWARD_DQ_ROWS") == nullptr && vector_alu_is_faster(p)) return ARENO_ERR_UNSUPPORTED;
   }
-  const int64_t dq_blocks = (p.q_tokens + kBmWaves * dq_rows - 1) / (kBmWaves * dq_rows);
-  bwd_fn dq;
-  DkvLaunch dkv;
+  BwdLaunch dq, dkv;
   int64_t dkv_groups = 0;  // workgroups of a kv head
-  if (p.head_dim == 64) {
-    dq = dq_rows == 32 ? (bf16 ? bwd_mfma32_dq_kernel<KV_BF16, 64> : bwd_mfma32_dq_kernel<KV_F16, 64>)
-                       : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 64> : bwd_mfma_dq_kernel<KV_F16, 64>);
-    dkv = dkv32_launch(p, &dkv_groups);
-  } else if (p.head_dim == 192) {
-    dq = bf16 ? bwd_mfma_dq_kernel<KV_BF16, 192> : bwd_mfma_dq_kernel<KV_F16, 192>;
-    dkv = bf16 ? dkv_launch<KV_BF16, 192>() : dkv_launch<KV_F16, 192>();
-  } else if (p.head_dim == 256) {
-    dq = bf16 ? bwd_mfma_dq_kernel<KV_BF16, 256> : bwd_mfma_dq_kernel<KV_F16, 256>;
-    dkv = bf16 ? dkv_launch<KV_BF16, 256>() : dkv_launch<KV_F16, 256>();
+  if (p.head_dim > 128) {
+    dq = dq32_wide_launch(p);
+    dkv = dkv32_wide_launch(p, &dkv_groups);
   } else {
-    dq = dq_rows == 32 ? (bf16 ? bwd_mfma32_dq_kernel<KV_BF16, 128> : bwd_mfma32_dq_kernel<KV_F16, 128>)
-                       : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 128> : bwd_mfma_dq_kernel<KV_F16, 128>);
+    bwd_fn fn;
+    if (p.head_dim == 64) {
+      fn = dq_rows == 32 ? (bf16 ? bwd_mfma32_dq_kernel<KV_BF16, 64> : bwd_mfma32_dq_kernel<KV_F16, 64>)
+                         : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 64> : bwd_mfma_dq_kernel<KV_F16, 64>);
+    } else {
+      fn = dq_rows == 32 ? (bf16 ? bwd_mfma32_dq_kernel<KV_BF16, 128> : bwd_mfma32_dq_kernel<KV_F16, 128>)
+                         : (bf16 ? bwd_mfma_dq_kernel<KV_BF16, 128> : bwd_mfma_dq_kernel<KV_F16, 128>);
+    }
+    dq = BwdLaunch{fn, 0, kBmThreads, kBmWaves * dq_rows};
     dkv = dkv32_launch(p, &dkv_groups);
   }
   const char* op = "areno_hip_attention_backward";
-  if (dkv.fn == nullptr) return fail(ARENO_ERR_LAUNCH, "%s: the dkv kernel's LDS size was refused", op);
+  if (dq.fn == nullptr || dkv.fn == nullptr) return fail(ARENO_ERR_LAUNCH, "%s: the kernels' LDS size was refused", op);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (q_blocks > 0) {
-    hipLaunchKernelGGL(dq, dim3(static_cast<unsigned>(dq_blocks * p.q_heads)), dim3(kBmThreads), 0, s, p);
+    const int64_t dq_blocks = (p.q_tokens + dq.rows - 1) / dq.rows;
+    hipLaunchKernelGGL(dq.fn, dim3(static_cast<unsigned>(dq_blocks * p.q_heads)), dim3(dq.threads), dq.lds_bytes, s, p);
     if (int rc = check_launch(op)) return rc;
   }
   if (k_blocks > 0) {
-    if (dkv_groups == 0) dkv_groups = (p.k_tokens + dkv.key_rows - 1) / dkv.key_rows;
     hipLaunchKernelGGL(dkv.fn, dim3(static_cast<unsigned>(dkv_groups * p.kv_heads)), dim3(dkv.threads), dkv.lds_bytes, s, p);
     if (int rc = check_launch(op)) return rc;
   }

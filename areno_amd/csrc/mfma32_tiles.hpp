@@ -83,6 +83,11 @@ struct LdsTile {
 __device__ __forceinline__ void fetch_to_lds(const char* base, uint32_t offset, uint32_t lds) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(offset), "s"(base), "{m0}"(lds) : "memory");
 }
+// The same for the offsets of a tile that the sequence ends in.  (Another text, so that the compiler keeps the two paths
+// apart instead of clamping every tile's rows.)
+__device__ __forceinline__ void fetch_end_to_lds(const char* base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 ; end" : : "v"(offset), "s"(base), "{m0}"(lds) : "memory");
+}
 // the same for 64 words of 4 bytes
 __device__ __forceinline__ void fetch_words_to_lds(const char* base, uint32_t offset, uint32_t lds) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(offset), "s"(base), "{m0}"(lds) : "memory");
@@ -92,6 +97,16 @@ __device__ __forceinline__ void fetched() { asm volatile("s_waitcnt vmcnt(0) lgk
 // The wave's fetches have landed and its LDS reads are in registers; then every wave's have: the tiles asked for may be
 // read and the tiles read so far may be fetched over.
 __device__ __forceinline__ void fetched_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory"); }
+
+// Every wave's LDS accesses are done; fetches stay in flight.
+__device__ __forceinline__ void handed_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : : : "memory"); }
+
+// The lane's number, worked out where it is needed (the sums leave no register to keep it in).
+__device__ __forceinline__ int lane_now() {
+  int x;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(x));
+  return x;
+}
 
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
   return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)p));

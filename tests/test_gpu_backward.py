@@ -264,6 +264,26 @@ def test_key_gradients_where_blocks_and_tiles_end(dtype, parts, hq, hkv, d, wind
         assert err <= unit * max(want.norm().item(), scale), f"{name} {dtype} {hq}/{hkv} d={d} lens={lens}: {err / want.norm().item():.3g}"
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("parts", ["1", "2"])
+@pytest.mark.parametrize("hq,hkv,d,window_left", [(4, 2, 256, None), (3, 3, 192, 33), (4, 1, 192, None), (2, 1, 256, 31)])
+@pytest.mark.parametrize("lens", [[63, 64, 65, 1, 129], [33, 0, 31, 2, 97], [32]])
+def test_wide_heads_where_blocks_and_tiles_end(dtype, parts, hq, hkv, d, window_left, lens, monkeypatch):
+    """Head dims 192 and 256, the dkv kernel with its stream of tiles in one part and in two: sequences one off blocks of 64
+    and 32 rows and off tiles, windows one off a tile.  The bar is that of the 32-bit weights above."""
+    monkeypatch.setenv("ARENO_BACKWARD_PARTS", parts)
+    monkeypatch.setenv("ARENO_BACKWARD_DQ_ROWS", "16")  # (and not the kernels that a launch's estimate may prefer)
+    g = torch.Generator().manual_seed(d + len(lens))
+    t = sum(lens)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=DEV)
+    q, k, v, go = (torch.randn(t, h, d, generator=g).to(dtype).to(DEV) for h in (hq, hkv, hkv, hq))
+    out = ops.areno_varlen_causal_attention(q, k, v, cu, window_left=window_left)
+    got = _c_backward(go, q, k, v, out, cu, torch.float32, d**-0.5, -1 if window_left is None else window_left)
+    for x, want, name in zip(got, _gradients_in_64_bits(go, q, k, v, out, lens, window_left, d**-0.5), ("dq", "dk", "dv")):
+        err = ((x.cpu().double() - want).norm() / want.norm()).item()
+        assert err <= 4e-6, f"{name} {dtype} {hq}/{hkv} d={d} lens={lens}: {err:.3g}"
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("query_start,window_left", [(0, None), (7, None), (3, 5)])
 def test_dense_backward(dtype, query_start, window_left):
