@@ -901,33 +901,52 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
   }
 }
 
-// Merge of the items cut by unit borders.  Workgroup (u, kv head) takes the last item of unit u, if that item starts
-// in unit u and runs on into later units: it combines the partials of all units the item touches, normalises and
-// writes the item's rows.
+// Merge of the items cut by unit borders.  Workgroup (i, kv head, part) takes the i-th unit whose last item starts in it
+// and runs on into later units: it combines the partials of all units the item touches, normalises and writes its
+// part of the item's rows.
 //
 // What the item is, unit u has left in `cuts`: finding it again from the sequences' lengths, as every workgroup did,
-// is a walk through more code than there is work (28 / 4 heads of 128: 42 -> 22 us for the follow-ups of
-// 4 sequences, up to 64 tokens on 4 k cached ones, about 11 pieces per item; 32 / 8 heads, 16 chunks of up to 512 tokens on
-// 16 k cached ones: 30 -> 15 us).  Bound by latency and by how many compute
-// units pull: a workgroup is a chain of round trips to partials that other XCDs wrote.  So an item's rows are spread
-// over many small workgroups (blockIdx.z; each thread has kMergeChunks 16-byte chunks of every partial), and
-// kMergeBatch partials are asked for before the first of them is used.
+// is a walk through more code than there is work.  Bound by latency, by how many compute units pull, and by the
+// dispatch of workgroups (3 ns each: with one for every unit and part, whether or not the unit has left an item, most of a
+// small launch was empty workgroups).  So the launch has no more of them than the token count allows items, an
+// item's rows are spread over many small workgroups (blockIdx.z; each thread has kMergeChunks 16-byte chunks of every
+// partial), and kMergeBatch partials are asked for before the first of them is used.
+// Kernel time, us: 28 / 4 heads of 128, the follow-ups of 4 sequences, up to 64 tokens on 4 k cached ones, about 11
+// partials per item: 22.5 -> 10.9 (with one chunk per thread 12.0, with batches of 4 12.4); 32 / 8 heads, 16 chunks of up to
+// 512 tokens on 16 k cached ones, an item to merge in almost every unit: 15.
 constexpr int kMergeThreads = 256;
 constexpr int kMergeChunks = 2;
-constexpr int kMergeBatch = 4;
+constexpr int kMaxMergeRounds = kMaxPrefillUnits / kWave;
 
+template <int kMergeBatch>
 __global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(PrefillParams p) {
   const int tid = threadIdx.x;
-  const int unit = blockIdx.x;
-  const CutItem cut = p.cuts[unit];
+  const int lane = tid & (kWave - 1);
+  // the blockIdx.x-th unit that has left something; where the launch has a workgroup for every unit: that unit, or nothing
+  int unit = blockIdx.x;
+  if (static_cast<int>(gridDim.x) < p.units) {
+    int first[kMaxMergeRounds], nth = unit;
+    unit = -1;
+#pragma unroll
+    for (int r = 0; r < kMaxMergeRounds; ++r) first[r] = kWave * r + lane < p.units ? p.cuts[kWave * r + lane].first_slot : -1;
+#pragma unroll
+    for (int r = 0; r < kMaxMergeRounds; ++r) {
+      const uint64_t has = __builtin_amdgcn_ballot_w64(first[r] >= 0);
+      const bool mine = first[r] >= 0 && __builtin_popcountll(has & ((uint64_t{1} << lane) - 1)) == nth;
+      const uint64_t chosen = __builtin_amdgcn_ballot_w64(mine);
+      if (unit < 0 && chosen != 0) unit = kWave * r + __builtin_ctzll(chosen);
+      nth -= __builtin_popcountll(has);  // (below zero behind the chosen one: no lane has that rank)
+    }
+  }
+  const CutItem cut = p.cuts[max(unit, 0)];
   if (cut.end < p.tokens) {  // rows behind the last sequence, the end of a padded pack, become zeros
     const int64_t words_per_row = static_cast<int64_t>(p.q_heads) * (p.head_dim / 4), words = p.tokens * words_per_row;
     const int64_t wgs = static_cast<int64_t>(gridDim.x) * gridDim.y * gridDim.z;
-    const int64_t wg = (static_cast<int64_t>(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + unit;
+    const int64_t wg = (static_cast<int64_t>(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
     for (int64_t w = cut.end * words_per_row + wg * kMergeThreads + tid; w < words; w += wgs * kMergeThreads)
       *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + w * 8) = uint2_t{0u, 0u};
   }
-  if (cut.first_slot < 0) return;
+  if (unit < 0 || cut.first_slot < 0) return;
   const int vhead = blockIdx.y;
   const int kvh = p.head_parts > 1 ? vhead / p.head_parts : vhead;
   const int head0 = kvh * p.group + 16 * (vhead - kvh * p.head_parts);
@@ -1208,8 +1227,12 @@ int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out
   const dim3 grid(p.units, vheads);
   hipLaunchKernelGGL(fn, grid, dim3(kPrefillThreads), 0, static_cast<hipStream_t>(stream), p);
   if (int rc = check_launch(op)) return rc;
+  // (at least one: the merge also writes the zeros behind the last sequence)
+  const int64_t cut_items = std::max<int64_t>(std::min<int64_t>(p.units, tokens / block_tokens + num_seqs), 1);
   const int merge_parts = (rows_per_wg * (cache->head_dim / 4) + kMergeChunks * kMergeThreads - 1) / (kMergeChunks * kMergeThreads);
-  hipLaunchKernelGGL(prefill_merge_kernel, dim3(p.units, vheads, merge_parts), dim3(kMergeThreads), 0,
+  // (fewer items than units: several partials each, all of them asked for at once)
+  hipLaunchKernelGGL(cut_items < p.units ? prefill_merge_kernel<12> : prefill_merge_kernel<4>,
+                     dim3(static_cast<unsigned>(cut_items), vheads, merge_parts), dim3(kMergeThreads), 0,
                      static_cast<hipStream_t>(stream), p);
   return check_launch(op);
 }

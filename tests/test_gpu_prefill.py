@@ -251,6 +251,17 @@ def test_prefill_one_query_block_cut_by_many_shares(kv):
     assert_close(_run_prefill(w), _expected_prefill(w), *tolerances(kv), what="one block, many shares")
 
 
+@pytest.mark.parametrize("hq,hkv", [(4, 1), (8, 2), (16, 8), (40, 2)])
+@pytest.mark.parametrize("lens,ctxs", [([5], [1600]), ([3, 70], [0, 900]), ([1, 0, 2, 90], [700, 5, 350, 0]), ([200] * 9, [40] * 9)])
+def test_prefill_few_items_over_many_shares(hq, hkv, lens, ctxs):
+    """The merge looks its items up among the units (256 of a lone kv head) when the tokens allow fewer items than units:
+    one item in dozens of pieces (and batches), items in units far apart, units without steps, as many items as units.
+    The bar is the file's."""
+    w = workloads.make_prefill_workload("few items", seed=hq, new_lens=torch.tensor(lens), ctx_lens=torch.tensor(ctxs), hq=hq, hkv=hkv,
+                                        d=64, bs=16, kv="bf16", device=DEV, quantize_fn=gpu_quantize)  # fmt: skip
+    assert_close(_run_prefill(w), _expected_prefill(w), *tolerances("bf16"), what=f"{hq}/{hkv} {lens[:4]}")
+
+
 def test_prefill_sequences_without_new_tokens_and_single_tokens():
     """Empty chunks (cu_seqlens repeats) between chunks of 1, 33 and 200 tokens; contexts 0, tile-aligned and odd."""
     new = torch.tensor([0, 1, 0, 33, 1, 0, 200, 0])
