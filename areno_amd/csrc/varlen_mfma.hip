@@ -254,26 +254,45 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
     const int k0 = t * TK;
     if (!wave_live || k0 > wave_qmax) return;
     if (p.window_left >= 0 && k0 + TK - 1 < wave_qmin - p.window_left) return;
-    const char* kt_lds = vm_lds + buf * S::kBuffer;
+    char* kt_lds = vm_lds + buf * S::kBuffer;
     char* vt_lds = vm_lds + buf * S::kBuffer + T::kBytes;
     float16_t s[KT];
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) s[kt] = zero16();
+    // Wide heads: the products' operands in one stream, each read kAhead products in front of its own (the compiler, short of
+    // registers, waits for most of them right behind the read): rows of K, then columns of V.  2 x 4 500 tokens, 16 / 8 heads of
+    // 256, window 1 024: 165 -> 160 us; up to head dim 128 it changes the time by -7 to +3 % and is not used.
+    constexpr int kScores = NKS * KT, kReads = kScores + 2 * KT * NB, kAhead = D == 256 ? 3 : 4;
+    auto read = [&](int x) {
+      if (x < kScores) return tile_rows<KIND, T>(kt_lds, at_rows, 32 * (x % KT), x / KT);
+      return tile_columns<KIND, T>(vt_lds, at_columns, 16 * ((x - kScores) / NB), (x - kScores) % NB);
+    };
+    V8 operand[kAhead];
+    if constexpr (D > 128) {
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
+      for (int x = 0; x < kAhead; ++x) operand[x] = read(x);
 #pragma unroll
-      for (int kt = 0; kt < KT; ++kt) s[kt] = M::mfma(tile_rows<KIND, T>(kt_lds, at_rows, 32 * kt, ks), qop[ks], s[kt]);
+      for (int x = 0; x < kScores; ++x) {
+        __builtin_amdgcn_sched_barrier(0);
+        s[x % KT] = M::mfma(operand[x % kAhead], qop[x / KT], s[x % KT]);
+        operand[x % kAhead] = read(x + kAhead);
+      }
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) s[kt] = M::mfma(tile_rows<KIND, T>(kt_lds, at_rows, 32 * kt, ks), qop[ks], s[kt]);
+      }
+      // four operand reads ahead of the products: left alone the compiler waits for
+      // every pair of reads right behind it (4 x 4 096 tokens, 32 / 8 heads of 128: 577 -> 557 us)
+      __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, kAhead, 0);
+#pragma unroll
+      for (int x = 0; x < NKS * KT - kAhead; ++x) {
+        __builtin_amdgcn_sched_group_barrier(kSchedMatrix, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(kSchedMatrix, kAhead, 0);
     }
-    // four operand reads ahead of the products (two where registers are short): left alone the compiler waits for
-    // every pair of reads right behind it (4 x 4 096 tokens, 32 / 8 heads of 128: 577 -> 557 us)
-    constexpr int kAhead = D <= 128 ? 4 : 2;
-    __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, kAhead, 0);
-#pragma unroll
-    for (int x = 0; x < NKS * KT - kAhead; ++x) {
-      __builtin_amdgcn_sched_group_barrier(kSchedMatrix, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(kSchedLdsRead, 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(kSchedMatrix, kAhead, 0);
     if (k0 + TK - 1 > wave_qmin || (p.window_left >= 0 && k0 < wave_qmax - p.window_left)) {
       const int hi = q_pos - k0 - 4 * h;
       const int lo = p.window_left >= 0 ? hi - p.window_left : -0x40000000;
@@ -333,7 +352,16 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
 #pragma unroll
     for (int b = 0; b < 2 * KT; ++b) {
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) acc[nb] = M::mfma(tile_columns<KIND, T>(vt_lds, at_columns, 16 * b, nb), pop[b], acc[nb]);
+      for (int nb = 0; nb < NB; ++nb) {
+        const int x = kScores + b * NB + nb;
+        if constexpr (D > 128) {
+          __builtin_amdgcn_sched_barrier(0);
+          acc[nb] = M::mfma(operand[x % kAhead], pop[b], acc[nb]);
+          if (x + kAhead < kReads) operand[x % kAhead] = read(x + kAhead);
+        } else {
+          acc[nb] = M::mfma(read(x), pop[b], acc[nb]);
+        }
+      }
     }
   };
 
