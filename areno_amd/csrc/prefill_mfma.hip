@@ -901,14 +901,14 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
   }
 }
 
-// Merge of the items cut by unit borders.  Workgroup (i, kv head, part) takes the i-th unit whose last item starts in it
-// and runs on into later units: it combines the partials of all units the item touches, normalises and writes its
-// part of the item's rows.
+// Merge of the items cut by unit borders.  Workgroup (i, kv head, part) takes unit i, or with PER_ITEM the i-th unit, whose last
+// item starts in it and runs on into later units: it combines the partials of all units the item touches, normalises
+// and writes its part of the item's rows.
 //
 // What the item is, unit u has left in `cuts`: finding it again from the sequences' lengths, as every workgroup did,
 // is a walk through more code than there is work.  Bound by latency, by how many compute units pull, and by the
 // dispatch of workgroups (3 ns each: with one for every unit and part, whether or not the unit has left an item, most of a
-// small launch was empty workgroups).  So the launch has no more of them than the token count allows items, an
+// small launch was empty workgroups).  So such a launch has no more of them than the token count allows items, an
 // item's rows are spread over many small workgroups (blockIdx.z; each thread has kMergeChunks 16-byte chunks of every
 // partial), and kMergeBatch partials are asked for before the first of them is used.
 // Kernel time, us: 28 / 4 heads of 128, the follow-ups of 4 sequences, up to 64 tokens on 4 k cached ones, about 11
@@ -916,29 +916,38 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
 // 512 tokens on 16 k cached ones, an item to merge in almost every unit: 15.
 constexpr int kMergeThreads = 256;
 constexpr int kMergeChunks = 2;
-constexpr int kMaxMergeRounds = kMaxPrefillUnits / kWave;
 
-template <int kMergeBatch>
+template <bool PER_ITEM>
 __global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(PrefillParams p) {
+  constexpr int kMergeBatch = PER_ITEM ? 12 : 4;
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
-  // the blockIdx.x-th unit that has left something; where the launch has a workgroup for every unit: that unit, or nothing
   int unit = blockIdx.x;
-  if (static_cast<int>(gridDim.x) < p.units) {
-    int first[kMaxMergeRounds], nth = unit;
+  CutItem cut;
+  if constexpr (!PER_ITEM) {
+    cut = p.cuts[unit];
+  } else {  // the blockIdx.x-th unit that has left something
+    // a lane looks at a unit, and the chosen one hands over what it has read; the next 64 are asked for meanwhile
+    int nth = unit;
     unit = -1;
-#pragma unroll
-    for (int r = 0; r < kMaxMergeRounds; ++r) first[r] = kWave * r + lane < p.units ? p.cuts[kWave * r + lane].first_slot : -1;
-#pragma unroll
-    for (int r = 0; r < kMaxMergeRounds; ++r) {
-      const uint64_t has = __builtin_amdgcn_ballot_w64(first[r] >= 0);
-      const bool mine = first[r] >= 0 && __builtin_popcountll(has & ((uint64_t{1} << lane) - 1)) == nth;
-      const uint64_t chosen = __builtin_amdgcn_ballot_w64(mine);
-      if (unit < 0 && chosen != 0) unit = kWave * r + __builtin_ctzll(chosen);
-      nth -= __builtin_popcountll(has);  // (below zero behind the chosen one: no lane has that rank)
+    CutItem next = p.cuts[min(lane, p.units - 1)];
+    for (int u0 = 0; u0 < p.units && unit < 0; u0 += kWave) {
+      const CutItem mine = next;
+      if (u0 + kWave < p.units) next = p.cuts[min(u0 + kWave + lane, p.units - 1)];
+      const uint64_t has = __builtin_amdgcn_ballot_w64(u0 + lane < p.units && mine.first_slot >= 0);
+      const bool here = (has >> lane & 1) != 0 && __builtin_popcountll(has & ((uint64_t{1} << lane) - 1)) == nth;
+      const uint64_t chosen = __builtin_amdgcn_ballot_w64(here);
+      const int from = chosen != 0 ? __builtin_ctzll(chosen) : 0;
+      if (chosen != 0) unit = u0 + from;
+      nth -= __builtin_popcountll(has);
+      cut.first_slot = __builtin_amdgcn_readlane(mine.first_slot, from);
+      cut.total = __builtin_amdgcn_readlane(mine.total, from);
+      cut.step_end = __builtin_amdgcn_readlane(mine.step_end, from);
+      cut.token0 = __builtin_amdgcn_readlane(mine.token0, from);
+      cut.tokens = __builtin_amdgcn_readlane(mine.tokens, from);
+      cut.end = __builtin_amdgcn_readlane(mine.end, from);
     }
   }
-  const CutItem cut = p.cuts[max(unit, 0)];
   if (cut.end < p.tokens) {  // rows behind the last sequence, the end of a padded pack, become zeros
     const int64_t words_per_row = static_cast<int64_t>(p.q_heads) * (p.head_dim / 4), words = p.tokens * words_per_row;
     const int64_t wgs = static_cast<int64_t>(gridDim.x) * gridDim.y * gridDim.z;
@@ -1227,12 +1236,20 @@ int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out
   const dim3 grid(p.units, vheads);
   hipLaunchKernelGGL(fn, grid, dim3(kPrefillThreads), 0, static_cast<hipStream_t>(stream), p);
   if (int rc = check_launch(op)) return rc;
-  // (at least one: the merge also writes the zeros behind the last sequence)
-  const int64_t cut_items = std::max<int64_t>(std::min<int64_t>(p.units, tokens / block_tokens + num_seqs), 1);
-  const int merge_parts = (rows_per_wg * (cache->head_dim / 4) + kMergeChunks * kMergeThreads - 1) / (kMergeChunks * kMergeThreads);
-  // (fewer items than units: several partials each, all of them asked for at once)
-  hipLaunchKernelGGL(cut_items < p.units ? prefill_merge_kernel<12> : prefill_merge_kernel<4>,
-                     dim3(static_cast<unsigned>(cut_items), vheads, merge_parts), dim3(kMergeThreads), 0,
+  // Far fewer items than units, and more workgroups than compute units if each unit had its own: a workgroup per item that
+  // there can be (at least one: the merge also writes the zeros behind the last sequence), several partials each, all of
+  // them asked for at once.  Otherwise one per unit: finding the item costs a round trip, and fewer workgroups of 170
+  // registers fit.  Norm, rotary, write and attention with a workgroup per unit and per item, us: 28 / 4 heads (64 units, blocks of
+  // 36 tokens), 1 x 8 tokens on 4 k cached 43.0, 36.4; 1 x 512 on 1 k 50.4, 41.8; 8 x 32 on 300 30.5, 25.6; 16 x 100 on 8 k 130.5,
+  // 134.5; 16 / 16 heads (16 units, blocks of 256): 1 x 512 on 1 k 61.1, 30.3; 8 x 32 on 300 22.9, 25.9; 1 x 8 on 4 k 22.2, 23.0 (the two that lose stay with units);
+  // 8 / 2 heads (128 units, blocks of 64): 8 x 32 on 300 25.9, 21.4; 1 x 8 on 4 k 45.5, 46.5 (its loss is accepted).
+  const int64_t items = std::max<int64_t>(tokens / block_tokens + num_seqs, 1);
+  const int64_t rows = std::min<int64_t>(rows_per_wg, tokens * fold);  // of an item
+  const int merge_parts = static_cast<int>((rows * (cache->head_dim / 4) + kMergeChunks * kMergeThreads - 1) / (kMergeChunks * kMergeThreads));
+  const bool per_item = 4 * items <= p.units && static_cast<int64_t>(p.units) * vheads * merge_parts > 256;
+  const unsigned cut_items = static_cast<unsigned>(per_item ? items : p.units);
+  hipLaunchKernelGGL(per_item ? prefill_merge_kernel<true> : prefill_merge_kernel<false>,
+                     dim3(cut_items, vheads, merge_parts), dim3(kMergeThreads), 0,
                      static_cast<hipStream_t>(stream), p);
   return check_launch(op);
 }
