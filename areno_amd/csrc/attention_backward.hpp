@@ -64,18 +64,20 @@ __device__ inline __attribute__((always_inline)) void store_grad4(void* base, in
     *reinterpret_cast<f16x4*>(static_cast<_Float16*>(base) + i) = __builtin_convertvector(v, f16x4);
   }
 }
-// the last sequence that starts at or in front of `row` (the one that holds it, when the row exists)
+// The last sequence that starts at or in front of `row` (the one that holds it, when the row exists).  Every lane looks at one
+// of 64 places, so up to 64 sequences take one round trip to memory where halving took one per bit of their number, with
+// nothing else under way.  (All lanes of the wave take part; `row` is the same for them.)
 __device__ inline __attribute__((always_inline)) int seq_of_row(const int32_t* cu, int num_seqs, int64_t row) {
-  int lo = 0, hi = num_seqs;
-  while (lo + 1 < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (static_cast<int64_t>(cu[mid]) <= row) {
-      lo = mid;
-    } else {
-      hi = mid;
-    }
+  const int lane = static_cast<int>(threadIdx.x) & 63;
+  int first = 0;
+  for (int left = num_seqs; left > 1;) {  // among [first, first + left)
+    const int apart = (left + 63) >> 6, at = lane * apart;
+    const bool starts = at < left && static_cast<int64_t>(cu[first + at]) <= row;
+    const int behind = (__builtin_popcountll(__builtin_amdgcn_ballot_w64(starts)) - 1) * apart;
+    if (behind > 0) first += behind, left -= behind;
+    left = left < apart ? left : apart;
   }
-  return lo;
+  return first;
 }
 
 // a kernel with its launch shape

@@ -102,9 +102,13 @@ __device__ __forceinline__ float operand_element(uint32_t word, int hi) {
 // Bound by what a wave issues and waits for between its products, so a tile has one barrier (two LDS buffers), a
 // row's softmax reference mostly stays where it is (no lane swaps, no rescaling), and dP - dO . O comes out of the
 // product, which starts at -(dO . O); the dkv kernel's does too (forward and backward of 2 x 2 048 tokens, 28 / 4 heads of
-// 128, bf16: 435 -> 427 us).
+// 128, bf16: 435 -> 427 us).  Short sequences are mostly a block's start: its sequence is found in one round trip, the first
+// tile is on its way together with Q.  In a step the operands are read ahead of their products and the exponentials go
+// between the products of dP.  Forward and backward, us, before and with these: 16 x 20 .. 600 tokens, 16 heads of 64, fp16: 83.6,
+// 80.8; 12 x 100 .. 900, 32 / 8 heads of 64, bf16: 134.7, 131.1 (137 with three waves per SIMD, hence the bound of four); 6 x 60 ..
+// 450, 28 / 4 heads of 128, fp16: 90.0, 86.9.
 template <int KIND, int D>
-__global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p) {
+__global__ __launch_bounds__(kBmThreads, D == 64 ? 4 : 2) void bwd_mfma_dq_kernel(BwdParams p) {
   using Ops = MfmaOps<KIND>;
   using V8 = typename Ops::vec8;
   using T = BmTile<D>;
@@ -129,73 +133,75 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
   row = wave_row0 + lr;
 
   int covered = 0;  // (where the sequences seen so far end)
-  for (int s = seq_of_row(p.cu_q, p.num_seqs, r0); s < p.num_seqs; ++s) {
-    const int64_t sq0 = p.cu_q[s], sq1 = covered = p.cu_q[s + 1];
-    if (sq0 >= block_end) break;
+  int s = uniform(seq_of_row(p.cu_q, p.num_seqs, r0));
+  for (int64_t sq0 = uniform(p.cu_q[s]), sq1; s < p.num_seqs && sq0 < block_end; ++s, sq0 = sq1) {
+    // (asked for together)
+    const int q_end = p.cu_q[s + 1], k_begin = p.cu_k[s], k_end = p.cu_k[s + 1], before = p.ctx != nullptr ? p.ctx[s] : 0;
+    sq1 = covered = uniform(q_end);
     const int64_t q_lo = sq0 > r0 ? sq0 : r0, q_hi = sq1 < block_end ? sq1 : block_end;
     if (q_lo >= q_hi) continue;
-    const int ctx = p.ctx != nullptr ? p.ctx[s] : 0;
-    const int64_t k_base = p.cu_k[s];
-    const int n_k = p.cu_k[s + 1] - p.cu_k[s];
-    bool live;
-    int pos;
-    bool wave_live = false, wave_full = true;
-    live = row >= q_lo && row < q_hi;
-    pos = live ? ctx + static_cast<int>(row - sq0) : -1;
+    const int ctx = uniform(before);
+    const int64_t k_base = uniform(k_begin);
+    const int n_k = uniform(k_end) - static_cast<int>(k_base);
+    const bool live = row >= q_lo && row < q_hi;
+    const int pos = live ? ctx + static_cast<int>(row - sq0) : -1;
     const uint64_t live_lanes = __builtin_amdgcn_ballot_w64(live);
-    wave_live = wave_live || live_lanes != 0;
-    wave_full = wave_full && live_lanes == ~0ull;
+    const bool wave_live = live_lanes != 0, wave_full = live_lanes == ~0ull;
     // (the positions of the wave's query rows, when all of them belong to this sequence)
     const int wave_pos_lo = ctx + static_cast<int>(wave_row0 - sq0), wave_pos_hi = wave_pos_lo + kWaveRows - 1;
     const int pos_min = ctx + static_cast<int>(q_lo - sq0), pos_max = ctx + static_cast<int>(q_hi - 1 - sq0);
     const int key_lo = p.window_left >= 0 ? (pos_min - p.window_left > 0 ? pos_min - p.window_left : 0) : 0;
     const int key_hi = pos_max < n_k - 1 ? pos_max : n_k - 1;
 
-    // this lane's parts of its rows of Q and dO (B operands), and dO . O
-    int64_t row_elem;
-    V8 qop[NS], gop[NS];
-    float delta;
-    float4_t acc[NB];
-    float m_run, l_lane;
-    row_elem = (row * p.q_heads + h) * D;
-    float d = 0.0f;
+    const int t0 = key_lo / kBmTile, t1 = key_hi / kBmTile;
+    uint4_t kreg[T::kChunks], vreg[T::kChunks];
+    auto fetch = [&](int t) {
 #pragma unroll
-    for (int sl = 0; sl < NS; ++sl) {
-      uint4_t qw = {0u, 0u, 0u, 0u}, gw = qw, ow = qw;
-      if (live) {
-        const int64_t off = (row_elem + (D / 4) * lk + 8 * sl) * 2;
-        qw = load16(p.q, off);
-        gw = load16(p.grad_out, off);
-        ow = load16(p.out, off);
+      for (int i = 0; i < T::kChunks; ++i) {
+        const int c = tid + kBmThreads * i;
+        const int r = c / T::kChunksPerRow, col = c % T::kChunksPerRow;
+        const int key = kBmTile * t + r < n_k ? kBmTile * t + r : n_k - 1;  // rows past the end repeat the last key
+        const int64_t off = ((k_base + key) * p.kv_heads + kvh) * (D * 2) + col * 16;
+        kreg[i] = load16(p.k, off);
+        vreg[i] = load16(p.v, off);
       }
-      qop[sl] = __builtin_bit_cast(V8, qw);
-      gop[sl] = __builtin_bit_cast(V8, gw);
+    };
+    // this lane's parts of its rows of Q and dO (B operands), and dO . O; the first tile is asked for behind them, so that
+    // both are on their way together
+    const int64_t row_elem = (row * p.q_heads + h) * D;
+    V8 qop[NS], gop[NS];
+    float4_t acc[NB];
+    float m_run = kBmNegInf, l_lane = 0.0f, d = 0.0f;
+    {
+      uint4_t qw[NS], gw[NS], ow[NS];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        d += operand_element<KIND>(gw[j], 0) * operand_element<KIND>(ow[j], 0) +
-             operand_element<KIND>(gw[j], 1) * operand_element<KIND>(ow[j], 1);
+      for (int sl = 0; sl < NS; ++sl) qw[sl] = gw[sl] = ow[sl] = uint4_t{0u, 0u, 0u, 0u};
+      if (live) {
+#pragma unroll
+        for (int sl = 0; sl < NS; ++sl) {
+          const int64_t off = (row_elem + (D / 4) * lk + 8 * sl) * 2;
+          qw[sl] = load16(p.q, off);
+          gw[sl] = load16(p.grad_out, off);
+          ow[sl] = load16(p.out, off);
+        }
+      }
+      if (key_hi >= key_lo) fetch(t0);
+#pragma unroll
+      for (int sl = 0; sl < NS; ++sl) {
+        qop[sl] = __builtin_bit_cast(V8, qw[sl]);
+        gop[sl] = __builtin_bit_cast(V8, gw[sl]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          d += operand_element<KIND>(gw[sl][j], 0) * operand_element<KIND>(ow[sl][j], 0) +
+               operand_element<KIND>(gw[sl][j], 1) * operand_element<KIND>(ow[sl][j], 1);
+        }
       }
     }
-    delta = rows_sum(d);
+    const float delta = rows_sum(d);
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[nb] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    m_run = kBmNegInf;
-    l_lane = 0.0f;
 
     if (key_hi >= key_lo) {  // (the same for the whole workgroup)
-      const int t0 = key_lo / kBmTile, t1 = key_hi / kBmTile;
-      uint4_t kreg[T::kChunks], vreg[T::kChunks];
-      auto fetch = [&](int t) {
-#pragma unroll
-        for (int i = 0; i < T::kChunks; ++i) {
-          const int c = tid + kBmThreads * i;
-          const int r = c / T::kChunksPerRow, col = c % T::kChunksPerRow;
-          const int key = kBmTile * t + r < n_k ? kBmTile * t + r : n_k - 1;  // rows past the end repeat the last key
-          const int64_t off = ((k_base + key) * p.kv_heads + kvh) * (D * 2) + col * 16;
-          kreg[i] = load16(p.k, off);
-          vreg[i] = load16(p.v, off);
-        }
-      };
       auto publish = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < T::kChunks; ++i) {
@@ -210,42 +216,37 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
         char* const s_v = v_lds + buf * (kBmTile * T::RS);
         if (t < t1) fetch(t + 1);
         if (wave_live) {
-          float sc[2][4], dp[2][4];
-          auto first_products = [&](auto masked) {
-#pragma unroll
-            for (int tg = 0; tg < 2; ++tg) {
-              float4_t c1, c2;
-              c1 = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-              c2 = float4_t{-delta, -delta, -delta, -delta};  // dP comes out less dO . O
-#pragma unroll
-              for (int sl = 0; sl < NS; ++sl) {
-                const V8 k_rows = tile_row_operand<KIND, T, D>(s_k, tg, sl, lr, lk);
-                const V8 v_rows = tile_row_operand<KIND, T, D>(s_v, tg, sl, lr, lk);
-                c1 = Ops::mfma(k_rows, qop[sl], c1);
-                c2 = Ops::mfma(v_rows, gop[sl], c2);
-              }
-#pragma unroll
-              for (int j = 0; j < 4; ++j) {
-                sc[tg][j] = c1[j];  // (the softmax scale goes in with the reference, below)
-                if constexpr (decltype(masked)::value) {
-                  const int key = kBmTile * t + 16 * tg + 4 * lk + j;
-                  const bool ok =
-                      key <= pos && key < n_k && (p.window_left < 0 || key >= pos - p.window_left);
-                  sc[tg][j] = ok ? sc[tg][j] : kBmNegInf;
-                }
-                dp[tg][j] = c2[j];
-              }
-            }
+          // the products' operands in one stream, each read kAhead products in front of its own: rows of K and of V (the
+          // two groups of 16 in turn, so that a product does not wait for the one before), columns of K
+          constexpr int kAhead = 4, kRowReads = 2 * NS, kReads = 2 * kRowReads + NB;
+          auto read = [&](int x) {
+            if (x < kRowReads) return tile_row_operand<KIND, T, D>(s_k, x & 1, x >> 1, lr, lk);
+            if (x < 2 * kRowReads) return tile_row_operand<KIND, T, D>(s_v, x & 1, (x - kRowReads) >> 1, lr, lk);
+            return tile_transposed_operand<KIND, T>(s_k, x - 2 * kRowReads, lr, lk);
           };
+          V8 operand[kAhead];
+#pragma unroll
+          for (int x = 0; x < kAhead; ++x) operand[x] = read(x);
+          float4_t sc[2] = {}, dp[2];
+#pragma unroll
+          for (int x = 0; x < kRowReads; ++x) {
+            __builtin_amdgcn_sched_barrier(0);
+            sc[x & 1] = Ops::mfma(operand[x % kAhead], qop[x >> 1], sc[x & 1]);
+            operand[x % kAhead] = read(x + kAhead);
+          }
           // most tiles lie below the diagonal and inside the window as a whole: every query row of this wave sees
           // every key of the tile, and nothing needs a mask
           const int key_first = kBmTile * t, key_last = key_first + kBmTile - 1;
           const bool plain = wave_full && key_last < n_k && key_last <= wave_pos_lo &&
                              (p.window_left < 0 || key_first >= wave_pos_hi - p.window_left);
-          if (plain) {
-            first_products(std::false_type{});
-          } else {
-            first_products(std::true_type{});
+          if (!plain) {
+            const int base = key_first + 4 * lk;  // keys base + 16 tg + j
+            const int last = min(pos, n_k - 1) - base, first = p.window_left < 0 ? -base : pos - p.window_left - base;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const int key = 16 * (e >> 2) + (e & 3);
+              sc[e >> 2][e & 3] = key >= first && key <= last ? sc[e >> 2][e & 3] : kBmNegInf;
+            }
           }
           // The reference of a row is raised only when a score of the wave exceeds its row's by more than 2^kLazy: most
           // tiles then take no lane swaps and no rescaling.  bf16 has room for probabilities up to 2^8 in dS; fp16 may
@@ -272,27 +273,37 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma_dq_kernel(BwdParams p)
             }
           }
           const float m_ref = m_run == kBmNegInf ? 0.0f : m_run;
-          float ds[2][4];
+          dp[0] = dp[1] = float4_t{-delta, -delta, -delta, -delta};  // dP comes out less dO . O
 #pragma unroll
-          for (int tg = 0; tg < 2; ++tg) {
+          for (int x = 0; x < kRowReads; ++x) {
+            __builtin_amdgcn_sched_barrier(0);
+            dp[x & 1] = Ops::mfma(operand[(kRowReads + x) % kAhead], gop[x >> 1], dp[x & 1]);
+            operand[(kRowReads + x) % kAhead] = read(kRowReads + x + kAhead);
+            // the exponentials between the products of dP (exp2(-inf) = 0: masked keys)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              // (exp2(-inf) = 0: masked keys)
-              const float pe = fast_exp2(__builtin_fmaf(sc[tg][j], p.scale_log2e, -m_ref));
+            for (int e = 8 / kRowReads * x; e < 8 / kRowReads * (x + 1); ++e) {
+              const float pe = fast_exp2(__builtin_fmaf(sc[e >> 2][e & 3], p.scale_log2e, -m_ref));
+              sc[e >> 2][e & 3] = pe;
               l_lane += pe;
-              ds[tg][j] = pe * dp[tg][j];
             }
           }
+          __builtin_amdgcn_sched_barrier(0);
+          float ds[2][4];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) ds[e >> 2][e & 3] = sc[e >> 2][e & 3] * dp[e >> 2][e & 3];
           const V8 dsop = streamed_operand<KIND>(ds);
 #pragma unroll
-          for (int nb = 0; nb < NB; ++nb)
-            acc[nb] = Ops::mfma(tile_transposed_operand<KIND, T>(s_k, nb, lr, lk), dsop, acc[nb]);
+          for (int nb = 0; nb < NB; ++nb) {
+            const int x = 2 * kRowReads + nb;
+            __builtin_amdgcn_sched_barrier(0);
+            acc[nb] = Ops::mfma(operand[x % kAhead], dsop, acc[nb]);
+            if (x + kAhead < kReads) operand[x % kAhead] = read(x + kAhead);
+          }
         }
         // (tile t - 1, which lay where t + 1 goes, was read in front of the last barrier)
         if (t < t1) publish(buf ^ 1);
         __syncthreads();
       };
-      fetch(t0);
       __syncthreads();  // the tiles' previous readers (an earlier sequence of this block) are done
       publish(0);
       __syncthreads();

@@ -284,6 +284,26 @@ def test_wide_heads_where_blocks_and_tiles_end(dtype, parts, hq, hkv, d, window_
         assert err <= 4e-6, f"{name} {dtype} {hq}/{hkv} d={d} lens={lens}: {err:.3g}"
 
 
+@pytest.mark.parametrize("seqs", [1, 63, 64, 65, 130])
+@pytest.mark.parametrize("dq_rows", ["16", "32"])
+@pytest.mark.parametrize("hq,hkv,d,dtype", [(2, 1, 64, torch.float16), (2, 2, 128, torch.bfloat16), (2, 1, 256, torch.bfloat16)])
+def test_blocks_find_their_sequence_among_many(seqs, dq_rows, hq, hkv, d, dtype, monkeypatch):
+    """A block looks its sequence up 64 at a time: around 64 and 128 of them, empty ones between them and at both ends, and
+    more than one block long.  The bar of the 16-bit kernels above, one unit of the inputs' type, in the 2-norm."""
+    monkeypatch.setenv("ARENO_BACKWARD_DQ_ROWS", dq_rows)
+    g = torch.Generator().manual_seed(seqs)
+    lens = [(0, 3, 37, 0, 141, 1, 65)[i % 7] for i in range(seqs)] if seqs > 1 else [150]
+    t = sum(lens)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=DEV)
+    q, k, v, go = (torch.randn(t, h, d, generator=g).to(dtype).to(DEV) for h in (hq, hkv, hkv, hq))
+    out = ops.areno_varlen_causal_attention(q, k, v, cu)
+    got = _c_backward(go, q, k, v, out, cu, torch.float32, d**-0.5)
+    unit = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    for x, want, name in zip(got, _gradients_in_64_bits(go, q, k, v, out, lens, None, d**-0.5), ("dq", "dk", "dv")):
+        err = ((x.cpu().double() - want).norm() / want.norm()).item()
+        assert err <= unit, f"{name} {dtype} d={d} seqs={seqs}: {err:.3g}"
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("query_start,window_left", [(0, None), (7, None), (3, 5)])
 def test_dense_backward(dtype, query_start, window_left):
