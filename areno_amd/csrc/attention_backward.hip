@@ -33,6 +33,7 @@ constexpr int kBwdWaves = 4;
 constexpr int kLanesPerKey = 4;
 constexpr int kKeysPerPass = kWave / kLanesPerKey;  // 16
 constexpr float kNegInfB = -__builtin_huge_valf();
+constexpr int32_t kWidestWindow = 1 << 30;
 
 __device__ __forceinline__ int find_seq(const int32_t* cu, int num_seqs, int64_t token) {
   int lo = 0, hi = num_seqs;
@@ -354,7 +355,8 @@ extern "C" int areno_hip_attention_backward_typed(const void* grad_out, const vo
   p.num_seqs = num_seqs;
   p.q_heads = q_heads;
   p.kv_heads = kv_heads;
-  p.window_left = window_left;
+  // (the kernels add the window to positions in 32 bits: a wider one than any keys in memory shows as much as this)
+  p.window_left = window_left < kWidestWindow ? window_left : kWidestWindow;
   p.head_dim = head_dim;
   p.dtype = dtype;
   p.grad_dtype = grad_dtype;

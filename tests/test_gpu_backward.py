@@ -304,6 +304,20 @@ def test_blocks_find_their_sequence_among_many(seqs, dq_rows, hq, hkv, d, dtype,
         assert err <= unit, f"{name} {dtype} d={d} seqs={seqs}: {err:.3g}"
 
 
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float16, 128), (torch.bfloat16, 192), (torch.float16, 256), (torch.bfloat16, 96), (torch.float32, 64)])
+@pytest.mark.parametrize("window_left", [2**31 - 1, 2**31 - 100, 2**30, 2**30 - 1])
+def test_a_window_as_wide_as_its_type_holds_is_none(dtype, d, window_left):
+    """Gradients with the widest windows: those without one, bit for bit (positions and the window are added in 32 bits)."""
+    g = torch.Generator().manual_seed(d)
+    cu = torch.tensor([0, 70, 73, 273], dtype=torch.int32, device=DEV)
+    q, k, v, go = (torch.randn(273, h, d, generator=g).to(dtype).to(DEV) for h in (4, 2, 2, 4))
+    out = ops.areno_varlen_causal_attention(q, k, v, cu)
+    want = _c_backward(go, q, k, v, out, cu, torch.float32, d**-0.5)
+    assert all(x.abs().max() > 0 for x in want)
+    for got, x, name in zip(_c_backward(go, q, k, v, out, cu, torch.float32, d**-0.5, window_left), want, ("dq", "dk", "dv")):
+        assert torch.equal(got, x), f"{name} {dtype} d={d} window={window_left}"
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("query_start,window_left", [(0, None), (7, None), (3, 5)])
 def test_dense_backward(dtype, query_start, window_left):
