@@ -1,11 +1,12 @@
 // dK and dV of the causal varlen / dense attention ops on 32 x 32 x 16 matrix products (gfx950): 16-bit inputs, head dims
-// 64 and 128.  The second launch of attention_backward_mfma.hip, for sequences long enough to fill its tiles; reads the
-// rows' statistics that the dq kernel left.  The reference: areno/accel/csrc/attention.cu:244-524.
+// 64 and 128.  The second launch of attention_backward_mfma.hip; reads the rows' statistics that the dq kernel left.  The reference: areno/accel/csrc/attention.cu:244-524.
 //
 // A wave owns 32 packed key rows of one kv head: K and V of them as B operands and both sums in registers.  It goes
 // through the query rows that may see them, for every q head of the group, in tiles of 32 that the memory pipe puts into
-// LDS:  S = Q . K^T,  dP = dO . V^T - dO . O,  P = exp2(S - lse),  dS = P * dP,  dV^T += dO^T . P,  dK^T += Q^T . dS.  A
-// C tile of the first two is the B operand of the last two as it lies (mfma32_tiles.hpp).
+// LDS:  S = Q . K^T,  dP = dO . V^T - dO . O,  P = exp2(scale S - lse),  dS = P * dP,  dV^T += dO^T . P,  dK^T += Q^T . dS.  A
+// C tile of the first two is the B operand of the last two as it lies (mfma32_tiles.hpp).  S is summed in the order of the
+// dq kernel with 32 rows per wave; the one with 16 sums it in another, so that behind it S and the log-sum-exp differ by
+// S's own roundings (32 bits in both).
 //
 // A workgroup is four waves: KW waves own neighbouring keys and share a stream of tiles, and P such parts own the same keys
 // and take every P-th tile of the stream each; the sums of parts 1 .. P - 1 go to part 0 through LDS at the end, in a fixed
@@ -49,21 +50,9 @@ struct Dkv32Shape {
 };
 extern __shared__ __attribute__((aligned(1024))) char dkv32_lds[];
 
-// x as an A operand whose row sums are x: three bf16 parts (24 bits) in the first elements of lane half 0, and zeros
-__device__ __forceinline__ bf16x8_t three_parts(float x, int half) {
-  uint32_t w[2], u = half == 0 ? __builtin_bit_cast(uint32_t, x) : 0u;
-  const float rest = __builtin_bit_cast(float, u) - __builtin_bit_cast(float, u & 0xffff0000u);  // (exact)
-  const uint32_t v = __builtin_bit_cast(uint32_t, rest);
-  const float last = rest - __builtin_bit_cast(float, v & 0xffff0000u);
-  w[0] = __builtin_amdgcn_perm(v, u, 0x07060302u);  // the upper halves, u's in the low one
-  w[1] = __builtin_bit_cast(uint32_t, last) >> 16;
-  return __builtin_bit_cast(bf16x8_t, uint4_t{w[0], w[1], 0u, 0u});
-}
-
 template <int KIND, int D, int KW, int P, int OCC>
 __global__ __launch_bounds__((Dkv32Shape<D, KW, P>::kThreads)) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void bwd_mfma32_dkv_kernel(BwdParams p) {
   using M = Mfma32<KIND>;
-  using Start = Mfma32<KV_BF16>;
   using V8 = typename M::vec8;
   using L = Dkv32Shape<D, KW, P>;
   using T = typename L::Tile;
@@ -86,8 +75,6 @@ __global__ __launch_bounds__((Dkv32Shape<D, KW, P>::kThreads)) __attribute__((am
   // (with the part's place: a multiple of 256, which the reads' exclusive-ors leave alone)
   static_assert(L::kPart % 256 == 0, "the parts' places");
   uint32_t at_rows = T::rows_base(l32, half) + part * L::kPart, at_columns = T::columns_base(lane) + part * L::kPart;
-  const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, uint4_t{0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u});
-  const float unscale = __builtin_bit_cast(float, uniform(__builtin_bit_cast(int, 1.0f / p.scale_log2e)));  // (the scale is positive)
   const uint32_t lds0 = lds_address(dkv32_lds) + part * L::kPart;
   const uint32_t stride = static_cast<uint32_t>(p.q_heads) * (D * 2);
   // Fetch f of a wave fills kFetchRows rows; the chunk a lane fetches is the one that belongs where its bytes land.  A wave
@@ -220,7 +207,7 @@ __global__ __launch_bounds__((Dkv32Shape<D, KW, P>::kThreads)) __attribute__((am
           }
         }
         if (wave == 0) {
-          fetch_words_to_lds(sb, static_cast<uint32_t>(min(lane >> 1, last)) * 8u + (lane & 1) * 4u,
+          fetch_words_to_lds(sb, static_cast<uint32_t>(min(lane & 31, last)) * 8u + (lane >> 5) * 4u,
                              lds0 + static_cast<uint32_t>(buf * L::kBuffer + 2 * T::kBytes));
         }
         ahead += P;
@@ -257,19 +244,31 @@ __global__ __launch_bounds__((Dkv32Shape<D, KW, P>::kThreads)) __attribute__((am
         };
         constexpr int kReads = 2 * NKS + 4 * NB;
         V8 operand[kAhead];
-        // The statistics go into the products as one more contraction step, so that a lane reads those of one row
-        // instead of sixteen: what is added to S and dP, -lse / scale and -(dO . O), in three bf16 parts times ones.
-        const float2_t stat = *reinterpret_cast<const float2_t*>(q_lds + 2 * T::kBytes + part * L::kPart + 8 * (lane_now() & 31));
+        // The statistics of the rows that this lane has values of, the log-sum-exps and (128 bytes on) -(dO . O): of rows
+        // 8 c + 4 (lane / 32) .. + 3 at 32 c.  P's exponent is rounded once, in its fma: put into the products as a
+        // contraction step (a row's log-sum-exp over the scale in three bf16 parts) it was rounded three times, took two
+        // products more and no less time: backward of 4 x 4 096 tokens, 32 / 8 heads of 128, bf16: 1 851 -> 1 812 us; 12 x 100 .. 900,
+        // 32 / 8 heads of 64: 123 -> 120.
+        const char* const stats = q_lds + 2 * T::kBytes + part * L::kPart + 16 * (lane_now() >> 5);
+        auto stat = [&](int which, int c) { return *reinterpret_cast<const float4_t*>(stats + 128 * which + 32 * c); };
 #pragma unroll
         for (int x = 0; x < kAhead; ++x) operand[x] = read(x);
-        float16_t sc = zero16();
+        float16_t sc = zero16(), dp;
+        float4_t lse[4];  // (each read one group of rows in front of its use)
 #pragma unroll
         for (int x = 0; x < NKS; ++x) {
           __builtin_amdgcn_sched_barrier(0);
           sc = M::mfma(operand[x % kAhead], kop[x], sc);
           operand[x % kAhead] = read(x + kAhead);
+          // (dP comes out less dO . O)
+#pragma unroll
+          for (int c = 4 * x / NKS; c < 4 * (x + 1) / NKS; ++c) {
+            const float4_t start = stat(1, c);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) dp[4 * c + j] = start[j];
+          }
         }
-        sc = Start::mfma(three_parts(max_f32(stat[0] * -unscale, -3e38f), half), ones, sc);
+        if constexpr (!kTight) lse[0] = stat(0, 0);
         if (t < plain_lo || t > plain_hi) {
           const int lane = lane_now();
           const int base = kDkvTile * t + 4 * (lane >> 5);  // queries base + 8 c + j
@@ -284,30 +283,32 @@ __global__ __launch_bounds__((Dkv32Shape<D, KW, P>::kThreads)) __attribute__((am
             sc[e] = q >= first && q <= last ? sc[e] : kDkvNegInf;
           }
         }
-        float16_t dp = zero16();
         V8 pop[2], dsop[2];
         uint32_t w[8], dw[8];
-        // (a query without visible keys has +inf as its log-sum-exp: exp2 of what comes of it is 0)
+        // (a query without visible keys has +inf as its log-sum-exp: exp2(-inf) = 0)
 #pragma unroll
         for (int x = 0; x < NKS; ++x) {
           __builtin_amdgcn_sched_barrier(0);
           dp = M::mfma(operand[(NKS + x) % kAhead], vop[x], dp);
           operand[(NKS + x) % kAhead] = read(NKS + x + kAhead);
+          if (!kTight && 4 * (x + 1) % NKS == 0 && x + 1 < NKS) lse[4 * (x + 1) / NKS] = stat(0, 4 * (x + 1) / NKS);
           if constexpr (!kTight) {  // the exponentials between the products of dP
 #pragma unroll
             for (int e = 16 / NKS * x; e < 16 / NKS * (x + 1); e += 2) {
-              sc[e] = fast_exp2(sc[e] * p.scale_log2e);
-              sc[e + 1] = fast_exp2(sc[e + 1] * p.scale_log2e);
+              sc[e] = fast_exp2(__builtin_fmaf(sc[e], p.scale_log2e, -lse[e >> 2][e & 3]));
+              sc[e + 1] = fast_exp2(__builtin_fmaf(sc[e + 1], p.scale_log2e, -lse[e >> 2][(e & 3) + 1]));
               w[e / 2] = pack_pair<KIND>(sc[e], sc[e + 1]);
             }
           }
         }
-        dp = Start::mfma(three_parts(stat[1], half), ones, dp);
         if constexpr (kTight) {  // (P and dS at once, so that packed ones take the registers of those they come from)
+          lse[0] = stat(0, 0);
 #pragma unroll
           for (int e = 0; e < 16; e += 2) {
             __builtin_amdgcn_sched_barrier(0);
-            const float p0 = fast_exp2(sc[e] * p.scale_log2e), p1 = fast_exp2(sc[e + 1] * p.scale_log2e);
+            if (e % 4 == 0 && e < 12) lse[e / 4 + 1] = stat(0, e / 4 + 1);
+            const float p0 = fast_exp2(__builtin_fmaf(sc[e], p.scale_log2e, -lse[e >> 2][e & 3]));
+            const float p1 = fast_exp2(__builtin_fmaf(sc[e + 1], p.scale_log2e, -lse[e >> 2][(e & 3) + 1]));
             w[e / 2] = pack_pair<KIND>(p0, p1);
             dw[e / 2] = pack_pair<KIND>(p0 * dp[e], p1 * dp[e + 1]);
           }

@@ -618,8 +618,6 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
   // the kernels mask raw scores and take row maxima before scaling: any other scale is for the vector-ALU kernels, as in
   // the forward (launch_prefill_mfma)
   if (!(p.scale_log2e > 0.0f)) return ARENO_ERR_UNSUPPORTED;
-  // (the dkv kernels up to head dim 128 divide a row's log-sum-exp by the scale: 128 / 1e-36 has to stay a number)
-  if (p.head_dim <= 128 && p.scale_log2e < 1e-36f) return ARENO_ERR_UNSUPPORTED;
   if (p.q_heads > 65535 || p.kv_heads > 65535) return ARENO_ERR_UNSUPPORTED;
   const int64_t q_blocks = (p.q_tokens + kBmRows - 1) / kBmRows, k_blocks = (p.k_tokens + kBmRows - 1) / kBmRows;
   if (q_blocks * p.q_heads > 0x7fffffffLL || k_blocks * p.kv_heads > 0x7fffffffLL) return ARENO_ERR_UNSUPPORTED;

@@ -8,6 +8,7 @@ format's rounding at that magnitude, plus the rounding of the saved output that 
 use for dO . O), 1e-4 for fp32."""
 
 import ctypes
+import math
 
 import pytest
 import torch
@@ -247,8 +248,7 @@ def test_wide_heads_keep_their_weights_in_32_bits(dtype, hq, hkv, d, window_left
 @pytest.mark.parametrize("lens,scale", [([31, 33, 32, 97, 128, 129], 0.1), ([1], 0.1), ([161, 0, 1, 2, 95], 2.0), ([64, 65, 63], 1e-3), ([33], 1e-37)])
 def test_key_gradients_where_blocks_and_tiles_end(dtype, parts, hq, hkv, d, window_left, lens, scale, monkeypatch):
     """The dkv kernel of head dims 64 and 128 in each of its shapes and as the launch's size picks them: sequences one off
-    its blocks (32, 64, 128 keys) and tiles, windows one off a tile, rows' statistics divided by small and large scales (the
-    smallest leaves the matrix cores).  The bar, in the 2-norm: P and dS are rounded to the inputs' type, by half a unit
+    its blocks (32, 64, 128 keys) and tiles, windows one off a tile, small and large scales.  The bar, in the 2-norm: P and dS are rounded to the inputs' type, by half a unit
     in the last place at most; one unit."""
     if parts is not None:
         monkeypatch.setenv("ARENO_BACKWARD_PARTS", parts)
@@ -262,6 +262,27 @@ def test_key_gradients_where_blocks_and_tiles_end(dtype, parts, hq, hkv, d, wind
     for x, want, name in zip(got, _gradients_in_64_bits(go, q, k, v, out, lens, window_left, scale), ("dq", "dk", "dv")):
         err = (x.cpu().double() - want).norm().item()
         assert err <= unit * max(want.norm().item(), scale), f"{name} {dtype} {hq}/{hkv} d={d} lens={lens}: {err / want.norm().item():.3g}"
+
+
+@pytest.mark.parametrize("parts", ["1", "2", "4"])
+@pytest.mark.parametrize("dq_rows", ["16", "32"])
+@pytest.mark.parametrize("d", [64, 128])
+def test_probabilities_of_large_scores(d, dq_rows, parts, monkeypatch):
+    """Single tokens with integer queries and keys (every sum of their products is exact): P is 1, dO is 1 and dV is what
+    the dkv kernel made of P.  Its exponent is a difference of a score and a log-sum-exp of the same size, x, which holds
+    the score rounded once (half a unit in the last place, 2^-24 x at most; a quarter more for the exponential and the
+    logarithm); then P is rounded to fp16 (2^-11 at most)."""
+    monkeypatch.setenv("ARENO_BACKWARD_PARTS", parts)
+    monkeypatch.setenv("ARENO_BACKWARD_DQ_ROWS", dq_rows)
+    g = torch.Generator().manual_seed(d)
+    t, h, scale = 200, 4, 0.0917
+    q, k = (torch.randint(-300, 301, (t, h, d), generator=g).to(torch.float16).to(DEV) for _ in range(2))
+    v = torch.randn(t, h, d, generator=g).to(torch.float16).to(DEV)
+    cu = torch.arange(t + 1, dtype=torch.int32, device=DEV)
+    dv = _c_backward(torch.ones_like(v), q, k, v, v, cu, torch.float32, scale)[2].double()
+    x = scale / math.log(2) * (q.double() * k.double()).sum(-1, keepdim=True).abs()
+    assert x.max() > 3e4
+    assert ((dv - 1).abs() <= 1.25 * math.log(2) * 2.0**-24 * x + 2.0**-11).all()
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
