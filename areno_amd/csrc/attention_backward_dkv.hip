@@ -12,7 +12,9 @@
 // and take every P-th tile of the stream each; the sums of parts 1 .. P - 1 go to part 0 through LDS at the end, in a fixed
 // order.  (4, 1) for large launches, two workgroups per compute unit; (2, 2); (1, 4) for small ones, whose time is that of
 // their longest block: there a wave has its tiles for itself, no barrier, and 512 registers.  In a (1, 4) launch of about
-// one workgroup per compute unit it takes block i and then block `blocks - 1 - i`: their costs add up to the same.
+// one workgroup per compute unit it takes block i and then block `blocks - 1 - i`: their costs add up to the same.  (1, 1) is
+// a workgroup of one wave, for many short sequences: in a block of 128 keys each of them is a stream that one wave of four
+// computes on while all wait at its barriers.
 //
 // Bound: (4, 1) by the matrix cores (54 % of the cycles, at the clock that they then leave, 1.66 GHz) and LDS; (1, 4) by
 // what one wave issues, 350 instructions and 34 products of 32 cycles in 2 500.  Where the time was: 16 x 16 x 32 products
@@ -405,8 +407,10 @@ BwdLaunch launch_of() {
   if (!allow_lds<L::kLdsBytes>(fn, allowed_on)) return BwdLaunch{nullptr, 0, 0, 0};
   return BwdLaunch{fn, L::kLdsBytes, L::kThreads, L::kKeys};
 }
+constexpr int kLoneWave = 0;  // for the parts: one wave
 template <int KIND, int D>
 BwdLaunch launch_of(int parts) {
+  if (parts == kLoneWave) return launch_of<KIND, D, 1, 1, D == 64 ? 2 : 1>();
   if (parts == 4) return launch_of<KIND, D, 1, 4, 1>();
   if (parts == 2) return launch_of<KIND, D, 2, 2, 2>();
   return launch_of<KIND, D, 4, 1, 2>();
@@ -425,6 +429,14 @@ constexpr int64_t kComputeUnits = 256;
 // 126, 113, 95 (119); 48 x 256 (1 536) 239, 262, 276 (262); 4 x 4 096, 32 / 8 (4 096) 1 977, 2 056, 2 214 (2 248); 8 / 8 heads, 32 x 128
 // (1 024) 36.0, 37.6, 59 (35.5).  D = 64: 2 x 2 048, 32 / 8 (1 024) 266, 186, 182 (213); 3 x 4 096, 28 / 4 (1 536) 958, 723, 773 (994);
 // 16 / 16 heads: 8 x 128 (512) 22.1, 20.4, 24.6 (21.1); 16 x 310 (2 480) 66, 69, 102 (65).
+// One wave by itself instead of one part, where a block holds several sequences or its streams are a few steps: it has a
+// block of 32 keys to find and to write, so in a launch that fills the chip many times over the streams have to be
+// shorter, at head dim 128 more than at 64.  One part, one wave (the 16-row kernels), us, D = 128: 16 / 16 heads, 4 096 x 8 tokens
+// (16 384 blocks) 910, 774 (954); 64 x 32 (1 024) 31.5, 28.3 (29.5); 300 x 48 (7 200) 212, 199 (228); 100 x 100 (5 000) 149, 146 (168);
+// 16 x 160 (1 280) 47.3, 42.7 (50.4); 32 x 128 (2 048) 52.0, 54.5 (59.0); 100 x 160 (8 000) 226, 239 (247); 8 / 8, 16 x 200 (800) 42.5, 38.1
+// (42.3); 8 / 2, 300 x 48 (900) 92.0, 74.9 (84.2); 24 / 8, 60 x 60 (904) 76.0, 62.9 (71.7); 300 x 80 (6 000) 382, 388 (427).  D = 64: 16 / 16 heads,
+// 4 096 x 8 496, 353 (484); 512 x 16 (4 096) 73.3, 56.7 (71.5); 32 x 96 (1 536) 26.5, 22.7 (25.8); 16 x 160 27.8, 22.4 (26.8); 64 x 200 (6 400)
+// 105, 103 (114); 200 x 128 (12 800) 179, 185 (187); 8 / 2, 300 x 48 55.7, 44.7 (49.9); 28 / 4, 4 096 x 16 (8 192) 700, 554 (690).
 BwdLaunch dkv32_launch(const BwdParams& p, int64_t* groups) {
   const int64_t blocks = (p.k_tokens + 31) / 32, workgroups = blocks * p.kv_heads;
   const int64_t seqs = std::max<int64_t>(p.num_seqs, 1), mean = std::max<int64_t>(p.q_tokens / seqs, 1), group = p.q_heads / p.kv_heads;
@@ -435,13 +447,18 @@ BwdLaunch dkv32_launch(const BwdParams& p, int64_t* groups) {
     parts = 4;
   } else if (workgroups <= (chain >= 64 ? 2304 : chain < 8 ? (mean < 32 ? 1280 : 768) : p.head_dim == 64 ? 2048 : 1280)) {
     parts = 2;
+  } else if (workgroups <= 0x7fffffffLL && (chain <= 3 || (chain <= 6 && workgroups <= (p.head_dim == 64 ? 8192 : 1536)))) {
+    parts = kLoneWave;
   }
   // Pairs of blocks where every one of them then has a compute unit (two share one at head dim 64) and single blocks would not
   const int64_t units = (p.head_dim == 64 ? 2 : 1) * kComputeUnits;
   bool pairs = workgroups > units && (blocks + 1) / 2 * p.kv_heads <= units;
-  // ARENO_BACKWARD_PARTS=1|2|4 (read at every launch; 4 in pairs) fixes the choice: the same dK and dV up to the order of
-  // the last sums, so this is for tests of the kernels a launch of the test's size would not take, and for timing
+  // ARENO_BACKWARD_PARTS=1w|1|2|4s|4 (read at every launch; one wave, 4 with single blocks and in pairs) fixes the choice: the
+  // same dK and dV up to the order of the last sums, so this is for tests of the kernels a launch of the test's size would
+  // not take, and for timing
   if (const char* e = getenv("ARENO_BACKWARD_PARTS")) {
+    if (strcmp(e, "1w") == 0 && workgroups <= 0x7fffffffLL) parts = kLoneWave;
+    if (strcmp(e, "4s") == 0 && workgroups <= 0x7fffffffLL) parts = 4, pairs = false;
     if (strcmp(e, "1") == 0) parts = 1;
     if (strcmp(e, "2") == 0) parts = 2;
     if (strcmp(e, "4") == 0 && workgroups <= 0x7fffffffLL) parts = 4, pairs = true;
@@ -452,7 +469,7 @@ BwdLaunch dkv32_launch(const BwdParams& p, int64_t* groups) {
   } else {
     launch = p.dtype == ARENO_DT_BF16 ? launch_of<KV_BF16, 128>(parts) : launch_of<KV_F16, 128>(parts);
   }
-  *groups = parts < 4 ? (p.k_tokens + launch.rows - 1) / std::max(launch.rows, 1) : pairs ? (blocks + 1) / 2 : blocks;
+  *groups = parts != 4 ? (p.k_tokens + launch.rows - 1) / std::max(launch.rows, 1) : pairs ? (blocks + 1) / 2 : blocks;
   return launch;
 }
 

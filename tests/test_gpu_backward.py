@@ -264,7 +264,28 @@ def test_key_gradients_where_blocks_and_tiles_end(dtype, parts, hq, hkv, d, wind
         assert err <= unit * max(want.norm().item(), scale), f"{name} {dtype} {hq}/{hkv} d={d} lens={lens}: {err / want.norm().item():.3g}"
 
 
-@pytest.mark.parametrize("parts", ["1", "2", "4"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("parts", ["1w", "4s", None])
+@pytest.mark.parametrize("hq,hkv,d,window_left", [(4, 1, 128, None), (16, 16, 128, 33), (8, 2, 64, None), (16, 16, 64, 31)])
+@pytest.mark.parametrize("lens", [[31, 33, 32, 97, 128, 129], [1], [161, 0, 1, 2, 95], [40] * 42 + [0, 7, 1]])
+def test_key_gradients_of_lone_waves_and_of_single_blocks(dtype, parts, hq, hkv, d, window_left, lens, monkeypatch):
+    """The dkv kernel's workgroups of one wave (which a launch of 42 short sequences and 16 kv heads takes by itself) and of four
+    parts with a block each, sequences one off blocks and tiles.  The bar is that of the other shapes."""
+    if parts is not None:
+        monkeypatch.setenv("ARENO_BACKWARD_PARTS", parts)
+    g = torch.Generator().manual_seed(d + len(lens))
+    t = sum(lens)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32, device=DEV)
+    q, k, v, go = (torch.randn(t, h, d, generator=g).to(dtype).to(DEV) for h in (hq, hkv, hkv, hq))
+    out = ops.areno_varlen_causal_attention(q, k, v, cu, window_left=window_left)
+    got = _c_backward(go, q, k, v, out, cu, torch.float32, d**-0.5, -1 if window_left is None else window_left)
+    unit = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    for x, want, name in zip(got, _gradients_in_64_bits(go, q, k, v, out, lens, window_left, d**-0.5), ("dq", "dk", "dv")):
+        err = (x.cpu().double() - want).norm().item()
+        assert err <= unit * max(want.norm().item(), d**-0.5), f"{name} {dtype} {hq}/{hkv} d={d} lens={lens[:6]}: {err / want.norm().item():.3g}"
+
+
+@pytest.mark.parametrize("parts", ["1w", "1", "2", "4"])
 @pytest.mark.parametrize("dq_rows", ["16", "32"])
 @pytest.mark.parametrize("d", [64, 128])
 def test_probabilities_of_large_scores(d, dq_rows, parts, monkeypatch):
