@@ -622,16 +622,21 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
   const int64_t q_blocks = (p.q_tokens + kBmRows - 1) / kBmRows, k_blocks = (p.k_tokens + kBmRows - 1) / kBmRows;
   if (q_blocks * p.q_heads > 0x7fffffffLL || k_blocks * p.kv_heads > 0x7fffffffLL) return ARENO_ERR_UNSUPPORTED;
   const bool bf16 = p.dtype == ARENO_DT_BF16;
-  // The dq kernel with 32 rows per wave over long sequences: 512 tokens on the average at head dim 128, 1 024 at head dim 64
-  // where the launch also has 4 workgroups of 64 rows per compute unit.  The backward with 16 and 32 rows, us: D = 128:
-  // 4 x 4 096 tokens, 32 / 8 heads (32 per unit) 2 183, 1 791; 2 x 2 048, 28 / 4 heads (7) 304, 264; 4 x 600, 32 / 8 (4.6) 140, 134;
-  // 1 x 2 048, 8 heads (1) 97, 93; 1 x 1 024, 8 / 2 heads (0.5) 78, 78; 16 x 256, 28 / 4 (7) 94, 95.  D = 64: 4 x 4 096, 32 / 8 (32) 1 144, 1 054;
-  // 6 x 1 024, 16 heads (6) 91, 87; 1 x 2 048, 28 / 4 (3.5) 125, 124; 1 x 2 048, 16 heads (2) 79, 81; 64 x 512, 28 / 4 (56) 418, 410; 12 x 512,
-  // 16 heads (6) 67.7, 68.6.  A block of many short sequences, which it takes one after the other, is a longer chain in
-  // the larger block: 28 / 4 heads of 128, 512 x 8 tokens (7) 162, 221; 256 x 128 (56) 497, 538; of 64, 256 x 128 (56) 248, 271.
+  // The dq kernel with 32 rows per wave where a row sees many keys and the launch has several workgroups per compute unit:
+  // small launches are their longest block, whose start and end take longer with twice the rows, and so are blocks of
+  // many short sequences, which it takes one after the other.  The backward with 16 and 32 rows, us (in brackets workgroups of 64
+  // rows per unit), D = 128: 4 x 4 096 tokens, 32 / 8 heads (32) 2 194, 1 802; 2 x 2 048, 28 / 4 (7) 286, 255; 1 x 4 096, 16 / 16 (4) 302, 263; 6 / 6
+  // (1.5) 187, 179; 1 x 2 048, 16 / 16 (2) 109, 106; 6 / 6 (0.8) 95.2, 97.1; 4 x 1 024, 16 / 16 (4) 108, 101; 2 x 1 024 (2) 65.3, 66.9; 1 x 1 024 (1) 55.2,
+  // 58.4; 1 x 600 (0.6) 39.0, 44.3; 28 / 4 heads, 4 x 600 (4.2) 161, 155; 64 x 512 (56) 769, 755; 16 x 256 (7) 85.9, 89.9; 256 x 128 (56) 465, 537;
+  // 512 x 8 (7) 158, 229; windows over 4 x 2 048 (14): 1 024 440, 382; 512 296, 271; 256 195, 198; 128 149, 163.  D = 64: 4 x 4 096, 32 / 8 (32)
+  // 1 178, 1 044; 4 x 1 024, 16 / 16 (4) 60.6, 59.4; 2 x 1 024 (2) 40.7, 42.1; 12 x 512 (6) 60.1, 62.3; 28 / 4 heads, 64 x 512 (56) 402, 406; 256 x 128
+  // (56) 243, 272; windows over 4 x 2 048: 512 155, 151; 256 105, 107; 128 75.8, 85.5.
   // ARENO_BACKWARD_DQ_ROWS=16|32 (read at every launch) fixes the choice, for tests and timing.
   const int64_t mean_length = p.q_tokens / (p.num_seqs > 0 ? p.num_seqs : 1);
-  int dq_rows = mean_length >= (p.head_dim == 128 ? 512 : 1024) && (p.head_dim == 128 || q_blocks * p.q_heads >= 4 * kBmComputeUnits) ? 32 : 16;
+  const int64_t seen = p.window_left >= 0 ? std::min<int64_t>(mean_length, p.window_left + int64_t{1}) : mean_length;
+  const int64_t workgroups = q_blocks * p.q_heads;  // (of 64 rows)
+  int dq_rows = p.head_dim == 128 ? ((seen >= 512 && workgroups >= 3 * kBmComputeUnits) || (seen > 1024 && workgroups >= kBmComputeUnits * 3 / 2) ? 32 : 16)
+                                  : (seen >= 512 && mean_length >= 1024 && workgroups >= 4 * kBmComputeUnits ? 32 : 16);
   if (const char* e = getenv("ARENO_BACKWARD_DQ_ROWS")) {
     if (strcmp(e, "32") == 0) dq_rows = 32;
     if (strcmp(e, "16") == 0) dq_rows = 16;
