@@ -955,7 +955,10 @@ __global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(PrefillPar
     for (int64_t w = cut.end * words_per_row + wg * kMergeThreads + tid; w < words; w += wgs * kMergeThreads)
       *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + w * 8) = uint2_t{0u, 0u};
   }
-  if (unit < 0 || cut.first_slot < 0) return;
+  if constexpr (PER_ITEM) {
+    if (unit < 0) return;
+  }
+  if (cut.first_slot < 0) return;  // (by itself: with both in one condition the slots' products took more instructions)
   const int vhead = blockIdx.y;
   const int kvh = p.head_parts > 1 ? vhead / p.head_parts : vhead;
   const int head0 = kvh * p.group + 16 * (vhead - kvh * p.head_parts);
@@ -1239,10 +1242,11 @@ int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out
   // Far fewer items than units, and more workgroups than compute units if each unit had its own: a workgroup per item that
   // there can be (at least one: the merge also writes the zeros behind the last sequence), several partials each, all of
   // them asked for at once.  Otherwise one per unit: finding the item costs a round trip, and fewer workgroups of 170
-  // registers fit.  Norm, rotary, write and attention with a workgroup per unit and per item, us: 28 / 4 heads (64 units, blocks of
-  // 36 tokens), 1 x 8 tokens on 4 k cached 43.0, 36.4; 1 x 512 on 1 k 50.4, 41.8; 8 x 32 on 300 30.5, 25.6; 16 x 100 on 8 k 130.5,
-  // 134.5; 16 / 16 heads (16 units, blocks of 256): 1 x 512 on 1 k 61.1, 30.3; 8 x 32 on 300 22.9, 25.9; 1 x 8 on 4 k 22.2, 23.0 (the two that lose stay with units);
-  // 8 / 2 heads (128 units, blocks of 64): 8 x 32 on 300 25.9, 21.4; 1 x 8 on 4 k 45.5, 46.5 (its loss is accepted).
+  // registers fit.  The attention with a workgroup per unit and per item, us (workgroups of the units in brackets): 28 / 4 heads (64
+  // units, blocks of 36 tokens), 1 x 8 tokens on 4 k cached (1 024) 38.6, 31.9; 8 x 32 on 300 (2 560) 25.1, 20.3; 8 / 1 (256 units, blocks
+  // of 32), 1 x 8 (1 024) 66.4, 50.3; heads of 64, 1 x 8 on 2 k (512) 50.8, 38.1; 8 / 2 (128 units, blocks of 64), 1 x 32 on 2 k 60.9, 31.4;
+  // 4 x 6 on 700 (1 024) 18.7, 19.1; 16 / 16 (16 units, blocks of 256), 1 x 512 on 1 k, with norm, rotary and write, 61.1, 30.3; items
+  // close to the units: 28 / 4, 16 x 100 on 8 k 130.5, 134.5; 16 / 16, 8 x 32 on 300 22.9, 25.9 (the two that lose stay with units).
   const int64_t items = std::max<int64_t>(tokens / block_tokens + num_seqs, 1);
   const int64_t rows = std::min<int64_t>(rows_per_wg, tokens * fold);  // of an item
   const int merge_parts = static_cast<int>((rows * (cache->head_dim / 4) + kMergeChunks * kMergeThreads - 1) / (kMergeChunks * kMergeThreads));
