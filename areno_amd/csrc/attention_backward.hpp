@@ -4,6 +4,8 @@
 #pragma once
 
 #include <stdint.h>
+#include <stdlib.h>
+#include <string.h>
 
 #include <atomic>
 
@@ -78,6 +80,12 @@ __device__ inline __attribute__((always_inline)) int seq_of_row(const int32_t* c
     left = left < apart ? left : apart;
   }
   return first;
+}
+
+// whether a switch has this value (read at every launch)
+inline bool fixed_by(const char* name, const char* value) {
+  const char* const e = getenv(name);
+  return e != nullptr && strcmp(e, value) == 0;
 }
 
 // a kernel with its launch shape

@@ -22,9 +22,6 @@
 // the spilled addresses of a step (a scratch load waits for all the fetches in front of it).  Forward and backward, us:
 // 4 x 4 096 tokens, 32 / 8 heads of 128, bf16: 2 904 -> 2 429 (the kernel 1 600 -> 1 000); 2 x 2 048, 28 / 4 heads: 393 -> 340
 // (245 -> 145).
-#include <stdlib.h>
-#include <string.h>
-
 #include <algorithm>
 #include <atomic>
 
@@ -469,12 +466,13 @@ BwdLaunch dkv32_launch(const BwdParams& p, int64_t* groups) {
   // ARENO_BACKWARD_PARTS=1w|1|2|4s|4 (read at every launch; one wave, 4 with single blocks and in pairs) fixes the choice: the
   // same dK and dV up to the order of the last sums, so this is for tests of the kernels a launch of the test's size would
   // not take, and for timing
-  if (const char* e = getenv("ARENO_BACKWARD_PARTS")) {
-    if (strcmp(e, "1w") == 0 && workgroups <= 0x7fffffffLL) parts = kLoneWave;
-    if (strcmp(e, "4s") == 0 && workgroups <= 0x7fffffffLL) parts = 4, pairs = false;
-    if (strcmp(e, "1") == 0) parts = 1;
-    if (strcmp(e, "2") == 0) parts = 2;
-    if (strcmp(e, "4") == 0 && workgroups <= 0x7fffffffLL) parts = 4, pairs = true;
+  const char* const name = "ARENO_BACKWARD_PARTS";
+  if (fixed_by(name, "1")) parts = 1;
+  if (fixed_by(name, "2")) parts = 2;
+  if (workgroups <= 0x7fffffffLL) {
+    if (fixed_by(name, "1w")) parts = kLoneWave;
+    if (fixed_by(name, "4s")) parts = 4, pairs = false;
+    if (fixed_by(name, "4")) parts = 4, pairs = true;
   }
   BwdLaunch launch;
   if (p.head_dim == 64) {

@@ -25,12 +25,7 @@
 // packed rows may hold rows of several sequences; it goes through them one after the other, the rows of the others
 // masked.
 
-#include <stdlib.h>
-#include <string.h>
-
 #include <algorithm>
-#include <atomic>
-#include <type_traits>
 
 #include "attention_backward.hpp"
 #include "backward_order.hpp"
@@ -631,19 +626,20 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
   // 512 x 8 (7) 158, 229; windows over 4 x 2 048 (14): 1 024 440, 382; 512 296, 271; 256 195, 198; 128 149, 163.  D = 64: 4 x 4 096, 32 / 8 (32)
   // 1 178, 1 044; 4 x 1 024, 16 / 16 (4) 60.6, 59.4; 2 x 1 024 (2) 40.7, 42.1; 12 x 512 (6) 60.1, 62.3; 28 / 4 heads, 64 x 512 (56) 402, 406; 256 x 128
   // (56) 243, 272; windows over 4 x 2 048: 512 155, 151; 256 105, 107; 128 75.8, 85.5.
-  // ARENO_BACKWARD_DQ_ROWS=16|32 (read at every launch) fixes the choice, for tests and timing.
+  // ARENO_BACKWARD_DQ_ROWS=16|32 (read at every launch) fixes the choice, for tests and timing; at head dims 192 and 256,
+  // which have one form, either value asks for it whatever the estimate says, as ARENO_BACKWARD_PARTS does.
   const int64_t mean_length = p.q_tokens / (p.num_seqs > 0 ? p.num_seqs : 1);
   const int64_t seen = p.window_left >= 0 ? std::min<int64_t>(mean_length, p.window_left + int64_t{1}) : mean_length;
   const int64_t workgroups = q_blocks * p.q_heads;  // (of 64 rows)
   int dq_rows = p.head_dim == 128 ? ((seen >= 512 && workgroups >= 3 * kBmComputeUnits) || (seen > 1024 && workgroups >= kBmComputeUnits * 3 / 2) ? 32 : 16)
                                   : (seen >= 512 && mean_length >= 1024 && workgroups >= 4 * kBmComputeUnits ? 32 : 16);
-  if (const char* e = getenv("ARENO_BACKWARD_DQ_ROWS")) {
-    if (strcmp(e, "32") == 0) dq_rows = 32;
-    if (strcmp(e, "16") == 0) dq_rows = 16;
-  }
-  // (head dims 192 and 256: not for many very short sequences, unless a switch fixes the shapes)
+  if (fixed_by("ARENO_BACKWARD_DQ_ROWS", "32")) dq_rows = 32;
+  if (fixed_by("ARENO_BACKWARD_DQ_ROWS", "16")) dq_rows = 16;
+  // (head dims 192 and 256: not for many very short sequences, unless a switch asks for these kernels)
   if (p.head_dim > 128) {
-    if (getenv("ARENO_BACKWARD_DQ_ROWS") == nullptr && vector_alu_is_faster(p)) return ARENO_ERR_UNSUPPORTED;
+    const bool asked_for = fixed_by("ARENO_BACKWARD_DQ_ROWS", "16") || fixed_by("ARENO_BACKWARD_DQ_ROWS", "32") ||
+                           fixed_by("ARENO_BACKWARD_PARTS", "1") || fixed_by("ARENO_BACKWARD_PARTS", "2");
+    if (!asked_for && vector_alu_is_faster(p)) return ARENO_ERR_UNSUPPORTED;
   }
   BwdLaunch dq, dkv;
   int64_t dkv_groups = 0;  // workgroups of a kv head

@@ -15,9 +15,6 @@
 // cycles a step, a third of the time in waits; dq: two).  Against 16 x 16 x 32 products with 16 rows per wave, both kernels, us: 2 717 tokens in four sequences, 16 / 8
 // heads of 256, window 512, bf16: 372 -> 271; 1 x 1 000, 8 / 1 heads: 917 -> 230.  Relative error of dV against 64 bits, before
 // and now: 2.74e-7, 2.64e-7 (bf16), 2.83e-7, 2.71e-7 (fp16); queries four times as large: 6.2e-7, 5.7e-7.
-#include <stdlib.h>
-#include <string.h>
-
 #include <algorithm>
 #include <atomic>
 
@@ -721,11 +718,9 @@ BwdLaunch dq32_wide_launch(const BwdParams& p) {
 // window (4 096) 2 052, 2 267 (2 576).
 BwdLaunch dkv32_wide_launch(const BwdParams& p, int64_t* groups) {
   int parts = dkv32_wide_parts(p);
-  // (ARENO_BACKWARD_PARTS=1|2, read at every launch, fixes it, for tests and timing)
-  if (const char* e = getenv("ARENO_BACKWARD_PARTS")) {
-    if (strcmp(e, "1") == 0) parts = 1;
-    if (strcmp(e, "2") == 0) parts = 2;
-  }
+  // (ARENO_BACKWARD_PARTS=1|2 fixes it, for tests and timing)
+  if (fixed_by("ARENO_BACKWARD_PARTS", "1")) parts = 1;
+  if (fixed_by("ARENO_BACKWARD_PARTS", "2")) parts = 2;
   BwdLaunch launch;
   if (p.head_dim == 192) {
     launch = p.dtype == ARENO_DT_BF16 ? launch_of<KV_BF16, 192>(parts) : launch_of<KV_F16, 192>(parts);

@@ -326,6 +326,28 @@ def test_wide_heads_where_blocks_and_tiles_end(dtype, parts, hq, hkv, d, window_
         assert err <= 4e-6, f"{name} {dtype} {hq}/{hkv} d={d} lens={lens}: {err:.3g}"
 
 
+@pytest.mark.parametrize("name,value,asked", [("PARTS", "1", True), ("PARTS", "2", True), ("DQ_ROWS", "32", True), ("DQ_ROWS", "48", False), ("PARTS", "4", False)])
+@pytest.mark.parametrize("d", [192, 256])
+def test_switches_ask_for_the_wide_heads_matrix_core_kernels(d, name, value, asked, monkeypatch):
+    """Single tokens of wide heads are the vector-ALU kernels'; a switch with a value that names one of the matrix-core
+    kernels' shapes takes them there (other bits come out of it), any other value changes nothing."""
+    g = torch.Generator().manual_seed(d)
+    t = 64
+    cu = torch.tensor(list(range(0, 2 * t, 2)) + [2 * t], dtype=torch.int32, device=DEV)
+    q, k, v, go = (torch.randn(2 * t, h, d, generator=g).to(torch.bfloat16).to(DEV) for h in (32, 1, 1, 32))
+    out = ops.areno_varlen_causal_attention(q, k, v, cu)
+    grads = lambda: _c_backward(go, q, k, v, out, cu, torch.float32, d**-0.5)  # noqa: E731
+    plain = grads()
+    monkeypatch.setenv("ARENO_BACKWARD_DQ_ROWS", "16")
+    matrix = grads()
+    assert not torch.equal(plain[1], matrix[1])
+    monkeypatch.delenv("ARENO_BACKWARD_DQ_ROWS")
+    monkeypatch.setenv(f"ARENO_BACKWARD_{name}", value)
+    got = grads()
+    assert torch.equal(got[1], plain[1]) != asked
+    assert torch.equal(got[0], (matrix if asked else plain)[0])
+
+
 @pytest.mark.parametrize("seqs", [1, 63, 64, 65, 130])
 @pytest.mark.parametrize("dq_rows", ["16", "32"])
 @pytest.mark.parametrize("hq,hkv,d,dtype", [(2, 1, 64, torch.float16), (2, 2, 128, torch.bfloat16), (2, 1, 256, torch.bfloat16)])

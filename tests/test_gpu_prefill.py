@@ -252,7 +252,7 @@ def test_prefill_one_query_block_cut_by_many_shares(kv):
 
 
 @pytest.mark.parametrize("hq,hkv", [(4, 1), (8, 2), (16, 8), (40, 2)])
-@pytest.mark.parametrize("lens,ctxs", [([5], [1600]), ([3, 70], [0, 900]), ([1, 0, 2, 90], [700, 5, 350, 0]), ([200] * 9, [40] * 9)])
+@pytest.mark.parametrize("lens,ctxs", [([5], [1600]), ([40], [1600]), ([3, 70], [0, 900]), ([1, 0, 2, 90], [700, 5, 350, 0]), ([200] * 9, [40] * 9)])
 def test_prefill_few_items_over_many_shares(hq, hkv, lens, ctxs):
     """The merge looks its items up among the units (256 of a lone kv head) when the tokens allow fewer items than units:
     one item in dozens of pieces (and batches), items in units far apart, units without steps, as many items as units.
