@@ -578,10 +578,11 @@ constexpr int64_t kBmComputeUnits = 256;
 // Whether the vector-ALU kernels take a launch of wide heads in less time.  A matrix-core workgroup goes through the
 // sequences of its block one after the other, at least one tile each (the dkv kernel for every q head of the group);
 // the vector-ALU kernels have a wave per row and do not care.  For sequences of 64 tokens and more the matrix cores
-// win by up to 30 times, for many single tokens they lose by as much; in between both are estimated, in us, from what
-// launches of 1 .. 300 sequences of 1 .. 64 tokens took (head dims 192 and 256, four head ratios; the matrix cores within 23 %
-// of 9 in 10).  vector ALU, matrix cores, in us, 16 / 8 heads of 256, bf16: 8 x 4 tokens 58, 96; 64 x 1 59, 467; 64 x 4 155, 145; 8 x 16
-// 86, 54; 300 x 2 383, 275.
+// win by up to 30 times, for many single tokens they lose by as much; in between both are estimated, in us, from what 2 034
+// launches of 1 .. 300 sequences of 1 .. 64 tokens took (head dims 192 and 256, six head ratios, equal and ragged lengths, a window).
+// The choice takes 0.02 % longer than the better of both over equal lengths (4 % at most) and 0.2 % over ragged ones (more than a
+// tenth in 10 of 1 170, 24 % at most).  vector ALU, matrix cores, in us, 16 / 8 heads of 256, bf16: 8 x 4 tokens 53, 91; 64 x 1 53, 460;
+// 64 x 4 149, 140; 8 x 16 81, 48; 300 x 2 377, 270; 8 / 1 heads, 8 x 12 71, 99; 6 / 6 heads, 16 x 12 101, 72.
 bool vector_alu_is_faster(const BwdParams& p) {
   const bool d256 = p.head_dim == 256;
   auto ceil_div = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
@@ -589,20 +590,21 @@ bool vector_alu_is_faster(const BwdParams& p) {
   const int64_t seqs = p.num_seqs, group = p.q_heads / p.kv_heads;
   const int64_t queries = std::max<int64_t>(p.q_tokens / seqs, 1), keys = std::max<int64_t>(p.k_tokens / seqs, 1);
   const int64_t reach = p.window_left >= 0 ? p.window_left + int64_t{1} : INT32_MAX;
-  // matrix cores: sequences in a block, steps of each, rounds of workgroups
+  // matrix cores: sequences in a block (which ends inside one as often as not), steps of each, rounds of workgroups
+  auto in_block = [&](int64_t rows, int64_t length) { return std::min(static_cast<double>(seqs), ceil_div(rows, length) + 0.5); };
   const int parts = dkv32_wide_parts(p);
   const int64_t dkv_rows = 64 / parts, dkv_rounds = ceil_div(ceil_div(p.k_tokens, dkv_rows) * p.kv_heads, kBmComputeUnits);
-  const int64_t dkv_steps = std::min(seqs, std::max<int64_t>(dkv_rows / keys, 1)) *
-                            ceil_div(ceil_div(std::min(queries, reach + dkv_rows), kBmTile) * group, parts) * dkv_rounds;
-  const int64_t dq_steps = std::min(seqs, std::max<int64_t>(kBmRows / queries, 1)) * ceil_div(std::min(keys, reach + kBmRows), kBmTile) *
-                           ceil_div(ceil_div(p.q_tokens, kBmRows) * p.q_heads, 2 * kBmComputeUnits);
-  const double matrix_cores = d256 ? 21 * dkv_rounds + 2.8 * dkv_steps + 6.5 * dq_steps : 16.5 * dkv_rounds + 2.4 * dkv_steps + 4.4 * dq_steps;
-  // vector ALU: all rows' work, or one row's chain, 16 keys or pairs at a time
-  const double seen = static_cast<double>(std::min(keys, reach)), pairs = static_cast<double>(std::min(queries, reach) * group);
-  const double work = (d256 ? 0.0245 : 0.0182) * (static_cast<double>(p.q_tokens * p.q_heads) * std::max(1.0, seen / 24) +
-                                                  static_cast<double>(p.k_tokens * p.kv_heads) * std::max(1.0, pairs / 48));
-  const double chain = d256 ? 43 + 4.6 * pairs / 16 + 5.0 * seen / 16 : 33 + 3.0 * pairs / 16 + 3.5 * seen / 16;
-  return std::max(work, chain) * 1.1 < matrix_cores;
+  const double dkv_steps = in_block(dkv_rows, keys) *
+                           ceil_div(ceil_div(std::min(queries, reach + dkv_rows), kBmTile) * group, parts) * dkv_rounds;
+  const double dq_steps = in_block(kBmRows, queries) * ceil_div(std::min(keys, reach + kBmRows), kBmTile) *
+                          ceil_div(ceil_div(p.q_tokens, kBmRows) * p.q_heads, 2 * kBmComputeUnits);
+  const double matrix_cores = d256 ? 14.5 * dkv_rounds + 2.75 * dkv_steps + 6.3 * dq_steps : 11 * dkv_rounds + 2.3 * dkv_steps + 4.2 * dq_steps;
+  // vector ALU: a wave per row, one of them per SIMD; a row's start and its keys or pairs, 16 at a time
+  const int64_t seen = std::min(keys, reach), pairs = std::min(queries, reach) * group, waves = 4 * kBmComputeUnits;
+  const int64_t q_rounds = ceil_div(p.q_tokens * p.q_heads, waves), k_rounds = ceil_div(p.k_tokens * p.kv_heads, waves);
+  const double vector_alu = d256 ? q_rounds * (21.2 + 2.29 * ceil_div(seen, 16)) + k_rounds * (24.1 + 4.25 * ceil_div(pairs, 16))
+                                 : q_rounds * (16 + 1.41 * ceil_div(seen, 16)) + k_rounds * (18.1 + 2.74 * ceil_div(pairs, 16));
+  return vector_alu < matrix_cores;
 }
 
 }  // namespace
