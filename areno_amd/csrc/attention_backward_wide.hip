@@ -193,6 +193,9 @@ __global__ __launch_bounds__(kWideDqWaves* kWave) __attribute__((amdgpu_waves_pe
   float4_t* const hand = reinterpret_cast<float4_t*>(wide_lds + L::kHands + wave * L::kHand) + lane;
   float* const reference = reinterpret_cast<float*>(wide_lds + L::kHands + wave * L::kHand + 2 * 16 * kWave * 4) + lane;
 
+  // (the block's first sequence is looked up while the rows below are on their way)
+  int s = uniform(seq_of_row(p.cu_q, p.num_seqs, r0));
+  int64_t sq0 = uniform(p.cu_q[s]), sq1;
   V8 own[NKS];  // this lane's parts of its row of Q or dO (B operands)
   float delta = 0.0f;
   {
@@ -224,8 +227,7 @@ __global__ __launch_bounds__(kWideDqWaves* kWave) __attribute__((amdgpu_waves_pe
   }
 
   int covered = 0;  // (where the sequences seen so far end)
-  int s = uniform(seq_of_row(p.cu_q, p.num_seqs, r0));
-  for (int64_t sq0 = uniform(p.cu_q[s]), sq1; s < p.num_seqs && sq0 < block_end; ++s, sq0 = sq1) {
+  for (; s < p.num_seqs && sq0 < block_end; ++s, sq0 = sq1) {
     // (asked for together)
     const int q_end = p.cu_q[s + 1], k_begin = p.cu_k[s], k_end = p.cu_k[s + 1], before = p.ctx != nullptr ? p.ctx[s] : 0;
     sq1 = covered = uniform(q_end);
@@ -450,6 +452,9 @@ __global__ __launch_bounds__((WideShape<D, KW, P>::kThreads)) __attribute__((amd
     fetch_offset[f] = static_cast<uint32_t>(r) * stride + static_cast<uint32_t>((slot % T::kChunksPerRow) ^ T::twist(r)) * 16u;
   }
 
+  // (the block's first sequence is looked up while the rows below are on their way)
+  int s = uniform(seq_of_row(p.cu_k, p.num_seqs, r0));
+  int64_t sk0 = uniform(p.cu_k[s]), sk1;
   V8 own[NKS];  // this lane's parts of its row of K or V (B operands)
   const int64_t row = r0 + 32 * wave + (lane & 31);
   {
@@ -474,8 +479,7 @@ __global__ __launch_bounds__((WideShape<D, KW, P>::kThreads)) __attribute__((amd
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) acc[nb] = zero16();
 
-  int s = uniform(seq_of_row(p.cu_k, p.num_seqs, r0));
-  for (int64_t sk0 = uniform(p.cu_k[s]), sk1; s < p.num_seqs && sk0 < block_end; ++s, sk0 = sk1) {
+  for (; s < p.num_seqs && sk0 < block_end; ++s, sk0 = sk1) {
     // (asked for together)
     const int k_end = p.cu_k[s + 1], q_begin = p.cu_q[s], q_end = p.cu_q[s + 1], before = p.ctx != nullptr ? p.ctx[s] : 0;
     sk1 = uniform(k_end);
