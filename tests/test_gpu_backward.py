@@ -60,10 +60,10 @@ def test_varlen_backward(dtype, window_left, hq, hkv, d):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("hq,hkv,d,window_left", [(8, 2, 128, None), (4, 4, 64, None), (6, 1, 64, 40), (4, 2, 128, 200), (2, 1, 128, 0)])
 def test_varlen_backward_long_sequences_on_the_matrix_core_kernels(dtype, hq, hkv, d, window_left, parts, dq_rows, last, monkeypatch):
-    """16-bit inputs at head dims 64 / 128 take the matrix-core backward: sequences longer than its blocks of 64 rows
-    and tiles of 32, blocks that hold several sequences (and empty ones), query groups, windows shorter and longer
-    than a tile.  The dkv kernel in each of its shapes: key blocks of 64 rows with the stream of query tiles in one
-    part or split over two, key blocks of 32 rows with four parts (the library reads the variable at every launch;
+    """16-bit inputs at head dims 64 / 128 take the matrix-core backward: sequences longer than its blocks (of 64 or 128
+    query rows, of 128, 64 or 32 keys) and tiles of 32, blocks that hold several sequences (and empty ones), query groups,
+    windows shorter and longer than a tile.  The dkv kernel in three of its shapes: key blocks of 128 rows, of 64 with the
+    stream of query tiles in two parts, of 32 with four parts and in pairs (the library reads the variable at every launch;
     left alone it picks by the size of the launch).  The last sequence's length makes the number of 32-row blocks
     even (1 327 tokens: every block has a partner in the four-part shape's pairs) or odd (1 359: the middle one has
     none)."""
@@ -89,8 +89,8 @@ def test_varlen_backward_long_sequences_on_the_matrix_core_kernels(dtype, hq, hk
 @pytest.mark.parametrize("hq,hkv,d,window_left", [(4, 2, 256, None), (6, 2, 256, 70), (3, 3, 192, None), (4, 1, 192, 97), (2, 1, 256, 0)])
 @pytest.mark.parametrize("lens", [[300, 1, 0, 130, 5, 95, 97, 161], [127], [129, 31], [1]])
 def test_varlen_backward_of_wide_heads_on_the_matrix_core_kernels(dtype, hq, hkv, d, window_left, lens, monkeypatch):
-    """Head dims 192 and 256: sequences longer than the dkv kernel's blocks (96 and 128 packed keys), blocks that hold
-    several sequences, lengths one off a block and a tile, windows shorter and longer than a block.  The bar is the
+    """Head dims 192 and 256: sequences longer than the dkv kernel's blocks (64 or 32 packed keys), blocks that hold
+    several sequences, lengths one off a tile, windows shorter and longer than a block.  The bar is the
     file's."""
     monkeypatch.setenv("ARENO_BACKWARD_DQ_ROWS", "16")  # (and not the kernels that a launch's estimate may prefer)
     g = torch.Generator().manual_seed(hq * 31 + d + len(lens))
@@ -150,15 +150,15 @@ def test_varlen_backward_with_a_scale_that_is_not_positive(dtype, scale, d):
         _close(got, ref, REL[dtype], f"{name} {dtype} d={d} scale={scale}")
 
 
-def _c_backward(go, q, k, v, out, cu, grad_dtype, scale, window_left=-1):
+def _c_backward(go, q, k, v, out, cu, grad_dtype, scale, window_left=-1, cu_k=None, ctx=None):
     """The C entry on gradient buffers full of NaN: what it leaves unwritten shows."""
     t, hq, d = q.shape
     grads = [torch.full(x.shape, float("nan"), dtype=grad_dtype, device=DEV) for x in (q, k, v)]
     workspace = torch.empty(t * hq * 8, dtype=torch.uint8, device=DEV)
-    ptr = lambda x: ctypes.c_void_p(x.data_ptr())  # noqa: E731
+    ptr = lambda x: None if x is None else ctypes.c_void_p(x.data_ptr())  # noqa: E731
     status = cabi.lib().areno_hip_attention_backward_typed(
         *map(ptr, (go, q, k, v, out, *grads)), cabi.dtype_code(grads[0]), cabi.dtype_code(q), ctypes.c_int64(t),
-        ctypes.c_int64(k.shape[0]), hq, k.shape[1], d, ptr(cu), None, None, cu.numel() - 1, window_left, ctypes.c_float(scale),
+        ctypes.c_int64(k.shape[0]), hq, k.shape[1], d, ptr(cu), ptr(cu_k), ptr(ctx), cu.numel() - 1, window_left, ctypes.c_float(scale),
         ptr(workspace), ctypes.c_size_t(workspace.numel()), ctypes.c_void_p(cabi.current_stream_ptr()))  # fmt: skip
     cabi.check(status, "areno_hip_attention_backward_typed")
     return grads
@@ -380,6 +380,57 @@ def test_a_window_as_wide_as_its_type_holds_is_none(dtype, d, window_left):
     assert all(x.abs().max() > 0 for x in want)
     for got, x, name in zip(_c_backward(go, q, k, v, out, cu, torch.float32, d**-0.5, window_left), want, ("dq", "dk", "dv")):
         assert torch.equal(got, x), f"{name} {dtype} d={d} window={window_left}"
+
+
+def _with_contexts(q, k, v, go, q_lens, k_lens, ctxs, window_left, scale):
+    """The forward's output (in the inputs' type) and dQ, dK, dV in 64 bits where sequence s has its queries at positions ctxs[s]
+    and on, and keys of its own."""
+    unit = q.dtype
+    q, k, v, go = (x.double().cpu() for x in (q, k, v, go))
+    out, grads, group = torch.zeros_like(q), [torch.zeros_like(x) for x in (q, k, v)], q.shape[1] // k.shape[1]
+    q0 = k0 = 0
+    for n_q, n_k, ctx in zip(q_lens, k_lens, ctxs):
+        rows, keys = slice(q0, q0 + n_q), slice(k0, k0 + n_k)
+        q0, k0 = q0 + n_q, k0 + n_k
+        i, j = ctx + torch.arange(n_q)[:, None], torch.arange(n_k)[None]
+        seen = (j <= i) & (j >= i - (i + 1 if window_left is None else window_left))
+        for h in range(q.shape[1]):
+            qh, kh, vh, gh = q[rows, h], k[keys, h // group], v[keys, h // group], go[rows, h]
+            prob = torch.softmax((scale * qh @ kh.T).masked_fill(~seen, float("-inf")), -1)
+            out[rows, h] = (prob @ vh).to(unit).double()
+            ds = prob * (gh @ vh.T - (gh * out[rows, h]).sum(-1, keepdim=True))
+            grads[0][rows, h] = scale * ds @ kh
+            grads[1][keys, h // group] += scale * ds.T @ qh
+            grads[2][keys, h // group] += prob.T @ gh
+    return out.to(unit).to(DEV), grads
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("window_left", [None, 33, 100])
+@pytest.mark.parametrize("hq,hkv,d", [(4, 2, 64), (4, 1, 128), (2, 2, 128), (4, 2, 192), (3, 3, 256)])
+@pytest.mark.parametrize("parts,dq_rows", [("1w", "16"), ("1", "16"), ("2", "32"), ("4s", "16"), ("4", "32")])
+def test_queries_behind_cached_keys_on_the_matrix_core_kernels(dtype, window_left, hq, hkv, d, parts, dq_rows, monkeypatch):
+    """Contexts (fewer queries than keys) in every form of the dq and dkv kernels: queries that start inside a tile, at its edge
+    and one off it, in the first and in later blocks of keys, keys behind the last query's position, fewer keys than positions,
+    a sequence of keys alone.  The bar, in the 2-norm: P and dS are rounded to the inputs' type, by half a unit in the last
+    place at most; one unit (wide heads do not round them: their own bar)."""
+    if d > 128 and parts not in ("1", "2"):
+        pytest.skip("wide heads have two shapes")
+    monkeypatch.setenv("ARENO_BACKWARD_PARTS", parts)
+    monkeypatch.setenv("ARENO_BACKWARD_DQ_ROWS", dq_rows)
+    g = torch.Generator().manual_seed(d + hq)
+    q_lens, ctxs = [70, 1, 0, 161, 33, 40, 5], [45, 200, 7, 96, 0, 129, 31]
+    k_lens = [n + c + more for n, c, more in zip(q_lens, ctxs, (3, 0, 2, 40, 0, -5, 0))]
+    cu, cu_k = (torch.tensor([0] + list(torch.tensor(x).cumsum(0)), dtype=torch.int32, device=DEV) for x in (q_lens, k_lens))
+    ctx = torch.tensor(ctxs, dtype=torch.int32, device=DEV)
+    q, go = (torch.randn(sum(q_lens), hq, d, generator=g).to(dtype).to(DEV) for _ in range(2))
+    k, v = (torch.randn(sum(k_lens), hkv, d, generator=g).to(dtype).to(DEV) for _ in range(2))
+    out, want = _with_contexts(q, k, v, go, q_lens, k_lens, ctxs, window_left, d**-0.5)
+    got = _c_backward(go, q, k, v, out, cu, torch.float32, d**-0.5, -1 if window_left is None else window_left, cu_k, ctx)
+    unit = 4e-6 if d > 128 else 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    for x, ref, name in zip(got, want, ("dq", "dk", "dv")):
+        err = ((x.cpu().double() - ref).norm() / ref.norm()).item()
+        assert err <= unit, f"{name} {dtype} {hq}/{hkv} d={d} window={window_left}: {err:.3g}"
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
