@@ -432,7 +432,7 @@ constexpr int64_t kComputeUnits = 256;
 // 12 steps) 30.8, 28.3; 1 x 200 (112, 6) 22.7, 21.6; 24 x 40, 28 / 4 (120, 7) 54.9, 38.0; 8 / 2 (60, 4) 38.0, 28.1; 4 x 300, 24 / 8 (304, 27) 55.5, 60.4; 2 x 600, 16 / 16 (608, 18) 57.6, 72.8;
 // 16 x 150, 32 / 8 (600, 16) 72.1, 83.2; 8 x 300 (600, 36) 97.5, 92.8; window 128: 1 x 600, 24 / 8 (152, 15) 38.2, 32.6; 2 x 600, 16 / 16 (608, 5) 39.2,
 // 57.7; 1 x 4 096, 32 / 8 (1 024, 20) 92.3, 119.  D = 64: 2 x 600, 16 / 16 37.8, 52.0; 1 x 600 (304, 18) 27.4, 29.0; 4 x 300, 24 / 8 38.1, 32.3; 32 / 8, window
-// 128 (304, 20) 35.3, 33.6; 4 x 600, 6 / 6 // (450, 18) 34.7, 37.1; 1 x 4 096, 6 / 6, window 128 (768, 5) 21.2, 36.6.
+// 128 (304, 20) 35.3, 33.6; 4 x 600, 6 / 6 (450, 18) 34.7, 37.1; 1 x 4 096, 6 / 6, window 128 (768, 5) 21.2, 36.6.
 // One wave by itself instead of one part (of few steps: or two), where a block holds several sequences or its streams are a few steps: it has a
 // block of 32 keys to find and to write, so in a launch that fills the chip many times over the streams have to be
 // shorter, at head dim 128 more than at 64.  One part, one wave (the 16-row kernels), us, D = 128: 16 / 16 heads, 4 096 x 8 tokens

@@ -87,11 +87,6 @@ __device__ __forceinline__ typename MfmaOps<KIND>::vec8 streamed_operand(const f
   return __builtin_bit_cast(V8, uint4_t{pack_pair<KIND>(x[0][0], x[0][1]), pack_pair<KIND>(x[0][2], x[0][3]),
                                         pack_pair<KIND>(x[1][0], x[1][1]), pack_pair<KIND>(x[1][2], x[1][3])});
 }
-template <int KIND>
-__device__ __forceinline__ float operand_element(uint32_t word, int hi) {
-  const uint32_t bits = hi ? word >> 16 : word & 0xffffu;
-  return KIND == KV_BF16 ? bf16_bits_to_float(bits) : f16_bits_to_float(bits);
-}
 
 // ---- dQ (and the rows' statistics) ------------------------------------------------------------------------------------
 // Bound by what a wave issues and waits for between its products, so a tile has one barrier (two LDS buffers), a

@@ -29,18 +29,12 @@ constexpr int kWideTile = 32;  // query rows per step
 constexpr float kWideNegInf = -__builtin_huge_valf();
 extern __shared__ __attribute__((aligned(1024))) char wide_lds[];
 
-template <int KIND>
-__device__ __forceinline__ float element(uint32_t word, int hi) {
-  const uint32_t bits = hi ? word >> 16 : word & 0xffffu;
-  return KIND == KV_BF16 ? bf16_bits_to_float(bits) : f16_bits_to_float(bits);
-}
-
 // Sixteen values of a column (with the other lane half's, thirty-two) as three 16-bit B operands of either block of 16 rows
 // that add up to them, times a power of two in fp16: the 16-bit inputs of wide heads had fp32 kernels until the matrix
 // cores took them, and lose nothing by it.
 // bf16 holds eight significant bits with fp32's exponents: the upper half of a value's word, that of the rest and what is
 // left then are its 24.  fp16 holds eleven in a narrow range: the values of a column are first scaled together, so that the
-// largest comes to lie in [2^14, 2^15); what three parts leave is 2^-40 of it and less.
+// largest comes to lie in [2^14, 2^15); what three parts leave, below fp16's smallest step of 2^-24, is less than 2^-38 of it.
 template <int KIND>
 struct WideWeights {
   typename Mfma32<KIND>::vec8 part[3][2];
@@ -219,7 +213,8 @@ __global__ __launch_bounds__(kWideDqWaves* kWave) __attribute__((amdgpu_waves_pe
       if (second) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          delta += element<KIND>(w[ks][j], 0) * element<KIND>(o[ks][j], 0) + element<KIND>(w[ks][j], 1) * element<KIND>(o[ks][j], 1);
+          delta += operand_element<KIND>(w[ks][j], 0) * operand_element<KIND>(o[ks][j], 0) +
+                   operand_element<KIND>(w[ks][j], 1) * operand_element<KIND>(o[ks][j], 1);
         }
       }
     }
@@ -415,8 +410,8 @@ struct WideShape {
   static constexpr int kLdsBytes = kTiles + P * KW * kHand;
 };
 
-template <int KIND, int D, int KW, int P, int OCC>
-__global__ __launch_bounds__((WideShape<D, KW, P>::kThreads)) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void bwd_mfma32_wide_dkv_kernel(BwdParams p) {
+template <int KIND, int D, int KW, int P>
+__global__ __launch_bounds__((WideShape<D, KW, P>::kThreads)) __attribute__((amdgpu_waves_per_eu(1, 1))) void bwd_mfma32_wide_dkv_kernel(BwdParams p) {
   using M = Mfma32<KIND>;
   using V8 = typename M::vec8;
   using L = WideShape<D, KW, P>;
@@ -439,8 +434,8 @@ __global__ __launch_bounds__((WideShape<D, KW, P>::kThreads)) __attribute__((amd
 
   static_assert(L::kPart % 256 == 0 && T::kBytes % 256 == 0, "places that the reads' exclusive-ors leave alone");
   // a wave's rows operand comes from the one tile, its columns operand from the other
-  uint32_t at_rows = T::rows_base(lane & 31, lane >> 5) + part * L::kPart + (second ? T::kBytes : 0);
-  uint32_t at_columns = T::columns_base(lane) + part * L::kPart + (second ? 0 : T::kBytes);
+  const uint32_t at_rows = T::rows_base(lane & 31, lane >> 5) + part * L::kPart + (second ? T::kBytes : 0);
+  const uint32_t at_columns = T::columns_base(lane) + part * L::kPart + (second ? 0 : T::kBytes);
   const uint32_t lds0 = lds_address(wide_lds) + part * L::kPart;
   const uint32_t stride = static_cast<uint32_t>(p.q_heads) * (D * 2);
   float4_t* const hand = reinterpret_cast<float4_t*>(wide_lds + L::kTiles + (part * KW + wave) * L::kHand);
@@ -560,7 +555,6 @@ __global__ __launch_bounds__((WideShape<D, KW, P>::kThreads)) __attribute__((amd
       to_next_heads();
     };
     auto step = [&](int i, int buf) {
-      if constexpr (OCC > 1) asm volatile("" : "+v"(at_rows), "+v"(at_columns));  // (addresses worked out where they are used)
       fetched_barrier();  // the step's tile (asked for a step ago) is there, and every wave has left the one before
       if (i + 1 < steps) fetch(buf ^ 1);
       const int t = tile;
@@ -689,17 +683,17 @@ __global__ __launch_bounds__((WideShape<D, KW, P>::kThreads)) __attribute__((amd
   }
 }
 
-template <int KIND, int D, int KW, int P, int OCC>
+template <int KIND, int D, int KW, int P>
 BwdLaunch launch_of() {
   using L = WideShape<D, KW, P>;
-  const bwd_fn fn = bwd_mfma32_wide_dkv_kernel<KIND, D, KW, P, OCC>;
+  const bwd_fn fn = bwd_mfma32_wide_dkv_kernel<KIND, D, KW, P>;
   static std::atomic<uint64_t> allowed_on{0};
   if (!allow_lds<L::kLdsBytes>(fn, allowed_on)) return BwdLaunch{nullptr, 0, 0, 0};
   return BwdLaunch{fn, L::kLdsBytes, L::kThreads, L::kKeys};
 }
 template <int KIND, int D>
 BwdLaunch launch_of(int parts) {
-  return parts == 2 ? launch_of<KIND, D, 1, 2, 1>() : launch_of<KIND, D, 2, 1, 1>();
+  return parts == 2 ? launch_of<KIND, D, 1, 2>() : launch_of<KIND, D, 2, 1>();
 }
 
 }  // namespace

@@ -1,4 +1,4 @@
-// What the kernels on 32 x 32 x 16 matrix products share (varlen_mfma.hip): the products, LDS tiles that
+// What the kernels on 32 x 32 x 16 matrix products share (varlen_mfma.hip, attention_backward_*.hip): the products, LDS tiles that
 // the memory pipe fills directly (no registers, no staging instructions), and the two ways a wave reads an operand out
 // of such a tile.
 //
@@ -40,6 +40,13 @@ struct Mfma32<KV_F16> {
     return __builtin_amdgcn_fdot2(__builtin_bit_cast(half2_t, pair), ones, c, false);
   }
 };
+
+// one of the two 16-bit elements of an operand's word
+template <int KIND>
+__device__ __forceinline__ float operand_element(uint32_t word, int hi) {
+  const uint32_t bits = hi ? word >> 16 : word & 0xffffu;
+  return KIND == KV_BF16 ? bf16_bits_to_float(bits) : f16_bits_to_float(bits);
+}
 
 __device__ __forceinline__ float16_t zero16() {
   float16_t z;
