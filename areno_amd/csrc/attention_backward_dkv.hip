@@ -382,16 +382,18 @@ __global__ __launch_bounds__((Dkv32Shape<D, KW, P>::kThreads)) __attribute__((am
     const int64_t out_row = r0 + 32 * wave + (lane_ & 31);
     if (part == 0 && out_row < p.k_tokens) {
       const int64_t out_elem = (out_row * p.kv_heads + kvh) * D + 4 * (lane_ >> 5);
+      store_grads<typename M::elem>(p.grad_dtype, [&](auto store) {
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
+        for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int64_t at_elem = out_elem + 32 * nb + 8 * c;
-          store_grad4(p.grad_k, at_elem, acc_k[nb][4 * c] * p.scale, acc_k[nb][4 * c + 1] * p.scale, acc_k[nb][4 * c + 2] * p.scale,
-                      acc_k[nb][4 * c + 3] * p.scale, p.grad_dtype);
-          store_grad4(p.grad_v, at_elem, acc_v[nb][4 * c], acc_v[nb][4 * c + 1], acc_v[nb][4 * c + 2], acc_v[nb][4 * c + 3], p.grad_dtype);
+          for (int c = 0; c < 4; ++c) {
+            const int64_t at_elem = out_elem + 32 * nb + 8 * c;
+            store(p.grad_k, at_elem, acc_k[nb][4 * c] * p.scale, acc_k[nb][4 * c + 1] * p.scale, acc_k[nb][4 * c + 2] * p.scale,
+                  acc_k[nb][4 * c + 3] * p.scale);
+            store(p.grad_v, at_elem, acc_v[nb][4 * c], acc_v[nb][4 * c + 1], acc_v[nb][4 * c + 2], acc_v[nb][4 * c + 3]);
+          }
         }
-      }
+      });
     }
   }
 }

@@ -307,11 +307,11 @@ __global__ __launch_bounds__(kBmThreads, D == 64 ? 4 : 2) void bwd_mfma_dq_kerne
     const float l_tot = rows_sum(l_lane);
     if (live) {
       const float f = l_tot > 0.0f ? p.scale / l_tot : 0.0f;
+      store_grads<typename Mfma32<KIND>::elem>(p.grad_dtype, [&](auto store) {
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        store_grad4(p.grad_q, row_elem + 4 * lk + 16 * nb, acc[nb][0] * f, acc[nb][1] * f,
-                    acc[nb][2] * f, acc[nb][3] * f, p.grad_dtype);
-      }
+        for (int nb = 0; nb < NB; ++nb)
+          store(p.grad_q, row_elem + 4 * lk + 16 * nb, acc[nb][0] * f, acc[nb][1] * f, acc[nb][2] * f, acc[nb][3] * f);
+      });
       if (lk == 0) {
         float* st = p.row_stats + (h * p.q_tokens + row) * 2;
         // a row without visible keys gets a reference no score reaches: its probabilities come out as zeros
@@ -322,8 +322,10 @@ __global__ __launch_bounds__(kBmThreads, D == 64 ? 4 : 2) void bwd_mfma_dq_kerne
   }
   if (row >= covered && row < p.q_tokens) {  // behind the last sequence, the end of a padded pack
     const int64_t row_elem = (row * p.q_heads + h) * D;
+    store_grads<typename Mfma32<KIND>::elem>(p.grad_dtype, [&](auto store) {
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) store_grad4(p.grad_q, row_elem + 4 * lk + 16 * nb, 0.0f, 0.0f, 0.0f, 0.0f, p.grad_dtype);
+      for (int nb = 0; nb < NB; ++nb) store(p.grad_q, row_elem + 4 * lk + 16 * nb, 0.0f, 0.0f, 0.0f, 0.0f);
+    });
   }
 }
 
@@ -546,14 +548,16 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
     const float l_tot = both_halves(l_lane, sum);
     if (live) {
       const float f = l_tot > 0.0f ? p.scale / l_tot : 0.0f;
+      store_grads<typename M::elem>(p.grad_dtype, [&](auto store) {
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
+        for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          store_grad4(p.grad_q, row_elem + 32 * nb + 8 * c + 4 * half, acc[nb][4 * c] * f, acc[nb][4 * c + 1] * f,
-                      acc[nb][4 * c + 2] * f, acc[nb][4 * c + 3] * f, p.grad_dtype);
+          for (int c = 0; c < 4; ++c) {
+            store(p.grad_q, row_elem + 32 * nb + 8 * c + 4 * half, acc[nb][4 * c] * f, acc[nb][4 * c + 1] * f, acc[nb][4 * c + 2] * f,
+                  acc[nb][4 * c + 3] * f);
+          }
         }
-      }
+      });
       if (half == 0) {
         float* st = p.row_stats + (h * p.q_tokens + row) * 2;
         st[0] = l_tot > 0.0f ? m_run + __builtin_log2f(l_tot) : __builtin_huge_valf();
@@ -563,8 +567,10 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
   }
   if (row >= covered && row < p.q_tokens) {  // behind the last sequence, the end of a padded pack
     const int64_t row_elem = (row * p.q_heads + h) * D;
+    store_grads<typename M::elem>(p.grad_dtype, [&](auto store) {
 #pragma unroll
-    for (int c = 0; c < D / 8; ++c) store_grad4(p.grad_q, row_elem + 8 * c + 4 * half, 0.0f, 0.0f, 0.0f, 0.0f, p.grad_dtype);
+      for (int c = 0; c < D / 8; ++c) store(p.grad_q, row_elem + 8 * c + 4 * half, 0.0f, 0.0f, 0.0f, 0.0f);
+    });
   }
 }
 

@@ -370,14 +370,16 @@ __global__ __launch_bounds__(kWideDqWaves* kWave) __attribute__((amdgpu_waves_pe
     const float l_tot = *reference;
     if (live) {
       const float f = l_tot > 0.0f ? p.scale / l_tot : 0.0f;
+      store_grads<typename M::elem>(p.grad_dtype, [&](auto store) {
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
+        for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          store_grad4(p.grad_q, row_elem + 64 * nb + (second ? 32 : 0) + 8 * c + 4 * half, acc[nb][4 * c] * f, acc[nb][4 * c + 1] * f,
-                      acc[nb][4 * c + 2] * f, acc[nb][4 * c + 3] * f, p.grad_dtype);
+          for (int c = 0; c < 4; ++c) {
+            store(p.grad_q, row_elem + 64 * nb + (second ? 32 : 0) + 8 * c + 4 * half, acc[nb][4 * c] * f, acc[nb][4 * c + 1] * f,
+                  acc[nb][4 * c + 2] * f, acc[nb][4 * c + 3] * f);
+          }
         }
-      }
+      });
       if (half == 0) {
         // a row without visible keys gets a reference no score reaches: its probabilities come out as zeros
         p.row_stats[(h * p.q_tokens + row) * 2 + (second ? 1 : 0)] =
@@ -386,11 +388,13 @@ __global__ __launch_bounds__(kWideDqWaves* kWave) __attribute__((amdgpu_waves_pe
     }
   }
   if (row >= covered && row < p.q_tokens) {  // behind the last sequence, the end of a padded pack
+    store_grads<typename M::elem>(p.grad_dtype, [&](auto store) {
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
+      for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) store_grad4(p.grad_q, row_elem + 64 * nb + (second ? 32 : 0) + 8 * c + 4 * half, 0.0f, 0.0f, 0.0f, 0.0f, p.grad_dtype);
-    }
+        for (int c = 0; c < 4; ++c) store(p.grad_q, row_elem + 64 * nb + (second ? 32 : 0) + 8 * c + 4 * half, 0.0f, 0.0f, 0.0f, 0.0f);
+      }
+    });
   }
 }
 
@@ -674,12 +678,14 @@ __global__ __launch_bounds__((WideShape<D, KW, P>::kThreads)) __attribute__((amd
     void* const out = second ? p.grad_k : p.grad_v;
     const float f = second ? p.scale : 1.0f;
     const int64_t elem = (out_row * p.kv_heads + kvh) * D + 4 * (l >> 5);
+    store_grads<typename M::elem>(p.grad_dtype, [&](auto store) {
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
+      for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
-        store_grad4(out, elem + 32 * nb + 8 * c, acc[nb][4 * c] * f, acc[nb][4 * c + 1] * f, acc[nb][4 * c + 2] * f, acc[nb][4 * c + 3] * f, p.grad_dtype);
-    }
+        for (int c = 0; c < 4; ++c)
+          store(out, elem + 32 * nb + 8 * c, acc[nb][4 * c] * f, acc[nb][4 * c + 1] * f, acc[nb][4 * c + 2] * f, acc[nb][4 * c + 3] * f);
+      }
+    });
   }
 }
 

@@ -19,6 +19,7 @@ template <int KIND>
 struct Mfma32;
 template <>
 struct Mfma32<KV_BF16> {
+  using elem = __bf16;
   using vec8 = bf16x8_t;
   static __device__ __forceinline__ float16_t mfma(vec8 a, vec8 b, float16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
@@ -31,6 +32,7 @@ struct Mfma32<KV_BF16> {
 };
 template <>
 struct Mfma32<KV_F16> {
+  using elem = _Float16;
   using vec8 = half8_t;
   static __device__ __forceinline__ float16_t mfma(vec8 a, vec8 b, float16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);

@@ -43,8 +43,7 @@ HIP_DEVICE_FLAGS = [
     # matrix products accumulate in vector registers: left to itself the compiler puts the decode kernels'
     # accumulators into accumulation registers and copies all 36 of them out and back around the rescaling of every
     # tile step (117 copies per step at head dim 128); of the instances that fill the 256 vector registers some spill
-    # (prefill at head dim 512; of the backward the dq kernels at 192 and 256 and with 32 rows at 128, the dkv kernel's forms
-    # with two waves per SIMD at 128)
+    # (prefill at head dim 512; of the backward the dq kernel with 32 rows at 128, outside its tile loop)
     "-mllvm", "-amdgpu-mfma-vgpr-form",
     "-DARENO_DEVICE_FLAGS_OK=1",  # device_common.hpp refuses to compile without the two flags above
 ] + [f"-D{name}={os.environ[name]}" for name in ("ARENO_MFMA_NW", "ARENO_TRACE", "ARENO_MFMA_QUANT_OCC", "ARENO_MFMA_WIDE_OCC", "ARENO_PREFILL_WAVES") if os.environ.get(name)]  # fmt: skip
