@@ -419,52 +419,45 @@ constexpr int64_t kComputeUnits = 256;
 
 }  // namespace
 
-// The shape, from the launch's size (blocks of 32 keys of a kv head) and what a block's stream is for sequences of the mean
-// length, of which a window shows a block of keys its own queries and as many behind them: `per_seq` steps for a sequence,
-// `steps` for all that a block holds.  Four parts want streams that keep all four
-// busy for longer than handing their sums over takes, and pay until their workgroups, one per compute unit, come round a
-// second or third time; one part wants the chip filled twice with blocks of 128 keys.  The backward in us, in one part, two,
-// four (what the 16-row kernels took): D = 128, 28 / 4 heads: 2 x 2 048 tokens (512 blocks) 565, 397, 261 (310); 4 x 2 048
-// (1 024) 679, 569, 524 (573); 6 x 2 048 (1 536) 842, 745, 792 (891); 8 x 2 048 (2 048) 1 006, 963, 1 053 (1 154); 16 x 256 (512)
-// 126, 113, 95 (119); 48 x 256 (1 536) 239, 262, 276 (262); 4 x 4 096, 32 / 8 (4 096) 1 977, 2 056, 2 214 (2 248); 8 / 8 heads, 32 x 128
-// (1 024) 36.0, 37.6, 59 (35.5).  D = 64: 2 x 2 048, 32 / 8 (1 024) 266, 186, 182 (213); 3 x 4 096, 28 / 4 (1 536) 958, 723, 773 (994);
-// 16 / 16 heads: 8 x 128 (512) 22.1, 20.4, 24.6 (21.1); 16 x 310 (2 480) 66, 69, 102 (65).
-// In one round of workgroups a stream of 12 steps is enough for four parts, of four and more q heads one of 4; where they
-// share the units, or come round again, it has to be longer.  Two, four parts, us, D = 128: 1 x 400 tokens, 16 / 16 heads (208 blocks,
-// 12 steps) 30.8, 28.3; 1 x 200 (112, 6) 22.7, 21.6; 24 x 40, 28 / 4 (120, 7) 54.9, 38.0; 8 / 2 (60, 4) 38.0, 28.1; 4 x 300, 24 / 8 (304, 27) 55.5, 60.4; 2 x 600, 16 / 16 (608, 18) 57.6, 72.8;
-// 16 x 150, 32 / 8 (600, 16) 72.1, 83.2; 8 x 300 (600, 36) 97.5, 92.8; window 128: 1 x 600, 24 / 8 (152, 15) 38.2, 32.6; 2 x 600, 16 / 16 (608, 5) 39.2,
-// 57.7; 1 x 4 096, 32 / 8 (1 024, 20) 92.3, 119.  D = 64: 2 x 600, 16 / 16 37.8, 52.0; 1 x 600 (304, 18) 27.4, 29.0; 4 x 300, 24 / 8 38.1, 32.3; 32 / 8, window
-// 128 (304, 20) 35.3, 33.6; 4 x 600, 6 / 6 (450, 18) 34.7, 37.1; 1 x 4 096, 6 / 6, window 128 (768, 5) 21.2, 36.6.
-// One wave by itself instead of one part (of few steps: or two), where a block holds several sequences or its streams are a few steps: it has a
-// block of 32 keys to find and to write, so in a launch that fills the chip many times over the streams have to be
-// shorter, at head dim 128 more than at 64.  One part, one wave (the 16-row kernels), us, D = 128: 16 / 16 heads, 4 096 x 8 tokens
-// (16 384 blocks) 910, 774 (954); 64 x 32 (1 024) 31.5, 28.3 (29.5); 300 x 48 (7 200) 212, 199 (228); 100 x 100 (5 000) 149, 146 (168);
-// 16 x 160 (1 280) 47.3, 42.7 (50.4); 32 x 128 (2 048) 52.0, 54.5 (59.0); 100 x 160 (8 000) 226, 239 (247); 8 / 8, 16 x 200 (800) 42.5, 38.1
-// (42.3); 8 / 2, 300 x 48 (900) 92.0, 74.9 (84.2); 24 / 8, 60 x 60 (904) 76.0, 62.9 (71.7); 300 x 80 (6 000) 382, 388 (427).  D = 64: 16 / 16 heads,
-// 4 096 x 8 496, 353 (484); 512 x 16 (4 096) 73.3, 56.7 (71.5); 32 x 96 (1 536) 26.5, 22.7 (25.8); 16 x 160 27.8, 22.4 (26.8); 64 x 200 (6 400)
-// 105, 103 (114); 200 x 128 (12 800) 179, 185 (187); 8 / 2, 300 x 48 55.7, 44.7 (49.9); 28 / 4, 4 096 x 16 (8 192) 700, 554 (690).  Two parts,
-// one wave: 8 / 8, 16 x 160 (640) 31.4, 27.2 and 21.0, 18.4; 6 / 6, 16 x 150 (450) 30.2, 31.1 and 20.0, 20.8.
+// The shape, from the launch's size (blocks of 32 keys of a kv head) and the steps of a block's streams, for sequences of the
+// mean length, of which a window shows a block of keys its own queries and as many behind them.  Up to a workgroup per
+// compute unit a launch is its longest block: four parts, unless its streams are so few steps that handing the sums
+// over takes longer.  Blocks of several sequences are one wave's: in a wider one each sequence is a stream that one wave
+// computes on while the others wait.  The more workgroups there are the longer a stream has to be for four parts and for two;
+// one part, which two waves per SIMD share, is for launches that fill the chip many times over.
+// Lines drawn through 4 074 launches of 1 .. 1 000 sequences of 1 .. 4 096 tokens, ten head ratios, equal and ragged lengths,
+// windows: the choice takes 0.65 % longer than the best of all shapes, and nowhere 3 % longer than the 16-row kernels did.  The
+// backward in us; in brackets blocks, steps.  One wave, two parts, four:  D = 128: 16 / 16 heads, 1 x 26 (16, 1) 11.1, 12.5, 14.3; 24 / 8, 8 x 160
+// (328, 15) 54.6, 48.5, 45.9; 6 / 6, 5 x 474 (450, 14) 45.0, 43.3, 49.7; 32 / 2, 347 x 14 (316, 48) 208, 198, 163; D = 64: 28 / 4, 9 x 617 (696, 133)
+// 175, 130, 110; 24 / 8, 36 x 75 (680, 6) 39.6, 36.5, 44.3; 28 / 4, 12 x 347 (524, 70) 155, 112, 87; 28 / 4, 38 x 92 (440, 14) 49.0, 43.6, 47.1.
+// One wave, one part, two:  D = 64: 16 / 16, 11 x 716 (3 952, 22) 124, 109, 123; 361 x 132, window 128 (23 840, 4) 432, 408, 460; D = 128: 16 / 8, 196 x
+// 128 (6 272, 8) 279, 259, 272; 16 / 16, 67 x 180, window 128 (6 032, 5) 184, 173, 191.  One part, two, four:  D = 128, 28 / 4: 8 x 2 048 (2 048) 1 006,
+// 963, 1 053; 4 x 4 096, 32 / 8 (4 096) 1 977, 2 056, 2 214.
 BwdLaunch dkv32_launch(const BwdParams& p, int64_t* groups) {
   const int64_t blocks = (p.k_tokens + 31) / 32, workgroups = blocks * p.kv_heads;
   const int64_t seqs = std::max<int64_t>(p.num_seqs, 1), mean = std::max<int64_t>(p.q_tokens / seqs, 1), group = p.q_heads / p.kv_heads;
   const int64_t seen = p.window_left >= 0 ? std::min<int64_t>(mean, p.window_left + int64_t{32}) : mean;
-  const int64_t chain = seen / kDkvTile * group, per_seq = std::max(chain, group);
-  const int64_t steps = mean < 32 ? per_seq * std::min(seqs, 32 / mean) : per_seq;
-  const int64_t units = (p.head_dim == 64 ? 2 : 1) * kComputeUnits;  // (for workgroups of four parts: at head dim 64 two share one)
-  const int64_t most_for_two = chain >= 64 ? 2304 : chain < 8 ? (mean < 32 ? 1280 : 768) : p.head_dim == 64 ? 2048 : 1280;
-  const bool lone = workgroups > 512 && workgroups <= 0x7fffffffLL &&
-                    (chain <= 3 || (chain <= 6 && workgroups <= (p.head_dim == 64 ? 8192 : 1536)));
-  int parts = 1;
-  if (workgroups <= (chain >= 128 ? 1152 : 640) && per_seq >= 4 &&
-      steps >= (workgroups <= kComputeUnits ? (group >= 4 ? 4 : 12) : mean < 32 ? 16 : workgroups <= units ? 20 : 32)) {
-    parts = 4;
-  } else if (workgroups <= most_for_two && !(lone && mean >= 32 && chain <= 5)) {
-    parts = 2;
-  } else if (lone) {
-    parts = kLoneWave;
+  const int64_t steps = std::max<int64_t>(seen / kDkvTile, 1) * group * std::min(seqs, 1 + 31 / mean);  // (a block of 32 keys ends inside a sequence)
+  const bool d64 = p.head_dim == 64, several = mean < 32;
+  int parts;
+  if (workgroups <= kComputeUnits) {
+    parts = steps >= (!several ? 2 : seqs == 1 ? 4 : 6) ? 4 : kLoneWave;
+  } else if (several) {
+    parts = workgroups <= 2 * kComputeUnits && steps >= (d64 ? 12 : 48) ? 4 : kLoneWave;
+  } else if (workgroups <= 2 * kComputeUnits) {
+    parts = steps >= (workgroups <= 384 ? 12 : 20) ? 4 : steps > 3 ? 2 : kLoneWave;
+  } else if (workgroups <= 1152) {
+    parts = steps >= (d64 ? 96 : 33) ? 4 : steps > 5 ? 2 : kLoneWave;
+  } else {
+    parts = steps <= (workgroups > (d64 ? 8192 : 4096) ? 3 : d64 ? 16 : 6) ? kLoneWave : workgroups <= 3000 ? 2 : 1;
   }
-  // Pairs of blocks where every one of them then has a compute unit and single blocks would not
-  bool pairs = workgroups > units && (blocks + 1) / 2 * p.kv_heads <= units;
+  if (parts == kLoneWave && workgroups > 0x7fffffffLL) parts = 1;
+  // Pairs of blocks, whose costs add up to the same for one sequence, or two, where every pair then has a compute unit
+  // and single blocks come round a second time: 1 x 1 978, 16 / 8 heads of 128 (496 blocks): the backward 117 us, 120 with single ones; 2 x 2 819,
+  // 8 / 2 (354): 221, 232.  Far fewer pairs than units leave these idle (2 x 2 341, 8 / 2, 294: 256, 215), of many sequences single
+  // blocks end closer together (13 x 451, 8 / 2, 368: 91.9, 76.6), and at head dim 64, where two workgroups share a unit, they
+  // always do (1 x 3 091, 6 / 6, 582: 105, 95).
+  bool pairs = !d64 && p.num_seqs <= 2 && workgroups >= kComputeUnits * 5 / 4 && (blocks + 1) / 2 * p.kv_heads <= kComputeUnits;
   // ARENO_BACKWARD_PARTS=1w|1|2|4s|4 (read at every launch; one wave, 4 with single blocks and in pairs) fixes the choice: the
   // same dK and dV up to the order of the last sums, so this is for tests of the kernels a launch of the test's size would
   // not take, and for timing
