@@ -423,15 +423,19 @@ constexpr int64_t kComputeUnits = 256;
 // mean length, of which a window shows a block of keys its own queries and as many behind them.  Up to a workgroup per
 // compute unit a launch is its longest block: four parts, unless its streams are so few steps that handing the sums
 // over takes longer.  Blocks of several sequences are one wave's: in a wider one each sequence is a stream that one wave
-// computes on while the others wait.  The more workgroups there are the longer a stream has to be for four parts and for two;
-// one part, which two waves per SIMD share, is for launches that fill the chip many times over.
-// Lines drawn through 4 074 launches of 1 .. 1 000 sequences of 1 .. 4 096 tokens, ten head ratios, equal and ragged lengths,
-// windows: the choice takes 0.65 % longer than the best of all shapes, and nowhere 3 % longer than the 16-row kernels did.  The
-// backward in us; in brackets blocks, steps.  One wave, two parts, four:  D = 128: 16 / 16 heads, 1 x 26 (16, 1) 11.1, 12.5, 14.3; 24 / 8, 8 x 160
+// computes on while the others wait.  The more workgroups there are the longer a stream has to be for four parts and for two,
+// and four pay only where a few blocks' streams are far longer than the rest (not in a window); one part, which two waves
+// per SIMD share, is for launches that fill the chip many times over, sooner where no block of 128 holds two sequences.
+// Lines drawn through 8 753 launches of 1 .. 1 000 sequences of 1 .. 4 096 tokens, ten head ratios, equal and ragged lengths,
+// windows: the choice takes 0.8 % longer than the best of all shapes, and 3 % longer than the 16-row kernels in one.  The backward in us; in brackets blocks, steps.  One wave, two parts, four:  D = 128: 16 / 16 heads, 1 x 26 (16, 1) 11.1, 12.5, 14.3; 6 / 6, 6 x 64
+// (72, 2) 13.9, 16.6, 16.7; 24 / 8, 8 x 160
 // (328, 15) 54.6, 48.5, 45.9; 6 / 6, 5 x 474 (450, 14) 45.0, 43.3, 49.7; 32 / 2, 347 x 14 (316, 48) 208, 198, 163; D = 64: 28 / 4, 9 x 617 (696, 133)
-// 175, 130, 110; 24 / 8, 36 x 75 (680, 6) 39.6, 36.5, 44.3; 28 / 4, 12 x 347 (524, 70) 155, 112, 87; 28 / 4, 38 x 92 (440, 14) 49.0, 43.6, 47.1.
+// 175, 130, 110; 24 / 8, 36 x 75 (680, 6) 39.6, 36.5, 44.3; 28 / 4, 12 x 347 (524, 70) 155, 112, 87; 28 / 4, 38 x 92 (440, 14) 49.0, 43.6, 47.1;
+// D = 128: 8 / 1, 29 x 768, window 512 (696, 136) 258, 197, 245; 32 / 2, 37 x 448 (1 036, 224) 566, 431, 538; 32 / 8, 2 x 1 380 (696, 172): two parts
+// 1.33 times four.
 // One wave, one part, two:  D = 64: 16 / 16, 11 x 716 (3 952, 22) 124, 109, 123; 361 x 132, window 128 (23 840, 4) 432, 408, 460; D = 128: 16 / 8, 196 x
-// 128 (6 272, 8) 279, 259, 272; 16 / 16, 67 x 180, window 128 (6 032, 5) 184, 173, 191.  One part, two, four:  D = 128, 28 / 4: 8 x 2 048 (2 048) 1 006,
+// 128 (6 272, 8) 279, 259, 272; 16 / 16, 67 x 180, window 128 (6 032, 5) 184, 173, 191; 32 x 128 (2 048, 4) 57, 50, 56; 32 / 8, 61 x 128
+// (1 952, 16) 138, 127, 134.  One part, two, four:  D = 128, 28 / 4: 8 x 2 048 (2 048) 1 006,
 // 963, 1 053; 4 x 4 096, 32 / 8 (4 096) 1 977, 2 056, 2 214.
 BwdLaunch dkv32_launch(const BwdParams& p, int64_t* groups) {
   const int64_t blocks = (p.k_tokens + 31) / 32, workgroups = blocks * p.kv_heads;
@@ -439,17 +443,23 @@ BwdLaunch dkv32_launch(const BwdParams& p, int64_t* groups) {
   const int64_t seen = p.window_left >= 0 ? std::min<int64_t>(mean, p.window_left + int64_t{32}) : mean;
   const int64_t steps = std::max<int64_t>(seen / kDkvTile, 1) * group * std::min(seqs, 1 + 31 / mean);  // (a block of 32 keys ends inside a sequence)
   const bool d64 = p.head_dim == 64, several = mean < 32;
+  // equal lengths, as far as the sizes tell, whose ends are those of blocks of 32 keys, or of 128: no block has a second stream
+  const bool whole = seqs == 1 || (p.q_tokens == seqs * mean && mean % 32 == 0), whole128 = whole && mean % 128 == 0;
   int parts;
   if (workgroups <= kComputeUnits) {
-    parts = steps >= (!several ? 2 : seqs == 1 ? 4 : 6) ? 4 : kLoneWave;
+    parts = steps >= (whole ? (d64 ? 4 : 7) : several ? 6 : 2) ? 4 : kLoneWave;
   } else if (several) {
     parts = workgroups <= 2 * kComputeUnits && steps >= (d64 ? 12 : 48) ? 4 : kLoneWave;
   } else if (workgroups <= 2 * kComputeUnits) {
-    parts = steps >= (workgroups <= 384 ? 12 : 20) ? 4 : steps > 3 ? 2 : kLoneWave;
+    parts = steps >= (whole || workgroups > 384 ? 20 : 12) ? 4 : steps > (whole ? 6 : 3) ? 2 : kLoneWave;
   } else if (workgroups <= 1152) {
-    parts = steps >= (d64 ? 96 : 33) ? 4 : steps > 5 ? 2 : kLoneWave;
+    const bool few = seen == mean && workgroups <= 1024 && !(whole && seqs > 12);  // blocks with the longest streams
+    parts = few && steps >= (d64 ? 64 : workgroups <= 640 ? 28 : 80) ? 4 : steps > 5 ? 2 : kLoneWave;
   } else {
-    parts = steps <= (workgroups > (d64 ? 8192 : 4096) ? 3 : d64 ? 16 : 6) ? kLoneWave : workgroups <= 3000 ? 2 : 1;
+    // (one part: 512 workgroups of 128 keys are a full round)
+    const bool one = d64 ? workgroups > 3000 : whole128 ? workgroups > 1536 : workgroups > 3000 || (workgroups > 1792 && workgroups <= 2048 && steps <= 64);
+    const int64_t lone = workgroups > (d64 ? 8192 : 4096) ? 3 : d64 ? 16 : one && whole128 ? 3 : 6;
+    parts = steps <= lone ? kLoneWave : one ? 1 : 2;
   }
   if (parts == kLoneWave && workgroups > 0x7fffffffLL) parts = 1;
   // Pairs of blocks, whose costs add up to the same for one sequence, or two, where every pair then has a compute unit
