@@ -122,11 +122,8 @@ bool allow_lds(bwd_fn fn, std::atomic<uint64_t>& allowed_on) {
 // of a kv head
 BwdLaunch dkv32_launch(const BwdParams& p, int64_t* groups);
 // head dims 192 and 256 (attention_backward_wide.hip): the dkv kernel over blocks of 64 keys, or of 32 with its stream in two
-// parts while these do not fill the chip twice and a sequence has a step for either part
-inline int dkv32_wide_parts(const BwdParams& p) {
-  const int64_t mean = p.num_seqs > 0 ? p.q_tokens / p.num_seqs : 0;
-  return (p.k_tokens + 31) / 32 * p.kv_heads <= 512 && (mean > 32 || p.q_heads > p.kv_heads) ? 2 : 1;
-}
+// parts, by the blocks of 32 and the steps of their streams
+int dkv32_wide_parts(const BwdParams& p);
 BwdLaunch dq32_wide_launch(const BwdParams& p);
 BwdLaunch dkv32_wide_launch(const BwdParams& p, int64_t* groups);
 #endif

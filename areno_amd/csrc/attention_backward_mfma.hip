@@ -579,11 +579,11 @@ constexpr int64_t kBmComputeUnits = 256;
 // Whether the vector-ALU kernels take a launch of wide heads in less time.  A matrix-core workgroup goes through the
 // sequences of its block one after the other, at least one tile each (the dkv kernel for every q head of the group);
 // the vector-ALU kernels have a wave per row and do not care.  For sequences of 64 tokens and more the matrix cores
-// win by up to 30 times, for many single tokens they lose by as much; in between both are estimated, in us, from what 2 034
-// launches of 1 .. 300 sequences of 1 .. 64 tokens took (head dims 192 and 256, six head ratios, equal and ragged lengths, a window).
-// The choice takes 0.02 % longer than the better of both over equal lengths (4 % at most) and 0.2 % over ragged ones (more than a
-// tenth in 10 of 1 170, 24 % at most).  vector ALU, matrix cores, in us, 16 / 8 heads of 256, bf16: 8 x 4 tokens 53, 91; 64 x 1 53, 460;
-// 64 x 4 149, 140; 8 x 16 81, 48; 300 x 2 377, 270; 8 / 1 heads, 8 x 12 71, 99; 6 / 6 heads, 16 x 12 101, 72.
+// win by up to 30 times, for many single tokens they lose by as much; in between both are estimated, in us, from what 1 494
+// launches of 1 .. 400 sequences took, most of 1 .. 64 tokens (head dims 192 and 256, ten head ratios, equal and ragged lengths,
+// windows).  The choice takes 0.1 % longer than the better of both (more than a tenth in 6, 44 % at most, of ragged lengths).
+// vector ALU, matrix cores, in us, heads of 256: 12 / 4, 4 x 21 tokens 70, 46; 5 x 5 53, 58; 8 / 2, 31 x 7 80, 87; 44 x 8 104, 67; 16 / 8,
+// 77 x 2 124, 180; of 192: 8 / 1, 2 x 12 54, 37; 24 / 8, 6 x 12 63, 52; 12 / 4, 18 x 7 58, 73.
 bool vector_alu_is_faster(const BwdParams& p) {
   const bool d256 = p.head_dim == 256;
   auto ceil_div = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
@@ -599,7 +599,7 @@ bool vector_alu_is_faster(const BwdParams& p) {
                            ceil_div(ceil_div(std::min(queries, reach + dkv_rows), kBmTile) * group, parts) * dkv_rounds;
   const double dq_steps = in_block(kBmRows, queries) * ceil_div(std::min(keys, reach + kBmRows), kBmTile) *
                           ceil_div(ceil_div(p.q_tokens, kBmRows) * p.q_heads, 2 * kBmComputeUnits);
-  const double matrix_cores = d256 ? 14.5 * dkv_rounds + 2.75 * dkv_steps + 6.3 * dq_steps : 11 * dkv_rounds + 2.3 * dkv_steps + 4.2 * dq_steps;
+  const double matrix_cores = d256 ? 11.5 * dkv_rounds + 2.85 * dkv_steps + 4.2 * dq_steps : 10.5 * dkv_rounds + 2.5 * dkv_steps + 3.4 * dq_steps;
   // vector ALU: a wave per row, one of them per SIMD; a row's start and its keys or pairs, 16 at a time
   const int64_t seen = std::min(keys, reach), pairs = std::min(queries, reach) * group, waves = 4 * kBmComputeUnits;
   const int64_t q_rounds = ceil_div(p.q_tokens * p.q_heads, waves), k_rounds = ceil_div(p.k_tokens * p.kv_heads, waves);

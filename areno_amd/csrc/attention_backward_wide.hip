@@ -716,10 +716,20 @@ BwdLaunch dq32_wide_launch(const BwdParams& p) {
   if (p.head_dim == 192) return p.dtype == ARENO_DT_BF16 ? dq_launch_of<KV_BF16, 192>() : dq_launch_of<KV_F16, 192>();
   return p.dtype == ARENO_DT_BF16 ? dq_launch_of<KV_BF16, 256>() : dq_launch_of<KV_F16, 256>();
 }
-// The dkv kernel's shape: blocks of 64 keys, or of 32 with the stream in two parts.  Both kernels of the backward in us, in
-// one part and two (what the 16-row kernels took), blocks of 32 in brackets: heads of 256, window 512: 1 x 1 000 tokens, 8 / 1
-// heads (32) 383, 230 (917); 4 x 300, 16 / 8 (304) 127, 102 (208); 2 717 in four sequences, 16 / 8 (680) 271, 282 (372); 8 x 2 048, no
-// window (4 096) 2 052, 2 267 (2 576).
+// The dkv kernel's shape: blocks of 64 keys, or of 32 with the stream in two parts, which end sooner where the launch is its
+// longest blocks; with more than three rounds of workgroups what counts is the tiles' traffic, half of it per key in the larger
+// blocks (and where blocks hold several sequences, the waves that wait in these).  The backward in us, in one part and two
+// (what the 16-row kernels took); in brackets blocks of 32, steps: heads of 192: 16 / 16, 5 x 34 tokens (96, 1) 39.1, 31.0 (47.6); 24 / 8,
+// 2 x 1 580 (792, 147) 683, 455 (599); 32 / 8, 248 x 12 (744, 12) 214, 170 (209); 8 / 2, 15 x 1 066 (1 000, 132) 764, 622 (678); 6 / 6, 8 x 1 926
+// (2 892, 60) 687, 744 (725); 28 / 4, 3 x 3 196 (1 200, 693) 4 158, 3 608 (3 022); of 256: 6 / 6, 4 x 535 (402, 16) 105, 93 (176); 32 / 8, 2 x 720 (360, 88) 356, 252 (633); 12 / 4, 5 x 1 306
+// (820, 120) 539, 664 (978); 32 / 8, 6 x 1 161 (1 744, 144) 1 227, 1 268 (1 612).  Over 1 971 launches 0.5 % more than the better one.
+int dkv32_wide_parts(const BwdParams& p) {
+  const int64_t seqs = std::max<int64_t>(p.num_seqs, 1), mean = std::max<int64_t>(p.q_tokens / seqs, 1), blocks = (p.k_tokens + 31) / 32 * p.kv_heads;
+  const int64_t seen = p.window_left >= 0 ? std::min<int64_t>(mean, p.window_left + int64_t{32}) : mean;
+  const int64_t steps = std::max<int64_t>(seen / kWideTile, 1) * (p.q_heads / p.kv_heads) * std::min(seqs, 1 + 31 / mean);
+  const bool short_or_long = mean < 32 ? steps >= 7 : p.head_dim == 192 && steps >= 512;
+  return steps >= (blocks > 256 ? 4 : mean > 32 ? 1 : 2) && blocks <= (short_or_long ? 2048 : p.head_dim == 192 ? 1024 : 512) ? 2 : 1;
+}
 BwdLaunch dkv32_wide_launch(const BwdParams& p, int64_t* groups) {
   int parts = dkv32_wide_parts(p);
   // (ARENO_BACKWARD_PARTS=1|2 fixes it, for tests and timing)
