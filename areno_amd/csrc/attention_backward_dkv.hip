@@ -16,12 +16,12 @@
 // a workgroup of one wave, for many short sequences: in a block of 128 keys each of them is a stream that one wave of four
 // computes on while all wait at its barriers.
 //
-// Bound: (4, 1) by the matrix cores (54 % of the cycles, at the clock that they then leave, 1.66 GHz) and LDS; (1, 4) by
+// Bound: (4, 1) by the matrix cores (busy 58 % of the cycles, at the clock that they then leave, 1.7 GHz) and LDS; (1, 4) by
 // what one wave issues, 350 instructions and 34 products of 32 cycles in 2 500.  Where the time was: 16 x 16 x 32 products
 // read an operand of 1 KB each where these read one per two; the compiler waited for every operand right behind its read;
-// the spilled addresses of a step (a scratch load waits for all the fetches in front of it).  Forward and backward, us:
-// 4 x 4 096 tokens, 32 / 8 heads of 128, bf16: 2 904 -> 2 429 (the kernel 1 600 -> 1 000); 2 x 2 048, 28 / 4 heads: 393 -> 340
-// (245 -> 145).
+// the spilled addresses of a step (a scratch load waits for all the fetches in front of it).  Forward and backward, us, with the
+// 16-row kernel and this (the kernel by itself under the profiler): 4 x 4 096 tokens, 32 / 8 heads of 128, bf16: 2 886, 2 357 (1 763, 1 123);
+// 2 x 2 048, 28 / 4 heads: 394, 324 (256, 147).
 #include <algorithm>
 #include <atomic>
 
@@ -427,16 +427,18 @@ constexpr int64_t kComputeUnits = 256;
 // and four pay only where a few blocks' streams are far longer than the rest (not in a window); one part, which two waves
 // per SIMD share, is for launches that fill the chip many times over, sooner where no block of 128 holds two sequences.
 // Lines drawn through 8 753 launches of 1 .. 1 000 sequences of 1 .. 4 096 tokens, ten head ratios, equal and ragged lengths,
-// windows: the choice takes 0.8 % longer than the best of all shapes, and 3 % longer than the 16-row kernels in one.  The backward in us; in brackets blocks, steps.  One wave, two parts, four:  D = 128: 16 / 16 heads, 1 x 26 (16, 1) 11.1, 12.5, 14.3; 6 / 6, 6 x 64
-// (72, 2) 13.9, 16.6, 16.7; 24 / 8, 8 x 160
-// (328, 15) 54.6, 48.5, 45.9; 6 / 6, 5 x 474 (450, 14) 45.0, 43.3, 49.7; 32 / 2, 347 x 14 (316, 48) 208, 198, 163; D = 64: 28 / 4, 9 x 617 (696, 133)
-// 175, 130, 110; 24 / 8, 36 x 75 (680, 6) 39.6, 36.5, 44.3; 28 / 4, 12 x 347 (524, 70) 155, 112, 87; 28 / 4, 38 x 92 (440, 14) 49.0, 43.6, 47.1;
-// D = 128: 8 / 1, 29 x 768, window 512 (696, 136) 258, 197, 245; 32 / 2, 37 x 448 (1 036, 224) 566, 431, 538; 32 / 8, 2 x 1 380 (696, 172): two parts
-// 1.33 times four.
-// One wave, one part, two:  D = 64: 16 / 16, 11 x 716 (3 952, 22) 124, 109, 123; 361 x 132, window 128 (23 840, 4) 432, 408, 460; D = 128: 16 / 8, 196 x
-// 128 (6 272, 8) 279, 259, 272; 16 / 16, 67 x 180, window 128 (6 032, 5) 184, 173, 191; 32 x 128 (2 048, 4) 57, 50, 56; 32 / 8, 61 x 128
-// (1 952, 16) 138, 127, 134.  One part, two, four:  D = 128, 28 / 4: 8 x 2 048 (2 048) 1 006,
-// 963, 1 053; 4 x 4 096, 32 / 8 (4 096) 1 977, 2 056, 2 214.
+// windows: the choice takes 0.8 % longer than the best of all shapes, and 3 % longer than the 16-row kernels in one.  The backward
+// in us, sequences x tokens (blocks, steps):
+//   one wave, two parts, four.  D = 128: 16 / 16 heads, 1 x 26 (16, 1) 11.1, 12.5, 14.3; 6 / 6, 6 x 64 (72, 2) 13.9, 16.6, 16.8; 24 / 8, 8 x 160 (328, 15)
+// 54.6, 48.5, 45.9; 6 / 6, 5 x 474 (450, 14) 45.0, 43.3, 49.7; 32 / 2, 347 x 14 (316, 48) 208, 198, 163; 8 / 1, 29 x 768, window 512 (696, 136) 258, 197, 245;
+// 32 / 2, 37 x 448 (1 036, 224) 566, 431, 538; 32 / 8, 2 x 1 380 (696, 172) 266, 230, 172.  D = 64: 28 / 4, 9 x 617 (696, 133) 175, 130, 110; 24 / 8, 36 x 75
+// (680, 6) 39.6, 36.5, 44.3; 28 / 4, 12 x 347 (524, 70) 155, 112, 87; 28 / 4, 38 x 92 (440, 14) 49.0, 43.6, 47.1; 32 / 8, 2 x 2 048 (1 024, 256) 220, 172, 172.
+//   one wave, one part, two (the 16-row kernels).  D = 128: 16 / 16, 4 096 x 8 (16 384, 4) 717, 854, 899 (948); 512 x 16 (4 096, 2) 111, 125, 135 (133); 32 x 128 (2 048, 4) 55.0,
+// 50.6, 56.5 (57.3); 32 / 8, 61 x 128 (1 952, 16) 139, 127, 133 (155); 16 / 8, 196 x 128 (6 272, 8) 279, 259, 272; 16 / 16, 67 x 180, window 128 (6 032, 5) 184, 173, 191.
+// D = 64: 16 / 16, 4 096 x 8 335, 485, 518 (481); 512 x 8 (2 048, 4) 42, 60, 64 (66); 512 x 4 (1 024, 8) 49, 78, 64 (71); 11 x 716 (3 952, 22) 124, 109, 123; 361 x 132, window 128
+// (23 840, 4) 432, 408, 460.
+//   one part, two, four.  D = 128: 28 / 4, 8 x 2 048 (2 048, 448) 997, 926, 980 (1 182); 32 / 8, 4 x 4 096 (4 096, 512) 1 822, 1 864, 2 027 (2 382); D = 64: 28 / 4, 3 x 4 096
+// (1 536, 896) 887, 704, 764 (1 008).
 BwdLaunch dkv32_launch(const BwdParams& p, int64_t* groups) {
   const int64_t blocks = (p.k_tokens + 31) / 32, workgroups = blocks * p.kv_heads;
   const int64_t seqs = std::max<int64_t>(p.num_seqs, 1), mean = std::max<int64_t>(p.q_tokens / seqs, 1), group = p.q_heads / p.kv_heads;
@@ -457,7 +459,7 @@ BwdLaunch dkv32_launch(const BwdParams& p, int64_t* groups) {
     parts = few && steps >= (d64 ? 64 : workgroups <= 640 ? 28 : 80) ? 4 : steps > 5 ? 2 : kLoneWave;
   } else {
     // (one part: 512 workgroups of 128 keys are a full round)
-    const bool one = d64 ? workgroups > 3000 : whole128 ? workgroups > 1536 : workgroups > 3000 || (workgroups > 1792 && workgroups <= 2048 && steps <= 64);
+    const bool one = workgroups > 3000 || (!d64 && steps <= 64 && (whole128 ? workgroups > 1536 : workgroups > 1792 && workgroups <= 2048));
     const int64_t lone = workgroups > (d64 ? 8192 : 4096) ? 3 : d64 ? 16 : one && whole128 ? 3 : 6;
     parts = steps <= lone ? kLoneWave : one ? 1 : 2;
   }
