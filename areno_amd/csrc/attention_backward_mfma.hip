@@ -332,7 +332,7 @@ __global__ __launch_bounds__(kBmThreads, D == 64 ? 4 : 2) void bwd_mfma_dq_kerne
 // The same with 32 query rows per wave, 128 per workgroup, on 32 x 32 x 16 products, for long sequences: an operand read
 // from LDS serves a product of twice the size, the K and V tiles are fetched straight into LDS (mfma32_tiles.hpp), an
 // operand is read four products in front of its own and the exponentials go between the products of dP.  Bound by the
-// matrix cores (56 % of the cycles at the clock that they then leave, 1.4 to 2 GHz) and the vector ALU.  Forward and
+// matrix cores (busy 53 % of the cycles, at the clock that they then leave, 1.7 GHz) and the vector ALU.  Forward and
 // backward of 4 x 4 096 tokens, 32 / 8 heads of 128, bf16: 2 429 -> 2 375 us with the operands read ahead.  (Registers spill
 // at head dim 128 once per sequence of a block, not in the tile loop.)
 template <int KIND, int D>

@@ -12,8 +12,9 @@
 // in the same order in both kernels, so that its roundings do not count between P and the log-sum-exp.
 //
 // Bound: what one wave issues and waits for (dkv: one wave per SIMD, 500 vector instructions and 64 products of 32
-// cycles a step, a third of the time in waits; dq: two).  Against 16 x 16 x 32 products with 16 rows per wave, both kernels, us: 2 717 tokens in four sequences, 16 / 8
-// heads of 256, window 512, bf16: 372 -> 271; 1 x 1 000, 8 / 1 heads: 917 -> 230.  Relative error of dV against 64 bits, before
+// cycles a step, a third of the time in waits; dq: two).  Against 16 x 16 x 32 products with 16 rows per wave, the backward, us: 2 717
+// tokens in four sequences, 16 / 8 heads of 256, window 512, bf16: 357 -> 197 (under the profiler dkv 239 -> 135, dq 109 -> 83);
+// 1 x 1 000, 8 / 1 heads: 911 -> 216.  Relative error of dV against 64 bits, before
 // and now: 2.74e-7, 2.64e-7 (bf16), 2.83e-7, 2.71e-7 (fp16); queries four times as large: 6.2e-7, 5.7e-7.
 #include <algorithm>
 #include <atomic>
@@ -721,8 +722,9 @@ BwdLaunch dq32_wide_launch(const BwdParams& p) {
 // blocks (and where blocks hold several sequences, the waves that wait in these).  The backward in us, in one part and two
 // (what the 16-row kernels took); in brackets blocks of 32, steps: heads of 192: 16 / 16, 5 x 34 tokens (96, 1) 39.1, 31.0 (47.6); 24 / 8,
 // 2 x 1 580 (792, 147) 683, 455 (599); 32 / 8, 248 x 12 (744, 12) 214, 170 (209); 8 / 2, 15 x 1 066 (1 000, 132) 764, 622 (678); 6 / 6, 8 x 1 926
-// (2 892, 60) 687, 744 (725); 28 / 4, 3 x 3 196 (1 200, 693) 4 158, 3 608 (3 022); of 256: 6 / 6, 4 x 535 (402, 16) 105, 93 (176); 32 / 8, 2 x 720 (360, 88) 356, 252 (633); 12 / 4, 5 x 1 306
-// (820, 120) 539, 664 (978); 32 / 8, 6 x 1 161 (1 744, 144) 1 227, 1 268 (1 612).  Over 1 971 launches 0.5 % more than the better one.
+// (2 892, 60) 687, 744 (725); 28 / 4, 3 x 3 196 (1 200, 693) 4 158, 3 608 (3 022); of 256: 6 / 6,
+// 4 x 535 (402, 16) 105, 93 (176); 32 / 8, 2 x 720 (360, 88) 356, 252 (633); 8 / 1, 1 x 1 000, window 512 (32, 136) 367, 216 (911); 12 / 4, 5 x 1 306 (820, 120)
+// 539, 664 (978); 32 / 8, 6 x 1 161 (1 744, 144) 1 227, 1 268 (1 612); 28 / 4, 8 x 2 048 (2 048, 448) 3 684, 3 831 (4 569).  Over 1 971 launches 0.5 % more than the better one.
 int dkv32_wide_parts(const BwdParams& p) {
   const int64_t seqs = std::max<int64_t>(p.num_seqs, 1), mean = std::max<int64_t>(p.q_tokens / seqs, 1), blocks = (p.k_tokens + 31) / 32 * p.kv_heads;
   const int64_t seen = p.window_left >= 0 ? std::min<int64_t>(mean, p.window_left + int64_t{32}) : mean;

@@ -912,8 +912,10 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
 // item's rows are spread over many small workgroups (blockIdx.z; each thread has kMergeChunks 16-byte chunks of every
 // partial), and kMergeBatch partials are asked for before the first of them is used.
 // Kernel time, us: 28 / 4 heads of 128, the follow-ups of 4 sequences, up to 64 tokens on 4 k cached ones, about 11
-// partials per item: 22.5 -> 10.9 (with one chunk per thread 12.0, with batches of 4 12.4); 32 / 8 heads, 16 chunks of up to
-// 512 tokens on 16 k cached ones, an item to merge in almost every unit: 15.
+// partials per item: 22.5 -> 10.9 (with one chunk per thread 12.0); 32 / 8 heads, 16 chunks of up to 512 tokens on 16 k cached
+// ones, an item to merge in almost every unit: 15.  The batch where a workgroup has an item: the attention's us with 4, 8, 12, 16,
+// 24: 8 / 1 heads, 1 x 8 tokens on 4 k 66.8, 65.6, 64.8, 65.0, 67.0; on 16 k 105.9, 101.7, 99.9, 98.7, 102.7; 28 / 4, 1 x 8 on 4 k 38.0, 37.0, 36.8,
+// 36.4, 37.3; 4 x 64 on 4 k 48.2, 48.3, 49.4, 49.3, 52.6; 8 x 32 on 300 29.4, 29.5, 28.5, 28.5, 33.7.
 constexpr int kMergeThreads = 256;
 constexpr int kMergeChunks = 2;
 

@@ -260,8 +260,8 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) s[kt] = zero16();
     // Wide heads: the products' operands in one stream, each read kAhead products in front of its own (the compiler, short of
-    // registers, waits for most of them right behind the read): rows of K, then columns of V.  2 x 4 500 tokens, 16 / 8 heads of
-    // 256, window 1 024: 165 -> 160 us; up to head dim 128 it changes the time by -7 to +3 % and is not used.
+    // registers, waits for most of them right behind the read): rows of K, then columns of V.  Two sequences of 3 000 .. 6 000
+    // tokens, 16 / 8 heads of 256, window 1 024: 162 -> 158 us (under the profiler); up to head dim 128 it changes the time by -7 to +3 % and is not used.
     constexpr int kScores = NKS * KT, kReads = kScores + 2 * KT * NB, kAhead = D == 256 ? 3 : 4;
     auto read = [&](int x) {
       if (x < kScores) return tile_rows<KIND, T>(kt_lds, at_rows, 32 * (x % KT), x / KT);
