@@ -538,3 +538,19 @@ def test_gradients_in_the_input_dtype_are_the_fp32_gradients_rounded_once(dtype,
     for a, b, name in zip(wide, typed, ("dq", "dk", "dv")):
         assert a.dtype == torch.float32 and b.dtype == dtype
         assert torch.equal(a.to(dtype), b), f"{name} {dtype} d={d}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,parts,dq_rows", [(64, "1w", "16"), (64, "4s", "32"), (128, "1", "32"), (128, "2", "16"), (192, "1", "16"), (192, "2", "16"), (256, "1", "16"), (256, "2", "16")])
+def test_gradients_in_the_inputs_type_are_the_fp32_ones_rounded_in_every_form(dtype, d, parts, dq_rows, monkeypatch):
+    """The kernels' stores in either type, rows behind the last sequence (zeros) included: bit for bit the same sums, rounded
+    once."""
+    monkeypatch.setenv("ARENO_BACKWARD_PARTS", parts)
+    monkeypatch.setenv("ARENO_BACKWARD_DQ_ROWS", dq_rows)
+    g = torch.Generator().manual_seed(d)
+    cu = torch.tensor([0, 33, 33, 170], dtype=torch.int32, device=DEV)
+    q, k, v, go = (torch.randn(203, h, d, generator=g).to(dtype).to(DEV) for h in (4, 2, 2, 4))
+    out = ops.areno_varlen_causal_attention(q, k, v, cu)
+    wide, narrow = (_c_backward(go, q, k, v, out, cu, t, d**-0.5) for t in (torch.float32, dtype))
+    for w, n, name in zip(wide, narrow, ("dq", "dk", "dv")):
+        assert w[:170].abs().max() > 0 and torch.equal(w.to(dtype), n), f"{name} {dtype} d={d} parts={parts}"
