@@ -360,6 +360,7 @@ extern "C" int areno_hip_attention_backward_typed(const void* grad_out, const vo
   p.head_dim = head_dim;
   p.dtype = dtype;
   p.grad_dtype = grad_dtype;
+  p.q_order = p.k_order = BlockOrder{};
   p.scale = softmax_scale;
   p.scale_log2e = softmax_scale * kLog2e;
   // 16-bit inputs at head dims 64, 128, 192 and 256 run on the matrix cores (ARENO_BACKWARD_KERNEL=valu: a diagnosis switch

@@ -26,7 +26,6 @@
 #include <atomic>
 
 #include "attention_backward.hpp"
-#include "backward_order.hpp"
 #include "mfma32_tiles.hpp"
 
 namespace areno {
@@ -58,6 +57,7 @@ __global__ __launch_bounds__((Dkv32Shape<D, KW, P>::kThreads)) __attribute__((am
   constexpr int NKS = D / 16, NB = D / 32, NF = T::kFetches;
   constexpr bool kTight = D > 64 && OCC > 1;  // sums, K and V and the scores leave 32 registers for all the rest
 
+  ask_for_arguments(p, p.k_order);
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave_of_block = uniform(tid >> 6);
@@ -69,7 +69,7 @@ __global__ __launch_bounds__((Dkv32Shape<D, KW, P>::kThreads)) __attribute__((am
   const int wg = static_cast<int>(blockIdx.x / static_cast<unsigned>(p.kv_heads));
   // (launched with a workgroup per pair of blocks, or with one per block: then in cost order, one block each)
   const bool paired = gridDim.x / static_cast<unsigned>(p.kv_heads) < static_cast<unsigned>(k_blocks);
-  const int first_block = paired ? wg : uniform(static_cast<int>(block_in_cost_order(wg, k_blocks, p.num_seqs, false)));
+  const int first_block = paired ? wg : uniform(block_in_launch_order(wg, p.k_order, L::kKeys, false));
 
   // (with the part's place: a multiple of 256, which the reads' exclusive-ors leave alone)
   static_assert(L::kPart % 256 == 0, "the parts' places");

@@ -14,7 +14,7 @@
 //                of the group, the query rows that may see them:  S = Q . K^T,  dP = dO . V^T,  P = exp2(S - lse),
 //                dS = P * (dP - dO . O),  dV^T += dO^T . P  and  dK^T += Q^T . dS.  Every gradient element has one owner.
 // Head dims 192 and 256 have both kernels in attention_backward_wide.hip.
-// Both launches take their blocks in an order that lets their workgroups end together: see block_in_cost_order.
+// Both launches take their blocks in an order that lets their workgroups end together: see block_in_launch_order.
 //
 // The streamed index of a tile (keys in the dq kernel, queries in the dkv kernel) is the contraction index of the
 // second pair of products; a 16 x 16 product leaves element 4 g + j of that index in lane group g, which is exactly
@@ -28,7 +28,6 @@
 #include <algorithm>
 
 #include "attention_backward.hpp"
-#include "backward_order.hpp"
 #include "decode_mfma_kernels.hpp"
 #include "mfma32_tiles.hpp"
 
@@ -108,6 +107,7 @@ __global__ __launch_bounds__(kBmThreads, D == 64 ? 4 : 2) void bwd_mfma_dq_kerne
   __shared__ __attribute__((aligned(16))) char k_lds[2 * kBmTile * T::RS];
   __shared__ __attribute__((aligned(16))) char v_lds[2 * kBmTile * T::RS];
 
+  ask_for_arguments(p, p.q_order);
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = uniform(tid >> 6);  // (in a scalar register: what follows from it is scalar work and scalar branches)
@@ -115,8 +115,7 @@ __global__ __launch_bounds__(kBmThreads, D == 64 ? 4 : 2) void bwd_mfma_dq_kerne
   // workgroups in launch order: the heads of a block next to each other, the blocks by cost
   const int h = static_cast<int>(blockIdx.x % static_cast<unsigned>(p.q_heads));
   const int kvh = h / (p.q_heads / p.kv_heads);
-  const int64_t q_blocks = (p.q_tokens + kRows - 1) / kRows;
-  const int64_t r0 = block_in_cost_order(blockIdx.x / static_cast<unsigned>(p.q_heads), q_blocks, p.num_seqs, true) * kRows;
+  const int64_t r0 = int64_t{block_in_launch_order(static_cast<int>(blockIdx.x / static_cast<unsigned>(p.q_heads)), p.q_order, kRows, true)} * kRows;
   const int64_t block_end = r0 + kRows < p.q_tokens ? r0 + kRows : p.q_tokens;
   const int64_t wave_row0 = r0 + kWaveRows * wave;
   int64_t row;  // this lane's query rows (columns of the products)
@@ -345,15 +344,14 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
   constexpr int kBuffer = 2 * T::kBytes;  // K, V
   __shared__ __attribute__((aligned(1024))) char lds[2 * kBuffer];
 
+  ask_for_arguments(p, p.q_order);
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = uniform(tid >> 6);
   const int l32 = lane & 31, half = lane >> 5;
   const int h = static_cast<int>(blockIdx.x % static_cast<unsigned>(p.q_heads));
   const int kvh = h / (p.q_heads / p.kv_heads);
-  const int64_t q_blocks = (p.q_tokens + kRows - 1) / kRows;
-  const int block = uniform(static_cast<int>(
-      block_in_cost_order(blockIdx.x / static_cast<unsigned>(p.q_heads), q_blocks, p.num_seqs, true)));
+  const int block = uniform(block_in_launch_order(static_cast<int>(blockIdx.x / static_cast<unsigned>(p.q_heads)), p.q_order, kRows, true));
   const int64_t r0 = static_cast<int64_t>(block) * kRows;
   const int64_t block_end = r0 + kRows < p.q_tokens ? r0 + kRows : p.q_tokens;
   const int64_t wave_row0 = r0 + 32 * wave;
@@ -664,13 +662,16 @@ int launch_attention_backward_mfma(const BwdParams& p, void* stream) {
   const char* op = "areno_hip_attention_backward";
   if (dq.fn == nullptr || dkv.fn == nullptr) return fail(ARENO_ERR_LAUNCH, "%s: the kernels' LDS size was refused", op);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  BwdParams params = p;
+  params.q_order = block_order(p.q_tokens, dq.rows, p.num_seqs);
+  params.k_order = block_order(p.k_tokens, dkv.rows, p.num_seqs);
   if (q_blocks > 0) {
     const int64_t dq_blocks = (p.q_tokens + dq.rows - 1) / dq.rows;
-    hipLaunchKernelGGL(dq.fn, dim3(static_cast<unsigned>(dq_blocks * p.q_heads)), dim3(dq.threads), dq.lds_bytes, s, p);
+    hipLaunchKernelGGL(dq.fn, dim3(static_cast<unsigned>(dq_blocks * p.q_heads)), dim3(dq.threads), dq.lds_bytes, s, params);
     if (int rc = check_launch(op)) return rc;
   }
   if (k_blocks > 0) {
-    hipLaunchKernelGGL(dkv.fn, dim3(static_cast<unsigned>(dkv_groups * p.kv_heads)), dim3(dkv.threads), dkv.lds_bytes, s, p);
+    hipLaunchKernelGGL(dkv.fn, dim3(static_cast<unsigned>(dkv_groups * p.kv_heads)), dim3(dkv.threads), dkv.lds_bytes, s, params);
     if (int rc = check_launch(op)) return rc;
   }
   return ARENO_OK;

@@ -20,7 +20,6 @@
 #include <atomic>
 
 #include "attention_backward.hpp"
-#include "backward_order.hpp"
 #include "mfma32_tiles.hpp"
 
 namespace areno {
@@ -151,6 +150,7 @@ __global__ __launch_bounds__(kWideDqWaves* kWave) __attribute__((amdgpu_waves_pe
   using T = typename L::Tile;
   constexpr int NKS = D / 16, NB = D / 64, NF = T::kFetches;  // NB: a wave's blocks of 32 columns of dQ, every second one
 
+  ask_for_arguments(p, p.q_order);
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave_of_block = uniform(tid >> 6);
@@ -159,9 +159,7 @@ __global__ __launch_bounds__(kWideDqWaves* kWave) __attribute__((amdgpu_waves_pe
   const int half = lane >> 5;
   const int h = static_cast<int>(blockIdx.x % static_cast<unsigned>(p.q_heads));
   const int kvh = h / (p.q_heads / p.kv_heads);
-  const int64_t q_blocks = (p.q_tokens + L::kRows - 1) / L::kRows;
-  const int block = uniform(static_cast<int>(
-      block_in_cost_order(blockIdx.x / static_cast<unsigned>(p.q_heads), q_blocks, p.num_seqs, true)));
+  const int block = uniform(block_in_launch_order(static_cast<int>(blockIdx.x / static_cast<unsigned>(p.q_heads)), p.q_order, L::kRows, true));
   const int64_t r0 = static_cast<int64_t>(block) * L::kRows;
   const int64_t block_end = r0 + L::kRows < p.q_tokens ? r0 + L::kRows : p.q_tokens;
   const int64_t wave_row0 = r0 + 32 * wave;
@@ -423,6 +421,7 @@ __global__ __launch_bounds__((WideShape<D, KW, P>::kThreads)) __attribute__((amd
   using T = typename L::Tile;
   constexpr int NKS = D / 16, NB = D / 32, NF = T::kFetches;
 
+  ask_for_arguments(p, p.k_order);
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave_of_block = uniform(tid >> 6);
@@ -431,9 +430,7 @@ __global__ __launch_bounds__((WideShape<D, KW, P>::kThreads)) __attribute__((amd
   const bool second = part_wave & 1;  // V and dK
   const int kvh = static_cast<int>(blockIdx.x % static_cast<unsigned>(p.kv_heads));
   const int group = p.q_heads / p.kv_heads;
-  const int k_blocks = static_cast<int>((p.k_tokens + L::kKeys - 1) / L::kKeys);
-  const int block = uniform(static_cast<int>(
-      block_in_cost_order(blockIdx.x / static_cast<unsigned>(p.kv_heads), k_blocks, p.num_seqs, false)));
+  const int block = uniform(block_in_launch_order(static_cast<int>(blockIdx.x / static_cast<unsigned>(p.kv_heads)), p.k_order, L::kKeys, false));
   const int64_t r0 = static_cast<int64_t>(block) * L::kKeys;
   const int64_t block_end = r0 + L::kKeys < p.k_tokens ? r0 + L::kKeys : p.k_tokens;
 
@@ -722,15 +719,14 @@ BwdLaunch dq32_wide_launch(const BwdParams& p) {
 // blocks (and where blocks hold several sequences, the waves that wait in these).  The backward in us, in one part and two
 // (what the 16-row kernels took); in brackets blocks of 32, steps: heads of 192: 16 / 16, 5 x 34 tokens (96, 1) 39.1, 31.0 (47.6); 24 / 8,
 // 2 x 1 580 (792, 147) 683, 455 (599); 32 / 8, 248 x 12 (744, 12) 214, 170 (209); 8 / 2, 15 x 1 066 (1 000, 132) 764, 622 (678); 6 / 6, 8 x 1 926
-// (2 892, 60) 687, 744 (725); 28 / 4, 3 x 3 196 (1 200, 693) 4 158, 3 608 (3 022); of 256: 6 / 6,
+// (2 892, 60) 687, 744 (725); of 256: 6 / 6,
 // 4 x 535 (402, 16) 105, 93 (176); 32 / 8, 2 x 720 (360, 88) 356, 252 (633); 8 / 1, 1 x 1 000, window 512 (32, 136) 367, 216 (911); 12 / 4, 5 x 1 306 (820, 120)
 // 539, 664 (978); 32 / 8, 6 x 1 161 (1 744, 144) 1 227, 1 268 (1 612); 28 / 4, 8 x 2 048 (2 048, 448) 3 684, 3 831 (4 569).  Over 1 971 launches 0.5 % more than the better one.
 int dkv32_wide_parts(const BwdParams& p) {
   const int64_t seqs = std::max<int64_t>(p.num_seqs, 1), mean = std::max<int64_t>(p.q_tokens / seqs, 1), blocks = (p.k_tokens + 31) / 32 * p.kv_heads;
   const int64_t seen = p.window_left >= 0 ? std::min<int64_t>(mean, p.window_left + int64_t{32}) : mean;
   const int64_t steps = std::max<int64_t>(seen / kWideTile, 1) * (p.q_heads / p.kv_heads) * std::min(seqs, 1 + 31 / mean);
-  const bool short_or_long = mean < 32 ? steps >= 7 : p.head_dim == 192 && steps >= 512;
-  return steps >= (blocks > 256 ? 4 : mean > 32 ? 1 : 2) && blocks <= (short_or_long ? 2048 : p.head_dim == 192 ? 1024 : 512) ? 2 : 1;
+  return steps >= (blocks > 256 ? 4 : mean > 32 ? 1 : 2) && blocks <= (mean < 32 && steps >= 7 ? 2048 : p.head_dim == 192 ? 1024 : 512) ? 2 : 1;
 }
 BwdLaunch dkv32_wide_launch(const BwdParams& p, int64_t* groups) {
   int parts = dkv32_wide_parts(p);
