@@ -20,8 +20,8 @@
 // what one wave issues, 350 instructions and 34 products of 32 cycles in 2 500.  Where the time was: 16 x 16 x 32 products
 // read an operand of 1 KB each where these read one per two; the compiler waited for every operand right behind its read;
 // the spilled addresses of a step (a scratch load waits for all the fetches in front of it).  Forward and backward, us, with the
-// 16-row kernel and this (the kernel by itself under the profiler): 4 x 4 096 tokens, 32 / 8 heads of 128, bf16: 2 886, 2 357 (1 763, 1 123);
-// 2 x 2 048, 28 / 4 heads: 394, 324 (256, 147).
+// 16-row kernel and this (the kernel by itself under the profiler): 4 x 4 096 tokens, 32 / 8 heads of 128, bf16: 2 886, 2 357 (1 763, 1 091);
+// 2 x 2 048, 28 / 4 heads: 394, 324 (256, 143).
 #include <algorithm>
 #include <atomic>
 

@@ -13,8 +13,8 @@
 //
 // Bound: what one wave issues and waits for (dkv: one wave per SIMD, 500 vector instructions and 64 products of 32
 // cycles a step, a third of the time in waits; dq: two).  Against 16 x 16 x 32 products with 16 rows per wave, the backward, us: 2 717
-// tokens in four sequences, 16 / 8 heads of 256, window 512, bf16: 357 -> 197 (under the profiler dkv 239 -> 135, dq 109 -> 83);
-// 1 x 1 000, 8 / 1 heads: 911 -> 216.  Relative error of dV against 64 bits, before
+// tokens in four sequences, 16 / 8 heads of 256, window 512, bf16: 354 -> 198 (the profiler's dkv 239 -> 133, dq 109 -> 77);
+// 1 x 1 000, 8 / 1 heads: 910 -> 217.  Relative error of dV against 64 bits, before
 // and now: 2.74e-7, 2.64e-7 (bf16), 2.83e-7, 2.71e-7 (fp16); queries four times as large: 6.2e-7, 5.7e-7.
 #include <algorithm>
 #include <atomic>
