@@ -15,6 +15,7 @@ from areno_amd.accel.attention import (
     areno_qk_norm_rope_cache_write,
     areno_rope_rows,
     areno_varlen_causal_attention,
+    areno_varlen_causal_attention_cache_write,
 )
 
 __all__ = [
@@ -26,4 +27,5 @@ __all__ = [
     "areno_qk_norm_rope_cache_write",
     "areno_rope_rows",
     "areno_varlen_causal_attention",
+    "areno_varlen_causal_attention_cache_write",
 ]

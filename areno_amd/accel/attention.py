@@ -80,10 +80,12 @@ class _VarlenCausalAttention(torch.autograd.Function):
     return fp32 gradients that are cast to the inputs' dtypes."""
 
     @staticmethod
-    def forward(ctx, q, k, v, cu_seqlens, window_left: int, softmax_scale: float):
-        out = _extension().areno_varlen_causal_attention_forward(
-            q.contiguous(), k.contiguous(), v.contiguous(), cu_seqlens.contiguous(), window_left, softmax_scale
-        )
+    def forward(ctx, q, k, v, cu_seqlens, window_left: int, softmax_scale: float, pages=None):
+        args = (q.contiguous(), k.contiguous(), v.contiguous(), cu_seqlens.contiguous(), window_left, softmax_scale)
+        if pages is None:
+            out = _extension().areno_varlen_causal_attention_forward(*args)
+        else:  # (a tuple: the caches take no part in the graph, as in areno_paged_cache_write)
+            out = _extension().areno_varlen_causal_attention_forward_cache_write(*args, *pages)
         ctx.save_for_backward(q, k, v, out, cu_seqlens)
         ctx.window_left = window_left
         ctx.softmax_scale = softmax_scale
@@ -98,7 +100,7 @@ class _VarlenCausalAttention(torch.autograd.Function):
         )  # fmt: skip
         # (the kernels round their fp32 sums to the inputs' dtype at the store: the casts of the reference's wrapper,
         # ``areno/accel/attention.py:117-118`` there, without fp32 tensors in between)
-        return dq, dk, dv, None, None, None
+        return dq, dk, dv, None, None, None, None
 
 
 class _PagedDecode(torch.autograd.Function):
@@ -377,18 +379,7 @@ def areno_paged_causal_attention_decode(
     return call()
 
 
-@torch._dynamo.disable
-def areno_varlen_causal_attention(
-    q: torch.Tensor,
-    k: torch.Tensor,
-    v: torch.Tensor,
-    cu_seqlens: torch.Tensor,
-    *,
-    window_left: int | None = None,
-    softmax_scale: float | None = None,
-) -> torch.Tensor:
-    """Apply packed causal attention to flat ``(tokens, heads, head_dim)`` tensors."""
-    op = "areno_varlen_causal_attention"
+def _check_varlen(op: str, q, k, v, cu_seqlens) -> None:
     if not _all_on_gpu(q, k, v, cu_seqlens):
         raise RuntimeError(f"{op} requires CUDA q, k, v, and cu_seqlens tensors")
     if q.dim() != 3 or k.dim() != 3 or v.dim() != 3:
@@ -401,6 +392,20 @@ def areno_varlen_causal_attention(
         raise ValueError(f"{op} expects q heads to be divisible by kv heads")
     if q.shape[2] != k.shape[2] or q.shape[2] != v.shape[2]:
         raise ValueError(f"{op} head dim mismatch")
+
+
+@torch._dynamo.disable
+def areno_varlen_causal_attention(
+    q: torch.Tensor,
+    k: torch.Tensor,
+    v: torch.Tensor,
+    cu_seqlens: torch.Tensor,
+    *,
+    window_left: int | None = None,
+    softmax_scale: float | None = None,
+) -> torch.Tensor:
+    """Apply packed causal attention to flat ``(tokens, heads, head_dim)`` tensors."""
+    _check_varlen("areno_varlen_causal_attention", q, k, v, cu_seqlens)
     if q.dtype == torch.float64 and k.dtype == torch.float64 and v.dtype == torch.float64:
         # the reference's kernels read doubles and compute in fp32 (attention.cu:846 there): the same through casts
         return _VarlenCausalAttention.apply(q.float(), k.float(), v.float(), cu_seqlens, _window_left(window_left),
@@ -445,6 +450,24 @@ def areno_causal_attention(
     return _CausalAttention.apply(q, k, v, int(query_start), _window_left(window_left), _scale(q, softmax_scale))
 
 
+def _check_cache_write(op: str, k, v, k_cache, v_cache, cache_block_ids, cache_block_offsets, k_scale, v_scale) -> None:
+    if not _all_on_gpu(k, v, k_cache, v_cache, cache_block_ids, cache_block_offsets, k_scale, v_scale):
+        raise RuntimeError(f"{op} requires CUDA tensors")
+    if k.dim() != 3 or v.dim() != 3:
+        raise ValueError(f"{op} expects k/v shaped (tokens, kv_heads, head_dim)")
+    if k_cache.dim() != 4 or v_cache.dim() != 4:
+        raise ValueError(f"{op} expects 4D paged cache tensors")
+    if cache_block_ids.dim() != 1 or cache_block_offsets.dim() != 1:
+        raise ValueError(f"{op} expects 1D cache_block_ids and cache_block_offsets")
+    if cache_block_ids.dtype != torch.int64 or cache_block_offsets.dtype != torch.int64:
+        raise ValueError(f"{op} expects int64 cache_block_ids and cache_block_offsets")
+    _check_scales(op, k_cache, k_scale, v_scale)
+    if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
+        raise ValueError(f"{op} expects contiguous cache tensors (they are updated in place)")
+    if k_scale is not None and not (k_scale.is_contiguous() and v_scale.is_contiguous()):
+        raise ValueError(f"{op} expects contiguous scale tensors (they are updated in place)")
+
+
 @torch._dynamo.disable
 def areno_paged_cache_write(
     k: torch.Tensor,
@@ -462,26 +485,36 @@ def areno_paged_cache_write(
     For ``int8`` / ``float8_e4m3fn`` caches each ``(token, kv head)`` row gets its own scale,
     written to ``k_scale``/``v_scale`` at the same ``(block, slot)``.
     """
-    op = "areno_paged_cache_write"
-    if not _all_on_gpu(k, v, k_cache, v_cache, cache_block_ids, cache_block_offsets, k_scale, v_scale):
-        raise RuntimeError(f"{op} requires CUDA tensors")
-    if k.dim() != 3 or v.dim() != 3:
-        raise ValueError(f"{op} expects k/v shaped (tokens, kv_heads, head_dim)")
-    if k_cache.dim() != 4 or v_cache.dim() != 4:
-        raise ValueError(f"{op} expects 4D paged cache tensors")
-    if cache_block_ids.dim() != 1 or cache_block_offsets.dim() != 1:
-        raise ValueError(f"{op} expects 1D cache_block_ids and cache_block_offsets")
-    if cache_block_ids.dtype != torch.int64 or cache_block_offsets.dtype != torch.int64:
-        raise ValueError(f"{op} expects int64 cache_block_ids and cache_block_offsets")
-    _check_scales(op, k_cache, k_scale, v_scale)
-    if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
-        raise ValueError(f"{op} expects contiguous cache tensors (they are updated in place)")
-    if k_scale is not None and not (k_scale.is_contiguous() and v_scale.is_contiguous()):
-        raise ValueError(f"{op} expects contiguous scale tensors (they are updated in place)")
+    _check_cache_write("areno_paged_cache_write", k, v, k_cache, v_cache, cache_block_ids, cache_block_offsets, k_scale, v_scale)
     _extension().areno_paged_cache_write(
         k.contiguous(), v.contiguous(), k_cache, v_cache,
         cache_block_ids.contiguous(), cache_block_offsets.contiguous(), k_scale, v_scale,
     )  # fmt: skip
+
+
+@torch._dynamo.disable
+def areno_varlen_causal_attention_cache_write(
+    q: torch.Tensor,
+    k: torch.Tensor,
+    v: torch.Tensor,
+    cu_seqlens: torch.Tensor,
+    k_cache: torch.Tensor,
+    v_cache: torch.Tensor,
+    cache_block_ids: torch.Tensor,
+    cache_block_offsets: torch.Tensor,
+    *,
+    window_left: int | None = None,
+    softmax_scale: float | None = None,
+    k_scale: torch.Tensor | None = None,
+    v_scale: torch.Tensor | None = None,
+) -> torch.Tensor:
+    """:func:`areno_paged_cache_write` of ``k`` / ``v`` and :func:`areno_varlen_causal_attention` over them, the prefill
+    of fresh prompts: neither needs the other's result, and where the sizes allow it one launch does both.  Pages and
+    output are the same bits as those of the two ops."""
+    _check_cache_write("areno_paged_cache_write", k, v, k_cache, v_cache, cache_block_ids, cache_block_offsets, k_scale, v_scale)
+    _check_varlen("areno_varlen_causal_attention", q, k, v, cu_seqlens)
+    pages = (k_cache, v_cache, cache_block_ids.contiguous(), cache_block_offsets.contiguous(), k_scale, v_scale)
+    return _VarlenCausalAttention.apply(q, k, v, cu_seqlens, _window_left(window_left), _scale(q, softmax_scale), pages)
 
 
 @torch._dynamo.disable

@@ -111,22 +111,6 @@ struct BwdLaunch {
   bwd_fn fn;  // nullptr: its LDS size was refused
   int lds_bytes, threads, rows;  // (rows of a block)
 };
-// more than 64 KB of LDS has to be allowed once per device; one bit per device (the attribute belongs to the device's copy)
-template <int BYTES>
-bool allow_lds(bwd_fn fn, std::atomic<uint64_t>& allowed_on) {
-  if constexpr (BYTES > 64 * 1024) {
-    int device = 0;
-    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return false;
-    if ((allowed_on.load(std::memory_order_acquire) >> device & 1) == 0) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, BYTES) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-      }
-      allowed_on.fetch_or(uint64_t{1} << device, std::memory_order_release);
-    }
-  }
-  return true;
-}
 // the kernels on 32 x 32 x 16 products (attention_backward_dkv.hip), head dims 64 and 128, 16-bit types; `groups`: workgroups
 // of a kv head
 BwdLaunch dkv32_launch(const BwdParams& p, int64_t* groups);

@@ -403,7 +403,7 @@ BwdLaunch launch_of() {
   using L = Dkv32Shape<D, KW, P>;
   const bwd_fn fn = bwd_mfma32_dkv_kernel<KIND, D, KW, P, OCC>;
   static std::atomic<uint64_t> allowed_on{0};
-  if (!allow_lds<L::kLdsBytes>(fn, allowed_on)) return BwdLaunch{nullptr, 0, 0, 0};
+  if (!allow_lds<L::kLdsBytes>(reinterpret_cast<const void*>(fn), allowed_on)) return BwdLaunch{nullptr, 0, 0, 0};
   return BwdLaunch{fn, L::kLdsBytes, L::kThreads, L::kKeys};
 }
 constexpr int kLoneWave = 0;  // for the parts: one wave

@@ -692,7 +692,7 @@ BwdLaunch launch_of() {
   using L = WideShape<D, KW, P>;
   const bwd_fn fn = bwd_mfma32_wide_dkv_kernel<KIND, D, KW, P>;
   static std::atomic<uint64_t> allowed_on{0};
-  if (!allow_lds<L::kLdsBytes>(fn, allowed_on)) return BwdLaunch{nullptr, 0, 0, 0};
+  if (!allow_lds<L::kLdsBytes>(reinterpret_cast<const void*>(fn), allowed_on)) return BwdLaunch{nullptr, 0, 0, 0};
   return BwdLaunch{fn, L::kLdsBytes, L::kThreads, L::kKeys};
 }
 template <int KIND, int D>
@@ -707,7 +707,7 @@ BwdLaunch dq_launch_of() {
   using L = WideDqShape<D>;
   const bwd_fn fn = bwd_mfma32_wide_dq_kernel<KIND, D>;
   static std::atomic<uint64_t> allowed_on{0};
-  if (!allow_lds<L::kLdsBytes>(fn, allowed_on)) return BwdLaunch{nullptr, 0, 0, 0};
+  if (!allow_lds<L::kLdsBytes>(reinterpret_cast<const void*>(fn), allowed_on)) return BwdLaunch{nullptr, 0, 0, 0};
   return BwdLaunch{fn, L::kLdsBytes, kWideDqWaves * kWave, L::kRows};
 }
 BwdLaunch dq32_wide_launch(const BwdParams& p) {

@@ -85,10 +85,23 @@ __device__ __forceinline__ uint32_t pack_two_16(float lo, float hi, int dtype) {
                                 : (float_to_f16_bits(lo) | (float_to_f16_bits(hi) << 16));
 }
 
+// (the steps of wave_max_fast: LPR lanes next to each other, a power of two)
 template <int LPR>
 __device__ __forceinline__ float lane_group_max(float x) {
-#pragma unroll
-  for (int m = 1; m < LPR; m <<= 1) x = fmaxf(x, wave_xor(x, m));
+  if constexpr (LPR >= 2) x = max_f32(x, dpp_lanes<kDppQuadSwap1>(x));
+  if constexpr (LPR >= 4) x = max_f32(x, dpp_lanes<kDppQuadSwap2>(x));
+  if constexpr (LPR >= 8) x = max_f32(x, dpp_lanes<kDppRowHalfMirror>(x));
+  if constexpr (LPR >= 16) x = max_f32(x, dpp_lanes<kDppRowMirror>(x));
+  if constexpr (LPR >= 32) {
+    uint32_t a = __builtin_bit_cast(uint32_t, x), b = a;
+    swap_rows16(a, b);
+    x = max_f32(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+  }
+  if constexpr (LPR >= 64) {
+    uint32_t a = __builtin_bit_cast(uint32_t, x), b = a;
+    swap_rows32(a, b);
+    x = max_f32(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+  }
   return x;
 }
 

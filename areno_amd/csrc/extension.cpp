@@ -242,9 +242,7 @@ at::Tensor paged_decode_forward(at::Tensor q, at::Tensor k_update, at::Tensor v_
                                    num_splits, softmax_scale, c10::nullopt, c10::nullopt, 0, c10::nullopt, nullptr);
 }
 
-at::Tensor varlen_forward(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor cu_seqlens, int64_t window_left,
-                          double softmax_scale) {
-  const char* op = "areno_varlen_causal_attention";
+void check_varlen(const char* op, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& cu_seqlens) {
   TORCH_CHECK(q.is_cuda(), op, " q must be CUDA");
   TORCH_CHECK(k.is_cuda(), op, " k must be CUDA");
   TORCH_CHECK(v.is_cuda(), op, " v must be CUDA");
@@ -262,6 +260,12 @@ at::Tensor varlen_forward(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor c
   TORCH_CHECK(q.size(1) % k.size(1) == 0, op, " q heads must be divisible by kv heads");
   TORCH_CHECK(q.size(2) == k.size(2) && q.size(2) == v.size(2), op, " head dim mismatch");
   TORCH_CHECK(cu_seqlens.size(0) >= 2, op, " cu_seqlens must contain at least one sequence");
+}
+
+at::Tensor varlen_forward(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor cu_seqlens, int64_t window_left,
+                          double softmax_scale) {
+  const char* op = "areno_varlen_causal_attention";
+  check_varlen(op, q, k, v, cu_seqlens);
   const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(q));
   auto out = at::empty_like(q);
   const size_t ws_bytes =
@@ -276,9 +280,9 @@ at::Tensor varlen_forward(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor c
   return out;
 }
 
-void cache_write(at::Tensor k, at::Tensor v, at::Tensor k_cache, at::Tensor v_cache, at::Tensor block_ids,
-                 at::Tensor block_offsets, c10::optional<at::Tensor> k_scale, c10::optional<at::Tensor> v_scale) {
-  const char* op = "areno_paged_cache_write";
+areno_paged_cache check_cache_write(const char* op, const at::Tensor& k, const at::Tensor& v, const at::Tensor& k_cache,
+                                    const at::Tensor& v_cache, const at::Tensor& block_ids, const at::Tensor& block_offsets,
+                                    const c10::optional<at::Tensor>& k_scale, const c10::optional<at::Tensor>& v_scale) {
   TORCH_CHECK(k.is_cuda() && v.is_cuda(), op, " k and v must be CUDA");
   TORCH_CHECK(block_ids.is_cuda() && block_offsets.is_cuda(), op, " block ids/offsets must be CUDA");
   TORCH_CHECK(k.is_contiguous() && v.is_contiguous(), op, " k and v must be contiguous");
@@ -294,11 +298,40 @@ void cache_write(at::Tensor k, at::Tensor v, at::Tensor k_cache, at::Tensor v_ca
               " token count mismatch");
   TORCH_CHECK(k.size(1) == k_cache.size(2) && v.size(1) == v_cache.size(2), op, " head mismatch");
   TORCH_CHECK(k.size(2) == k_cache.size(3) && v.size(2) == v_cache.size(3), op, " head dim mismatch");
+  return cache;
+}
+
+void cache_write(at::Tensor k, at::Tensor v, at::Tensor k_cache, at::Tensor v_cache, at::Tensor block_ids,
+                 at::Tensor block_offsets, c10::optional<at::Tensor> k_scale, c10::optional<at::Tensor> v_scale) {
+  const char* op = "areno_paged_cache_write";
+  const areno_paged_cache cache = check_cache_write(op, k, v, k_cache, v_cache, block_ids, block_offsets, k_scale, v_scale);
   const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(k));
   const int status =
       areno_hip_cache_write(&cache, k.data_ptr(), v.data_ptr(), dtype_code(k, op, "k"), k.size(0),
                             block_ids.data_ptr<int64_t>(), block_offsets.data_ptr<int64_t>(), current_stream(k));
   check_status(status, op);
+}
+
+// areno_paged_cache_write of k and v and areno_varlen_causal_attention over them, by one launch where the sizes allow it
+at::Tensor varlen_forward_cache_write(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor cu_seqlens, int64_t window_left,
+                                      double softmax_scale, at::Tensor k_cache, at::Tensor v_cache, at::Tensor block_ids,
+                                      at::Tensor block_offsets, c10::optional<at::Tensor> k_scale,
+                                      c10::optional<at::Tensor> v_scale) {
+  const areno_paged_cache cache = check_cache_write("areno_paged_cache_write", k, v, k_cache, v_cache, block_ids, block_offsets,
+                                                    k_scale, v_scale);
+  const char* op = "areno_varlen_causal_attention";
+  check_varlen(op, q, k, v, cu_seqlens);
+  const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(device_of(q));
+  auto out = at::empty_like(q);
+  const size_t ws_bytes = areno_hip_prefill_workspace_bytes(cache.kv_heads, cache.head_dim);
+  auto workspace = at::empty({static_cast<int64_t>(ws_bytes)}, q.options().dtype(at::kByte));
+  const int status = areno_hip_varlen_attention_cache_write(
+      &cache, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), dtype_code(q, op, "q"), q.size(0),
+      static_cast<int32_t>(q.size(1)), cu_seqlens.data_ptr<int32_t>(), static_cast<int32_t>(cu_seqlens.size(0) - 1),
+      static_cast<int32_t>(window_left), static_cast<float>(softmax_scale), block_ids.data_ptr<int64_t>(),
+      block_offsets.data_ptr<int64_t>(), workspace.data_ptr(), ws_bytes, current_stream(q));
+  check_status(status, op);
+  return out;
 }
 
 at::Tensor paged_varlen_forward(at::Tensor q, at::Tensor k_cache, at::Tensor v_cache, at::Tensor block_table,
@@ -679,6 +712,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("areno_paged_decode_plan", &paged_decode_plan, "work list of a decode step, built once for all its layers");
   m.def("areno_paged_causal_attention_decode_forward_planned", &paged_decode_forward_planned,
         "paged decode forward with a per-step plan");
+  m.def("areno_varlen_causal_attention_forward_cache_write", &varlen_forward_cache_write,
+        "KV cache write and varlen causal attention forward over the same K and V");
   m.def("areno_paged_cache_write", &cache_write, "quantize-and-scatter KV cache write");
   m.def("areno_rope_rows", &rope_rows, "rotary rows of a step's tokens, rounded for an activation dtype");
   m.def("areno_qk_norm_rope_cache_write_rows", &qk_norm_rope_cache_write_rows,

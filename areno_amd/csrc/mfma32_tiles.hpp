@@ -9,6 +9,8 @@
 // is read in as well (tile_columns below).
 #pragma once
 
+#include <atomic>
+
 #include "decode_mfma_kernels.hpp"
 
 namespace areno {
@@ -148,6 +150,23 @@ __device__ __forceinline__ typename Mfma32<KIND>::vec8 tile_columns(char* tile, 
     w[2 * half + 1] = u[1];
   }
   return __builtin_bit_cast(typename Mfma32<KIND>::vec8, uint4_t{w[0], w[1], w[2], w[3]});
+}
+
+// more than 64 KB of LDS has to be allowed once per device; one bit per device (the attribute belongs to the device's copy)
+template <int BYTES>
+bool allow_lds(const void* fn, std::atomic<uint64_t>& allowed_on) {
+  if constexpr (BYTES > 64 * 1024) {
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return false;
+    if ((allowed_on.load(std::memory_order_acquire) >> device & 1) == 0) {
+      if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, BYTES) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+      }
+      allowed_on.fetch_or(uint64_t{1} << device, std::memory_order_release);
+    }
+  }
+  return true;
 }
 
 }  // namespace areno

@@ -46,6 +46,7 @@
 // context 0 it is the reference's varlen kernel (areno/accel/csrc/attention.cu:145-242).
 
 #include "decode_mfma_kernels.hpp"
+#include "page_write.hpp"
 #include "prefill_steps.hpp"
 
 namespace areno {
@@ -1139,14 +1140,14 @@ size_t prefill_mfma_workspace_bytes(int32_t kv_heads, int32_t head_dim) {
 // Defined in varlen_mfma.hip: packed K/V, one workgroup per query block.
 int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, int32_t dtype, int64_t tokens,
                        int32_t q_heads, int32_t kv_heads, int32_t head_dim, const int32_t* cu_seqlens, int32_t num_seqs,
-                       int32_t window_left, float softmax_scale, void* stream);
+                       int32_t window_left, float softmax_scale, const PageWrite* pages, void* stream);
 
 // block_table == nullptr selects packed K/V: cache->k / cache->v then point at (tokens, kv_heads, D) tensors and
-// context_lens may be nullptr (no cached context).
+// context_lens may be nullptr (no cached context).  `pages` (packed K/V only): also stores K and V there, or refuses.
 int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out, int32_t q_dtype, int64_t tokens,
                         int32_t q_heads, int32_t num_seqs, const int32_t* block_table, int32_t max_blocks,
                         const int32_t* cu_seqlens_q, const int32_t* context_lens, int32_t window_left,
-                        float softmax_scale, void* workspace, size_t workspace_bytes, void* stream) {
+                        float softmax_scale, void* workspace, size_t workspace_bytes, const PageWrite* pages, void* stream) {
   const char* op = "areno_hip_paged_varlen_prefill";
   const int group = q_heads / cache->kv_heads;
   if (q_dtype != ARENO_DT_F16 && q_dtype != ARENO_DT_BF16) return ARENO_ERR_UNSUPPORTED;
@@ -1200,9 +1201,10 @@ int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out
                 workspace_bytes);
   if (block_table == nullptr && context_lens == nullptr) {
     const int rc = launch_varlen_mfma(q, cache->k, cache->v, out, q_dtype, tokens, q_heads, cache->kv_heads, cache->head_dim,
-                                      cu_seqlens_q, num_seqs, window_left, softmax_scale, stream);
+                                      cu_seqlens_q, num_seqs, window_left, softmax_scale, pages, stream);
     if (rc != ARENO_ERR_UNSUPPORTED) return rc;
   }
+  if (pages != nullptr) return ARENO_ERR_UNSUPPORTED;
 
   PrefillParams p;
   p.q = q;

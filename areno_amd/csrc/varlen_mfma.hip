@@ -19,9 +19,12 @@
 // per query block with nothing beside it, the partials of cut blocks (up to 67 MB written and read), a third of the
 // loop's vector instructions (staging, half the lane swaps).  Bound at length by the matrix cores and the LDS
 // reads behind them (an operand read per product), at short lengths by a block's chain of steps.
+#include <atomic>
 #include <type_traits>
 
+#include "cache_row_quant.hpp"
 #include "mfma32_tiles.hpp"
+#include "page_write.hpp"
 #include "varlen_blocks.hpp"
 
 namespace areno {
@@ -49,6 +52,7 @@ struct VarlenMfmaParams {
   BlockDivision block_division;
   int32_t window_left;
   float scale_log2e;
+  PageWrite pages;  // (of the instances that write them)
 };
 
 // Whole-wave reductions of integers, by the steps of wave_max_fast
@@ -126,20 +130,52 @@ __device__ __forceinline__ bool find_block(const VarlenMfmaParams& p, int i, Blo
 extern __shared__ __attribute__((aligned(1024))) char vm_lds[];
 constexpr int kSchedMatrix = 0x8, kSchedLdsRead = 0x100;  // instruction classes of sched_group_barrier
 
-template <int D>
+template <int D, bool WRITE>
 struct VmShape {
   static constexpr int kTile = D <= 128 ? 64 : 32;  // keys per step
   using Tile = LdsTile<D, kTile, kVmWaves>;
   static constexpr int kBuffer = 2 * Tile::kBytes;  // K, V
-  static constexpr int kLdsBytes = 2 * kBuffer;
+  static constexpr int kPlaces = 2 * kBuffer;  // the pages of the block's tokens, then their places in these
+  static constexpr int kLdsBytes = WRITE ? kPlaces + 2 * kVmRows * 8 : kPlaces;
 };
+
+// A token's row of one kv head (of K, or `second`: of V) into the pages: quantized or copied, chunk `sub` of 16 bytes per
+// lane, a row's lanes next to each other.  The bits are those of areno_hip_cache_write: the same closed forms over the same lanes.
+template <int KIND, int D>
+__device__ __forceinline__ void write_page_chunk(const PageWrite& w, uint4_t raw, bool second, int64_t id, int64_t slot, int kvh, int kv_heads, int sub, bool live) {
+  const bool store = live && id >= 0 && id < w.num_blocks && slot >= 0 && slot < w.block_size;
+  const int64_t dst_row = (id * w.block_size + slot) * kv_heads + kvh;
+  void* const pool = second ? w.v : w.k;
+  constexpr bool kWholeGroups = (D & (D - 1)) == 0;  // a row's lanes are a power of two, as its maximum wants them
+  if (kWholeGroups && is_quantized_dtype(w.cache_dtype)) {
+    float x[8], amax = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      x[2 * j] = operand_element<KIND>(raw[j], 0);
+      x[2 * j + 1] = operand_element<KIND>(raw[j], 1);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(x[j]));
+    amax = lane_group_max<kWholeGroups ? D / 8 : 1>(amax);
+    if (store) store_row_slice(x, amax, sub, dst_row, D, pool, second ? w.v_scale : w.k_scale, w.cache_dtype, w.scale_dtype);
+  } else if (store) {
+    // (whole rows that nothing here reads again: kept out of the way of the tiles in L2; the case below 57.5 -> 55.1 us)
+    __builtin_nontemporal_store(raw, reinterpret_cast<uint4_t*>(static_cast<char*>(pool) + (dst_row * D + sub * 8) * 2));
+  }
+}
 
 // (Two waves per SIMD, four at head dim 64, are what the tiles leave room for, and the scheduler is told so: where it
 // takes three to be within reach it saves registers for them and waits for every operand read right behind it --
 // 8 192 tokens, 8 / 1 heads of 128: 208 instead of 172 us.)
-template <int KIND, int D>
+//
+// WRITE: the launch also stores the tokens' K and V in the pages of a cache, which nothing in it reads.  A block's workgroup
+// has the rows of its own tokens in LDS when it is done -- they are the last keys that its rows see -- so they cost no
+// fetch, and their stores go out behind the output's, while the next workgroup starts.  The pass with a launch of its own for
+// the pages and with this, us: 32 prompts of 33 .. 512 tokens, 28 / 4 heads of 128, bf16: 61.5 -> 57.6; 2 x 3 000 .. 6 000, 16 / 8
+// heads of 256, window 1 024: 176.6 -> 165; 24 x 48 .. 387 into fp8 pages 40.0 -> 38.8; 2 x 9 .. 74: 21.7 -> 17.7 (the host's).
+template <int KIND, int D, bool WRITE>
 __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D == 64 ? 4 : 2))) void varlen_mfma_kernel(VarlenMfmaParams p) {
-  using S = VmShape<D>;
+  using S = VmShape<D, WRITE>;
   using T = typename S::Tile;
   using M = Mfma32<KIND>;
   using V8 = typename M::vec8;
@@ -174,9 +210,23 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
     if (!found) {
       // (the same for the whole workgroup; the grid covers the most blocks the token count allows and one more).  Rows
       // behind the last sequence -- the end of a padded pack -- become zeros, over the workgroups that have no block
-      const int end = p.cu_seqlens[p.num_seqs], rest = p.tokens - end;
-      if (rest <= 0) return;
+      const int end = p.cu_seqlens[p.num_seqs], rest = max(p.tokens - end, 0);
+      const int front = WRITE ? p.cu_seqlens[0] : 0;  // (tokens in front of the first sequence: their pages are written as well)
+      if (rest + front <= 0) return;
       const int idle = static_cast<int>(gridDim.x / static_cast<unsigned>(vheads)) - i + at.idle;  // so many
+      if constexpr (WRITE) {
+        constexpr int kChunks = D / 8;
+        if (head0 == kvh * p.group) {  // (the first of a kv head's parts)
+          const int64_t chunks = static_cast<int64_t>(rest + front) * kChunks;
+          for (int64_t c = at.idle * kVmThreads + tid; c < 2 * chunks; c += static_cast<int64_t>(idle) * kVmThreads) {
+            const bool second = c >= chunks;
+            const int64_t nth = (c - (second ? chunks : 0)) / kChunks, token = nth < front ? nth : nth - front + end;
+            const int sub = static_cast<int>(c % kChunks);
+            const uint4_t raw = load16(second ? p.v : p.k, ((token * p.kv_heads + kvh) * D + sub * 8) * 2);
+            write_page_chunk<KIND, D>(p.pages, raw, second, p.pages.block_ids[token], p.pages.block_offsets[token], kvh, p.kv_heads, sub, true);
+          }
+        }
+      }
       const int per_token = group_here * (D / 4);
       const int64_t words = static_cast<int64_t>(rest) * per_token;
       for (int64_t w = at.idle * kVmThreads + tid; w < words; w += static_cast<int64_t>(idle) * kVmThreads) {
@@ -366,6 +416,15 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
   };
 
   fetch(ta, 0);
+  // the tokens' places in the cache, into LDS with the first tile (asked for at the block's end, which is when they are
+  // needed, 1 560 blocks of 32 prompts of 33 .. 512 tokens take 56.2 us instead of 52.7, without a store)
+  const bool writes = WRITE && head0 == kvh * p.group;  // (the first of a kv head's parts)
+  if (writes && kWave * wave < 2 * tok_cnt) {
+    const uint32_t words = static_cast<uint32_t>(2 * tok_cnt), word = min(static_cast<uint32_t>(kWave * wave + lane), words - 1) * 4u;
+    const int64_t first = static_cast<int64_t>(q_begin + tok0) * 8;
+    fetch_words_to_lds(reinterpret_cast<const char*>(p.pages.block_ids) + first, word, lds0 + S::kPlaces + wave * (kWave * 4));
+    fetch_words_to_lds(reinterpret_cast<const char*>(p.pages.block_offsets) + first, word, lds0 + S::kPlaces + kVmRows * 8 + wave * (kWave * 4));
+  }
   // (the query rows are waited for here: left to their first use inside the loop, that wait would cover every step's
   // fetches as well)
 #pragma unroll
@@ -379,34 +438,60 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
     if (t + 1 <= tb) step(t + 1, 1);
   }
 
-  if (!live) return;
   uint32_t a = __builtin_bit_cast(uint32_t, l_lane), b = a;
   swap_rows32(a, b);
   const float l_tot = __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
-  const float inv = 1.0f / l_tot;
+  if (live) {
+    const float inv = 1.0f / l_tot;
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
+    for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const uint2_t w = {pack_pair<KIND>(acc[nb][4 * c] * inv, acc[nb][4 * c + 1] * inv),
-                         pack_pair<KIND>(acc[nb][4 * c + 2] * inv, acc[nb][4 * c + 3] * inv)};
-      *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + (row_elem + 32 * nb + 8 * c + 4 * h) * 2) = w;
+      for (int c = 0; c < 4; ++c) {
+        const uint2_t w = {pack_pair<KIND>(acc[nb][4 * c] * inv, acc[nb][4 * c + 1] * inv),
+                           pack_pair<KIND>(acc[nb][4 * c + 2] * inv, acc[nb][4 * c + 3] * inv)};
+        *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + (row_elem + 32 * nb + 8 * c + 4 * h) * 2) = w;
+      }
     }
+  }
+  if (!writes) return;
+  constexpr int kChunks = D / 8;  // of a row
+  const int chunks = tok_cnt * kChunks, thread = wave * kWave + lane_now();
+  const int64_t* const places = reinterpret_cast<const int64_t*>(vm_lds + S::kPlaces);
+  for (int first = 0; first < 2 * chunks; first += kVmThreads) {  // K's, then V's
+    const int c = min(first + thread, 2 * chunks - 1), sub = (first + thread) % kChunks;
+    const bool second = c >= chunks;
+    const int nth = (c - (second ? chunks : 0)) / kChunks;
+    const int key = tok0 + nth, t = key / TK, row = key % TK;
+    uint4_t raw;
+    if (t >= tb - 1) {  // the last two tiles lie in LDS, as their last barrier left them
+      raw = *reinterpret_cast<const uint4_t*>(vm_lds + ((t - ta) & 1) * S::kBuffer + (second ? T::kBytes : 0) + row * T::kRowBytes +
+                                              ((sub ^ T::twist(row)) << 4));
+    } else {
+      raw = load16(second ? v_base : k_base, static_cast<int64_t>(key) * stride + sub * 16);
+    }
+    write_page_chunk<KIND, D>(p.pages, raw, second, places[nth], places[kVmRows + nth], kvh, p.kv_heads, sub, first + thread < 2 * chunks);
   }
 }
 
 typedef void (*vm_fn)(VarlenMfmaParams);
 struct VmLaunch {
-  vm_fn fn;
+  vm_fn fn;  // nullptr: no such kernel, or its LDS size was refused
   int lds_bytes;
 };
-template <int KIND>
+template <int KIND, int D, bool WRITE>
+VmLaunch vm_launch_of() {
+  static std::atomic<uint64_t> allowed_on{0};
+  constexpr int kLdsBytes = VmShape<D, WRITE>::kLdsBytes;
+  const vm_fn fn = varlen_mfma_kernel<KIND, D, WRITE>;
+  return {allow_lds<kLdsBytes>(reinterpret_cast<const void*>(fn), allowed_on) ? fn : nullptr, kLdsBytes};
+}
+template <int KIND, bool WRITE>
 VmLaunch vm_lookup(int head_dim) {
   switch (head_dim) {
-    case 64: return {varlen_mfma_kernel<KIND, 64>, VmShape<64>::kLdsBytes};
-    case 128: return {varlen_mfma_kernel<KIND, 128>, VmShape<128>::kLdsBytes};
-    case 192: return {varlen_mfma_kernel<KIND, 192>, VmShape<192>::kLdsBytes};
-    case 256: return {varlen_mfma_kernel<KIND, 256>, VmShape<256>::kLdsBytes};
+    case 64: return vm_launch_of<KIND, 64, WRITE>();
+    case 128: return vm_launch_of<KIND, 128, WRITE>();
+    case 192: return vm_launch_of<KIND, 192, WRITE>();
+    case 256: return vm_launch_of<KIND, 256, WRITE>();
     default: return {nullptr, 0};
   }
 }
@@ -437,12 +522,14 @@ bool equal_shares_are_faster(int64_t tokens, int32_t num_seqs, int32_t q_heads, 
 
 // Called by launch_prefill_mfma behind its checks (types, scale, sizes, alignment, workspace), so that a packed call is
 // taken or refused, by the matrix cores or the generic kernel, as it is there.  ARENO_ERR_UNSUPPORTED: a launch for
-// the kernel of prefill_mfma.hip.
+// the kernel of prefill_mfma.hip.  `pages` (optional): where the launch also stores K and V.
 int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, int32_t dtype, int64_t tokens,
                        int32_t q_heads, int32_t kv_heads, int32_t head_dim, const int32_t* cu_seqlens, int32_t num_seqs,
-                       int32_t window_left, float softmax_scale, void* stream) {
+                       int32_t window_left, float softmax_scale, const PageWrite* pages, void* stream) {
   const char* op = "areno_hip_varlen_attention";
-  const VmLaunch l = dtype == ARENO_DT_BF16 ? vm_lookup<KV_BF16>(head_dim) : vm_lookup<KV_F16>(head_dim);
+  const bool bf16 = dtype == ARENO_DT_BF16;
+  const VmLaunch l = pages != nullptr ? (bf16 ? vm_lookup<KV_BF16, true>(head_dim) : vm_lookup<KV_F16, true>(head_dim))
+                                      : (bf16 ? vm_lookup<KV_BF16, false>(head_dim) : vm_lookup<KV_F16, false>(head_dim));
   if (l.fn == nullptr) return ARENO_ERR_UNSUPPORTED;
   const int group = q_heads / kv_heads;
   if (equal_shares_are_faster(tokens, num_seqs, q_heads, group, head_dim, window_left)) return ARENO_ERR_UNSUPPORTED;
@@ -468,6 +555,7 @@ int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, i
   p.block_division = block_division(p.block_tokens);
   p.window_left = window_left;
   p.scale_log2e = softmax_scale * kLog2e;
+  p.pages = pages != nullptr ? *pages : PageWrite{};
   const int64_t blocks = (tokens / p.block_tokens + num_seqs + 1) * vheads;
   if (blocks * kVmThreads > 0xffffffffLL) return ARENO_ERR_UNSUPPORTED;  // (a launch counts its work items in 32 bits)
   hipLaunchKernelGGL(l.fn, dim3(static_cast<unsigned>(blocks)), dim3(kVmThreads), l.lds_bytes,

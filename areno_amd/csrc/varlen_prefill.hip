@@ -7,6 +7,7 @@
 // dtype / head_dim <= 512 / head ratio and is the fallback for shapes the MFMA kernel does not cover.
 
 #include "device_common.hpp"
+#include "page_write.hpp"
 
 namespace areno {
 
@@ -147,7 +148,7 @@ int launch_generic(const VarlenParams& p, void* stream, const char* op) {
 int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out, int32_t q_dtype, int64_t tokens,
                         int32_t q_heads, int32_t num_seqs, const int32_t* block_table, int32_t max_blocks,
                         const int32_t* cu_seqlens_q, const int32_t* context_lens, int32_t window_left,
-                        float softmax_scale, void* workspace, size_t workspace_bytes, void* stream);
+                        float softmax_scale, void* workspace, size_t workspace_bytes, const PageWrite* pages, void* stream);
 size_t prefill_mfma_workspace_bytes(int32_t kv_heads, int32_t head_dim);
 
 }  // namespace areno
@@ -156,12 +157,13 @@ extern "C" size_t areno_hip_prefill_workspace_bytes(int32_t kv_heads, int32_t he
   return areno::prefill_mfma_workspace_bytes(kv_heads, head_dim);
 }
 
-extern "C" int areno_hip_varlen_attention(const void* q, const void* k, const void* v, void* out, int32_t dtype,
-                                          int64_t tokens, int32_t q_heads, int32_t kv_heads, int32_t head_dim,
-                                          const int32_t* cu_seqlens, int32_t num_seqs, int32_t window_left,
-                                          float softmax_scale, void* workspace, size_t workspace_bytes,
-                                          void* stream) {
-  using namespace areno;
+namespace areno {
+namespace {
+
+// `pages` (optional): K and V are stored there as well, by the same launch; ARENO_ERR_UNSUPPORTED where it cannot.
+int varlen_attention(const void* q, const void* k, const void* v, void* out, int32_t dtype, int64_t tokens, int32_t q_heads,
+                     int32_t kv_heads, int32_t head_dim, const int32_t* cu_seqlens, int32_t num_seqs, int32_t window_left,
+                     float softmax_scale, void* workspace, size_t workspace_bytes, const PageWrite* pages, void* stream) {
   const char* op = "areno_hip_varlen_attention";
   if (q == nullptr || k == nullptr || v == nullptr || out == nullptr || cu_seqlens == nullptr)
     return fail(ARENO_ERR_INVALID_ARGUMENT, "%s: NULL tensor pointer", op);
@@ -184,7 +186,8 @@ extern "C" int areno_hip_varlen_attention(const void* q, const void* k, const vo
     packed.cache_dtype = dtype;
     packed.scale_dtype = ARENO_DT_F32;
     const int rc = launch_prefill_mfma(&packed, q, out, dtype, tokens, q_heads, num_seqs, nullptr, 1, cu_seqlens,
-                                       nullptr, window_left, softmax_scale, workspace, workspace_bytes, stream);
+                                       nullptr, window_left, softmax_scale, workspace, workspace_bytes, pages, stream);
+    if (pages != nullptr) return rc;
     if (rc != ARENO_ERR_UNSUPPORTED) return rc;
   }
   VarlenParams p = {};
@@ -204,6 +207,66 @@ extern "C" int areno_hip_varlen_attention(const void* q, const void* k, const vo
   p.kv_dtype = dtype;
   p.scale_log2e = softmax_scale * kLog2e;
   return launch_generic(p, stream, op);
+}
+
+// Whether an attention launch over packed K / V can store them in the pages as areno_hip_cache_write would: that
+// kernel's 16-byte rows, and pages that none of the tensors the launch reads lies in (they would be read while they are written).
+bool pages_fit(const areno_paged_cache& c, const void* q, const void* k, const void* v, int32_t dtype, int64_t tokens, int32_t q_heads) {
+  const bool quantized = is_quantized(c.cache_dtype);
+  if (dtype != ARENO_DT_F16 && dtype != ARENO_DT_BF16) return false;
+  if (c.head_dim != 64 && c.head_dim != 128 && c.head_dim != 256 && (quantized || c.head_dim != 192)) return false;
+  if (!quantized && c.cache_dtype != dtype) return false;
+  if ((reinterpret_cast<uintptr_t>(c.k) | reinterpret_cast<uintptr_t>(c.v)) % 16 != 0) return false;
+  const int64_t rows = c.num_blocks * c.block_size * c.kv_heads;
+  struct Range {
+    const void* at;
+    int64_t bytes;
+  };
+  const int64_t row_bytes = static_cast<int64_t>(c.head_dim) * static_cast<int64_t>(dtype_size(c.cache_dtype));
+  const int64_t scale_bytes = quantized ? rows * static_cast<int64_t>(dtype_size(c.scale_dtype)) : 0;
+  const Range written[4] = {{c.k, rows * row_bytes}, {c.v, rows * row_bytes}, {c.k_scale, scale_bytes}, {c.v_scale, scale_bytes}};
+  const Range read[3] = {{q, tokens * q_heads * c.head_dim * 2}, {k, tokens * c.kv_heads * c.head_dim * 2}, {v, tokens * c.kv_heads * c.head_dim * 2}};
+  for (const Range& w : written) {
+    for (const Range& r : read) {
+      const uintptr_t a = reinterpret_cast<uintptr_t>(w.at), b = reinterpret_cast<uintptr_t>(r.at);
+      if (w.bytes > 0 && a < b + static_cast<uintptr_t>(r.bytes) && b < a + static_cast<uintptr_t>(w.bytes)) return false;
+    }
+  }
+  return true;
+}
+
+}  // namespace
+}  // namespace areno
+
+extern "C" int areno_hip_varlen_attention(const void* q, const void* k, const void* v, void* out, int32_t dtype,
+                                          int64_t tokens, int32_t q_heads, int32_t kv_heads, int32_t head_dim,
+                                          const int32_t* cu_seqlens, int32_t num_seqs, int32_t window_left,
+                                          float softmax_scale, void* workspace, size_t workspace_bytes,
+                                          void* stream) {
+  return areno::varlen_attention(q, k, v, out, dtype, tokens, q_heads, kv_heads, head_dim, cu_seqlens, num_seqs, window_left,
+                                 softmax_scale, workspace, workspace_bytes, nullptr, stream);
+}
+
+extern "C" int areno_hip_varlen_attention_cache_write(const areno_paged_cache* cache, const void* q, const void* k,
+                                                      const void* v, void* out, int32_t dtype, int64_t tokens,
+                                                      int32_t q_heads, const int32_t* cu_seqlens, int32_t num_seqs,
+                                                      int32_t window_left, float softmax_scale,
+                                                      const int64_t* block_ids, const int64_t* block_offsets,
+                                                      void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace areno;
+  if (int rc = validate_paged_cache(cache, "areno_hip_varlen_attention_cache_write")) return rc;
+  if (tokens > 0 && k != nullptr && v != nullptr && block_ids != nullptr && block_offsets != nullptr &&
+      pages_fit(*cache, q, k, v, dtype, tokens, q_heads)) {
+    const PageWrite pages = {cache->k, cache->v, cache->k_scale, cache->v_scale, block_ids, block_offsets, cache->num_blocks,
+                             cache->block_size, cache->cache_dtype, cache->scale_dtype};
+    const int rc = varlen_attention(q, k, v, out, dtype, tokens, q_heads, cache->kv_heads, cache->head_dim, cu_seqlens, num_seqs,
+                                    window_left, softmax_scale, workspace, workspace_bytes, &pages, stream);
+    if (rc != ARENO_ERR_UNSUPPORTED) return rc;
+  }
+  // two launches, the one behind the other
+  if (int rc = areno_hip_cache_write(cache, k, v, dtype, tokens, block_ids, block_offsets, stream)) return rc;
+  return areno_hip_varlen_attention(q, k, v, out, dtype, tokens, q_heads, cache->kv_heads, cache->head_dim, cu_seqlens, num_seqs,
+                                    window_left, softmax_scale, workspace, workspace_bytes, stream);
 }
 
 extern "C" int areno_hip_paged_varlen_prefill(const areno_paged_cache* cache, const void* q, void* out,
@@ -231,7 +294,7 @@ extern "C" int areno_hip_paged_varlen_prefill(const areno_paged_cache* cache, co
 
   const int rc = launch_prefill_mfma(cache, q, out, q_dtype, tokens, q_heads, num_seqs, block_table, max_blocks,
                                      cu_seqlens_q, context_lens, window_left, softmax_scale, workspace, workspace_bytes,
-                                     stream);
+                                     nullptr, stream);
   if (rc != ARENO_ERR_UNSUPPORTED) return rc;
 
   VarlenParams p = {};

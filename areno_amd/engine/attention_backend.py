@@ -5,9 +5,9 @@ Same call shape as the reference's ``FlashAttnInferBackend.forward``
 cache pools and an ``InferMeta``; two extra keyword arguments carry the scale pools of an int8 / fp8 cache.
 
 - prefill: the new K/V rows are quantized and scattered into the pages by ``(block_id, offset)``
-  (``areno_paged_cache_write`` in place of the ``index_put_`` pair of infer.py:245-263), then causal attention runs
-  over the packed new tokens (``areno_varlen_causal_attention``, infer.py:189-209) or, when the metadata carries
-  ``context_lens``, over the pages so a later chunk sees the earlier ones.
+  (``areno_paged_cache_write`` in place of the ``index_put_`` pair of infer.py:245-263) and causal attention runs
+  over the packed new tokens (``areno_varlen_causal_attention``, infer.py:189-209), both in one op, or, when the
+  metadata carries ``context_lens``, behind the write over the pages so a later chunk sees the earlier ones.
 - decode: one token per sequence; the op appends it to the page and attends over the whole history
   (``areno_paged_causal_attention_decode``, infer.py:212-242).
 """
@@ -22,6 +22,7 @@ from areno_amd.accel.attention import (
     areno_paged_causal_attention_decode,
     areno_paged_varlen_causal_attention,
     areno_varlen_causal_attention,
+    areno_varlen_causal_attention_cache_write,
 )
 from areno_amd.engine.metadata import InferMeta
 
@@ -79,6 +80,13 @@ class HipInferBackend(nn.Module):
             if update_cache:
                 if meta.cache_block_ids is None or meta.cache_block_offsets is None:
                     raise ValueError("prefill inference requires cache_block_ids and cache_block_offsets")
+                if meta.context_lens is None and value_dim == qk_dim == v_cache.shape[-1] and q.dtype != torch.float64:
+                    out = areno_varlen_causal_attention_cache_write(
+                        q_flat.contiguous(), k_flat.contiguous(), v_flat.contiguous(), meta.cu_seqlens.contiguous(),
+                        k_cache, v_cache, meta.cache_block_ids, meta.cache_block_offsets, window_left=window_left,
+                        softmax_scale=softmax_scale, k_scale=k_scale, v_scale=v_scale,
+                    )  # fmt: skip
+                    return out.reshape(q.shape[0], q.shape[1], q.shape[2], value_dim)
                 areno_paged_cache_write(
                     k_flat.contiguous(), pad_last_dim(v_flat, v_cache.shape[-1]).contiguous(), k_cache, v_cache,
                     meta.cache_block_ids, meta.cache_block_offsets, k_scale=k_scale, v_scale=v_scale,

@@ -237,6 +237,18 @@ int areno_hip_varlen_attention(const void* q, const void* k, const void* v, void
                                size_t workspace_bytes, void* stream);
 
 /*
+ * areno_hip_cache_write of k and v, and areno_hip_varlen_attention over them: the prefill of fresh prompts
+ * (areno/engine/layers/attention_backend/infer.py:186-209,245-263).  Neither needs the other's result, so where the
+ * matrix-core kernel takes the attention its launch stores the pages as well; otherwise two launches.  Arguments as
+ * there; the heads and the head dim of k and v are the cache's.  out and the pages are the same bits either way.
+ */
+int areno_hip_varlen_attention_cache_write(const areno_paged_cache* cache, const void* q, const void* k, const void* v,
+                                           void* out, int32_t dtype, int64_t tokens, int32_t q_heads,
+                                           const int32_t* cu_seqlens, int32_t num_seqs, int32_t window_left,
+                                           float softmax_scale, const int64_t* block_ids, const int64_t* block_offsets,
+                                           void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Causal prefill of new queries over paged (optionally quantized) KV; the new tokens' K/V must already be in
  * the cache (areno_hip_cache_write).  Query i of sequence s sits at absolute position context_lens[s] + i and sees
  * keys [0, that] (clipped on the left by window_left when >= 0).  No counterpart kernel in the reference (its

@@ -454,3 +454,66 @@ def test_varlen_of_many_sequences(dtype, hq, hkv, d, lens):
     out = ops.areno_varlen_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV))
     want = ar.ref_varlen(q, k, v, cu, -1, d**-0.5)
     assert_close(out, want, *tolerances("bf16"), what=f"varlen of {len(lens)} sequences {hq}/{hkv} d={d}")
+
+
+@pytest.mark.parametrize("kv", ["same", "int8", "fp8"])
+@pytest.mark.parametrize("act", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d", [(28, 4, 128), (16, 16, 64), (6, 6, 256), (8, 1, 256), (24, 8, 192), (40, 2, 128), (3, 3, 128)])
+def test_prefill_with_its_cache_write(kv, act, hq, hkv, d):
+    """One op for the cache write and the packed attention leaves the bits of the two ops: tokens of every place in a block and a
+    key tile, empty sequences, tokens in front of the first sequence and behind the last, ids outside the pool, a window."""
+    cache_dtype, scale_dtype = {"same": (act, None), "int8": (torch.int8, torch.float16), "fp8": (torch.float8_e4m3fn, torch.float32)}[kv]
+    lens, front, behind, bs = [1, 33, 0, 130, 64, 257, 18], 3, 5, 16
+    t = front + sum(lens) + behind
+    g = torch.Generator().manual_seed(d + hq)
+    q, k, v = (torch.randn(t, h, d, generator=g).to(act).to(DEV) for h in (hq, hkv, hkv))
+    k[7], v[9] = 0, 1e4
+    cu = (front + torch.tensor([0] + lens).cumsum(0)).to(torch.int32).to(DEV)
+    blocks = t // bs + 2
+    slots = torch.randperm(blocks * bs, generator=g)[:t].to(DEV)
+    ids, offs = slots // bs, slots % bs
+    ids[11], offs[12], ids[13], offs[14] = -1, bs, blocks, -1  # not stored
+
+    def pools():
+        shape = (blocks, bs, hkv, d)
+        made = [torch.full(shape, 3.0, device=DEV).to(cache_dtype) for _ in range(2)]
+        scales = [None, None] if scale_dtype is None else [torch.full(shape[:3], 7, device=DEV, dtype=scale_dtype) for _ in range(2)]
+        return made, dict(zip(("k_scale", "v_scale"), scales))
+
+    bits = lambda x: x.view(torch.uint8)  # noqa: E731
+    for window in (None, 40):
+        (k1, v1), s1 = pools()
+        ops.areno_paged_cache_write(k, v, k1, v1, ids, offs, **s1)
+        want = ops.areno_varlen_causal_attention(q, k, v, cu, window_left=window)
+        (k2, v2), s2 = pools()
+        out = ops.areno_varlen_causal_attention_cache_write(q, k, v, cu, k2, v2, ids, offs, window_left=window, **s2)
+        assert torch.equal(bits(out[front:]), bits(want[front:]))  # (no sequence's rows in front: not defined)
+        for a, b in [(k1, k2), (v1, v2), (s1["k_scale"], s2["k_scale"]), (s1["v_scale"], s2["v_scale"])]:
+            assert a is None or torch.equal(bits(a), bits(b))
+
+
+def test_prefill_whose_keys_lie_in_the_pages_it_writes():
+    """Keys that are read while pages are written must not be those pages: such a call stores first and attends then."""
+    t, bs = 64, 16
+    g = torch.Generator().manual_seed(3)
+    q, v = (torch.randn(t, h, 128, generator=g).to(torch.bfloat16).to(DEV) for h in (8, 2))
+    pool = torch.randn(t // bs, bs, 2, 128, generator=g).to(torch.bfloat16)
+    slots = torch.arange(t, device=DEV)  # every row is its own place, so that the store leaves the keys as they are
+    cu = torch.tensor([0, t], dtype=torch.int32, device=DEV)
+    ids, offs = slots // bs, slots % bs
+    want_pool, pool = pool.to(DEV).clone(), pool.to(DEV)
+    other = torch.zeros_like(pool)
+    want = ops.areno_varlen_causal_attention(q, want_pool.view(t, 2, 128), v, cu)
+    out = ops.areno_varlen_causal_attention_cache_write(q, pool.view(t, 2, 128), v, cu, pool, other, ids, offs)
+    assert torch.equal(out, want) and torch.equal(pool, want_pool) and torch.equal(other.view(t, 2, 128), v)
+
+
+def test_prefill_with_its_cache_write_takes_part_in_autograd():
+    q, k, v, cu = _packed([40, 9], 8, 2, 128, torch.bfloat16)
+    q, k, v = (x.to(DEV).requires_grad_(True) for x in (q, k, v))
+    slots = torch.arange(49, device=DEV)
+    pools = [torch.zeros(4, 16, 2, 128, device=DEV, dtype=torch.bfloat16) for _ in range(2)]
+    out = ops.areno_varlen_causal_attention_cache_write(q, k, v, cu.to(DEV), *pools, slots // 16, slots % 16)
+    grads = torch.autograd.grad(out, (q, k, v), torch.ones_like(out))
+    want = torch.autograd.grad(ops.areno_varlen_causal_attention(q, k, v, cu.to(DEV)), (q, k, v), torch.ones_like(out))
+    assert all(torch.equal(a, b) for a, b in zip(grads, want))
