@@ -171,7 +171,7 @@ __device__ __forceinline__ void write_page_chunk(const PageWrite& w, uint4_t raw
 // WRITE: the launch also stores the tokens' K and V in the pages of a cache, which nothing in it reads.  A block's workgroup
 // has the rows of its own tokens in LDS when it is done -- they are the last keys that its rows see -- so they cost no
 // fetch, and their stores go out behind the output's, while the next workgroup starts.  The pass with a launch of its own for
-// the pages and with this, us: 32 prompts of 33 .. 512 tokens, 28 / 4 heads of 128, bf16: 61.5 -> 57.6; 2 x 3 000 .. 6 000, 16 / 8
+// the pages and with this, us (both with the output's stores as they were then): 32 prompts of 33 .. 512 tokens, 28 / 4 heads of 128, bf16: 61.5 -> 57.6; 2 x 3 000 .. 6 000, 16 / 8
 // heads of 256, window 1 024: 176.6 -> 165; 24 x 48 .. 387 into fp8 pages 40.0 -> 38.8; 2 x 9 .. 74: 21.7 -> 17.7 (the host's).
 template <int KIND, int D, bool WRITE>
 __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D == 64 ? 4 : 2))) void varlen_mfma_kernel(VarlenMfmaParams p) {
@@ -438,38 +438,63 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
     if (t + 1 <= tb) step(t + 1, 1);
   }
 
+  if (writes) {
+    constexpr int kChunks = D / 8;  // of a row
+    const int chunks = tok_cnt * kChunks, thread = wave * kWave + lane_now();
+    const int64_t* const places = reinterpret_cast<const int64_t*>(vm_lds + S::kPlaces);
+    for (int first = 0; first < 2 * chunks; first += kVmThreads) {  // K's, then V's
+      const int c = min(first + thread, 2 * chunks - 1), sub = (first + thread) % kChunks;
+      const bool second = c >= chunks;
+      const int nth = (c - (second ? chunks : 0)) / kChunks;
+      const int key = tok0 + nth, t = key / TK, row = key % TK;
+      uint4_t raw;
+      if (t >= tb - 1) {  // the last two tiles lie in LDS, as their last barrier left them
+        raw = *reinterpret_cast<const uint4_t*>(vm_lds + ((t - ta) & 1) * S::kBuffer + (second ? T::kBytes : 0) + row * T::kRowBytes +
+                                                ((sub ^ T::twist(row)) << 4));
+      } else {
+        raw = load16(second ? v_base : k_base, static_cast<int64_t>(key) * stride + sub * 16);
+      }
+      write_page_chunk<KIND, D>(p.pages, raw, second, places[nth], places[kVmRows + nth], kvh, p.kv_heads, sub, first + thread < 2 * chunks);
+    }
+    handed_barrier();  // (the tile in front of the last is read)
+  }
+
+  // The output through LDS, where the tile in front of the last one lay (every wave has left it): a lane holds four elements
+  // here and there of a row, and stored from there they were 64 pieces of 8 bytes an instruction, which the memory
+  // pipe takes one by one.  As whole rows of 16-byte chunks, past L2, the kernel in us (whole rows kept in L2): 32 prompts of
+  // 33 .. 512 tokens, 28 / 4 heads of 128, with the pages: 57.8 -> 47.6 (50.0); 2 x 3 000 .. 6 000, 16 / 8 heads of 256, window 1 024: 197 ->
+  // 180 (187); 16 x 20 .. 600, 16 heads of 64: 16.5 -> 15.5 (16.8); 2 x 2 048: 84.8 -> 81.0 (82.7); 4 x 4 096, 32 / 8: 558 -> 545 (545).
   uint32_t a = __builtin_bit_cast(uint32_t, l_lane), b = a;
   swap_rows32(a, b);
   const float l_tot = __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
-  if (live) {
-    const float inv = 1.0f / l_tot;
+  const float inv = 1.0f / l_tot;  // (rows that do not exist are not stored)
+  char* const rows_lds = vm_lds + ((tb - ta + 1) & 1) * S::kBuffer + wave * (S::kBuffer / kVmWaves);
+  constexpr int kBlocks = S::kBuffer / kVmWaves / (32 * 64);  // blocks of 32 elements that a wave's part holds of its rows
+  constexpr int kRounds = (NB + kBlocks - 1) / kBlocks, kHere = NB / kRounds, kRowChunks = kHere * 4;
+  static_assert(NB % kRounds == 0 && 32 * kRowChunks % kWave == 0, "the output's parts");
+  const int l = lane_now(), column = l & 31;
+  auto place = [&](int row, int chunk) { return rows_lds + row * (kRowChunks * 16) + ((chunk ^ (row & (kRowChunks % 8 == 0 ? kRowChunks - 1 : 3))) << 4); };
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
+  for (int round = 0; round < kRounds; ++round) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const uint2_t w = {pack_pair<KIND>(acc[nb][4 * c] * inv, acc[nb][4 * c + 1] * inv),
-                           pack_pair<KIND>(acc[nb][4 * c + 2] * inv, acc[nb][4 * c + 3] * inv)};
-        *reinterpret_cast<uint2_t*>(static_cast<char*>(p.out) + (row_elem + 32 * nb + 8 * c + 4 * h) * 2) = w;
+    for (int x = 0; x < kRowChunks; ++x) {
+      const int nb = round * kHere + x / 4, c = x % 4;
+      const uint2_t w = {pack_pair<KIND>(acc[nb][4 * c] * inv, acc[nb][4 * c + 1] * inv),
+                         pack_pair<KIND>(acc[nb][4 * c + 2] * inv, acc[nb][4 * c + 3] * inv)};
+      *reinterpret_cast<uint2_t*>(place(column, x) + 8 * (l >> 5)) = w;
+    }
+    asm volatile("" : : : "memory");
+#pragma unroll
+    for (int x = 0; x < 32 * kRowChunks / kWave; ++x) {
+      const int i = x * kWave + l, row = i / kRowChunks, chunk = i % kRowChunks;
+      const int t_here = token_of_row(32 * wave + row), head_here = 32 * wave + row - t_here * p.fold;
+      const uint4_t w = *reinterpret_cast<const uint4_t*>(place(row, chunk));
+      if (t_here < tok_cnt && head_here < group_here) {
+        const int64_t elem = (static_cast<int64_t>(q_begin + tok0 + t_here) * p.q_heads + head0 + head_here) * D + round * (32 * kHere) + 8 * chunk;
+        __builtin_nontemporal_store(w, reinterpret_cast<uint4_t*>(static_cast<char*>(p.out) + elem * 2));
       }
     }
-  }
-  if (!writes) return;
-  constexpr int kChunks = D / 8;  // of a row
-  const int chunks = tok_cnt * kChunks, thread = wave * kWave + lane_now();
-  const int64_t* const places = reinterpret_cast<const int64_t*>(vm_lds + S::kPlaces);
-  for (int first = 0; first < 2 * chunks; first += kVmThreads) {  // K's, then V's
-    const int c = min(first + thread, 2 * chunks - 1), sub = (first + thread) % kChunks;
-    const bool second = c >= chunks;
-    const int nth = (c - (second ? chunks : 0)) / kChunks;
-    const int key = tok0 + nth, t = key / TK, row = key % TK;
-    uint4_t raw;
-    if (t >= tb - 1) {  // the last two tiles lie in LDS, as their last barrier left them
-      raw = *reinterpret_cast<const uint4_t*>(vm_lds + ((t - ta) & 1) * S::kBuffer + (second ? T::kBytes : 0) + row * T::kRowBytes +
-                                              ((sub ^ T::twist(row)) << 4));
-    } else {
-      raw = load16(second ? v_base : k_base, static_cast<int64_t>(key) * stride + sub * 16);
-    }
-    write_page_chunk<KIND, D>(p.pages, raw, second, places[nth], places[kVmRows + nth], kvh, p.kv_heads, sub, first + thread < 2 * chunks);
+    asm volatile("" : : : "memory");
   }
 }
 
