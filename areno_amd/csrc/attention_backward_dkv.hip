@@ -377,23 +377,45 @@ __global__ __launch_bounds__((Dkv32Shape<D, KW, P>::kThreads)) __attribute__((am
       }
     }
 
-    // every gradient element is written, also the zeros of keys no query sees
+    // Every gradient element is written, also the zeros of keys no query sees.  At head dim 64 16-bit ones as whole rows, through
+    // LDS (16 x 20 .. 600 tokens, 16 heads: 34.4 -> 33.2 us); at 128 that spilled registers of the loop in (4, 1) and (2, 2),
+    // and took the one wave that stores longer in (1, 4) (2 x 2 048, 28 / 4 heads: 139.4 -> 142.2).
+    constexpr bool kWholeRows = D == 64;
+    if constexpr (KW > 1 && kWholeRows) handed_barrier();  // (the other waves have read their last tile, or the sums)
     const int lane_ = lane_now();
-    const int64_t out_row = r0 + 32 * wave + (lane_ & 31);
-    if (part == 0 && out_row < p.k_tokens) {
-      const int64_t out_elem = (out_row * p.kv_heads + kvh) * D + 4 * (lane_ >> 5);
-      store_grads<typename M::elem>(p.grad_dtype, [&](auto store) {
+    const int64_t first_row = r0 + 32 * wave, out_row = first_row + (lane_ & 31);
+    if (kWholeRows && p.grad_dtype != ARENO_DT_F32) {
+      if (part == 0) {
+        using Stage = RowStage<4 * NB>;
+        char* const stage = dkv32_lds + wave * (32 * Stage::kRowBytes);
+        auto out = [&](void* grad, const float16_t (&acc)[NB], float f) {
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            const int64_t at_elem = out_elem + 32 * nb + 8 * c;
-            store(p.grad_k, at_elem, acc_k[nb][4 * c] * p.scale, acc_k[nb][4 * c + 1] * p.scale, acc_k[nb][4 * c + 2] * p.scale,
-                  acc_k[nb][4 * c + 3] * p.scale);
-            store(p.grad_v, at_elem, acc_v[nb][4 * c], acc_v[nb][4 * c + 1], acc_v[nb][4 * c + 2], acc_v[nb][4 * c + 3]);
+          for (int x = 0; x < 4 * NB; ++x) {
+            const int nb = x >> 2, c = 4 * (x & 3);
+            Stage::put(stage, lane_ & 31, x, lane_ >> 5, pack_pair<KIND>(acc[nb][c] * f, acc[nb][c + 1] * f), pack_pair<KIND>(acc[nb][c + 2] * f, acc[nb][c + 3] * f));
           }
+          Stage::template take<32>(stage, lane_, [&](int r, int chunk, uint4_t w) {
+            if (first_row + r < p.k_tokens) *reinterpret_cast<uint4_t*>(static_cast<char*>(grad) + (((first_row + r) * p.kv_heads + kvh) * D + 8 * chunk) * 2) = w;
+          });
+        };
+        out(p.grad_k, acc_k, p.scale);
+        out(p.grad_v, acc_v, 1.0f);
+      }
+    } else if (part == 0 && out_row < p.k_tokens) {
+      const int64_t out_elem = (out_row * p.kv_heads + kvh) * D + 4 * (lane_ >> 5);
+      auto out = [&](auto store) {
+#pragma unroll
+        for (int x = 0; x < 4 * NB; ++x) {
+          const int nb = x >> 2, c = 4 * (x & 3);
+          store(p.grad_k, out_elem + 8 * x, acc_k[nb][c] * p.scale, acc_k[nb][c + 1] * p.scale, acc_k[nb][c + 2] * p.scale, acc_k[nb][c + 3] * p.scale);
+          store(p.grad_v, out_elem + 8 * x, acc_v[nb][c], acc_v[nb][c + 1], acc_v[nb][c + 2], acc_v[nb][c + 3]);
         }
-      });
+      };
+      if constexpr (!kWholeRows) {
+        store_grads<typename M::elem>(p.grad_dtype, out);
+      } else {
+        out(GradStore<float>{});
+      }
     }
   }
 }

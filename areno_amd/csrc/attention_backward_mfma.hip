@@ -304,26 +304,41 @@ __global__ __launch_bounds__(kBmThreads, D == 64 ? 4 : 2) void bwd_mfma_dq_kerne
 
     // dQ = scale / l * sum_k p_k (dP_k - dO . O) K_k; the row's log-sum-exp (log2 domain) and -(dO . O) for the dkv kernel
     const float l_tot = rows_sum(l_lane);
-    if (live) {
-      const float f = l_tot > 0.0f ? p.scale / l_tot : 0.0f;
-      store_grads<typename Mfma32<KIND>::elem>(p.grad_dtype, [&](auto store) {
+    const float f = l_tot > 0.0f ? p.scale / l_tot : 0.0f;
+    const int l = lane_now(), lr_ = l & 15, lk_ = l >> 4;  // (worked out anew: kept, they would cost the loop registers)
+    const int64_t at = wave_row0 + lr_;
+    if (p.grad_dtype != ARENO_DT_F32) {  // as whole rows, through the tiles' LDS: they are read
+      using Stage = RowStage<2 * NB>;
+      char* const stage = k_lds + wave * (kWaveRows * Stage::kRowBytes);
+      static_assert(kBmWaves * kWaveRows * Stage::kRowBytes <= sizeof(k_lds), "the rows' place");
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+        Stage::put(stage, lr_, 2 * nb + (lk_ >> 1), lk_ & 1, pack_pair<KIND>(acc[nb][0] * f, acc[nb][1] * f), pack_pair<KIND>(acc[nb][2] * f, acc[nb][3] * f));
+      Stage::template take<kWaveRows>(stage, l, [&](int r, int chunk, uint4_t w) {
+        const int64_t to = wave_row0 + r;
+        if (to >= q_lo && to < q_hi) *reinterpret_cast<uint4_t*>(static_cast<char*>(p.grad_q) + ((to * p.q_heads + h) * D + 8 * chunk) * 2) = w;
+      });
+    }
+    if (at >= q_lo && at < q_hi) {
+      if (p.grad_dtype == ARENO_DT_F32) {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
-          store(p.grad_q, row_elem + 4 * lk + 16 * nb, acc[nb][0] * f, acc[nb][1] * f, acc[nb][2] * f, acc[nb][3] * f);
-      });
-      if (lk == 0) {
-        float* st = p.row_stats + (h * p.q_tokens + row) * 2;
+          GradStore<float>{}(p.grad_q, (at * p.q_heads + h) * D + 4 * lk_ + 16 * nb, acc[nb][0] * f, acc[nb][1] * f, acc[nb][2] * f, acc[nb][3] * f);
+      }
+      if (lk_ == 0) {
+        float* st = p.row_stats + (h * p.q_tokens + at) * 2;
         // a row without visible keys gets a reference no score reaches: its probabilities come out as zeros
         st[0] = l_tot > 0.0f ? m_run + __builtin_log2f(l_tot) : __builtin_huge_valf();
         st[1] = -delta;
       }
     }
   }
+  row = wave_row0 + (lane_now() & 15);
   if (row >= covered && row < p.q_tokens) {  // behind the last sequence, the end of a padded pack
-    const int64_t row_elem = (row * p.q_heads + h) * D;
+    const int64_t row_elem = (row * p.q_heads + h) * D + 4 * (lane_now() >> 4);
     store_grads<typename Mfma32<KIND>::elem>(p.grad_dtype, [&](auto store) {
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) store(p.grad_q, row_elem + 4 * lk + 16 * nb, 0.0f, 0.0f, 0.0f, 0.0f);
+      for (int nb = 0; nb < NB; ++nb) store(p.grad_q, row_elem + 16 * nb, 0.0f, 0.0f, 0.0f, 0.0f);
     });
   }
 }
@@ -544,30 +559,47 @@ __global__ __launch_bounds__(kBmThreads, 2) void bwd_mfma32_dq_kernel(BwdParams 
     }
 
     const float l_tot = both_halves(l_lane, sum);
-    if (live) {
-      const float f = l_tot > 0.0f ? p.scale / l_tot : 0.0f;
-      store_grads<typename M::elem>(p.grad_dtype, [&](auto store) {
+    const float f = l_tot > 0.0f ? p.scale / l_tot : 0.0f;
+    handed_barrier();  // (every wave has read its last tile)
+    const int l = lane_now();
+    const int64_t at = wave_row0 + (l & 31);
+    // (as whole rows, the kernel in us: 2 x 2 048 tokens, 28 / 4 heads of 128: 131 -> 123; 4 x 4 096, 32 / 8: 814 -> 790)
+    if (p.grad_dtype != ARENO_DT_F32) {
+      using Stage = RowStage<4 * NB>;
+      char* const stage = lds + wave * (32 * Stage::kRowBytes);
+      static_assert(kRows * Stage::kRowBytes <= sizeof(lds), "the rows' place");
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            store(p.grad_q, row_elem + 32 * nb + 8 * c + 4 * half, acc[nb][4 * c] * f, acc[nb][4 * c + 1] * f, acc[nb][4 * c + 2] * f,
-                  acc[nb][4 * c + 3] * f);
-          }
-        }
+      for (int x = 0; x < 4 * NB; ++x) {
+        const int nb = x >> 2, c = 4 * (x & 3);
+        Stage::put(stage, l & 31, x, l >> 5, pack_pair<KIND>(acc[nb][c] * f, acc[nb][c + 1] * f), pack_pair<KIND>(acc[nb][c + 2] * f, acc[nb][c + 3] * f));
+      }
+      Stage::template take<32>(stage, l, [&](int r, int chunk, uint4_t w) {
+        const int64_t to = wave_row0 + r;
+        if (to >= q_lo && to < q_hi) *reinterpret_cast<uint4_t*>(static_cast<char*>(p.grad_q) + ((to * p.q_heads + h) * D + 8 * chunk) * 2) = w;
       });
-      if (half == 0) {
-        float* st = p.row_stats + (h * p.q_tokens + row) * 2;
+    }
+    if (at >= q_lo && at < q_hi) {
+      if (p.grad_dtype == ARENO_DT_F32) {
+#pragma unroll
+        for (int x = 0; x < 4 * NB; ++x) {
+          const int nb = x >> 2, c = 4 * (x & 3);
+          GradStore<float>{}(p.grad_q, (at * p.q_heads + h) * D + 8 * x + 4 * (l >> 5), acc[nb][c] * f, acc[nb][c + 1] * f, acc[nb][c + 2] * f, acc[nb][c + 3] * f);
+        }
+      }
+      if (l < 32) {
+        float* st = p.row_stats + (h * p.q_tokens + at) * 2;
         st[0] = l_tot > 0.0f ? m_run + __builtin_log2f(l_tot) : __builtin_huge_valf();
         st[1] = -delta;
       }
     }
   }
-  if (row >= covered && row < p.q_tokens) {  // behind the last sequence, the end of a padded pack
-    const int64_t row_elem = (row * p.q_heads + h) * D;
+  const int l = lane_now();
+  const int64_t at = wave_row0 + (l & 31);
+  if (at >= covered && at < p.q_tokens) {  // behind the last sequence, the end of a padded pack
+    const int64_t elem = (at * p.q_heads + h) * D + 4 * (l >> 5);
     store_grads<typename M::elem>(p.grad_dtype, [&](auto store) {
 #pragma unroll
-      for (int c = 0; c < D / 8; ++c) store(p.grad_q, row_elem + 8 * c + 4 * half, 0.0f, 0.0f, 0.0f, 0.0f);
+      for (int c = 0; c < D / 8; ++c) store(p.grad_q, elem + 8 * c, 0.0f, 0.0f, 0.0f, 0.0f);
     });
   }
 }

@@ -367,31 +367,49 @@ __global__ __launch_bounds__(kWideDqWaves* kWave) __attribute__((amdgpu_waves_pe
     if (!second) *reference = both_halves_sum(l_lane);
     handed_barrier();
     const float l_tot = *reference;
-    if (live) {
-      const float f = l_tot > 0.0f ? p.scale / l_tot : 0.0f;
-      store_grads<typename M::elem>(p.grad_dtype, [&](auto store) {
+    const float f = l_tot > 0.0f ? p.scale / l_tot : 0.0f;
+    const int l = lane_now();  // (worked out anew: kept, what follows from it would cost the loop registers)
+    const int64_t at = wave_row0 + (l & 31);
+    if (p.grad_dtype != ARENO_DT_F32) {  // as whole blocks of 32 elements, through the tiles' LDS
+      using Stage = RowStage<4 * NB>;
+      char* const stage = wide_lds + wave_of_block * (32 * Stage::kRowBytes);
+      static_assert(kWideDqWaves * 32 * Stage::kRowBytes <= L::kHands, "the rows' place");
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            store(p.grad_q, row_elem + 64 * nb + (second ? 32 : 0) + 8 * c + 4 * half, acc[nb][4 * c] * f, acc[nb][4 * c + 1] * f,
-                  acc[nb][4 * c + 2] * f, acc[nb][4 * c + 3] * f);
-          }
-        }
+      for (int x = 0; x < 4 * NB; ++x) {
+        const int nb = x >> 2, c = 4 * (x & 3);
+        Stage::put(stage, l & 31, x, l >> 5, pack_pair<KIND>(acc[nb][c] * f, acc[nb][c + 1] * f), pack_pair<KIND>(acc[nb][c + 2] * f, acc[nb][c + 3] * f));
+      }
+      Stage::template take<32>(stage, l, [&](int r, int chunk, uint4_t w) {
+        const int64_t to = wave_row0 + r;
+        const int elem = 64 * (chunk >> 2) + (second ? 32 : 0) + 8 * (chunk & 3);
+        if (to >= q_lo && to < q_hi) *reinterpret_cast<uint4_t*>(static_cast<char*>(p.grad_q) + ((to * p.q_heads + h) * D + elem) * 2) = w;
       });
-      if (half == 0) {
+    }
+    if (at >= q_lo && at < q_hi) {
+      if (p.grad_dtype == ARENO_DT_F32) {
+#pragma unroll
+        for (int x = 0; x < 4 * NB; ++x) {
+          const int nb = x >> 2, c = 4 * (x & 3);
+          GradStore<float>{}(p.grad_q, (at * p.q_heads + h) * D + 64 * nb + (second ? 32 : 0) + 2 * c + 4 * (l >> 5), acc[nb][c] * f, acc[nb][c + 1] * f,
+                             acc[nb][c + 2] * f, acc[nb][c + 3] * f);
+        }
+      }
+      if (l < 32) {
         // a row without visible keys gets a reference no score reaches: its probabilities come out as zeros
-        p.row_stats[(h * p.q_tokens + row) * 2 + (second ? 1 : 0)] =
+        p.row_stats[(h * p.q_tokens + at) * 2 + (second ? 1 : 0)] =
             second ? -delta : l_tot > 0.0f ? m_run + __builtin_log2f(l_tot) : __builtin_huge_valf();
       }
     }
   }
-  if (row >= covered && row < p.q_tokens) {  // behind the last sequence, the end of a padded pack
+  const int l = lane_now();
+  const int64_t at = wave_row0 + (l & 31);
+  if (at >= covered && at < p.q_tokens) {  // behind the last sequence, the end of a padded pack
+    const int64_t elem = (at * p.q_heads + h) * D + (second ? 32 : 0) + 4 * (l >> 5);
     store_grads<typename M::elem>(p.grad_dtype, [&](auto store) {
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) store(p.grad_q, row_elem + 64 * nb + (second ? 32 : 0) + 8 * c + 4 * half, 0.0f, 0.0f, 0.0f, 0.0f);
+        for (int c = 0; c < 4; ++c) store(p.grad_q, elem + 64 * nb + 8 * c, 0.0f, 0.0f, 0.0f, 0.0f);
       }
     });
   }
@@ -657,32 +675,47 @@ __global__ __launch_bounds__((WideShape<D, KW, P>::kThreads)) __attribute__((amd
       }
     }
     __syncthreads();
-    if (part > 0) return;
+    if (part == 0) {
 #pragma unroll
-    for (int other = 0; other < P - 1; ++other) {
+      for (int other = 0; other < P - 1; ++other) {
 #pragma unroll
-      for (int x = 0; x < kFours; ++x) {
-        const float4_t theirs = sums[(other * kFours + x) * kStep];
+        for (int x = 0; x < kFours; ++x) {
+          const float4_t theirs = sums[(other * kFours + x) * kStep];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[x >> 2][4 * (x & 3) + j] += theirs[j];
+          for (int j = 0; j < 4; ++j) acc[x >> 2][4 * (x & 3) + j] += theirs[j];
+        }
       }
     }
   }
+  handed_barrier();  // (every wave has read its last tile, or the sums)
+  if (part > 0) return;
 
-  // every gradient element is written, also the zeros of keys no query sees
+  // every gradient element is written, also the zeros of keys no query sees; in 16 bits through LDS, as whole rows
   const int l = lane_now();
-  const int64_t out_row = r0 + 32 * wave + (l & 31);
-  if (out_row < p.k_tokens) {
-    void* const out = second ? p.grad_k : p.grad_v;
-    const float f = second ? p.scale : 1.0f;
-    const int64_t elem = (out_row * p.kv_heads + kvh) * D + 4 * (l >> 5);
-    store_grads<typename M::elem>(p.grad_dtype, [&](auto store) {
+  const int64_t first_row = r0 + 32 * wave;
+  void* const out = second ? p.grad_k : p.grad_v;
+  const float f = second ? p.scale : 1.0f;
+  if (p.grad_dtype == ARENO_DT_F32) {
+    const int64_t out_row = first_row + (l & 31);
+    if (out_row < p.k_tokens) {
+      const int64_t elem = (out_row * p.kv_heads + kvh) * D + 4 * (l >> 5);
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          store(out, elem + 32 * nb + 8 * c, acc[nb][4 * c] * f, acc[nb][4 * c + 1] * f, acc[nb][4 * c + 2] * f, acc[nb][4 * c + 3] * f);
+      for (int x = 0; x < 4 * NB; ++x) {
+        const int nb = x >> 2, c = 4 * (x & 3);
+        GradStore<float>{}(out, elem + 8 * x, acc[nb][c] * f, acc[nb][c + 1] * f, acc[nb][c + 2] * f, acc[nb][c + 3] * f);
       }
+    }
+  } else {
+    using Stage = RowStage<4 * NB>;
+    char* const stage = wide_lds + part_wave * (32 * Stage::kRowBytes);
+    static_assert(L::kPartWaves * 32 * Stage::kRowBytes <= L::kTiles, "the rows' place");
+#pragma unroll
+    for (int x = 0; x < 4 * NB; ++x) {
+      const int nb = x >> 2, c = 4 * (x & 3);
+      Stage::put(stage, l & 31, x, l >> 5, pack_pair<KIND>(acc[nb][c] * f, acc[nb][c + 1] * f), pack_pair<KIND>(acc[nb][c + 2] * f, acc[nb][c + 3] * f));
+    }
+    Stage::template take<32>(stage, l, [&](int r, int chunk, uint4_t w) {
+      if (first_row + r < p.k_tokens) *reinterpret_cast<uint4_t*>(static_cast<char*>(out) + (((first_row + r) * p.kv_heads + kvh) * D + 8 * chunk) * 2) = w;
     });
   }
 }

@@ -152,6 +152,37 @@ __device__ __forceinline__ typename Mfma32<KIND>::vec8 tile_columns(char* tile, 
   return __builtin_bit_cast(typename Mfma32<KIND>::vec8, uint4_t{w[0], w[1], w[2], w[3]});
 }
 
+// Rows of 16-bit elements on their way from a wave's registers to memory, through a part of LDS that is the wave's alone: a
+// lane of a C tile holds four elements here and there of a row, and stored from there they are 64 pieces of 8 bytes an
+// instruction, which the memory pipe takes one by one.  The 16-byte chunks of a row are permuted by a function of the row, so
+// that lanes that put the same chunk of different rows meet different banks.
+template <int CHUNKS>  // of a row
+struct RowStage {
+  static constexpr int kRowBytes = CHUNKS * 16;
+  static constexpr int kTwist = (CHUNKS & (CHUNKS - 1)) == 0 ? CHUNKS - 1 : 3;
+  static_assert(CHUNKS % 4 == 0, "the twist stays inside a row");
+  static __device__ __forceinline__ char* place(char* stage, int row, int chunk) {
+    return stage + row * kRowBytes + ((chunk ^ (row & kTwist)) << 4);
+  }
+  // four elements, the first or (`half`) the second ones of a chunk
+  static __device__ __forceinline__ void put(char* stage, int row, int chunk, int half, uint32_t lo, uint32_t hi) {
+    *reinterpret_cast<uint2_t*>(place(stage, row, chunk) + 8 * half) = uint2_t{lo, hi};
+  }
+  // The rows that were put, chunk by chunk: store(row, chunk, its 16 bytes), a row's lanes next to each other.  (The wave's LDS
+  // accesses take place in their order.)
+  template <int ROWS, typename Store>
+  static __device__ __forceinline__ void take(char* stage, int lane, const Store& store) {
+    static_assert(ROWS * CHUNKS % 64 == 0, "whole instructions");
+    asm volatile("" : : : "memory");
+#pragma unroll
+    for (int x = 0; x < ROWS * CHUNKS / 64; ++x) {
+      const int i = x * 64 + lane, row = i / CHUNKS, chunk = i % CHUNKS;
+      store(row, chunk, *reinterpret_cast<const uint4_t*>(place(stage, row, chunk)));
+    }
+    asm volatile("" : : : "memory");
+  }
+};
+
 // more than 64 KB of LDS has to be allowed once per device; one bit per device (the attribute belongs to the device's copy)
 template <int BYTES>
 bool allow_lds(const void* fn, std::atomic<uint64_t>& allowed_on) {

@@ -459,9 +459,8 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
     handed_barrier();  // (the tile in front of the last is read)
   }
 
-  // The output through LDS, where the tile in front of the last one lay (every wave has left it): a lane holds four elements
-  // here and there of a row, and stored from there they were 64 pieces of 8 bytes an instruction, which the memory
-  // pipe takes one by one.  As whole rows of 16-byte chunks, past L2, the kernel in us (whole rows kept in L2): 32 prompts of
+  // The output through LDS (RowStage), where the tile in front of the last one lay: every wave has left it.  Against pieces of
+  // 8 bytes from the accumulators, as whole rows past L2, the kernel in us (whole rows kept in L2): 32 prompts of
   // 33 .. 512 tokens, 28 / 4 heads of 128, with the pages: 57.8 -> 47.6 (50.0); 2 x 3 000 .. 6 000, 16 / 8 heads of 256, window 1 024: 197 ->
   // 180 (187); 16 x 20 .. 600, 16 heads of 64: 16.5 -> 15.5 (16.8); 2 x 2 048: 84.8 -> 81.0 (82.7); 4 x 4 096, 32 / 8: 558 -> 545 (545).
   uint32_t a = __builtin_bit_cast(uint32_t, l_lane), b = a;
@@ -471,30 +470,24 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
   char* const rows_lds = vm_lds + ((tb - ta + 1) & 1) * S::kBuffer + wave * (S::kBuffer / kVmWaves);
   constexpr int kBlocks = S::kBuffer / kVmWaves / (32 * 64);  // blocks of 32 elements that a wave's part holds of its rows
   constexpr int kRounds = (NB + kBlocks - 1) / kBlocks, kHere = NB / kRounds, kRowChunks = kHere * 4;
-  static_assert(NB % kRounds == 0 && 32 * kRowChunks % kWave == 0, "the output's parts");
-  const int l = lane_now(), column = l & 31;
-  auto place = [&](int row, int chunk) { return rows_lds + row * (kRowChunks * 16) + ((chunk ^ (row & (kRowChunks % 8 == 0 ? kRowChunks - 1 : 3))) << 4); };
+  static_assert(NB % kRounds == 0, "the output's parts");
+  using Stage = RowStage<kRowChunks>;
+  const int l = lane_now();
 #pragma unroll
   for (int round = 0; round < kRounds; ++round) {
 #pragma unroll
     for (int x = 0; x < kRowChunks; ++x) {
       const int nb = round * kHere + x / 4, c = x % 4;
-      const uint2_t w = {pack_pair<KIND>(acc[nb][4 * c] * inv, acc[nb][4 * c + 1] * inv),
-                         pack_pair<KIND>(acc[nb][4 * c + 2] * inv, acc[nb][4 * c + 3] * inv)};
-      *reinterpret_cast<uint2_t*>(place(column, x) + 8 * (l >> 5)) = w;
+      Stage::put(rows_lds, l & 31, x, l >> 5, pack_pair<KIND>(acc[nb][4 * c] * inv, acc[nb][4 * c + 1] * inv),
+                 pack_pair<KIND>(acc[nb][4 * c + 2] * inv, acc[nb][4 * c + 3] * inv));
     }
-    asm volatile("" : : : "memory");
-#pragma unroll
-    for (int x = 0; x < 32 * kRowChunks / kWave; ++x) {
-      const int i = x * kWave + l, row = i / kRowChunks, chunk = i % kRowChunks;
+    Stage::template take<32>(rows_lds, l, [&](int row, int chunk, uint4_t w) {
       const int t_here = token_of_row(32 * wave + row), head_here = 32 * wave + row - t_here * p.fold;
-      const uint4_t w = *reinterpret_cast<const uint4_t*>(place(row, chunk));
       if (t_here < tok_cnt && head_here < group_here) {
         const int64_t elem = (static_cast<int64_t>(q_begin + tok0 + t_here) * p.q_heads + head0 + head_here) * D + round * (32 * kHere) + 8 * chunk;
         __builtin_nontemporal_store(w, reinterpret_cast<uint4_t*>(static_cast<char*>(p.out) + elem * 2));
       }
-    }
-    asm volatile("" : : : "memory");
+    });
   }
 }
 
