@@ -410,7 +410,10 @@ def areno_varlen_causal_attention(
         # the reference's kernels read doubles and compute in fp32 (attention.cu:846 there): the same through casts
         return _VarlenCausalAttention.apply(q.float(), k.float(), v.float(), cu_seqlens, _window_left(window_left),
                                             _scale(q, softmax_scale)).double()  # fmt: skip
-    return _VarlenCausalAttention.apply(q, k, v, cu_seqlens, _window_left(window_left), _scale(q, softmax_scale))
+    args = (q, k, v, cu_seqlens, _window_left(window_left), _scale(q, softmax_scale))
+    # the extension's own autograd node; what it does not take (tracing, transforms, tangents) takes the class above
+    out = _extension().areno_varlen_causal_attention(*args)
+    return _VarlenCausalAttention.apply(*args) if out is None else out
 
 
 @torch._dynamo.disable

@@ -10,7 +10,12 @@
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
+
+#include <cmath>
 
 #include "../../include/areno_hip.h"
 
@@ -696,6 +701,119 @@ std::vector<at::Tensor> attention_backward(at::Tensor grad_out, at::Tensor q, at
   return {dq, dk, dv};
 }
 
+// ---- the ops' way from Python to the launch --------------------------------------------------------------------------
+// What these functions do not take as a matter of course they hand back as None, and the Python layer goes its own way:
+// tracing, functorch's transforms, dispatch modes, tensors of such, forward-mode tangents, and every call that the Python
+// layer's checks refuse (it then refuses by itself, with its own words).
+
+bool ordinary_call() {
+  return !torch::jit::tracer::isTracing() && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+         !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
+bool ordinary(const at::Tensor& t) {
+  constexpr c10::DispatchKeySet kWrapped({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
+                                          c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize});
+  return t.defined() && t.is_cuda() && !t.key_set().has_any(kWrapped) && !t._fw_grad(0).defined();
+}
+template <typename... Rest>
+bool ordinary(const at::Tensor& t, const Rest&... rest) {
+  return ordinary(t) && ordinary(rest...);
+}
+// an exception that a Python hook raised on the way (a saved-tensor hook's, say) stays that exception
+template <typename Call>
+pybind11::object as_python(const Call& call) {
+  try {
+    return pybind11::cast(call());
+  } catch (python_error& e) {
+    e.restore();
+    throw pybind11::error_already_set();
+  }
+}
+
+// The varlen op under autograd (_ArenoVarlenCausalAttention, areno/accel/attention.py:145-183 in the reference): saves q, k, v,
+// the output and cu_seqlens.  Forward and backward of small packs last as long as the host needs for them; with the Python class
+// of the same content and with this node, us: 5 sequences of 6 .. 49 tokens, 28 / 4 heads of 128: 79.1, 67.1; 16 x 20 .. 600, 16 heads
+// of 64: 80.6, 70.8.
+struct VarlenAttention : torch::autograd::Function<VarlenAttention> {
+  static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q, const at::Tensor& k,
+                            const at::Tensor& v, const at::Tensor& cu_seqlens, int64_t window_left, double softmax_scale) {
+    at::Tensor out = varlen_forward(q.contiguous(), k.contiguous(), v.contiguous(), cu_seqlens.contiguous(), window_left, softmax_scale);
+    ctx->save_for_backward({q, k, v, out, cu_seqlens});
+    ctx->saved_data["window_left"] = window_left;
+    ctx->saved_data["softmax_scale"] = softmax_scale;
+    return out;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    auto g = attention_backward(grads[0].contiguous(), saved[0].contiguous(), saved[1].contiguous(), saved[2].contiguous(),
+                                saved[3].contiguous(), saved[4].contiguous(), c10::nullopt, c10::nullopt,
+                                ctx->saved_data["window_left"].toInt(), ctx->saved_data["softmax_scale"].toDouble(), true);
+    return {g[0], g[1], g[2], at::Tensor(), at::Tensor(), at::Tensor()};
+  }
+};
+
+pybind11::object varlen_attention_op(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor cu_seqlens, int64_t window_left,
+                                     double softmax_scale) {
+  if (!ordinary_call() || !ordinary(q, k, v, cu_seqlens)) return pybind11::none();
+  return as_python([&] {
+    if (c10::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
+      return VarlenAttention::apply(q, k, v, cu_seqlens, window_left, softmax_scale);
+    return varlen_forward(q.contiguous(), k.contiguous(), v.contiguous(), cu_seqlens.contiguous(), window_left, softmax_scale);
+  });
+}
+
+// (1, T, heads, D) activations and the cache's pools as the inference backend gets them, where no gradient is wanted
+bool backend_call(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& k_cache, const at::Tensor& v_cache,
+                  const c10::optional<at::Tensor>& k_scale, const c10::optional<at::Tensor>& v_scale) {
+  if (!ordinary_call() || !ordinary(q, k, v, k_cache, v_cache)) return false;
+  const bool quantized = k_cache.scalar_type() == at::kChar || k_cache.scalar_type() == at::kFloat8_e4m3fn;
+  if (k_scale.has_value() != quantized || v_scale.has_value() != quantized) return false;
+  if (quantized && !(ordinary(*k_scale, *v_scale) && k_scale->is_contiguous() && v_scale->is_contiguous())) return false;
+  if (c10::GradMode::is_enabled() &&
+      (q.requires_grad() || k.requires_grad() || v.requires_grad() || k_cache.requires_grad() || v_cache.requires_grad()))
+    return false;
+  return q.dim() == 4 && k.dim() == 4 && v.dim() == 4 && k_cache.dim() == 4 && v_cache.dim() == 4 && k_cache.is_contiguous() &&
+         v_cache.is_contiguous() && q.scalar_type() != at::kDouble && v.size(3) == q.size(3) && v.size(3) == v_cache.size(3);
+}
+at::Tensor rows_of(const at::Tensor& x) { return x.reshape({-1, x.size(2), x.size(3)}).contiguous(); }
+double scale_or_default(const c10::optional<double>& scale, const at::Tensor& q) {
+  return scale.has_value() ? *scale : std::pow(static_cast<double>(q.size(3)), -0.5);
+}
+
+pybind11::object backend_decode(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor k_cache, at::Tensor v_cache, at::Tensor block_table,
+                                at::Tensor cache_seqlens, int64_t window_left, c10::optional<double> softmax_scale,
+                                c10::optional<at::Tensor> k_scale, c10::optional<at::Tensor> v_scale) {
+  if (!backend_call(q, k, v, k_cache, v_cache, k_scale, v_scale) || !ordinary(block_table, cache_seqlens)) return pybind11::none();
+  if (block_table.dim() != 2 || cache_seqlens.dim() != 1 || block_table.scalar_type() != at::kInt || cache_seqlens.scalar_type() != at::kInt)
+    return pybind11::none();
+  return as_python([&] {
+    return paged_decode_forward_impl(rows_of(q), rows_of(k), rows_of(v), k_cache, v_cache, block_table.contiguous(),
+                                     cache_seqlens.contiguous(), window_left, 8, scale_or_default(softmax_scale, q), k_scale, v_scale,
+                                     0, c10::nullopt, nullptr)
+        .view(q.sizes());
+  });
+}
+
+pybind11::object backend_prefill(at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor k_cache, at::Tensor v_cache, at::Tensor cu_seqlens,
+                                 at::Tensor block_ids, at::Tensor block_offsets, int64_t window_left,
+                                 c10::optional<double> softmax_scale, c10::optional<at::Tensor> k_scale,
+                                 c10::optional<at::Tensor> v_scale) {
+  if (!backend_call(q, k, v, k_cache, v_cache, k_scale, v_scale) || !ordinary(cu_seqlens, block_ids, block_offsets)) return pybind11::none();
+  if (cu_seqlens.dim() != 1 || cu_seqlens.scalar_type() != at::kInt || block_ids.dim() != 1 || block_offsets.dim() != 1 ||
+      block_ids.scalar_type() != at::kLong || block_offsets.scalar_type() != at::kLong)
+    return pybind11::none();
+  const int64_t tokens = q.size(0) * q.size(1);
+  if (k.size(0) * k.size(1) != tokens || v.size(0) * v.size(1) != tokens || k.size(2) != v.size(2) || k.size(2) == 0 ||
+      q.size(2) % k.size(2) != 0 || k.size(3) != q.size(3))
+    return pybind11::none();
+  return as_python([&] {
+    return varlen_forward_cache_write(rows_of(q), rows_of(k), rows_of(v), cu_seqlens.contiguous(), window_left,
+                                      scale_or_default(softmax_scale, q), k_cache, v_cache, block_ids.contiguous(),
+                                      block_offsets.contiguous(), k_scale, v_scale)
+        .view(q.sizes());
+  });
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -712,6 +830,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("areno_paged_decode_plan", &paged_decode_plan, "work list of a decode step, built once for all its layers");
   m.def("areno_paged_causal_attention_decode_forward_planned", &paged_decode_forward_planned,
         "paged decode forward with a per-step plan");
+  m.def("areno_varlen_causal_attention", &varlen_attention_op, "varlen causal attention, under autograd where that records; None: not taken");
+  m.def("backend_decode", &backend_decode, "the inference backend's decode pass; None: not taken");
+  m.def("backend_prefill", &backend_prefill, "the inference backend's pass over fresh prompts; None: not taken");
   m.def("areno_varlen_causal_attention_forward_cache_write", &varlen_forward_cache_write,
         "KV cache write and varlen causal attention forward over the same K and V");
   m.def("areno_paged_cache_write", &cache_write, "quantize-and-scatter KV cache write");

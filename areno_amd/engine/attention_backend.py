@@ -17,6 +17,7 @@ from __future__ import annotations
 import torch
 from torch import nn
 
+from areno_amd.accel._extension import extension as _extension
 from areno_amd.accel.attention import (
     areno_paged_cache_write,
     areno_paged_causal_attention_decode,
@@ -64,6 +65,9 @@ class HipInferBackend(nn.Module):
         k_scale: torch.Tensor | None = None,
         v_scale: torch.Tensor | None = None,
     ) -> torch.Tensor:
+        out = self._native(q, k, v, k_cache, v_cache, meta, window_size, softmax_scale, update_cache, k_scale, v_scale)
+        if out is not None:
+            return out
         q_flat = q.reshape(-1, q.shape[-2], q.shape[-1])
         k_flat = k.reshape(-1, k.shape[-2], k.shape[-1])
         v_flat = v.reshape(-1, v.shape[-2], v.shape[-1])
@@ -126,6 +130,29 @@ class HipInferBackend(nn.Module):
             return out.reshape(q.shape[0], q.shape[1], q.shape[2], value_dim)
 
         raise ValueError(f"unsupported inference mode: {meta.mode}")
+
+    @staticmethod
+    @torch._dynamo.disable
+    def _native(q, k, v, k_cache, v_cache, meta, window_size, softmax_scale, update_cache, k_scale, v_scale):
+        """The pass as one call of the extension: small ones last as long as the host needs for them.  Through the ops and as one
+        call, us: decode of one row with 4 k cached tokens 16.8, 13.7, of short rows 17.1, 11.7; prompts of a few tokens
+        (two ops) 21.3, 11.5.  None: whatever it does not take as a matter of course, and every call that the checks of the
+        ops refuse."""
+        if not q.is_cuda or not update_cache or (window_size is not None and window_size[1] != 0 and tuple(window_size) != (-1, -1)):
+            return None
+        window_left = -1 if window_size is None else int(window_size[0])
+        tensors = (q, k, v, k_cache, v_cache)
+        if meta.mode == "decode":
+            if meta.cache_seqlens is None or meta.block_table is None:
+                return None
+            return _extension().backend_decode(*tensors, meta.block_table, meta.cache_seqlens, window_left, softmax_scale,
+                                               k_scale, v_scale)  # fmt: skip
+        if meta.mode != "prefill" or meta.context_lens is not None or meta.max_seqlen is None or meta.block_table is None:
+            return None
+        if meta.cu_seqlens is None or meta.cache_block_ids is None or meta.cache_block_offsets is None:
+            return None
+        return _extension().backend_prefill(*tensors, meta.cu_seqlens, meta.cache_block_ids, meta.cache_block_offsets, window_left,
+                                            softmax_scale, k_scale, v_scale)  # fmt: skip
 
 
 def build_infer_attention_backend(attn_backend: str = "native") -> HipInferBackend:

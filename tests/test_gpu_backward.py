@@ -554,3 +554,81 @@ def test_gradients_in_the_inputs_type_are_the_fp32_ones_rounded_in_every_form(dt
     wide, narrow = (_c_backward(go, q, k, v, out, cu, t, d**-0.5) for t in (torch.float32, dtype))
     for w, n, name in zip(wide, narrow, ("dq", "dk", "dv")):
         assert w[:170].abs().max() > 0 and torch.equal(w.to(dtype), n), f"{name} {dtype} d={d} parts={parts}"
+
+
+def _small_varlen(dtype=torch.bfloat16):
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(49, h, 64, generator=g).to(dtype).to(DEV).requires_grad_(True) for h in (8, 2, 2))
+    return q, k, v, torch.tensor([0, 40, 49], dtype=torch.int32, device=DEV)
+
+
+def _through_the_python_class(q, k, v, cu):
+    return ops._VarlenCausalAttention.apply(q, k, v, cu, -1, 64**-0.5)
+
+
+def test_varlen_autograd_node_is_that_of_the_python_class():
+    """The extension's node and the Python class: the same gradients with every subset of inputs that want one, saved-tensor
+    hooks that see the same tensors, recomputation, non-contiguous inputs, no graph without a gradient to give."""
+    from torch.utils.checkpoint import checkpoint
+
+    q, k, v, cu = _small_varlen()
+    weight = torch.randn(49, 8, 64, device=DEV, dtype=torch.bfloat16)
+    want = torch.autograd.grad(_through_the_python_class(q, k, v, cu), (q, k, v), weight)
+    for wanted in ((0,), (1, 2), (0, 1, 2)):
+        args = [x.detach().requires_grad_(i in wanted) for i, x in enumerate((q, k, v))]
+        out = ops.areno_varlen_causal_attention(*args, cu)
+        grads = torch.autograd.grad(out, [args[i] for i in wanted], weight)
+        assert all(torch.equal(a, want[i]) for a, i in zip(grads, wanted))
+
+    def packed_by(op):
+        seen = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: (seen.append(t.clone()), t.cpu())[1], lambda t: t.to(DEV)):
+            out = op(q, k, v, cu)
+        grads = torch.autograd.grad(out, (q, k, v), weight)
+        return seen, grads
+
+    (seen, grads), (seen_class, _) = packed_by(ops.areno_varlen_causal_attention), packed_by(_through_the_python_class)
+    assert len(seen) == len(seen_class) and all(torch.equal(a, b) for a, b in zip(seen, seen_class))
+    assert all(torch.equal(a, b) for a, b in zip(grads, want))
+
+    def layer(a, b, c):
+        return ops.areno_varlen_causal_attention(a * 1, b * 1, c * 1, cu)  # (the recomputation stops as soon as it has what was saved)
+
+    grads = torch.autograd.grad(checkpoint(layer, q, k, v, use_reentrant=False), (q, k, v), weight)
+    assert all(torch.equal(a, b) for a, b in zip(grads, want))
+    wide = torch.randn(49, 8, 128, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    part = wide[..., ::2]
+    grad = torch.autograd.grad(ops.areno_varlen_causal_attention(part, k, v, cu), wide, weight)[0]
+    assert torch.equal(grad, torch.autograd.grad(_through_the_python_class(part, k, v, cu), wide, weight)[0])
+    with torch.no_grad():
+        assert not ops.areno_varlen_causal_attention(q, k, v, cu).requires_grad
+    out = ops.areno_varlen_causal_attention(q, k, v, cu)
+    with torch.no_grad():
+        q.mul_(2)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.backward(weight)
+    q, k, v, cu = _small_varlen()
+    out = ops.areno_varlen_causal_attention(q, k, v, cu)
+    out.backward(weight)
+    with pytest.raises(RuntimeError, match="second time"):
+        out.backward(weight)
+
+
+def test_varlen_calls_that_no_node_of_its_own_takes():
+    """Forward-mode tangents and vmap are refused as the Python class refuses them; a hook's exception stays itself."""
+    q, k, v, cu = _small_varlen()
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(q.detach(), torch.ones_like(q))
+        with pytest.raises(RuntimeError):
+            ops.areno_varlen_causal_attention(dual, k, v, cu)
+    with pytest.raises(RuntimeError, match="vmap"):
+        torch.vmap(lambda x: ops.areno_varlen_causal_attention(x, k, v, cu))(torch.stack([q.detach(), q.detach()]))
+
+    class Own(Exception):
+        pass
+
+    def refuse(t):
+        raise Own
+
+    with torch.autograd.graph.saved_tensors_hooks(refuse, lambda t: t), pytest.raises(Own):
+        ops.areno_varlen_causal_attention(q, k, v, cu)

@@ -166,3 +166,40 @@ def test_loop_driven_by_device_block_tables():
     decode([2, 1, 3], lens_dev, 9)  # row 3 reaches position 16 one step before row 1 reaches 48
     assert pages.row_pages(1) == [6, 7, 8, 10] and pages.row_pages(3) == [3, 9]
     same_pages()
+
+
+@pytest.mark.parametrize("kv", ["auto", "int8"])
+def test_a_pass_is_the_same_through_the_extension_and_the_ops(kv):
+    """The backend hands most calls to the extension as a whole; a call that wants a gradient, or whose values need padding,
+    goes through the ops.  Same output and pages either way, and the refusals are the ops'."""
+    gen = torch.Generator().manual_seed(9)
+    hq, hkv, d, t = 8, 2, 64, 45
+    backend = build_infer_attention_backend()
+    q, k, v = (torch.randn(1, t, h, d, generator=gen).to(torch.bfloat16).to(DEV) for h in (hq, hkv, hkv))
+    slots = torch.arange(t, device=DEV)
+    table = torch.arange(8, dtype=torch.int32, device=DEV).view(2, 4)
+    prefill = InferMeta(mode="prefill", cu_seqlens=torch.tensor([0, 40, t], dtype=torch.int32, device=DEV), max_seqlen=40,
+                        block_table=table, cache_block_ids=slots // BS, cache_block_offsets=slots % BS)  # fmt: skip
+    decode = InferMeta(mode="decode", cache_seqlens=torch.tensor([40, 5], dtype=torch.int32, device=DEV), block_table=table)
+    layers = [allocate_kv_caches(1, 8, BS, hkv, d, DEV, torch.bfloat16, kv)[0] for _ in range(2)]
+    for layer in layers:
+        for pool in (layer.k_cache, layer.v_cache):
+            pool.view(torch.uint8).zero_()
+    for meta, rows in ((prefill, t), (decode, 2)):
+        outs = []
+        for layer, wants_grad in zip(layers, (False, True)):
+            x = q[:, :rows].detach().requires_grad_(wants_grad)
+            outs.append(backend(x, k[:, :rows], v[:, :rows], layer.k_cache, layer.v_cache, meta, window_size=(20, 0),
+                                k_scale=layer.k_scale, v_scale=layer.v_scale))  # fmt: skip
+            assert outs[-1].requires_grad == wants_grad
+        assert torch.equal(outs[0], outs[1])
+        for a, b in ((layers[0].k_cache, layers[1].k_cache), (layers[0].v_cache, layers[1].v_cache)):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+        bad = [(dict(q=q[..., :32]), RuntimeError), (dict(k_cache=layers[0].k_cache[0]), ValueError), (dict(q=q.cpu()), RuntimeError)]
+        for changed, error in bad:
+            args = {**dict(q=q[:, :rows], k=k[:, :rows], v=v[:, :rows], k_cache=layers[0].k_cache), **changed}
+            if "q" in changed:
+                args["q"] = args["q"][:, :rows]
+            with pytest.raises((error, ValueError)):
+                backend(args["q"], args["k"], args["v"], args["k_cache"], layers[0].v_cache, meta, k_scale=layers[0].k_scale,
+                        v_scale=layers[0].v_scale)  # fmt: skip
