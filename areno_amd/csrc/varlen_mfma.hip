@@ -3,9 +3,9 @@
 //
 // A workgroup of four waves computes one query block of one kv head -- 128 rows, row r being (token r / fold, q head
 // r % fold) as in prefill_mfma.hip -- from its first visible key to its last.  No block is cut, so nothing is left
-// to merge; the blocks of a launch are taken longest first (varlen_blocks.hpp), and two workgroups share a compute unit
+// to merge; the blocks of a launch are taken longest first (varlen_blocks.hpp), and two or three workgroups share a compute unit
 // (four at head dim 64), so one's waits and softmax fall into the other's products.  Per step of 64 keys (32 at the wide
-// heads) a wave, which owns 32 of the rows:
+// heads, and at head dim 128 where short_tiles_are_faster) a wave, which owns 32 of the rows:
 //   * passes one barrier and asks for the next step's K and V tiles, which the memory pipe writes into LDS by itself
 //     (two buffers; mfma32_tiles.hpp);
 //   * S^T = K . Q^T on 32 x 32 x 16 products, Q in registers; a lane holds half of the keys of one query row;
@@ -19,6 +19,7 @@
 // per query block with nothing beside it, the partials of cut blocks (up to 67 MB written and read), a third of the
 // loop's vector instructions (staging, half the lane swaps).  Bound at length by the matrix cores and the LDS
 // reads behind them (an operand read per product), at short lengths by a block's chain of steps.
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -130,12 +131,13 @@ __device__ __forceinline__ bool find_block(const VarlenMfmaParams& p, int i, Blo
 extern __shared__ __attribute__((aligned(1024))) char vm_lds[];
 constexpr int kSchedMatrix = 0x8, kSchedLdsRead = 0x100;  // instruction classes of sched_group_barrier
 
-template <int D, bool WRITE>
+template <int D, bool WRITE, int TILE>
 struct VmShape {
-  static constexpr int kTile = D <= 128 ? 64 : 32;  // keys per step
+  static constexpr int kTile = TILE;  // keys per step
   using Tile = LdsTile<D, kTile, kVmWaves>;
   static constexpr int kBuffer = 2 * Tile::kBytes;  // K, V
-  static constexpr int kPlaces = 2 * kBuffer;  // the pages of the block's tokens, then their places in these
+  static constexpr int kQueries = kBuffer + (D <= 128 ? kVmRows * D * 2 : 0);  // the end of the query rows, which start where the second tile will lie
+  static constexpr int kPlaces = 2 * kBuffer > kQueries ? 2 * kBuffer : kQueries;  // the pages of the block's tokens, then their places in these
   static constexpr int kLdsBytes = WRITE ? kPlaces + 2 * kVmRows * 8 : kPlaces;
 };
 
@@ -164,7 +166,7 @@ __device__ __forceinline__ void write_page_chunk(const PageWrite& w, uint4_t raw
   }
 }
 
-// (Two waves per SIMD, four at head dim 64, are what the tiles leave room for, and the scheduler is told so: where it
+// (Two waves per SIMD -- three with steps of 32 keys at head dim 128, four at 64 -- are what the tiles leave room for, and the scheduler is told so: where it
 // takes three to be within reach it saves registers for them and waits for every operand read right behind it --
 // 8 192 tokens, 8 / 1 heads of 128: 208 instead of 172 us.)
 //
@@ -173,9 +175,9 @@ __device__ __forceinline__ void write_page_chunk(const PageWrite& w, uint4_t raw
 // fetch, and their stores go out behind the output's, while the next workgroup starts.  The pass with a launch of its own for
 // the pages and with this, us (both with the output's stores as they were then): 32 prompts of 33 .. 512 tokens, 28 / 4 heads of 128, bf16: 61.5 -> 57.6; 2 x 3 000 .. 6 000, 16 / 8
 // heads of 256, window 1 024: 176.6 -> 165; 24 x 48 .. 387 into fp8 pages 40.0 -> 38.8; 2 x 9 .. 74: 21.7 -> 17.7 (the host's).
-template <int KIND, int D, bool WRITE>
-__global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D == 64 ? 4 : 2))) void varlen_mfma_kernel(VarlenMfmaParams p) {
-  using S = VmShape<D, WRITE>;
+template <int KIND, int D, bool WRITE, int TILE>
+__global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(D == 128 && TILE == 32 ? 3 : 2, D == 64 ? 4 : D == 128 && TILE == 32 ? 3 : 2))) void varlen_mfma_kernel(VarlenMfmaParams p) {
+  using S = VmShape<D, WRITE, TILE>;
   using T = typename S::Tile;
   using M = Mfma32<KIND>;
   using V8 = typename M::vec8;
@@ -247,13 +249,31 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
   const int hh = r - t_row * p.fold;
   const bool live = t_row < tok_cnt && hh < group_here;
   const int q_pos = live ? tok0 + t_row : -1;
-  const int64_t row_elem = (static_cast<int64_t>(q_begin + tok0 + t_row) * p.q_heads + head0 + hh) * D;
+  // Up to head dim 128 the query rows come through LDS, where the second tile will lie, as whole rows: a lane needs 16 bytes
+  // here and there of one row, and asked for as such they are 64 pieces an instruction (the kernel with steps of 64 keys, us:
+  // 4 x 4 096, 32 / 8 heads: 548 -> 540; 16 x 20 .. 600, 16 heads of 64: 16.4 -> 15.9).  The wide heads' rows are twice what a buffer
+  // holds.  Rows that do not exist repeat the block's first.
+  constexpr bool kRowsThroughLds = D <= 128;
   V8 qop[NKS];
+  if constexpr (!kRowsThroughLds) {
+    const int64_t row_elem = (static_cast<int64_t>(q_begin + tok0 + t_row) * p.q_heads + head0 + hh) * D;
 #pragma unroll
-  for (int ks = 0; ks < NKS; ++ks) {
-    uint4_t w = {0u, 0u, 0u, 0u};
-    if (live) w = load16(p.q, (row_elem + 16 * ks + 8 * h) * 2);
-    qop[ks] = __builtin_bit_cast(V8, w);
+    for (int ks = 0; ks < NKS; ++ks) {
+      uint4_t w = {0u, 0u, 0u, 0u};
+      if (live) w = load16(p.q, (row_elem + 16 * ks + 8 * h) * 2);
+      qop[ks] = __builtin_bit_cast(V8, w);
+    }
+  } else {
+    const char* const rows = static_cast<const char*>(p.q) + (static_cast<int64_t>(q_begin + tok0) * p.q_heads + head0) * (D * 2);
+    constexpr int kFetchRows = 64 / T::kChunksPerRow;
+#pragma unroll
+    for (int f = 0; f < 32 / kFetchRows; ++f) {
+      const int row = kFetchRows * f + lane / T::kChunksPerRow, t = token_of_row(32 * wave + row), head = 32 * wave + row - t * p.fold;
+      const bool there = t < tok_cnt && head < group_here;
+      const uint32_t off = there ? static_cast<uint32_t>(t * p.q_heads + head) * (D * 2) : 0u;
+      fetch_to_lds(rows, off + static_cast<uint32_t>((lane % T::kChunksPerRow) ^ T::twist(row)) * 16u,
+                   lds_address(vm_lds) + S::kBuffer + wave * (32 * T::kRowBytes) + f * 1024);
+    }
   }
   const bool wave_live = 32 * wave < tok_cnt * p.fold;
   const int wave_qmin = tok0 + token_of_row(32 * wave);
@@ -355,11 +375,12 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
         }
       }
     }
-    // online softmax as in prefill_mfma.hip: the reference value is raised only when a tile exceeds it by 2^8
-    // (by 2^2 at the wide heads.  Relative error against 64 bits with 2^8 and 2^2, in bf16, and of the kernel that this one
-    // replaces: 256 wide, 300 .. 1 000 tokens, window 512: 2.026e-3, 1.992e-3, 2.020e-3; 192 wide: 1.985e-3, 1.955e-3,
-    // 1.957e-3; 2 x 2 048 tokens, 128 wide: 2.063e-3, 2.040e-3, 2.076e-3.  It costs 2 to 4 % of the time.)
-    constexpr float kLazy = D <= 128 ? 8.0f : 2.0f;
+    // online softmax as in prefill_mfma.hip: the reference value is raised only when a tile exceeds it by 2^8, by 2^2 with steps
+    // of 32 keys, whose first tile sets a lower one.  Relative error against 64 bits with 2^8 and 2^2, in bf16, and of the
+    // kernel with longer steps that it replaces: 256 wide, 300 .. 1 000 tokens, window 512: 2.026e-3, 1.992e-3, 2.020e-3; 192 wide:
+    // 1.985e-3, 1.955e-3, 1.957e-3; 128 wide, 33 .. 900 tokens: 1.973e-3, 1.949e-3, 1.960e-3 (fp16 2.467e-4, 2.436e-4, 2.450e-4).  It
+    // costs 2 to 4 % of the time.
+    constexpr float kLazy = TK == 64 ? 8.0f : 2.0f;
     float mt = max3_f32(s[0][0], s[0][1], s[0][2]);
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
@@ -424,6 +445,11 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(2, D
     const int64_t first = static_cast<int64_t>(q_begin + tok0) * 8;
     fetch_words_to_lds(reinterpret_cast<const char*>(p.pages.block_ids) + first, word, lds0 + S::kPlaces + wave * (kWave * 4));
     fetch_words_to_lds(reinterpret_cast<const char*>(p.pages.block_offsets) + first, word, lds0 + S::kPlaces + kVmRows * 8 + wave * (kWave * 4));
+  }
+  if constexpr (kRowsThroughLds) {
+    fetched();  // (its own rows: no barrier)
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) qop[ks] = tile_rows<KIND, T>(vm_lds + S::kBuffer + wave * (32 * T::kRowBytes), at_rows, 0, ks);
   }
   // (the query rows are waited for here: left to their first use inside the loop, that wait would cover every step's
   // fetches as well)
@@ -496,20 +522,20 @@ struct VmLaunch {
   vm_fn fn;  // nullptr: no such kernel, or its LDS size was refused
   int lds_bytes;
 };
-template <int KIND, int D, bool WRITE>
+template <int KIND, int D, bool WRITE, int TILE>
 VmLaunch vm_launch_of() {
   static std::atomic<uint64_t> allowed_on{0};
-  constexpr int kLdsBytes = VmShape<D, WRITE>::kLdsBytes;
-  const vm_fn fn = varlen_mfma_kernel<KIND, D, WRITE>;
+  constexpr int kLdsBytes = VmShape<D, WRITE, TILE>::kLdsBytes;
+  const vm_fn fn = varlen_mfma_kernel<KIND, D, WRITE, TILE>;
   return {allow_lds<kLdsBytes>(reinterpret_cast<const void*>(fn), allowed_on) ? fn : nullptr, kLdsBytes};
 }
 template <int KIND, bool WRITE>
-VmLaunch vm_lookup(int head_dim) {
+VmLaunch vm_lookup(int head_dim, bool short_tiles) {
   switch (head_dim) {
-    case 64: return vm_launch_of<KIND, 64, WRITE>();
-    case 128: return vm_launch_of<KIND, 128, WRITE>();
-    case 192: return vm_launch_of<KIND, 192, WRITE>();
-    case 256: return vm_launch_of<KIND, 256, WRITE>();
+    case 64: return vm_launch_of<KIND, 64, WRITE, 64>();
+    case 128: return short_tiles ? vm_launch_of<KIND, 128, WRITE, 32>() : vm_launch_of<KIND, 128, WRITE, 64>();
+    case 192: return vm_launch_of<KIND, 192, WRITE, 32>();
+    case 256: return vm_launch_of<KIND, 256, WRITE, 32>();
     default: return {nullptr, 0};
   }
 }
@@ -536,6 +562,20 @@ bool equal_shares_are_faster(int64_t tokens, int32_t num_seqs, int32_t q_heads, 
   return head_dim == 192 ? length >= 4096 && blocks <= 256 : length >= 2048 && blocks <= 320;
 }
 
+// Head dim 128: steps of 32 keys leave room for three workgroups per compute unit, whose starts, ends and softmax fall into
+// each other's products; steps of 64, two workgroups, are fewer, which counts where a launch is the chain of its longest
+// blocks.  So 32 for launches that fill the chip's places (blocks of the tokens, half a block more per sequence), the more so the
+// longer their chains, and for short sequences.  In us, 64 and 32 keys (workgroups, mean length): 28 / 4 heads, 64 x 12 .. 52 tokens (588, 32)
+// 11.7, 8.2; 16 x 200 (740) 17.8, 13.1; 64 x 25 .. 390 (2 913, 195) 60.8, 52; 16 x 64 .. 960 (1 716, 474) 52.3, 47; 4 x 4 096 (3 648) 476, 468; 32 / 8,
+// 1 x 4 096 (1 024) 146, 141.  Fewer, longer ones: 16 / 16, 4 x 250 (144) 11.8, 12.5; 4 x 1 343 (740) 48.4, 52; 28 / 4, 1 x 2 048 (452) 45.0, 49; 8 / 2, 4 x 3 334
+// (840) 137, 149.  Of 302 launches of 1 .. 64 sequences of 12 .. 6 600 tokens, five head ratios, equal and ragged lengths, the choice takes
+// 0.2 % more than the better one (6 % at most), 64 keys everywhere 4.8 %.  At head dim 64, where four workgroups share a unit with 64
+// keys, five with 32 gain and lose as much.
+bool short_tiles_are_faster(int64_t tokens, int32_t num_seqs, int64_t vheads, int block_tokens, int32_t window_left) {
+  const int64_t mean = tokens / num_seqs, seen = window_left >= 0 ? std::min<int64_t>(mean, window_left + int64_t{1} + block_tokens) : mean;
+  return seen <= 200 || (tokens / block_tokens + num_seqs / 2) * vheads >= 500 + seen / 4;
+}
+
 }  // namespace
 
 // Called by launch_prefill_mfma behind its checks (types, scale, sizes, alignment, workspace), so that a packed call is
@@ -546,15 +586,16 @@ int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, i
                        int32_t window_left, float softmax_scale, const PageWrite* pages, void* stream) {
   const char* op = "areno_hip_varlen_attention";
   const bool bf16 = dtype == ARENO_DT_BF16;
-  const VmLaunch l = pages != nullptr ? (bf16 ? vm_lookup<KV_BF16, true>(head_dim) : vm_lookup<KV_F16, true>(head_dim))
-                                      : (bf16 ? vm_lookup<KV_BF16, false>(head_dim) : vm_lookup<KV_F16, false>(head_dim));
+  const int group = q_heads / kv_heads, head_parts = (group + 15) / 16;
+  const bool short_tiles = short_tiles_are_faster(tokens, num_seqs, kv_heads * head_parts, kVmRows / (head_parts > 1 ? 16 : group), window_left);
+  const VmLaunch l = pages != nullptr ? (bf16 ? vm_lookup<KV_BF16, true>(head_dim, short_tiles) : vm_lookup<KV_F16, true>(head_dim, short_tiles))
+                                      : (bf16 ? vm_lookup<KV_BF16, false>(head_dim, short_tiles) : vm_lookup<KV_F16, false>(head_dim, short_tiles));
   if (l.fn == nullptr) return ARENO_ERR_UNSUPPORTED;
-  const int group = q_heads / kv_heads;
   if (equal_shares_are_faster(tokens, num_seqs, q_heads, group, head_dim, window_left)) return ARENO_ERR_UNSUPPORTED;
-  const int head_parts = (group + 15) / 16;
   const int64_t vheads = static_cast<int64_t>(kv_heads) * head_parts;
-  // offsets inside a key tile are 32 bits wide
+  // offsets inside a key tile and inside a block's query rows are 32 bits wide
   if (static_cast<int64_t>(kv_heads) * head_dim * 2 * 64 > 0x7fffffffLL) return ARENO_ERR_UNSUPPORTED;
+  if (static_cast<int64_t>(kVmRows / (head_parts > 1 ? 16 : group)) * q_heads * head_dim * 2 > 0xffffffffLL) return ARENO_ERR_UNSUPPORTED;
   VarlenMfmaParams p;
   p.q = q;
   p.k = k;

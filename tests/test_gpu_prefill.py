@@ -456,14 +456,26 @@ def test_varlen_of_many_sequences(dtype, hq, hkv, d, lens):
     assert_close(out, want, *tolerances("bf16"), what=f"varlen of {len(lens)} sequences {hq}/{hkv} d={d}")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("window_left", [None, 100])
+@pytest.mark.parametrize("lens,hq,hkv", [([701, 390], 28, 4), ([450, 351], 3, 3), ([701, 1, 64], 8, 2), ([129] * 40 + [1], 16, 16)])
+def test_varlen_steps_of_either_length(dtype, window_left, lens, hq, hkv):
+    """Head dim 128 has kernels with steps of 64 and of 32 keys: few long blocks, and short sequences or many blocks."""
+    q, k, v, cu = _packed(lens, hq, hkv, 128, dtype)
+    out = ops.areno_varlen_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV), window_left=window_left)
+    want = ar.ref_varlen(q, k, v, cu, ar.window_left_arg(window_left), 128**-0.5)
+    assert_close(out, want, *tolerances("bf16"), what="varlen")
+
+
 @pytest.mark.parametrize("kv", ["same", "int8", "fp8"])
 @pytest.mark.parametrize("act", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("hq,hkv,d", [(28, 4, 128), (16, 16, 64), (6, 6, 256), (8, 1, 256), (24, 8, 192), (40, 2, 128), (3, 3, 128)])
-def test_prefill_with_its_cache_write(kv, act, hq, hkv, d):
+@pytest.mark.parametrize("lens", [[1, 33, 0, 130, 64, 257, 18], [701, 390]])
+def test_prefill_with_its_cache_write(kv, act, hq, hkv, d, lens):
     """One op for the cache write and the packed attention leaves the bits of the two ops: tokens of every place in a block and a
     key tile, empty sequences, tokens in front of the first sequence and behind the last, ids outside the pool, a window."""
     cache_dtype, scale_dtype = {"same": (act, None), "int8": (torch.int8, torch.float16), "fp8": (torch.float8_e4m3fn, torch.float32)}[kv]
-    lens, front, behind, bs = [1, 33, 0, 130, 64, 257, 18], 3, 5, 16
+    front, behind, bs = 3, 5, 16
     t = front + sum(lens) + behind
     g = torch.Generator().manual_seed(d + hq)
     q, k, v = (torch.randn(t, h, d, generator=g).to(act).to(DEV) for h in (hq, hkv, hkv))
