@@ -221,6 +221,23 @@ __device__ __forceinline__ float max_all(const float (&v)[N]) {
 
 // a wave-uniform value that the compiler cannot prove uniform (it came out of LDS): move it to a scalar register
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+// Whole-wave reductions of integers, by the steps of wave_max_fast
+template <typename Op>
+__device__ __forceinline__ int wave_reduce(int x, Op op) {
+  auto lanes = [](int v, auto ctrl) {
+    return __builtin_bit_cast(int, dpp_lanes<decltype(ctrl)::value>(__builtin_bit_cast(float, v)));
+  };
+  x = op(x, lanes(x, std::integral_constant<int, kDppQuadSwap1>{}));
+  x = op(x, lanes(x, std::integral_constant<int, kDppQuadSwap2>{}));
+  x = op(x, lanes(x, std::integral_constant<int, kDppRowHalfMirror>{}));
+  x = op(x, lanes(x, std::integral_constant<int, kDppRowMirror>{}));
+  uint32_t a = static_cast<uint32_t>(x), b = a;
+  swap_rows16(a, b);
+  x = op(static_cast<int>(a), static_cast<int>(b));
+  a = b = static_cast<uint32_t>(x);
+  swap_rows32(a, b);
+  return uniform(op(static_cast<int>(a), static_cast<int>(b)));
+}
 
 // The item table in LDS as the cursor functions of decode_items.hpp want it; the lookups' indices are the same in
 // all lanes of a wave, so the values end up in scalar registers.

@@ -68,7 +68,7 @@ size_t prefill_mfma_workspace_bytes(int32_t kv_heads, int32_t head_dim);
 int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out, int32_t q_dtype, int64_t tokens,
                         int32_t q_heads, int32_t num_seqs, const int32_t* block_table, int32_t max_blocks,
                         const int32_t* cu_seqlens_q, const int32_t* context_lens, int32_t window_left,
-                        float softmax_scale, void* workspace, size_t workspace_bytes, void* stream);
+                        float softmax_scale, void* workspace, size_t workspace_bytes, const PageWrite* pages, void* stream);
 
 namespace {
 
@@ -86,8 +86,8 @@ constexpr int kMaxPrefillUnits = 512;   // per kv head
 // What a unit leaves for the merge: its last item, when that starts in the unit and is not finished there.
 struct CutItem {
   int32_t first_slot;  // of its partials, the others are at slot 2u of the units behind; -1: nothing to merge
-  int32_t total;       // tile steps of the launch
-  int32_t step_end;    // the item's steps end in front of this one
+  int32_t total;       // tile steps of the launch; 0: units that belong to one item each (place_of_unit)
+  int32_t step_end;    // the item's steps (total == 0: its units) end in front of this one
   int32_t token0;      // its first query token's row of q / out
   int32_t tokens;
   int32_t end;  // where the last sequence ends (also in units without anything to merge)
@@ -129,6 +129,7 @@ struct PrefillParams {
   int32_t q_dtype;
   int32_t units;        // per (kv head, part)
   int32_t rows_per_wg;  // query rows of one item: 64 per 16-row tile a wave owns
+  int32_t few_items;    // at most 64 items and sequences, fewer than units: place_of_unit
   float scale_log2e;
 };
 
@@ -217,6 +218,82 @@ __device__ __forceinline__ int unit_start_step(int total, int u, int units) {
   return static_cast<int>(q * static_cast<uint32_t>(u) + (n - q * d) * static_cast<uint32_t>(u) / d);
 }
 
+// Few items for many units: units that belong to one item each, instead of equal shares of all steps.  A unit that an item's
+// border cuts has two segments, and a segment costs ~10 us besides its steps (a fill, a query block, an end), as much as eight
+// steps: with six items over 64 units, six or seven steps each, the launch is those few units.  Here an item has as many
+// units as it needs at `share` steps each, the least share that does with the launch's units.  Every wave finds its place
+// by itself, a lane per sequence and then per item, with nothing to wait for but the lengths.  False: shares would become
+// a segment's cost larger than equal ones, or nothing to do.  The attention with equal shares and with this, us: 28 / 4 heads
+// of 128, 4 x 64 tokens on 4 k int8 ones: 33 -> 30; 8 x 512 on 4 k 101 -> 65; 2 x 512 on 64, 16 bits, 48.7 -> 30.8; 8 / 2,
+// 1 x 12 on 600 20.0 -> 11.8; of 411 launches of 1 .. 16 sequences of 1 .. 512 tokens on up to 16 k, by how many steps a share
+// is larger: none 0.82 of the time, 1 .. 3 0.82, 4 .. 7 0.89.  The look that finds it eight or more, and in vain, is 1 us:
+// 38.8 -> 39.8, 262 -> 266.
+struct UnitPlace {
+  StepPos pos;     // (item_x0 = 0: steps count from the item's first)
+  int x_begin, x_end;
+  int nth, of;     // which of the item's units this is
+  int end;         // where the last sequence ends
+};
+constexpr int kSegmentSteps = 8;  // what a segment costs besides its steps, in steps
+__device__ __forceinline__ bool place_of_unit(const PrefillParams& p, int tq, int unit, UnitPlace& at) {
+  const int lane = threadIdx.x & (kWave - 1), s = min(lane, p.num_seqs - 1);
+  const int q_begin = p.cu_seqlens_q[s], q_end = p.cu_seqlens_q[s + 1];
+  const int ctx = p.context_lens != nullptr ? p.context_lens[s] : 0;
+  const int n_new = lane < p.num_seqs ? max(q_end - q_begin, 0) : 0;
+  const int blocks = query_blocks(n_new, tq);
+  int items = 0, seq = 0, before = 0;
+  for (int i = 0; i < p.num_seqs; ++i) {
+    items += __builtin_amdgcn_readlane(blocks, i);
+    const bool behind = lane >= items;
+    seq += behind ? 1 : 0;
+    before = behind ? items : before;
+  }
+  if (items == 0 || items > kWave || items >= p.units) return false;
+  seq = min(seq, p.num_seqs - 1);
+  const int item_new = __shfl(n_new, seq, kWave), item_ctx = __shfl(ctx, seq, kWave), j = lane < items ? lane - before : 0;
+  const BlockTiles tiles = block_tiles(item_new, item_ctx, j, tq, p.window_left);
+  const uint32_t steps = lane < items ? static_cast<uint32_t>(max(tiles.count(), 1)) : 0u;
+  auto sum = [](uint32_t x) { return static_cast<uint32_t>(wave_reduce(static_cast<int>(x), [](int a, int b) { return a + b; })); };
+  auto units_at = [&](uint32_t share) { return (steps + share - 1) / share; };
+  const uint32_t total = sum(steps), units = static_cast<uint32_t>(p.units), spare = units - static_cast<uint32_t>(items);
+  const uint32_t equal = (total + units - 1) / units;
+  uint32_t lo = equal, hi = (total + spare - 1) / spare;  // (at which a unit more for every item does)
+  if (hi >= equal + kSegmentSteps) {
+    hi = equal + kSegmentSteps - 1;
+    if (sum(units_at(hi)) > units) return false;
+  }
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) / 2;
+    if (sum(units_at(mid)) <= units) {
+      hi = mid;
+    } else {
+      lo = mid + 1;
+    }
+  }
+  const int share = static_cast<int>(lo), of = static_cast<int>(units_at(lo));
+  int first = 0, chosen = -1, chosen_first = 0;
+  for (int i = 0; i < items; ++i) {
+    const int n = __builtin_amdgcn_readlane(of, i);
+    if (unit >= first && unit < first + n) chosen = i, chosen_first = first;
+    first += n;
+  }
+  at.end = __builtin_amdgcn_readlane(q_end, p.num_seqs - 1);
+  at.x_begin = at.x_end = 0;
+  if (chosen < 0) return true;  // (a unit without work)
+  at.nth = unit - chosen_first;
+  at.of = __builtin_amdgcn_readlane(of, chosen);
+  at.x_begin = at.nth * share;
+  at.x_end = min(at.x_begin + share, __builtin_amdgcn_readlane(static_cast<int>(steps), chosen));
+  at.pos.seq = __builtin_amdgcn_readlane(seq, chosen);
+  at.pos.j = __builtin_amdgcn_readlane(j, chosen);
+  at.pos.n_new = __builtin_amdgcn_readlane(item_new, chosen);
+  at.pos.ctx = __builtin_amdgcn_readlane(item_ctx, chosen);
+  at.pos.q_begin = __builtin_amdgcn_readlane(q_begin, at.pos.seq);
+  at.pos.tile = __builtin_amdgcn_readlane(tiles.tile_lo, chosen) + at.x_begin;
+  at.pos.item_x0 = 0;
+  return true;
+}
+
 // 16 codes of an 8-bit cache row (one 16-byte chunk) -> 16 fp16 values times the row's scale, as two 16-byte groups.
 // int8: (code ^ 0x80) under the exponent byte 0x64 is fp16 1152 + code, exactly; the packed subtract and multiply
 // that follow are exact resp. correctly rounded.  fp8: the hardware conversion is exact.
@@ -299,14 +376,20 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
   const int unit = blockIdx.x;
   const int tq = p.block_tokens;  // query tokens per item
 
-  prefix_tile_steps(p, tq, s_cum, s_wave_tot, &s_end);
-  const int total = s_cum[p.num_seqs];
-  const int x_begin = unit_start_step(total, unit, p.units);
-  const int x_end = unit_start_step(total, unit + 1, p.units);
+  UnitPlace place;
+  const bool one_item = p.few_items != 0 && place_of_unit(p, tq, unit, place);  // (the same for the whole launch)
+  if (!one_item) {
+    prefix_tile_steps(p, tq, s_cum, s_wave_tot, &s_end);
+    const int total = s_cum[p.num_seqs];
+    place.x_begin = unit_start_step(total, unit, p.units);
+    place.x_end = unit_start_step(total, unit + 1, p.units);
+    place.end = s_end;
+  }
+  const int x_begin = place.x_begin, x_end = place.x_end;
   if (x_begin >= x_end) {  // same for the whole workgroup
     if (vhead == 0 && tid == 0) {
       p.cuts[unit].first_slot = -1;
-      p.cuts[unit].end = s_end;
+      p.cuts[unit].end = place.end;
     }
     return;
   }
@@ -342,21 +425,34 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
   // One walk finds two places: the last wave looks up the unit's last step, for the merge, and the others its first,
   // which they hand to the last wave through LDS.
   const bool looks_at_end = wave == kPrefillWaves - 1;
-  StepPos pos = locate_step(p, s_cum, tq, looks_at_end ? x_end - 1 : x_begin);
+  StepPos pos;
+  if (one_item) {
+    pos = place.pos;
+  } else {
+    pos = locate_step(p, s_cum, tq, looks_at_end ? x_end - 1 : x_begin);
+  }
   if (looks_at_end && vhead == 0 && lane == 0) {
     const BlockTiles item = block_tiles(pos.n_new, pos.ctx, pos.j, tq, p.window_left);
     CutItem cut;
-    cut.step_end = pos.item_x0 + item.count();
-    cut.first_slot = cut.step_end > x_end && pos.item_x0 >= x_begin ? 2 * unit + (pos.item_x0 > x_begin ? 1 : 0) : -1;
-    cut.total = total;
+    if (one_item) {
+      cut.step_end = unit + place.of;
+      cut.first_slot = place.nth == 0 && place.of > 1 ? 2 * unit : -1;
+      cut.total = 0;
+    } else {
+      cut.step_end = pos.item_x0 + item.count();
+      cut.first_slot = cut.step_end > x_end && pos.item_x0 >= x_begin ? 2 * unit + (pos.item_x0 > x_begin ? 1 : 0) : -1;
+      cut.total = s_cum[p.num_seqs];
+    }
     cut.token0 = pos.q_begin + item.tok0;
     cut.tokens = item.cnt;
-    cut.end = s_end;
+    cut.end = place.end;
     p.cuts[unit] = cut;
   }
-  if (tid == 0) s_first = pos;
-  __syncthreads();
-  if (looks_at_end) pos = s_first;
+  if (!one_item) {
+    if (tid == 0) s_first = pos;
+    __syncthreads();
+    if (looks_at_end) pos = s_first;
+  }
   // (the same in every lane, and told so where vector registers are short: 1 024 sequences of 3 tokens, 16 heads of 512,
   // 619 -> 593 us; at the other head dims the scalar registers it takes are missed more, by up to 4 %)
   if constexpr (D > 256)
@@ -1009,14 +1105,19 @@ __global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(PrefillPar
           v[i][k] = *reinterpret_cast<const float2_t*>(ml + 2 * row[k]);
         }
         count = i + 1;
-        int at = unit_start_step(cut.total, u + 1, p.units);
-        for (++u; u < p.units; ++u) {
-          const int next = unit_start_step(cut.total, u + 1, p.units);
-          if (next > at) break;
-          at = next;
+        if (cut.total == 0) {  // the item's own units, one behind the other
+          ++u;
+          more = u < cut.step_end;
+        } else {
+          int at = unit_start_step(cut.total, u + 1, p.units);
+          for (++u; u < p.units; ++u) {
+            const int next = unit_start_step(cut.total, u + 1, p.units);
+            if (next > at) break;
+            at = next;
+          }
+          more = u < p.units && at < cut.step_end;
         }
         slot = 2 * u;
-        more = u < p.units && at < cut.step_end;
       }
     }
 #pragma unroll
@@ -1235,6 +1336,7 @@ int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out
   p.q_dtype = q_dtype;
   p.units = prefill_units(vheads);
   p.rows_per_wg = rows_per_wg;
+  p.few_items = num_seqs <= kWave && tokens / block_tokens + num_seqs <= std::min(kWave, p.units - 1) ? 1 : 0;
   p.scale_log2e = softmax_scale * kLog2e;
   p.cuts = static_cast<CutItem*>(workspace);
   char* const partials = static_cast<char*>(workspace) + kMaxPrefillUnits * sizeof(CutItem);

@@ -21,7 +21,6 @@
 // reads behind them (an operand read per product), at short lengths by a block's chain of steps.
 #include <algorithm>
 #include <atomic>
-#include <type_traits>
 
 #include "cache_row_quant.hpp"
 #include "mfma32_tiles.hpp"
@@ -55,24 +54,6 @@ struct VarlenMfmaParams {
   float scale_log2e;
   PageWrite pages;  // (of the instances that write them)
 };
-
-// Whole-wave reductions of integers, by the steps of wave_max_fast
-template <typename Op>
-__device__ __forceinline__ int wave_reduce(int x, Op op) {
-  auto lanes = [](int v, auto ctrl) {
-    return __builtin_bit_cast(int, dpp_lanes<decltype(ctrl)::value>(__builtin_bit_cast(float, v)));
-  };
-  x = op(x, lanes(x, std::integral_constant<int, kDppQuadSwap1>{}));
-  x = op(x, lanes(x, std::integral_constant<int, kDppQuadSwap2>{}));
-  x = op(x, lanes(x, std::integral_constant<int, kDppRowHalfMirror>{}));
-  x = op(x, lanes(x, std::integral_constant<int, kDppRowMirror>{}));
-  uint32_t a = static_cast<uint32_t>(x), b = a;
-  swap_rows16(a, b);
-  x = op(static_cast<int>(a), static_cast<int>(b));
-  a = b = static_cast<uint32_t>(x);
-  swap_rows32(a, b);
-  return uniform(op(static_cast<int>(a), static_cast<int>(b)));
-}
 
 // What the i-th workgroup of a head computes (block_place); false: nothing.  A lane
 // holds the blocks of sequences lane, lane + 64, ... in registers: a step of the bisection is a sum over the wave.

@@ -529,3 +529,24 @@ def test_prefill_with_its_cache_write_takes_part_in_autograd():
     grads = torch.autograd.grad(out, (q, k, v), torch.ones_like(out))
     want = torch.autograd.grad(ops.areno_varlen_causal_attention(q, k, v, cu.to(DEV)), (q, k, v), torch.ones_like(out))
     assert all(torch.equal(a, b) for a, b in zip(grads, want))
+
+
+@pytest.mark.parametrize("hq,hkv", [(28, 4), (32, 8), (8, 1), (16, 16), (40, 2)])
+@pytest.mark.parametrize("window_left", [None, 200])
+@pytest.mark.parametrize("new,ctx", [
+    ([1], [0]), ([1], [3001]), ([9], [5000]), ([64, 1, 33, 7], [2000, 33, 900, 0]), ([300], [40]), ([1] * 7, [0, 31, 32, 33, 1500, 64, 640]),
+    ([40, 0, 3, 0], [700, 50, 2, 0]), ([2] * 15, list(range(0, 600, 40))), ([5] * 70, [64] * 70),
+])  # fmt: skip
+def test_paged_prefill_of_few_items(hq, hkv, window_left, new, ctx):
+    """Where a launch has fewer items (query blocks) than units, every unit belongs to one item; where they are about as
+    many, or more, the units are equal shares of all steps.  Items of one step and of a hundred, sequences without new
+    tokens, more sequences than lanes, a packed end that no sequence holds."""
+    w = workloads.make_prefill_workload("few", seed=hq + len(new), new_lens=torch.tensor(new), ctx_lens=torch.tensor(ctx), hq=hq, hkv=hkv,
+                                        d=128, bs=16, kv="int8", device=DEV, quantize_fn=gpu_quantize)  # fmt: skip
+    t = w.q.shape[0]
+    q = torch.cat([w.q, w.q[:3]])
+    out = ops.areno_paged_varlen_causal_attention(q, w.k_cache, w.v_cache, w.block_table, w.cu_seqlens_q, w.context_lens,
+                                                  window_left=window_left, softmax_scale=w.softmax_scale, k_scale=w.k_scale,
+                                                  v_scale=w.v_scale)  # fmt: skip
+    assert_close(out[:t], _expected_prefill(w, window_left), *tolerances("int8"), what="prefill of few items")
+    assert not out[t:].any()
