@@ -130,6 +130,7 @@ struct PrefillParams {
   int32_t units;        // per (kv head, part)
   int32_t rows_per_wg;  // query rows of one item: 64 per 16-row tile a wave owns
   int32_t few_items;    // at most 64 items and sequences, fewer than units: place_of_unit
+  float cut_cost;       // there: what an item's being cut once more costs, in tile steps
   float scale_log2e;
 };
 
@@ -235,6 +236,13 @@ struct UnitPlace {
   int end;         // where the last sequence ends
 };
 constexpr int kSegmentSteps = 8;  // what a segment costs besides its steps, in steps
+// A unit of a cut item leaves a partial, 128 KB of a whole block at head dim 128, to be written, found and read again.  So a unit
+// has no fewer steps than makes the sum least of its own, of the partials' traffic and of the merge's chain over an
+// item's partials, which both fall as the steps grow: share + steps of an item * cut_cost / share is least at the root of the
+// product.  Above eight steps the rest of the launch hides that.  With one step a unit where the units allow it, and with
+// these, us: 8 / 2 heads of 128, 1 x 2 tokens on 8 k 45.1 -> 21.1, 2 x 5 on 4 k 33.1 -> 16.2; 28 / 4, 1 x 31 on 2 k 33.9 -> 21.5, 8 x 60 on
+// 64 30.8 -> 21.7; the 411 launches above 0.955 of the time (least 2: 0.953 and up to 1.07; without the longest item's chain 0.96).
+constexpr float kMostLeastSteps = 8.0f;
 __device__ __forceinline__ bool place_of_unit(const PrefillParams& p, int tq, int unit, UnitPlace& at) {
   const int lane = threadIdx.x & (kWave - 1), s = min(lane, p.num_seqs - 1);
   const int q_begin = p.cu_seqlens_q[s], q_end = p.cu_seqlens_q[s + 1];
@@ -256,8 +264,9 @@ __device__ __forceinline__ bool place_of_unit(const PrefillParams& p, int tq, in
   auto sum = [](uint32_t x) { return static_cast<uint32_t>(wave_reduce(static_cast<int>(x), [](int a, int b) { return a + b; })); };
   auto units_at = [&](uint32_t share) { return (steps + share - 1) / share; };
   const uint32_t total = sum(steps), units = static_cast<uint32_t>(p.units), spare = units - static_cast<uint32_t>(items);
-  const uint32_t equal = (total + units - 1) / units;
-  uint32_t lo = equal, hi = (total + spare - 1) / spare;  // (at which a unit more for every item does)
+  const float least = __builtin_amdgcn_sqrtf(p.cut_cost * static_cast<float>(total) * __builtin_amdgcn_rcpf(static_cast<float>(items)));
+  const uint32_t equal = max((total + units - 1) / units, static_cast<uint32_t>(min(max(least, 1.0f), kMostLeastSteps)));
+  uint32_t lo = equal, hi = max((total + spare - 1) / spare, equal);  // (at which a unit more for every item does)
   if (hi >= equal + kSegmentSteps) {
     hi = equal + kSegmentSteps - 1;
     if (sum(units_at(hi)) > units) return false;
@@ -1008,7 +1017,7 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
 // small launch was empty workgroups).  So such a launch has no more of them than the token count allows items, an
 // item's rows are spread over many small workgroups (blockIdx.z; each thread has kMergeChunks 16-byte chunks of every
 // partial), and kMergeBatch partials are asked for before the first of them is used.
-// Kernel time, us: 28 / 4 heads of 128, the follow-ups of 4 sequences, up to 64 tokens on 4 k cached ones, about 11
+// Kernel time with equal shares, us: 28 / 4 heads of 128, the follow-ups of 4 sequences, up to 64 tokens on 4 k cached ones, about 11
 // partials per item: 22.5 -> 10.9 (with one chunk per thread 12.0); 32 / 8 heads, 16 chunks of up to 512 tokens on 16 k cached
 // ones, an item to merge in almost every unit: 15.  The batch where a workgroup has an item: the attention's us with 4, 8, 12, 16,
 // 24: 8 / 1 heads, 1 x 8 tokens on 4 k 66.8, 65.6, 64.8, 65.0, 67.0; on 16 k 105.9, 101.7, 99.9, 98.7, 102.7; 28 / 4, 1 x 8 on 4 k 38.0, 37.0, 36.8,
@@ -1337,6 +1346,8 @@ int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out
   p.units = prefill_units(vheads);
   p.rows_per_wg = rows_per_wg;
   p.few_items = num_seqs <= kWave && tokens / block_tokens + num_seqs <= std::min(kWave, p.units - 1) ? 1 : 0;
+  // (all rows, 32 bits, written and read, at 6.7 MB a step: 0.65 us at twice what a large copy takes from memory, and one step)
+  p.cut_cost = 1.0f + static_cast<float>(vheads) * static_cast<float>(tokens) * static_cast<float>(fold * cache->head_dim) * (8.0f / 6.7e6f);
   p.scale_log2e = softmax_scale * kLog2e;
   p.cuts = static_cast<CutItem*>(workspace);
   char* const partials = static_cast<char*>(workspace) + kMaxPrefillUnits * sizeof(CutItem);
@@ -1348,7 +1359,7 @@ int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out
   // Far fewer items than units, and more workgroups than compute units if each unit had its own: a workgroup per item that
   // there can be (at least one: the merge also writes the zeros behind the last sequence), several partials each, all of
   // them asked for at once.  Otherwise one per unit: finding the item costs a round trip, and fewer workgroups of 170
-  // registers fit.  The attention with a workgroup per unit and per item, us (workgroups of the units in brackets): 28 / 4 heads (64
+  // registers fit.  The attention with a workgroup per unit and per item, us, with equal shares (workgroups of the units in brackets): 28 / 4 heads (64
   // units, blocks of 36 tokens), 1 x 8 tokens on 4 k cached (1 024) 38.6, 31.9; 8 x 32 on 300 (2 560) 25.1, 20.3; 8 / 1 (256 units, blocks
   // of 32), 1 x 8 (1 024) 66.4, 50.3; heads of 64, 1 x 8 on 2 k (512) 50.8, 38.1; 8 / 2 (128 units, blocks of 64), 1 x 32 on 2 k 60.9, 31.4;
   // 4 x 6 on 700 (1 024) 18.7, 19.1; 16 / 16 (16 units, blocks of 256), 1 x 512 on 1 k, with norm, rotary and write, 61.1, 30.3; items
