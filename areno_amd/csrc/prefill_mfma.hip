@@ -357,6 +357,15 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
   constexpr int RSV = 2 * D + 32;
   constexpr int NS = DW / 32;
   constexpr int NB = DW / 16;
+  // The products' operands are read kAhead in front of their own, V's first ones in front of the exponentials, in an order held by
+  // scheduling barriers: left alone, the compiler puts reads and their waits side by side and runs one chain of dependent
+  // products behind the other.  The pass, us, before and with it: 16 x up to 512 tokens on 16 k fp8 ones, 32 / 8 heads of 128, 796 ->
+  // 775; the attention: 8 x 512 on 4 k int8, 28 / 4 heads, 142 -> 133, 200 x 3 on 300 50.5 -> 47.5; heads of 64, 8 x 512 on 4 k, 16 bits,
+  // 76.4 -> 74.5; of 192 and 256 -1 %.  (Row maxima held between the products as well 783, conversion and stores of
+  // the staged chunks between them 849, the second row tile's exponentials between the first one's products 785.)  A head split
+  // over waves has no registers for it (16-bit pages, 512 wide, 8 x 512 tokens on 4 k: 205 -> 230).
+  constexpr int kAhead = DS == 1 ? 4 : 1;
+  constexpr int kSchedVector = 0x6;  // what may be moved across a scheduling barrier: vector and scalar ALU
   typedef typename std::conditional<SCALE16, uint16_t, float>::type scale_raw_t;
 
   __shared__ __attribute__((aligned(16))) char s_k[2][TK * RSK];
@@ -419,7 +428,7 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
 #pragma unroll
   for (int i = 0; i < NLD; ++i) {
     const int c = (kRoleSplit && role_v ? tid - kPrefillThreads / 2 : tid) + kPrefillThreads * i;
-    chunk_live[i] = (i + 1) * kPrefillThreads <= CHUNKS || c < CHUNKS;
+    chunk_live[i] = (kRoleSplit ? kPrefillThreads / 2 : (i + 1) * kPrefillThreads) <= CHUNKS || c < CHUNKS;
     chunk_tok[i] = min(c, CHUNKS - 1) / LPT;
     chunk_col[i] = min(c, CHUNKS - 1) % LPT;
   }
@@ -734,21 +743,25 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
     // raw scores of one key tile: S^T = K . Q^T
     float s_cur[kRowTiles][2][4];
     auto scores = [&](int tile, float (&s)[kRowTiles][2][4]) {
-      const char* kt = s_k[tile & 1];
+      const char* krow = s_k[tile & 1] + lr * RSK + (d0 + (DW / 4) * lk) * 2;
+      auto read = [&](int x) { return *reinterpret_cast<const V8*>(krow + 16 * (x & 1) * RSK + 16 * (x >> 1)); };
+      float4_t c[kRowTiles][2];
 #pragma unroll
-      for (int tg = 0; tg < 2; ++tg) {
-        const char* krow = kt + (16 * tg + lr) * RSK + (d0 + (DW / 4) * lk) * 2;
-        V8 kop[NS];
+      for (int nq = 0; nq < kRowTiles; ++nq) c[nq][0] = c[nq][1] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      V8 kop[kAhead];
 #pragma unroll
-        for (int sl = 0; sl < NS; ++sl) kop[sl] = *reinterpret_cast<const V8*>(krow + 16 * sl);
+      for (int x = 0; x < kAhead; ++x) kop[x] = read(x);
 #pragma unroll
-        for (int nq = 0; nq < kRowTiles; ++nq) {
-          float4_t c = {0.0f, 0.0f, 0.0f, 0.0f};
+      for (int x = 0; x < 2 * NS; ++x) {
+        if constexpr (DS == 1) __builtin_amdgcn_sched_barrier(kSchedVector);
 #pragma unroll
-          for (int sl = 0; sl < NS; ++sl) c = Ops::mfma(kop[sl], qop[nq][sl], c);
+        for (int nq = 0; nq < kRowTiles; ++nq) c[nq][x & 1] = Ops::mfma(kop[x % kAhead], qop[nq][x >> 1], c[nq][x & 1]);
+        if (x + kAhead < 2 * NS) kop[x % kAhead] = read(x + kAhead);
+      }
 #pragma unroll
-          for (int j = 0; j < 4; ++j) s[nq][tg][j] = c[j];
-        }
+      for (int nq = 0; nq < kRowTiles; ++nq) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[nq][0][j] = c[nq][0][j], s[nq][1][j] = c[nq][1][j];
       }
     };
 
@@ -779,6 +792,18 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
             }
             w[j] = __builtin_bit_cast(uint32_t, make_pair<Pair>(a, c));
           }
+          qop[nq][sl] = __builtin_bit_cast(V8, w);
+        }
+      }
+    }
+    // (Q is waited for here: left to the products, which a wave without rows skips, the wait is in every tile step as well)
+    if constexpr (DS == 1) {
+#pragma unroll
+      for (int nq = 0; nq < kRowTiles; ++nq) {
+#pragma unroll
+        for (int sl = 0; sl < NS; ++sl) {
+          uint4_t w = __builtin_bit_cast(uint4_t, qop[nq][sl]);
+          asm volatile("" : "+v"(w));
           qop[nq][sl] = __builtin_bit_cast(V8, w);
         }
       }
@@ -853,7 +878,8 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
           }
         }
       }
-      if constexpr (DS == 1) scores(t + 1, s_next);  // past tb this reads a buffer of clamped or stale keys; the result is dropped
+      // past tb this reads a buffer of clamped or stale keys; the result is dropped
+      if constexpr (DS == 1) scores(t + 1, s_next);
       // -- online softmax in the log2 domain; the (positive) softmax scale is applied to the row maximum and inside
       // the exponent's multiply-add -----------------------------------------------------------------------------------
       // The reference value m of a row only has to be the same for all its keys and to bound the scores well enough
@@ -899,6 +925,24 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
       float m_safe[kRowTiles];
 #pragma unroll
       for (int nq = 0; nq < kRowTiles; ++nq) m_safe[nq] = m_run[nq] == kNegInf ? 0.0f : m_run[nq];
+      // -- O^T += V^T . P^T: lane i of a 16-lane group supplies row (i / 4), 4 elements at column 16 nb + 4 (i % 4);
+      // two transpose reads of 4 tokens each, the first kAhead operands in front of the exponentials ----------------------
+      const char* vt = s_v[t & 1] + (d0 + 4 * (lr & 3)) * 2;
+      auto read = [&](int nb) {
+        uint32_t vw[4];
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          const char* a = vt + v_row_of(16 * half + 4 * lk + (lr >> 2)) * RSV + 32 * nb;
+          const short4_t r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)a);
+          const uint2_t u = __builtin_bit_cast(uint2_t, r);
+          vw[2 * half] = u[0];
+          vw[2 * half + 1] = u[1];
+        }
+        return __builtin_bit_cast(V8, uint4_t{vw[0], vw[1], vw[2], vw[3]});
+      };
+      V8 vop[kAhead];
+#pragma unroll
+      for (int nb = 0; nb < kAhead; ++nb) vop[nb] = read(nb);
       V8 pop[kRowTiles];
 #pragma unroll
       for (int nq = 0; nq < kRowTiles; ++nq) {
@@ -915,25 +959,12 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
         l_acc[nq] = Ops::mfma(ones_op, pop[nq], l_acc[nq]);  // sums the probabilities as rounded for the product
       }
 
-      // -- O^T += V^T . P^T: lane i of a 16-lane group supplies row (i / 4), 4 elements at column 16 nb + 4 (i % 4);
-      // two transpose reads of 4 tokens each -----------------------------------------------------------------------------
-      char* vt = s_v[t & 1];
-      const int r4 = lr >> 2;
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
-        uint32_t vw[4];
+        if constexpr (DS == 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          const int tok = 16 * half + 4 * lk + r4;
-          char* a = vt + v_row_of(tok) * RSV + (d0 + 16 * nb + 4 * (lr & 3)) * 2;
-          const short4_t r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)a);
-          const uint2_t u = __builtin_bit_cast(uint2_t, r);
-          vw[2 * half] = u[0];
-          vw[2 * half + 1] = u[1];
-        }
-        const V8 vop = __builtin_bit_cast(V8, uint4_t{vw[0], vw[1], vw[2], vw[3]});
-#pragma unroll
-        for (int nq = 0; nq < kRowTiles; ++nq) acc[nq][nb] = Ops::mfma(vop, pop[nq], acc[nq][nb]);
+        for (int nq = 0; nq < kRowTiles; ++nq) acc[nq][nb] = Ops::mfma(vop[nb % kAhead], pop[nq], acc[nq][nb]);
+        if (nb + kAhead < NB) vop[nb % kAhead] = read(nb + kAhead);
       }
     };
     for (int t = ta; t <= tb; t += 2) {
