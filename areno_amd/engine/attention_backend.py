@@ -65,9 +65,10 @@ class HipInferBackend(nn.Module):
         k_scale: torch.Tensor | None = None,
         v_scale: torch.Tensor | None = None,
     ) -> torch.Tensor:
-        out = self._native(q, k, v, k_cache, v_cache, meta, window_size, softmax_scale, update_cache, k_scale, v_scale)
-        if out is not None:
-            return out
+        if meta.context_lens is None or meta.mode == "decode":  # (a chunk is no such call)
+            out = self._native(q, k, v, k_cache, v_cache, meta, window_size, softmax_scale, update_cache, k_scale, v_scale)
+            if out is not None:
+                return out
         q_flat = q.reshape(-1, q.shape[-2], q.shape[-1])
         k_flat = k.reshape(-1, k.shape[-2], k.shape[-1])
         v_flat = v.reshape(-1, v.shape[-2], v.shape[-1])
@@ -147,7 +148,7 @@ class HipInferBackend(nn.Module):
                 return None
             return _extension().backend_decode(*tensors, meta.block_table, meta.cache_seqlens, window_left, softmax_scale,
                                                k_scale, v_scale)  # fmt: skip
-        if meta.mode != "prefill" or meta.context_lens is not None or meta.max_seqlen is None or meta.block_table is None:
+        if meta.mode != "prefill" or meta.max_seqlen is None or meta.block_table is None:
             return None
         if meta.cu_seqlens is None or meta.cache_block_ids is None or meta.cache_block_offsets is None:
             return None
