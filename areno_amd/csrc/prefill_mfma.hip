@@ -12,7 +12,8 @@
 // Balance: an item costs one "tile step" per 32-key tile it may see, and items differ by orders of magnitude (a
 // query block on a 16k context next to one on an empty context).  Every workgroup computes the prefix sum of tile
 // steps over the sequences in LDS and takes an equal share of the global tile-step range of its kv head (a "unit"),
-// whatever the length distribution.  A unit is a run of segments, each a range of key tiles of one item:
+// whatever the length distribution; with fewer items than units, units belong to one item each (place_of_unit).  A unit is a
+// run of segments, each a range of key tiles of one item:
 //   * an item that lies inside one unit is finished there and written to `out`;
 //   * an item cut by a unit border leaves un-normalised partials (running max, sum, accumulator) in the workspace
 //     -- slot 2u for the first item of unit u, slot 2u + 1 for its last -- and prefill_merge_kernel combines them.

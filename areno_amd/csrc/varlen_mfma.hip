@@ -13,8 +13,8 @@
 //   * O^T += V^T . P^T with the probabilities as they lie.
 // Measured against the kernel of prefill_mfma.hip and its merge, which it replaces for packed K / V but for few heads over
 // long sequences (equal_shares_are_faster), bf16, us: 32 prompts of 33 .. 512 tokens, 28 / 4 heads of 128, with the cache
-// write: 128 -> 60; 2 x 2 048: 166 -> 81; 4 x 4 096, 32 / 8 heads: 725 -> 540 (1 018 TFLOP/s); 256 tokens alone, 8 / 2 heads:
-// 46 -> 11; 256 x 24: 43 -> 34; 1 024 x 24: 154 -> 159; 4 x 300 .. 1 000, 16 / 8 heads of 256, window 512: 88 -> 39;
+// write: 128 -> 40; 2 x 2 048: 166 -> 74; 4 x 4 096, 32 / 8 heads: 725 -> 520 (1 060 TFLOP/s); 256 tokens alone, 8 / 2 heads:
+// 46 -> 11; 256 x 24: 43 -> 34; 1 024 x 24: 154 -> 159; 4 x 300 .. 1 000, 16 / 8 heads of 256, window 512: 88 -> 32;
 // 16 x 20 .. 600, 16 heads of 64, fp16: 50 -> 16.  What it does not spend any more: a ~10 us fill and drain
 // per query block with nothing beside it, the partials of cut blocks (up to 67 MB written and read), a third of the
 // loop's vector instructions (staging, half the lane swaps).  Bound at length by the matrix cores and the LDS
