@@ -103,6 +103,7 @@ def lib() -> ctypes.CDLL:
         handle.areno_hip_paged_decode_plan.argtypes = [_P, _P, _SZ, _P, _I32, _I32, _I32, _P, _I32, _P, _I32, _I32, _I32, _P, _P]
         handle.areno_hip_paged_decode_planned.argtypes = decode_args[:-2] + [_I32, _P, _P, _P, _SZ, _I32, _P]
         handle.areno_hip_varlen_attention.argtypes = [_P, _P, _P, _P, _I32, _I64, _I32, _I32, _I32, _P, _I32, _I32, _F, _P, _SZ, _P]  # fmt: skip
+        handle.areno_hip_varlen_attention_cache_write.argtypes = [_P, _P, _P, _P, _P, _I32, _I64, _I32, _P, _I32, _I32, _F, _P, _P, _P, _SZ, _P]  # fmt: skip
         handle.areno_hip_paged_varlen_prefill.argtypes = [_P, _P, _P, _I32, _I64, _I32, _I32, _P, _I32, _P, _P, _I32, _F, _P, _SZ, _P]  # fmt: skip
         handle.areno_hip_prefill_workspace_bytes.restype = _SZ
         handle.areno_hip_prefill_workspace_bytes.argtypes = [_I32, _I32]

@@ -209,32 +209,6 @@ int varlen_attention(const void* q, const void* k, const void* v, void* out, int
   return launch_generic(p, stream, op);
 }
 
-// Whether an attention launch over packed K / V can store them in the pages as areno_hip_cache_write would: that
-// kernel's 16-byte rows, and pages that none of the tensors the launch reads lies in (they would be read while they are written).
-bool pages_fit(const areno_paged_cache& c, const void* q, const void* k, const void* v, int32_t dtype, int64_t tokens, int32_t q_heads) {
-  const bool quantized = is_quantized(c.cache_dtype);
-  if (dtype != ARENO_DT_F16 && dtype != ARENO_DT_BF16) return false;
-  if (c.head_dim != 64 && c.head_dim != 128 && c.head_dim != 256 && (quantized || c.head_dim != 192)) return false;
-  if (!quantized && c.cache_dtype != dtype) return false;
-  if ((reinterpret_cast<uintptr_t>(c.k) | reinterpret_cast<uintptr_t>(c.v)) % 16 != 0) return false;
-  const int64_t rows = c.num_blocks * c.block_size * c.kv_heads;
-  struct Range {
-    const void* at;
-    int64_t bytes;
-  };
-  const int64_t row_bytes = static_cast<int64_t>(c.head_dim) * static_cast<int64_t>(dtype_size(c.cache_dtype));
-  const int64_t scale_bytes = quantized ? rows * static_cast<int64_t>(dtype_size(c.scale_dtype)) : 0;
-  const Range written[4] = {{c.k, rows * row_bytes}, {c.v, rows * row_bytes}, {c.k_scale, scale_bytes}, {c.v_scale, scale_bytes}};
-  const Range read[3] = {{q, tokens * q_heads * c.head_dim * 2}, {k, tokens * c.kv_heads * c.head_dim * 2}, {v, tokens * c.kv_heads * c.head_dim * 2}};
-  for (const Range& w : written) {
-    for (const Range& r : read) {
-      const uintptr_t a = reinterpret_cast<uintptr_t>(w.at), b = reinterpret_cast<uintptr_t>(r.at);
-      if (w.bytes > 0 && a < b + static_cast<uintptr_t>(r.bytes) && b < a + static_cast<uintptr_t>(w.bytes)) return false;
-    }
-  }
-  return true;
-}
-
 }  // namespace
 }  // namespace areno
 
@@ -256,7 +230,7 @@ extern "C" int areno_hip_varlen_attention_cache_write(const areno_paged_cache* c
   using namespace areno;
   if (int rc = validate_paged_cache(cache, "areno_hip_varlen_attention_cache_write")) return rc;
   if (tokens > 0 && k != nullptr && v != nullptr && block_ids != nullptr && block_offsets != nullptr &&
-      pages_fit(*cache, q, k, v, dtype, tokens, q_heads)) {
+      pages_fit(*cache, q, k, v, out, dtype, tokens, q_heads, cu_seqlens, num_seqs, block_ids, block_offsets)) {
     const PageWrite pages = {cache->k, cache->v, cache->k_scale, cache->v_scale, block_ids, block_offsets, cache->num_blocks,
                              cache->block_size, cache->cache_dtype, cache->scale_dtype};
     const int rc = varlen_attention(q, k, v, out, dtype, tokens, q_heads, cache->kv_heads, cache->head_dim, cu_seqlens, num_seqs,

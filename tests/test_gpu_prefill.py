@@ -1,6 +1,8 @@
 """Varlen prefill ops vs the CPU oracle: packed new-token attention (the reference's op) and
 causal prefill over paged, optionally quantized KV with a cached context (this build's extension)."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -518,6 +520,24 @@ def test_prefill_whose_keys_lie_in_the_pages_it_writes():
     want = ops.areno_varlen_causal_attention(q, want_pool.view(t, 2, 128), v, cu)
     out = ops.areno_varlen_causal_attention_cache_write(q, pool.view(t, 2, 128), v, cu, pool, other, ids, offs)
     assert torch.equal(out, want) and torch.equal(pool, want_pool) and torch.equal(other.view(t, 2, 128), v)
+
+
+@pytest.mark.parametrize("first_row", [0, 40, 63])
+def test_prefill_whose_output_lies_in_the_pages_it_writes(first_row):
+    """The C entry with ``out`` inside a pool (or behind its last row but one): the pages are stored first, then the output."""
+    t, bs, hq, hkv, d = 64, 16, 2, 2, 128
+    q, k, v, cu = (x.to(DEV) for x in _packed([40, 24], hq, hkv, d, torch.bfloat16))
+    slots = torch.arange(t, device=DEV)
+    ids, offs = slots // bs, slots % bs
+    memory = torch.zeros(first_row + t, hkv, d, device=DEV, dtype=torch.bfloat16)  # V's pool, and the output from first_row on
+    k_pool, v_pool, out = torch.zeros(t // bs, bs, hkv, d, device=DEV, dtype=torch.bfloat16), memory[:t].view(t // bs, bs, hkv, d), memory[first_row:]
+    workspace = torch.empty(cabi.prefill_workspace_bytes(hkv, d), dtype=torch.uint8, device=DEV)
+    cache = cabi.describe_cache(k_pool, v_pool)
+    cabi.check(cabi.lib().areno_hip_varlen_attention_cache_write(
+        ctypes.byref(cache), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), cabi.dtype_code(q), t, hq, cu.data_ptr(), 2, -1, d**-0.5,
+        ids.data_ptr(), offs.data_ptr(), workspace.data_ptr(), workspace.numel(), cabi.current_stream_ptr()), "prefill")  # fmt: skip
+    assert torch.equal(out, ops.areno_varlen_causal_attention(q, k, v, cu))
+    assert torch.equal(k_pool.view(t, hkv, d), k) and torch.equal(memory[:first_row], v[:first_row])
 
 
 def test_prefill_with_its_cache_write_takes_part_in_autograd():
