@@ -109,6 +109,8 @@ __device__ __forceinline__ bool find_block(const VarlenMfmaParams& p, int i, Blo
   return true;
 }
 
+// (the output is taken from 8-byte alignment on; the same instruction stores it)
+typedef uint4_t uint4_at8_t __attribute__((aligned(8)));
 extern __shared__ __attribute__((aligned(1024))) char vm_lds[];
 constexpr int kSchedMatrix = 0x8, kSchedLdsRead = 0x100;  // instruction classes of sched_group_barrier
 
@@ -492,7 +494,7 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(D ==
       const int t_here = token_of_row(32 * wave + row), head_here = 32 * wave + row - t_here * p.fold;
       if (t_here < tok_cnt && head_here < group_here) {
         const int64_t elem = (static_cast<int64_t>(q_begin + tok0 + t_here) * p.q_heads + head0 + head_here) * D + round * (32 * kHere) + 8 * chunk;
-        __builtin_nontemporal_store(w, reinterpret_cast<uint4_t*>(static_cast<char*>(p.out) + elem * 2));
+        __builtin_nontemporal_store(w, reinterpret_cast<uint4_at8_t*>(static_cast<char*>(p.out) + elem * 2));
       }
     });
   }

@@ -229,7 +229,8 @@ int areno_hip_paged_decode_planned(const areno_paged_cache* cache, const void* q
  *   cu_seqlens  device [num_seqs + 1] int32
  *   workspace   device, at least areno_hip_prefill_workspace_bytes(kv_heads, head_dim) bytes (may be NULL for F32): the
  *               launch's sizes decide whether it is used, and no 16-bit call is taken without it
- * Rows of out behind the last sequence (cu_seqlens[num_seqs] < tokens) become zeros.
+ * Rows of out behind the last sequence (cu_seqlens[num_seqs] < tokens) become zeros.  The matrix-core kernels take q, k and v
+ * of 16-byte and out of 8-byte alignment; the generic kernel takes what else there is.
  */
 int areno_hip_varlen_attention(const void* q, const void* k, const void* v, void* out, int32_t dtype, int64_t tokens,
                                int32_t q_heads, int32_t kv_heads, int32_t head_dim, const int32_t* cu_seqlens,

@@ -540,6 +540,21 @@ def test_prefill_whose_output_lies_in_the_pages_it_writes(first_row):
     assert torch.equal(k_pool.view(t, hkv, d), k) and torch.equal(memory[:first_row], v[:first_row])
 
 
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 64), (28, 4, 128), (6, 6, 192), (16, 8, 256)])
+@pytest.mark.parametrize("lens", [[5, 130, 33], [2] * 90])
+def test_packed_output_of_eight_byte_alignment(hq, hkv, d, lens):
+    """The C entry names no alignment for ``out``: from 8 bytes on it goes the way of an aligned one, to the bit."""
+    q, k, v, cu = (x.to(DEV) for x in _packed(lens, hq, hkv, d, torch.bfloat16))
+    workspace = torch.empty(cabi.prefill_workspace_bytes(hkv, d), dtype=torch.uint8, device=DEV)
+    memory = torch.full((q.numel() + 8,), float("nan"), device=DEV, dtype=torch.bfloat16)
+    out = memory[4 : 4 + q.numel()].view(q.shape)
+    cabi.check(cabi.lib().areno_hip_varlen_attention(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), cabi.dtype_code(q), q.shape[0], hq, hkv, d,
+        cu.data_ptr(), len(lens), -1, d**-0.5, workspace.data_ptr(), workspace.numel(), cabi.current_stream_ptr()), "varlen")  # fmt: skip
+    assert torch.equal(out, ops.areno_varlen_causal_attention(q, k, v, cu))
+    assert memory[:4].isnan().all() and memory[-4:].isnan().all()
+
+
 def test_prefill_with_its_cache_write_takes_part_in_autograd():
     q, k, v, cu = _packed([40, 9], 8, 2, 128, torch.bfloat16)
     q, k, v = (x.to(DEV).requires_grad_(True) for x in (q, k, v))
