@@ -768,7 +768,8 @@ bool backend_call(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
   if (!ordinary_call() || !ordinary(q, k, v, k_cache, v_cache)) return false;
   const bool quantized = k_cache.scalar_type() == at::kChar || k_cache.scalar_type() == at::kFloat8_e4m3fn;
   if (k_scale.has_value() != quantized || v_scale.has_value() != quantized) return false;
-  if (quantized && !(ordinary(*k_scale, *v_scale) && k_scale->is_contiguous() && v_scale->is_contiguous())) return false;
+  if (quantized && !(ordinary(*k_scale, *v_scale) && k_scale->dim() == 3 && v_scale->dim() == 3 && k_scale->is_contiguous() && v_scale->is_contiguous()))
+    return false;
   if (c10::GradMode::is_enabled() &&
       (q.requires_grad() || k.requires_grad() || v.requires_grad() || k_cache.requires_grad() || v_cache.requires_grad()))
     return false;

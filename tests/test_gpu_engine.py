@@ -5,6 +5,7 @@ on the (dequantized) cache contents."""
 import pytest
 import torch
 
+from areno_amd.accel import attention as ops
 from areno_amd.engine import InferMeta, allocate_kv_caches, build_infer_attention_backend
 from oracle import attention_ref as ar
 from tests.gpu_util import DEV, assert_close, dequant_cpu, tolerances
@@ -203,3 +204,62 @@ def test_a_pass_is_the_same_through_the_extension_and_the_ops(kv):
             with pytest.raises((error, ValueError)):
                 backend(args["q"], args["k"], args["v"], args["k_cache"], layers[0].v_cache, meta, k_scale=layers[0].k_scale,
                         v_scale=layers[0].v_scale)  # fmt: skip
+
+
+def _refusals(kv, mode):
+    """Calls of the backend that are refused: what they change of a good one, and of its metadata."""
+    scales = [] if kv == "auto" else [
+        ({"k_scale": lambda x: x[..., 0].contiguous()}, {}), ({"v_scale": lambda x: x[..., 0].contiguous()}, {}),
+        ({"k_scale": lambda x: x[None], "v_scale": lambda x: x[None]}, {}), ({"k_scale": lambda x: x.transpose(1, 2)}, {}),
+        ({"k_scale": lambda x: x.cpu()}, {}), ({"k_scale": lambda x: x[:4]}, {}), ({"k_scale": lambda x: None, "v_scale": lambda x: None}, {}),
+        ({"v_scale": lambda x: x.bfloat16()}, {}),
+    ]  # fmt: skip
+    metas = {"prefill": ("cu_seqlens", "cache_block_ids", "cache_block_offsets"), "decode": ("cache_seqlens", "block_table")}[mode]
+    return scales + [
+        ({"k_cache": lambda x: x[0]}, {}), ({"v_cache": lambda x: x.transpose(1, 2)}, {}), ({"k_cache": lambda x: x[:4]}, {}),
+        ({"v_cache": lambda x: x.cpu()}, {}), ({"q": lambda x: torch.cat([x, x], -1)}, {}), ({"q": lambda x: x.cpu()}, {}),
+        ({"q": lambda x: x.half()}, {}), ({"k": lambda x: x.half()}, {}), ({"v": lambda x: x.cpu()}, {}), ({"q": lambda x: x[:, :, :3]}, {}),
+    ] + [({}, {n: change}) for n in metas for change in (lambda x: x.float(), lambda x: x[None], lambda x: x.cpu())]  # fmt: skip
+
+
+@pytest.mark.parametrize("mode", ["prefill", "decode"])
+@pytest.mark.parametrize("kv", ["auto", "int8"])
+def test_a_refused_pass_is_refused_in_the_words_of_the_ops(kv, mode):
+    """Every call that the backend refuses raises what the ops raise that it stands for, type and message."""
+    hq, hkv, d, t = 8, 2, 64, 45
+    backend, dtype = build_infer_attention_backend(), torch.bfloat16
+    slots, table = torch.arange(t, device=DEV), torch.arange(8, dtype=torch.int32, device=DEV).view(2, 4)
+    fields, rows = {
+        "prefill": (dict(cu_seqlens=torch.tensor([0, 40, t], dtype=torch.int32, device=DEV), max_seqlen=40, block_table=table,
+                         cache_block_ids=slots // BS, cache_block_offsets=slots % BS), t),
+        "decode": (dict(cache_seqlens=torch.tensor([40, 5], dtype=torch.int32, device=DEV), block_table=table), 2),
+    }[mode]  # fmt: skip
+    layer = allocate_kv_caches(1, 8, BS, hkv, d, DEV, dtype, kv)[0]
+    good = {n: torch.zeros(1, rows, h, d, dtype=dtype, device=DEV) for n, h in (("q", hq), ("k", hkv), ("v", hkv))}
+    good.update(k_cache=layer.k_cache, v_cache=layer.v_cache, k_scale=layer.k_scale, v_scale=layer.v_scale)
+    scale_of = lambda x: dict(softmax_scale=x) if x is not None else {}  # noqa: E731
+
+    def by_the_ops(a, m, scale):
+        q, k, v = (a[n].reshape(-1, a[n].shape[-2], a[n].shape[-1]).contiguous() for n in "qkv")
+        scales = dict(k_scale=a["k_scale"], v_scale=a["v_scale"])
+        if mode == "decode":
+            for n in ("cache_seqlens", "block_table"):
+                if m[n].dtype != torch.int32:
+                    raise ValueError(f"native decode requires int32 {n}")
+            return ops.areno_paged_causal_attention_decode(q, k, v, a["k_cache"], a["v_cache"], m["block_table"].contiguous(),
+                                                           m["cache_seqlens"].contiguous(), **scales, **scale_of(scale))  # fmt: skip
+        ops.areno_paged_cache_write(k, v, a["k_cache"], a["v_cache"], m["cache_block_ids"], m["cache_block_offsets"], **scales)
+        return ops.areno_varlen_causal_attention(q, k, v, m["cu_seqlens"].contiguous(), **scale_of(scale))
+
+    for changes, meta_changes, *scale in _refusals(kv, mode):
+        scale = scale[0] if scale else None
+        a = {n: changes[n](x) if n in changes else x for n, x in good.items()}
+        m = {n: meta_changes[n](x) if n in meta_changes else x for n, x in fields.items()}
+        raised = []
+        for call in (lambda: by_the_ops(a, m, scale),
+                     lambda: backend(*(a[n] for n in ("q", "k", "v", "k_cache", "v_cache")), InferMeta(mode=mode, **m),
+                                     k_scale=a["k_scale"], v_scale=a["v_scale"], **scale_of(scale))):  # fmt: skip
+            with pytest.raises(Exception) as refused:
+                call()
+            raised.append((refused.type, str(refused.value).split("\n")[0]))
+        assert raised[0] == raised[1], (list(changes), list(meta_changes), scale)
