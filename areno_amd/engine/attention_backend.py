@@ -146,14 +146,20 @@ class HipInferBackend(nn.Module):
         if meta.mode == "decode":
             if meta.cache_seqlens is None or meta.block_table is None:
                 return None
-            return _extension().backend_decode(*tensors, meta.block_table, meta.cache_seqlens, window_left, softmax_scale,
-                                               k_scale, v_scale)  # fmt: skip
+            try:
+                return _extension().backend_decode(*tensors, meta.block_table, meta.cache_seqlens, window_left, softmax_scale,
+                                                   k_scale, v_scale)  # fmt: skip
+            except TypeError:  # (an argument that the binding does not convert: the ops may, or say so)
+                return None
         if meta.mode != "prefill" or meta.max_seqlen is None or meta.block_table is None:
             return None
         if meta.cu_seqlens is None or meta.cache_block_ids is None or meta.cache_block_offsets is None:
             return None
-        return _extension().backend_prefill(*tensors, meta.cu_seqlens, meta.cache_block_ids, meta.cache_block_offsets, window_left,
-                                            softmax_scale, k_scale, v_scale)  # fmt: skip
+        try:
+            return _extension().backend_prefill(*tensors, meta.cu_seqlens, meta.cache_block_ids, meta.cache_block_offsets, window_left,
+                                                softmax_scale, k_scale, v_scale)  # fmt: skip
+        except TypeError:
+            return None
 
 
 def build_infer_attention_backend(attn_backend: str = "native") -> HipInferBackend:

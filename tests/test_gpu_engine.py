@@ -219,7 +219,7 @@ def _refusals(kv, mode):
         ({"k_cache": lambda x: x[0]}, {}), ({"v_cache": lambda x: x.transpose(1, 2)}, {}), ({"k_cache": lambda x: x[:4]}, {}),
         ({"v_cache": lambda x: x.cpu()}, {}), ({"q": lambda x: torch.cat([x, x], -1)}, {}), ({"q": lambda x: x.cpu()}, {}),
         ({"q": lambda x: x.half()}, {}), ({"k": lambda x: x.half()}, {}), ({"v": lambda x: x.cpu()}, {}), ({"q": lambda x: x[:, :, :3]}, {}),
-    ] + [({}, {n: change}) for n in metas for change in (lambda x: x.float(), lambda x: x[None], lambda x: x.cpu())]  # fmt: skip
+    ] + [({}, {n: change}) for n in metas for change in (lambda x: x.float(), lambda x: x[None], lambda x: x.cpu())] + [({}, {}, "no number")]  # fmt: skip
 
 
 @pytest.mark.parametrize("mode", ["prefill", "decode"])
@@ -236,6 +236,7 @@ def test_a_refused_pass_is_refused_in_the_words_of_the_ops(kv, mode):
     }[mode]  # fmt: skip
     layer = allocate_kv_caches(1, 8, BS, hkv, d, DEV, dtype, kv)[0]
     good = {n: torch.zeros(1, rows, h, d, dtype=dtype, device=DEV) for n, h in (("q", hq), ("k", hkv), ("v", hkv))}
+    good["v"].normal_()
     good.update(k_cache=layer.k_cache, v_cache=layer.v_cache, k_scale=layer.k_scale, v_scale=layer.v_scale)
     scale_of = lambda x: dict(softmax_scale=x) if x is not None else {}  # noqa: E731
 
@@ -263,3 +264,6 @@ def test_a_refused_pass_is_refused_in_the_words_of_the_ops(kv, mode):
                 call()
             raised.append((refused.type, str(refused.value).split("\n")[0]))
         assert raised[0] == raised[1], (list(changes), list(meta_changes), scale)
+    out = [backend(*(good[n] for n in ("q", "k", "v", "k_cache", "v_cache")), InferMeta(mode=mode, **fields), k_scale=good["k_scale"],
+                   v_scale=good["v_scale"], softmax_scale=x) for x in (0.25, "0.25")]  # fmt: skip
+    assert torch.equal(*out)  # (whatever float() takes)
