@@ -515,7 +515,11 @@ def areno_varlen_causal_attention_cache_write(
     of fresh prompts: neither needs the other's result, and where the sizes allow it one launch does both.  Pages and
     output are the same bits as those of the two ops."""
     _check_cache_write("areno_paged_cache_write", k, v, k_cache, v_cache, cache_block_ids, cache_block_offsets, k_scale, v_scale)
-    _check_varlen("areno_varlen_causal_attention", q, k, v, cu_seqlens)
+    try:
+        _check_varlen("areno_varlen_causal_attention", q, k, v, cu_seqlens)
+    except (RuntimeError, ValueError):  # (the write comes first, and may refuse the call by itself)
+        areno_paged_cache_write(k, v, k_cache, v_cache, cache_block_ids, cache_block_offsets, k_scale=k_scale, v_scale=v_scale)
+        raise
     pages = (k_cache, v_cache, cache_block_ids.contiguous(), cache_block_offsets.contiguous(), k_scale, v_scale)
     return _VarlenCausalAttention.apply(q, k, v, cu_seqlens, _window_left(window_left), _scale(q, softmax_scale), pages)
 

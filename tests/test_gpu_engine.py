@@ -218,7 +218,8 @@ def _refusals(kv, mode):
     return scales + [
         ({"k_cache": lambda x: x[0]}, {}), ({"v_cache": lambda x: x.transpose(1, 2)}, {}), ({"k_cache": lambda x: x[:4]}, {}),
         ({"v_cache": lambda x: x.cpu()}, {}), ({"q": lambda x: torch.cat([x, x], -1)}, {}), ({"q": lambda x: x.cpu()}, {}),
-        ({"q": lambda x: x.half()}, {}), ({"k": lambda x: x.half()}, {}), ({"v": lambda x: x.cpu()}, {}), ({"q": lambda x: x[:, :, :3]}, {}),
+        ({"k": lambda x: x[:, :, :1]}, {}), ({"v": lambda x: torch.cat([x, x], 2)}, {}), ({"k": lambda x: x[:, :1]}, {}), ({"v": lambda x: x[:, :1]}, {}),
+        ({"k": lambda x: x[..., :32]}, {}), ({"q": lambda x: x.half()}, {}), ({"k": lambda x: x.half()}, {}), ({"v": lambda x: x.cpu()}, {}), ({"q": lambda x: x[:, :, :3]}, {}),
     ] + [({}, {n: change}) for n in metas for change in (lambda x: x.float(), lambda x: x[None], lambda x: x.cpu())] + [({}, {}, "no number")]  # fmt: skip
 
 
