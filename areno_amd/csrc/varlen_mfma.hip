@@ -266,6 +266,7 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(D ==
   const int key_hi = tok0 + tok_cnt - 1;  // the last key any row of the block sees
   const int key_lo = p.window_left >= 0 ? max(0, tok0 - p.window_left) : 0;
   const int ta = key_lo / TK, tb = key_hi / TK;
+  const float lazy = TK == 64 ? 8.0f : D == 128 && tb - ta < 4 ? 1.0f : 2.0f;  // (log2: by how much a score may exceed its row's reference)
   const int64_t stride = static_cast<int64_t>(p.kv_heads) * D * 2;
   const int64_t head_base = (static_cast<int64_t>(q_begin) * p.kv_heads + kvh) * (D * 2);
   const char* const k_base = static_cast<const char*>(p.k) + head_base;
@@ -359,18 +360,18 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(D ==
       }
     }
     // online softmax as in prefill_mfma.hip: the reference value is raised only when a tile exceeds it by 2^8, by 2^2 with steps
-    // of 32 keys, whose first tile sets a lower one.  Relative error against 64 bits with 2^8 and 2^2, in bf16, and of the
-    // kernel with longer steps that it replaces: 256 wide, 300 .. 1 000 tokens, window 512: 2.026e-3, 1.992e-3, 2.020e-3; 192 wide:
-    // 1.985e-3, 1.955e-3, 1.957e-3; 128 wide, 33 .. 900 tokens: 1.973e-3, 1.949e-3, 1.960e-3 (fp16 2.467e-4, 2.436e-4, 2.450e-4).  It
-    // costs 2 to 4 % of the time.
-    constexpr float kLazy = TK == 64 ? 8.0f : 2.0f;
+    // of 32 keys, whose first tile sets a lower one, and at head dim 128 by 2 where a block has no more than four of them.  Relative
+    // error against 64 bits with 2^8 and 2^2, in bf16, and of the kernel with longer steps that it replaces: 256 wide, 300 .. 1 000
+    // tokens, window 512: 2.026e-3, 1.992e-3, 2.020e-3; 192 wide: 1.985e-3, 1.955e-3, 1.957e-3; 128 wide, 33 .. 900 tokens: 1.973e-3,
+    // 1.949e-3, 1.960e-3 (fp16 2.467e-4, 2.436e-4, 2.450e-4).  It costs 2 to 4 % of the time.  With 2^2, with 2, and with longer steps, 128 wide,
+    // sequences of 64 tokens: 1.8202e-3, 1.8137e-3, 1.8177e-3, of 48: 1.7902e-3, 1.7872e-3, 1.7888e-3; 2 everywhere would cost 3 % more.
     float mt = max3_f32(s[0][0], s[0][1], s[0][2]);
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
 #pragma unroll
       for (int i = kt == 0 ? 3 : 0; i < 16; i += 2) mt = max3_f32(mt, s[kt][i], s[kt][i + 1 < 16 ? i + 1 : i]);
     }
-    if (__builtin_amdgcn_ballot_w64(mt * p.scale_log2e > m_run + kLazy) != 0) {
+    if (__builtin_amdgcn_ballot_w64(mt * p.scale_log2e > m_run + lazy) != 0) {
       uint32_t a = __builtin_bit_cast(uint32_t, mt), b = a;
       swap_rows32(a, b);
       mt = max_f32(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));

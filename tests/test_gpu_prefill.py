@@ -444,6 +444,36 @@ def test_paged_rows_behind_the_last_sequence_are_zeros(kv, d, page, behind):
     assert_close(out[: w.q.shape[0]], _run_prefill(w).cpu().float(), *tolerances(kv), what="rows in front of the padding")
 
 
+def _errors(out, q, k, v, lens, ctx):
+    """Relative distance from 64 bits of ``out``, and of attention whose only roundings are those of the probabilities, against
+    the row's largest score, and of the result; a row's sum is that of the rounded probabilities, as in the kernels."""
+    G, num, rounded, den, a, b = q.shape[1] // k.shape[1], 0.0, 0.0, 0.0, 0, 0
+    for n, c in zip(lens, ctx):
+        hidden = torch.arange(n + c)[None] > torch.arange(c, c + n)[:, None]
+        for h in range(q.shape[1]):
+            keys, values = k[b : b + n + c, h // G].double(), v[b : b + n + c, h // G].double()
+            s = (q[a : a + n, h].double() @ keys.T * q.shape[2] ** -0.5).masked_fill(hidden, -float("inf"))
+            p = (s - s.amax(1, keepdim=True)).exp()
+            p16 = p.to(out.dtype).double()
+            want, near = p @ values / p.sum(1, keepdim=True), p16 @ values / p16.sum(1, keepdim=True)
+            num += (out[a : a + n, h].double() - want).square().sum().item()
+            rounded += (near.to(out.dtype).double() - want).square().sum().item()
+            den += want.square().sum().item()
+        a, b = a + n, b + n + c
+    return (num / den) ** 0.5, (rounded / den) ** 0.5
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens", [[48] * 60, [64] * 60, list(range(33, 100))])
+def test_short_sequences_are_as_precise_as_their_rounded_probabilities(dtype, lens):
+    """Steps of 32 keys start a row with a reference that a later step may exceed; short sequences' probabilities are still
+    rounded as finely as against the row's maximum.  The bound's margin is for the sums' order, some 1e-4 of a rounding."""
+    q, k, v, cu = _packed(lens, 8, 2, 128, dtype)
+    out = ops.areno_varlen_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV)).cpu()
+    error, bound = _errors(out, q, k, v, lens, [0] * len(lens))
+    assert error <= bound * 1.0003, (error, bound)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("hq,hkv,d", [(7, 1, 128), (2, 2, 64), (3, 1, 192)])
 @pytest.mark.parametrize("lens", [
