@@ -235,6 +235,7 @@ struct UnitPlace {
   int x_begin, x_end;
   int nth, of;     // which of the item's units this is
   int end;         // where the last sequence ends
+  float lazy;      // (log2) by how much a score may exceed its row's reference; -inf: the reference follows every tile
 };
 constexpr int kSegmentSteps = 8;  // what a segment costs besides its steps, in steps
 // A unit of a cut item leaves a partial, 128 KB of a whole block at head dim 128, to be written, found and read again.  So a unit
@@ -288,6 +289,7 @@ __device__ __forceinline__ bool place_of_unit(const PrefillParams& p, int tq, in
     first += n;
   }
   at.end = __builtin_amdgcn_readlane(q_end, p.num_seqs - 1);
+  at.lazy = total < 4 * units ? kNegInf : 2.0f;
   at.x_begin = at.x_end = 0;
   if (chosen < 0) return true;  // (a unit without work)
   at.nth = unit - chosen_first;
@@ -404,6 +406,8 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
     place.x_end = unit_start_step(total, unit + 1, p.units);
     place.end = s_end;
   }
+  // (uniform, and told so)
+  const float lazy = __builtin_bit_cast(float, uniform(__builtin_bit_cast(int, one_item ? place.lazy : 8.0f)));
   const int x_begin = place.x_begin, x_end = place.x_end;
   if (x_begin >= x_end) {  // same for the whole workgroup
     if (vhead == 0 && tid == 0) {
@@ -888,7 +892,15 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
       // accumulators rescaled) only when a tile's scores exceed it by more than kLazy in the log2 domain (a factor
       // 2^kLazy in the probabilities, far inside fp16's range); each lane checks its own eight scores and one ballot
       // decides for the wave, which skips the cross-lane maximum and the rescale on most tiles.
-      constexpr float kLazy = 8.0f;
+      // In units of one item (place_of_unit), which have more steps than equal shares had, more keys would share a reference, and
+      // the probability that is exactly one, the largest, would be rounded in more rows.  There it is raised by a factor of
+      // 2^2; or, where equal shares would have fewer than four steps, it follows every tile's own maximum, also down, by at most
+      // kMostFall while the sum is small enough to grow by as much.  Relative error against 64 bits with equal shares, with units
+      // of one item and 2^8, and with this, 16-bit pages, heads of 128: 1 x 64 tokens on 600, 28 / 4 heads: 2.021e-3, 2.269e-3, 2.021e-3;
+      // 4 x 64 on 4 k: 2.253e-3, 2.281e-3, 2.209e-3; of 100 launches in two types no less precise.  It costs 2.7 % of the time
+      // (4 x 64 on 4 k, int8, with the write 34.2 -> 36.0 us; every tile's maximum in all of them 5.3 %; 2^4 or more in place of
+      // 2^2 gives less than half of that back and loses up to 1.4 % in precision).
+      constexpr float kMostFall = 8.0f, kMostSum = 16777216.0f;
       float mt_lane[kRowTiles];
       bool raise = false;
 #pragma unroll
@@ -897,13 +909,13 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
                                max3_f32(s_cur[nq][0][3], s_cur[nq][1][0], s_cur[nq][1][1]),
                                max3_f32(s_cur[nq][1][2], s_cur[nq][1][3], s_cur[nq][1][3]));
         // (-inf > -inf + kLazy is false: a fully masked row stays at -inf; anything finite beats -inf)
-        raise = raise | (mt_lane[nq] * p.scale_log2e > m_run[nq] + kLazy);  // no short circuit: straight-line code
+        raise = raise | (mt_lane[nq] * p.scale_log2e > m_run[nq] + lazy);  // no short circuit: straight-line code
       }
       if (__builtin_amdgcn_ballot_w64(raise) != 0) {
 #pragma unroll
         for (int nq = 0; nq < kRowTiles; ++nq) {
           const float mt = rows_max(mt_lane[nq]) * p.scale_log2e;
-          const float m_new = max_f32(m_run[nq], mt);
+          const float m_new = max_f32(m_run[nq] - (lazy < 0.0f && l_acc[nq][0] < kMostSum ? kMostFall : 0.0f), mt);
           const float m_ref = m_new == kNegInf ? 0.0f : m_new;
           const float alpha = settled(fast_exp2(m_run[nq] - m_ref));
           m_run[nq] = m_new;

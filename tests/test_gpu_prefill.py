@@ -475,6 +475,31 @@ def test_short_sequences_are_as_precise_as_their_rounded_probabilities(dtype, le
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d", [(28, 4, 128), (8, 1, 128), (8, 2, 64), (8, 4, 256)])
+@pytest.mark.parametrize("new,ctx", [([64], [600]), ([16], [3000]), ([60, 20, 50, 44], [400, 100, 300, 20])])
+def test_paged_prefill_of_few_items_is_as_precise_as_its_rounded_probabilities(dtype, hq, hkv, d, new, ctx):
+    """Units of one item have more steps than equal shares; their probabilities are rounded as finely as against the row's
+    maximum all the same."""
+    g = torch.Generator().manual_seed(d)
+    total, bs = [n + c for n, c in zip(new, ctx)], 16
+    k, v = (torch.randn(sum(total), hkv, d, generator=g).to(dtype) for _ in range(2))
+    q = torch.randn(sum(new), hq, d, generator=g).to(dtype)
+    pages = [-(-n // bs) for n in total]
+    table, ids, offs, first = torch.zeros(len(new), max(pages), dtype=torch.int32), [], [], 0
+    for i, n in enumerate(total):
+        table[i, : pages[i]] = torch.arange(first, first + pages[i])
+        ids.append(first + torch.arange(n) // bs)
+        offs.append(torch.arange(n) % bs)
+        first += pages[i]
+    k_cache, v_cache = (torch.zeros(first, bs, hkv, d, dtype=dtype, device=DEV) for _ in range(2))
+    ops.areno_paged_cache_write(k.to(DEV), v.to(DEV), k_cache, v_cache, torch.cat(ids).to(DEV), torch.cat(offs).to(DEV))
+    cu = torch.tensor([0] + new).cumsum(0).to(torch.int32)
+    out = ops.areno_paged_varlen_causal_attention(q.to(DEV), k_cache, v_cache, table.to(DEV), cu.to(DEV), torch.tensor(ctx, dtype=torch.int32, device=DEV)).cpu()
+    error, bound = _errors(out, q, k, v, new, ctx)
+    assert error <= bound * 1.001, (error, bound)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("hq,hkv,d", [(7, 1, 128), (2, 2, 64), (3, 1, 192)])
 @pytest.mark.parametrize("lens", [
     [2] * 256, [2] * 257, [1] * 1000 + [150] * 24, [7, 0] * 512, [0] * 1023 + [300], [40] + [0, 3] * 300, [1] * 1025,
