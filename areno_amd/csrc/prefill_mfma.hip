@@ -224,12 +224,12 @@ __device__ __forceinline__ int unit_start_step(int total, int u, int units) {
 // border cuts has two segments, and a segment costs ~10 us besides its steps (a fill, a query block, an end), as much as eight
 // steps: with six items over 64 units, six or seven steps each, the launch is those few units.  Here an item has as many
 // units as it needs at `share` steps each, the least share that does with the launch's units.  Every wave finds its place
-// by itself, a lane per sequence and then per item, with nothing to wait for but the lengths.  False: shares would become
-// a segment's cost larger than equal ones, or nothing to do.  The attention with equal shares and with this, us: 28 / 4 heads
+// by itself, a lane per sequence and then per item, with nothing to wait for but the lengths.  Where shares would become
+// a segment's cost larger than equal ones they stay equal, and what the lanes hold becomes the table that those are looked up in.  The attention with equal shares and with this, us: 28 / 4 heads
 // of 128, 4 x 64 tokens on 4 k int8 ones: 33 -> 30; 8 x 512 on 4 k 101 -> 65; 2 x 512 on 64, 16 bits, 48.7 -> 30.8; 8 / 2,
 // 1 x 12 on 600 20.0 -> 11.8; of 411 launches of 1 .. 16 sequences of 1 .. 512 tokens on up to 16 k, by how many steps a share
-// is larger: none 0.82 of the time, 1 .. 3 0.82, 4 .. 7 0.89.  The look that finds it eight or more, and in vain, is 1 us:
-// 38.8 -> 39.8, 262 -> 266.
+// is larger: none 0.82 of the time, 1 .. 3 0.82, 4 .. 7 0.89.  The look that finds it eight or more, and in vain, costs up
+// to 1 us, which the table gives back in part (48 such launches 0.993 of the time with a table of the lengths read again).
 struct UnitPlace {
   StepPos pos;     // (item_x0 = 0: steps count from the item's first)
   int x_begin, x_end;
@@ -245,20 +245,23 @@ constexpr int kSegmentSteps = 8;  // what a segment costs besides its steps, in 
 // these, us: 8 / 2 heads of 128, 1 x 2 tokens on 8 k 45.1 -> 21.1, 2 x 5 on 4 k 33.1 -> 16.2; 28 / 4, 1 x 31 on 2 k 33.9 -> 21.5, 8 x 60 on
 // 64 30.8 -> 21.7; the 411 launches above 0.955 of the time (least 2: 0.953 and up to 1.07; without the longest item's chain 0.96).
 constexpr float kMostLeastSteps = 8.0f;
-__device__ __forceinline__ bool place_of_unit(const PrefillParams& p, int tq, int unit, UnitPlace& at) {
+enum class Placed { kUnit, kTable, kNothing };  // the unit's place; where sequences begin and end on the line of steps (s_cum)
+__device__ __forceinline__ Placed place_of_unit(const PrefillParams& p, int tq, int unit, int* s_cum, UnitPlace& at) {
   const int lane = threadIdx.x & (kWave - 1), s = min(lane, p.num_seqs - 1);
   const int q_begin = p.cu_seqlens_q[s], q_end = p.cu_seqlens_q[s + 1];
   const int ctx = p.context_lens != nullptr ? p.context_lens[s] : 0;
   const int n_new = lane < p.num_seqs ? max(q_end - q_begin, 0) : 0;
   const int blocks = query_blocks(n_new, tq);
-  int items = 0, seq = 0, before = 0;
+  int items = 0, seq = 0, before = 0, first_item = 0;
   for (int i = 0; i < p.num_seqs; ++i) {
+    first_item = lane == i ? items : first_item;
     items += __builtin_amdgcn_readlane(blocks, i);
     const bool behind = lane >= items;
     seq += behind ? 1 : 0;
     before = behind ? items : before;
   }
-  if (items == 0 || items > kWave || items >= p.units) return false;
+  at.end = __builtin_amdgcn_readlane(q_end, p.num_seqs - 1);
+  if (items == 0 || items > kWave || items >= p.units) return Placed::kNothing;
   seq = min(seq, p.num_seqs - 1);
   const int item_new = __shfl(n_new, seq, kWave), item_ctx = __shfl(ctx, seq, kWave), j = lane < items ? lane - before : 0;
   const BlockTiles tiles = block_tiles(item_new, item_ctx, j, tq, p.window_left);
@@ -271,7 +274,19 @@ __device__ __forceinline__ bool place_of_unit(const PrefillParams& p, int tq, in
   uint32_t lo = equal, hi = max((total + spare - 1) / spare, equal);  // (at which a unit more for every item does)
   if (hi >= equal + kSegmentSteps) {
     hi = equal + kSegmentSteps - 1;
-    if (sum(units_at(hi)) > units) return false;
+    if (sum(units_at(hi)) > units) {
+      // the table that equal shares are looked up in, of what the lanes hold; every wave writes it, the same
+      uint32_t behind = steps;
+#pragma unroll
+      for (int off = 1; off < kWave; off <<= 1) {
+        const uint32_t before_it = __shfl_up(behind, off, kWave);
+        if (lane >= off) behind += before_it;
+      }
+      const int first_step = __shfl(static_cast<int>(behind - steps), min(first_item, kWave - 1), kWave);
+      if (lane < p.num_seqs) s_cum[lane] = first_item < items ? first_step : static_cast<int>(total);
+      if (lane == 0) s_cum[p.num_seqs] = static_cast<int>(total);
+      return Placed::kTable;
+    }
   }
   while (lo < hi) {
     const uint32_t mid = (lo + hi) / 2;
@@ -288,10 +303,9 @@ __device__ __forceinline__ bool place_of_unit(const PrefillParams& p, int tq, in
     if (unit >= first && unit < first + n) chosen = i, chosen_first = first;
     first += n;
   }
-  at.end = __builtin_amdgcn_readlane(q_end, p.num_seqs - 1);
   at.lazy = total < 4 * units ? kNegInf : 2.0f;
   at.x_begin = at.x_end = 0;
-  if (chosen < 0) return true;  // (a unit without work)
+  if (chosen < 0) return Placed::kUnit;  // (a unit without work)
   at.nth = unit - chosen_first;
   at.of = __builtin_amdgcn_readlane(of, chosen);
   at.x_begin = at.nth * share;
@@ -303,7 +317,7 @@ __device__ __forceinline__ bool place_of_unit(const PrefillParams& p, int tq, in
   at.pos.q_begin = __builtin_amdgcn_readlane(q_begin, at.pos.seq);
   at.pos.tile = __builtin_amdgcn_readlane(tiles.tile_lo, chosen) + at.x_begin;
   at.pos.item_x0 = 0;
-  return true;
+  return Placed::kUnit;
 }
 
 // 16 codes of an 8-bit cache row (one 16-byte chunk) -> 16 fp16 values times the row's scale, as two 16-byte groups.
@@ -398,16 +412,19 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
   const int tq = p.block_tokens;  // query tokens per item
 
   UnitPlace place;
-  const bool one_item = p.few_items != 0 && place_of_unit(p, tq, unit, place);  // (the same for the whole launch)
-  if (!one_item) {
+  const Placed placed = p.few_items != 0 ? place_of_unit(p, tq, unit, s_cum, place) : Placed::kNothing;  // (the same for the whole launch)
+  const bool one_item = placed == Placed::kUnit;
+  if (placed == Placed::kNothing) {
     prefix_tile_steps(p, tq, s_cum, s_wave_tot, &s_end);
+    place.end = s_end;
+  }
+  if (!one_item) {
     const int total = s_cum[p.num_seqs];
     place.x_begin = unit_start_step(total, unit, p.units);
     place.x_end = unit_start_step(total, unit + 1, p.units);
-    place.end = s_end;
   }
-  // (uniform, and told so)
-  const float lazy = __builtin_bit_cast(float, uniform(__builtin_bit_cast(int, one_item ? place.lazy : 8.0f)));
+  float lazy = one_item ? place.lazy : 8.0f;
+  asm("" : "+v"(lazy));  // (scalar registers are short)
   const int x_begin = place.x_begin, x_end = place.x_end;
   if (x_begin >= x_end) {  // same for the whole workgroup
     if (vhead == 0 && tid == 0) {
@@ -758,7 +775,7 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
       for (int x = 0; x < kAhead; ++x) kop[x] = read(x);
 #pragma unroll
       for (int x = 0; x < 2 * NS; ++x) {
-        if constexpr (DS == 1) __builtin_amdgcn_sched_barrier(kSchedVector);
+        if constexpr (kAhead > 1) __builtin_amdgcn_sched_barrier(kSchedVector);
 #pragma unroll
         for (int nq = 0; nq < kRowTiles; ++nq) c[nq][x & 1] = Ops::mfma(kop[x % kAhead], qop[nq][x >> 1], c[nq][x & 1]);
         if (x + kAhead < 2 * NS) kop[x % kAhead] = read(x + kAhead);
@@ -802,7 +819,7 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
       }
     }
     // (Q is waited for here: left to the products, which a wave without rows skips, the wait is in every tile step as well)
-    if constexpr (DS == 1) {
+    if constexpr (kAhead > 1) {
 #pragma unroll
       for (int nq = 0; nq < kRowTiles; ++nq) {
 #pragma unroll
@@ -912,10 +929,11 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
         raise = raise | (mt_lane[nq] * p.scale_log2e > m_run[nq] + lazy);  // no short circuit: straight-line code
       }
       if (__builtin_amdgcn_ballot_w64(raise) != 0) {
+        const float fall = __builtin_amdgcn_fmed3f(-lazy, 0.0f, kMostFall);
 #pragma unroll
         for (int nq = 0; nq < kRowTiles; ++nq) {
           const float mt = rows_max(mt_lane[nq]) * p.scale_log2e;
-          const float m_new = max_f32(m_run[nq] - (lazy < 0.0f && l_acc[nq][0] < kMostSum ? kMostFall : 0.0f), mt);
+          const float m_new = max_f32(m_run[nq] - (l_acc[nq][0] < kMostSum ? fall : 0.0f), mt);
           const float m_ref = m_new == kNegInf ? 0.0f : m_new;
           const float alpha = settled(fast_exp2(m_run[nq] - m_ref));
           m_run[nq] = m_new;
@@ -974,7 +992,7 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
 
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
-        if constexpr (DS == 1) __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kAhead > 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int nq = 0; nq < kRowTiles; ++nq) acc[nq][nb] = Ops::mfma(vop[nb % kAhead], pop[nq], acc[nq][nb]);
         if (nb + kAhead < NB) vop[nb % kAhead] = read(nb + kAhead);
