@@ -380,8 +380,9 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
   // 775; the attention: 8 x 512 on 4 k int8, 28 / 4 heads, 142 -> 133, 200 x 3 on 300 50.5 -> 47.5; heads of 64, 8 x 512 on 4 k, 16 bits,
   // 76.4 -> 74.5; of 192 and 256 -1 %.  (Row maxima held between the products as well 783, conversion and stores of
   // the staged chunks between them 849, the second row tile's exponentials between the first one's products 785.)  A head split
-  // over waves has no registers for it (16-bit pages, 512 wide, 8 x 512 tokens on 4 k: 205 -> 230).
-  constexpr int kAhead = DS == 1 ? 4 : 1;
+  // over waves has no registers for it (16-bit pages, 512 wide, 8 x 512 tokens on 4 k: 205 -> 230).  8-bit pages of heads of 64: of 60
+  // launches of more than 40 us, one, two and four ahead take 0.964, 0.948 and 0.955 of the time before.
+  constexpr int kAhead = DS > 1 ? 1 : D == 64 && ES == 1 ? 2 : 4;
   constexpr int kSchedVector = 0x6;  // what may be moved across a scheduling barrier: vector and scalar ALU
   typedef typename std::conditional<SCALE16, uint16_t, float>::type scale_raw_t;
 
