@@ -548,16 +548,24 @@ bool equal_shares_are_faster(int64_t tokens, int32_t num_seqs, int32_t q_heads, 
 
 // Head dim 128: steps of 32 keys leave room for three workgroups per compute unit, whose starts, ends and softmax fall into
 // each other's products; steps of 64, two workgroups, are fewer, which counts where a launch is the chain of its longest
-// blocks.  So 32 for launches that fill the chip's places (blocks of the tokens, half a block more per sequence), the more so the
-// longer their chains, and for short sequences.  In us, 64 and 32 keys (workgroups, mean length): 28 / 4 heads, 64 x 12 .. 52 tokens (588, 32)
-// 11.7, 8.2; 16 x 200 (740) 17.8, 13.1; 64 x 25 .. 390 (2 913, 195) 60.8, 52; 16 x 64 .. 960 (1 716, 474) 52.3, 47; 2 x 2 048 (912) 81, 74; 4 x 4 096 (3 648) 476, 468; 32 / 8,
-// 1 x 4 096 (1 024) 146, 141.  Fewer, longer ones: 16 / 16, 4 x 250 (144) 11.8, 12.5; 4 x 1 343 (688) 48.4, 53; 28 / 4, 1 x 2 048 (452) 45.0, 49; 8 / 2, 4 x 3 334
-// (840) 137, 149.  Of 302 launches of 1 .. 64 sequences of 12 .. 6 600 tokens, five head ratios, equal and ragged lengths, the choice takes
-// 0.2 % more than the better one (6 % at most), 64 keys everywhere 4.8 %.  At head dim 64, where four workgroups share a unit with 64
-// keys, five with 32 gain and lose as much.
+// blocks.  Sequences of up to 64 keys fill no more than one long step.  Where blocks cost alike -- a window, or sequences of equal
+// length as far as the sizes tell -- 32 wins as soon as there are more blocks than the 512 places of the longer steps, or a few less: a second
+// round is spared; the more keys, the more blocks it takes, up to 900.  Where lengths differ the longest ones decide for longer, and the line
+// lies higher, up to 1 400 blocks (of the tokens, half a block more per sequence).  In us, 64 and 32 keys (blocks, keys seen):
+//   equal: 28 / 4 heads, 16 x 200 (740, 200) 17.8, 13.1; 2 x 2 048 (912, 2 048) 81, 74; 4 x 4 096 (3 648) 476, 468; 32 / 8, 1 x 4 096 (1 024) 146, 141;
+// 16 / 16, 4 x 250 (144) 11.8, 12.5; 28 / 4, 1 x 2 048 (452) 45.0, 49;
+//   ragged: 28 / 4, 64 x 12 .. 52 (588, 32) 11.7, 8.2; 64 x 25 .. 390 (2 913, 195) 60.8, 52; 16 x 64 .. 960 (1 716, 474) 52.3, 47; 8 / 2, 4 x 3 334 on average
+// (840) 137, 149.
+// Of 2 576 launches of 1 .. 64 sequences of 12 .. 8 192 tokens, seven head ratios, equal and two kinds of ragged lengths, with and without a
+// window, most of them near the lines, the choice takes 1.3 % more than the better one, 64 keys everywhere 5.6 %, 32 everywhere 4.0 %, one line
+// for all of them (550 + 3 / 20 of the keys) 2.1 %; it is slower than 64 keys by more than 3 % in 165, most with one sequence far longer
+// than the rest, that line in 431.  At head dim 64, where four workgroups share a unit with 64 keys, five with 32 gain and lose as much.
 bool short_tiles_are_faster(int64_t tokens, int32_t num_seqs, int64_t vheads, int block_tokens, int32_t window_left) {
-  const int64_t mean = tokens / num_seqs, seen = window_left >= 0 ? std::min<int64_t>(mean, window_left + int64_t{1} + block_tokens) : mean;
-  return seen <= 200 || (tokens / block_tokens + num_seqs / 2) * vheads >= 550 + 3 * seen / 20;
+  const int64_t mean = tokens / num_seqs, window = window_left + int64_t{1} + block_tokens;
+  const int64_t seen = window_left >= 0 ? std::min(mean, window) : mean;
+  if (seen <= 64) return true;
+  const bool alike = num_seqs == 1 || (mean * num_seqs == tokens && mean % 16 == 0) || seen < mean;
+  return (tokens / block_tokens + num_seqs / 2) * vheads >= std::min<int64_t>(alike ? 425 + seen / 4 : 300 + 2 * seen, alike ? 900 : 1400);
 }
 
 }  // namespace

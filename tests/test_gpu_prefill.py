@@ -464,10 +464,10 @@ def _errors(out, q, k, v, lens, ctx):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("lens", [[48] * 60, [64] * 60, list(range(33, 100))])
+@pytest.mark.parametrize("lens", [[48] * 60, [64] * 60, list(range(33, 65)) * 2])
 def test_short_sequences_are_as_precise_as_their_rounded_probabilities(dtype, lens):
-    """Steps of 32 keys start a row with a reference that a later step may exceed; short sequences' probabilities are still
-    rounded as finely as against the row's maximum.  The bound's margin is for the sums' order, some 1e-4 of a rounding."""
+    """Steps of 32 keys (which launches of up to 64 tokens a sequence take) start a row with a reference that a later step may exceed;
+    short sequences' probabilities are still rounded as finely as against the row's maximum.  The bound's margin is for the sums' order, some 1e-4 of a rounding."""
     q, k, v, cu = _packed(lens, 8, 2, 128, dtype)
     out = ops.areno_varlen_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), cu.to(DEV)).cpu()
     error, bound = _errors(out, q, k, v, lens, [0] * len(lens))
