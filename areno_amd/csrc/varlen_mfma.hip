@@ -158,7 +158,9 @@ __device__ __forceinline__ void write_page_chunk(const PageWrite& w, uint4_t raw
 // fetch, and their stores go out behind the output's, while the next workgroup starts.  The pass with a launch of its own for
 // the pages and with this, us (both with the output's stores as they were then): 32 prompts of 33 .. 512 tokens, 28 / 4 heads of 128, bf16: 61.5 -> 57.6; 2 x 3 000 .. 6 000, 16 / 8
 // heads of 256, window 1 024: 176.6 -> 165; 24 x 48 .. 387 into fp8 pages 40.0 -> 38.8; 2 x 9 .. 74: 21.7 -> 17.7 (the host's).
-template <int KIND, int D, bool WRITE, int TILE>
+//
+// PAST_L2: the output's stores leave L2 to the tiles (output_past_l2).
+template <int KIND, int D, bool WRITE, int TILE, bool PAST_L2>
 __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(D == 128 && TILE == 32 ? 3 : 2, D == 64 ? 4 : D == 128 && TILE == 32 ? 3 : 2))) void varlen_mfma_kernel(VarlenMfmaParams p) {
   using S = VmShape<D, WRITE, TILE>;
   using T = typename S::Tile;
@@ -495,7 +497,12 @@ __global__ __launch_bounds__(kVmThreads) __attribute__((amdgpu_waves_per_eu(D ==
       const int t_here = token_of_row(32 * wave + row), head_here = 32 * wave + row - t_here * p.fold;
       if (t_here < tok_cnt && head_here < group_here) {
         const int64_t elem = (static_cast<int64_t>(q_begin + tok0 + t_here) * p.q_heads + head0 + head_here) * D + round * (32 * kHere) + 8 * chunk;
-        __builtin_nontemporal_store(w, reinterpret_cast<uint4_at8_t*>(static_cast<char*>(p.out) + elem * 2));
+        uint4_at8_t* const to = reinterpret_cast<uint4_at8_t*>(static_cast<char*>(p.out) + elem * 2);
+        if constexpr (PAST_L2) {
+          __builtin_nontemporal_store(w, to);
+        } else {
+          *to = w;
+        }
       }
     });
   }
@@ -506,23 +513,35 @@ struct VmLaunch {
   vm_fn fn;  // nullptr: no such kernel, or its LDS size was refused
   int lds_bytes;
 };
-template <int KIND, int D, bool WRITE, int TILE>
+template <int KIND, int D, bool WRITE, int TILE, bool PAST_L2>
 VmLaunch vm_launch_of() {
   static std::atomic<uint64_t> allowed_on{0};
   constexpr int kLdsBytes = VmShape<D, WRITE, TILE>::kLdsBytes;
-  const vm_fn fn = varlen_mfma_kernel<KIND, D, WRITE, TILE>;
+  const vm_fn fn = varlen_mfma_kernel<KIND, D, WRITE, TILE, PAST_L2>;
   return {allow_lds<kLdsBytes>(reinterpret_cast<const void*>(fn), allowed_on) ? fn : nullptr, kLdsBytes};
 }
-template <int KIND, bool WRITE>
+template <int KIND, bool WRITE, bool PAST_L2>
 VmLaunch vm_lookup(int head_dim, bool short_tiles) {
   switch (head_dim) {
-    case 64: return vm_launch_of<KIND, 64, WRITE, 64>();
-    case 128: return short_tiles ? vm_launch_of<KIND, 128, WRITE, 32>() : vm_launch_of<KIND, 128, WRITE, 64>();
-    case 192: return vm_launch_of<KIND, 192, WRITE, 32>();
-    case 256: return vm_launch_of<KIND, 256, WRITE, 32>();
+    case 64: return vm_launch_of<KIND, 64, WRITE, 64, PAST_L2>();
+    case 128: return short_tiles ? vm_launch_of<KIND, 128, WRITE, 32, PAST_L2>() : vm_launch_of<KIND, 128, WRITE, 64, PAST_L2>();
+    case 192: return vm_launch_of<KIND, 192, WRITE, 32, PAST_L2>();
+    case 256: return vm_launch_of<KIND, 256, WRITE, 32, PAST_L2>();
     default: return {nullptr, 0};
   }
 }
+template <int KIND>
+VmLaunch vm_lookup(int head_dim, bool short_tiles, bool write, bool past_l2) {
+  if (write) return past_l2 ? vm_lookup<KIND, true, true>(head_dim, short_tiles) : vm_lookup<KIND, true, false>(head_dim, short_tiles);
+  return past_l2 ? vm_lookup<KIND, false, true>(head_dim, short_tiles) : vm_lookup<KIND, false, false>(head_dim, short_tiles);
+}
+
+// The output's stores past L2 leave it to the tiles, 2 to 12 % of the kernel from 4 MB on, and cost the reader behind it nothing there; up to
+// 2 MB they gain nothing and cost it up to 2 us.  With and without, attention and a product with its output's width,
+// us: 16 heads of 64, 256 tokens (0.5 MB): 15.4, 13.8; 8 / 2 of 128, 500 (1 MB): 21.7, 19.4; 28 / 4, 500 (3.6 MB): 41.9, 42.8; 8 / 2,
+// 4 448 (9.1 MB): 33.6, 34.7; 28 / 4, 8 333 (60 MB): 210.1, 209.7; 16 / 8 of 256, 16 384 (134 MB): 903, 934.  (Two instances: decided inside the
+// kernel, per store or per block, it costs heads of 256 and short steps 2 to 4 %.)
+bool output_past_l2(int64_t tokens, int32_t q_heads, int32_t head_dim) { return tokens * q_heads * head_dim * 2 > (int64_t{2} << 20); }
 
 // Few heads over long sequences: such a launch has fewer blocks than the chip has places for, and lasts as long as its
 // longest block, one chain of steps over all its keys.  The kernel of prefill_mfma.hip, which cuts the blocks' steps
@@ -580,8 +599,8 @@ int launch_varlen_mfma(const void* q, const void* k, const void* v, void* out, i
   const bool bf16 = dtype == ARENO_DT_BF16;
   const int group = q_heads / kv_heads, head_parts = (group + 15) / 16;
   const bool short_tiles = short_tiles_are_faster(tokens, num_seqs, kv_heads * head_parts, kVmRows / (head_parts > 1 ? 16 : group), window_left);
-  const VmLaunch l = pages != nullptr ? (bf16 ? vm_lookup<KV_BF16, true>(head_dim, short_tiles) : vm_lookup<KV_F16, true>(head_dim, short_tiles))
-                                      : (bf16 ? vm_lookup<KV_BF16, false>(head_dim, short_tiles) : vm_lookup<KV_F16, false>(head_dim, short_tiles));
+  const bool past_l2 = output_past_l2(tokens, q_heads, head_dim);
+  const VmLaunch l = bf16 ? vm_lookup<KV_BF16>(head_dim, short_tiles, pages != nullptr, past_l2) : vm_lookup<KV_F16>(head_dim, short_tiles, pages != nullptr, past_l2);
   if (l.fn == nullptr) return ARENO_ERR_UNSUPPORTED;
   if (equal_shares_are_faster(tokens, num_seqs, q_heads, group, head_dim, window_left)) return ARENO_ERR_UNSUPPORTED;
   const int64_t vheads = static_cast<int64_t>(kv_heads) * head_parts;
