@@ -47,6 +47,7 @@
 // context 0 it is the reference's varlen kernel (areno/accel/csrc/attention.cu:145-242).
 
 #include "decode_mfma_kernels.hpp"
+#include "item_units.hpp"
 #include "page_write.hpp"
 #include "prefill_steps.hpp"
 
@@ -237,14 +238,12 @@ struct UnitPlace {
   int end;         // where the last sequence ends
   float lazy;      // (log2) by how much a score may exceed its row's reference; -inf: the reference follows every tile
 };
-constexpr int kSegmentSteps = 8;  // what a segment costs besides its steps, in steps
 // A unit of a cut item leaves a partial, 128 KB of a whole block at head dim 128, to be written, found and read again.  So a unit
 // has no fewer steps than makes the sum least of its own, of the partials' traffic and of the merge's chain over an
 // item's partials, which both fall as the steps grow: share + steps of an item * cut_cost / share is least at the root of the
 // product.  Above eight steps the rest of the launch hides that.  With one step a unit where the units allow it, and with
 // these, us: 8 / 2 heads of 128, 1 x 2 tokens on 8 k 45.1 -> 21.1, 2 x 5 on 4 k 33.1 -> 16.2; 28 / 4, 1 x 31 on 2 k 33.9 -> 21.5, 8 x 60 on
 // 64 30.8 -> 21.7; the 411 launches above 0.955 of the time (least 2: 0.953 and up to 1.07; without the longest item's chain 0.96).
-constexpr float kMostLeastSteps = 8.0f;
 enum class Placed { kUnit, kTable, kNothing };  // the unit's place; where sequences begin and end on the line of steps (s_cum)
 __device__ __forceinline__ Placed place_of_unit(const PrefillParams& p, int tq, int unit, int* s_cum, UnitPlace& at) {
   const int lane = threadIdx.x & (kWave - 1), s = min(lane, p.num_seqs - 1);
@@ -267,49 +266,33 @@ __device__ __forceinline__ Placed place_of_unit(const PrefillParams& p, int tq, 
   const BlockTiles tiles = block_tiles(item_new, item_ctx, j, tq, p.window_left);
   const uint32_t steps = lane < items ? static_cast<uint32_t>(max(tiles.count(), 1)) : 0u;
   auto sum = [](uint32_t x) { return static_cast<uint32_t>(wave_reduce(static_cast<int>(x), [](int a, int b) { return a + b; })); };
-  auto units_at = [&](uint32_t share) { return (steps + share - 1) / share; };
-  const uint32_t total = sum(steps), units = static_cast<uint32_t>(p.units), spare = units - static_cast<uint32_t>(items);
+  const uint32_t total = sum(steps);
   const float least = __builtin_amdgcn_sqrtf(p.cut_cost * static_cast<float>(total) * __builtin_amdgcn_rcpf(static_cast<float>(items)));
-  const uint32_t equal = max((total + units - 1) / units, static_cast<uint32_t>(min(max(least, 1.0f), kMostLeastSteps)));
-  uint32_t lo = equal, hi = max((total + spare - 1) / spare, equal);  // (at which a unit more for every item does)
-  if (hi >= equal + kSegmentSteps) {
-    hi = equal + kSegmentSteps - 1;
-    if (sum(units_at(hi)) > units) {
-      // the table that equal shares are looked up in, of what the lanes hold; every wave writes it, the same
-      uint32_t behind = steps;
+  const uint32_t share = share_of_items(total, static_cast<uint32_t>(items), static_cast<uint32_t>(p.units), least,
+                                        [&](uint32_t n) { return sum((steps + n - 1) / n); });
+  if (share == 0) {
+    // the table that equal shares are looked up in, of what the lanes hold; every wave writes it, the same
+    uint32_t behind = steps;
 #pragma unroll
-      for (int off = 1; off < kWave; off <<= 1) {
-        const uint32_t before_it = __shfl_up(behind, off, kWave);
-        if (lane >= off) behind += before_it;
-      }
-      const int first_step = __shfl(static_cast<int>(behind - steps), min(first_item, kWave - 1), kWave);
-      if (lane < p.num_seqs) s_cum[lane] = first_item < items ? first_step : static_cast<int>(total);
-      if (lane == 0) s_cum[p.num_seqs] = static_cast<int>(total);
-      return Placed::kTable;
+    for (int off = 1; off < kWave; off <<= 1) {
+      const uint32_t before_it = __shfl_up(behind, off, kWave);
+      if (lane >= off) behind += before_it;
     }
+    const int first_step = __shfl(static_cast<int>(behind - steps), min(first_item, kWave - 1), kWave);
+    if (lane < p.num_seqs) s_cum[lane] = first_item < items ? first_step : static_cast<int>(total);
+    if (lane == 0) s_cum[p.num_seqs] = static_cast<int>(total);
+    return Placed::kTable;
   }
-  while (lo < hi) {
-    const uint32_t mid = (lo + hi) / 2;
-    if (sum(units_at(mid)) <= units) {
-      hi = mid;
-    } else {
-      lo = mid + 1;
-    }
-  }
-  const int share = static_cast<int>(lo), of = static_cast<int>(units_at(lo));
-  int first = 0, chosen = -1, chosen_first = 0;
-  for (int i = 0; i < items; ++i) {
-    const int n = __builtin_amdgcn_readlane(of, i);
-    if (unit >= first && unit < first + n) chosen = i, chosen_first = first;
-    first += n;
-  }
-  at.lazy = total < 4 * units ? kNegInf : 2.0f;
+  const int of = static_cast<int>((steps + share - 1) / share);
+  const ItemUnit mine = item_of_unit(unit, items, [&](int i) { return __builtin_amdgcn_readlane(of, i); });
+  at.lazy = total < 4 * static_cast<uint32_t>(p.units) ? kNegInf : 2.0f;
   at.x_begin = at.x_end = 0;
-  if (chosen < 0) return Placed::kUnit;  // (a unit without work)
-  at.nth = unit - chosen_first;
+  if (mine.item < 0) return Placed::kUnit;
+  const int chosen = mine.item;
+  at.nth = mine.nth;
   at.of = __builtin_amdgcn_readlane(of, chosen);
-  at.x_begin = at.nth * share;
-  at.x_end = min(at.x_begin + share, __builtin_amdgcn_readlane(static_cast<int>(steps), chosen));
+  at.x_begin = at.nth * static_cast<int>(share);
+  at.x_end = min(at.x_begin + static_cast<int>(share), __builtin_amdgcn_readlane(static_cast<int>(steps), chosen));
   at.pos.seq = __builtin_amdgcn_readlane(seq, chosen);
   at.pos.j = __builtin_amdgcn_readlane(j, chosen);
   at.pos.n_new = __builtin_amdgcn_readlane(item_new, chosen);

@@ -2,9 +2,13 @@
 // steps in front of a query block and the bisection that finds the block of a step, held against a walk over the
 // blocks with block_tiles(), the one definition of which key tiles a block sees.  Built by
 // tests/test_prefill_steps_cpu.py with g++; no GPU code.
+#include <math.h>
 #include <stdint.h>
 #include <stdio.h>
 
+#include <vector>
+
+#include "../../areno_amd/csrc/item_units.hpp"
 #include "../../areno_amd/csrc/prefill_steps.hpp"
 
 using namespace areno;
@@ -62,5 +66,60 @@ extern "C" int prefill_steps_check_grid(int n_hi, int ctx_hi, const int* tqs, in
           ++shapes;
         }
   *shapes_out = shapes;
+  return 0;
+}
+
+// Every unit of a launch of few items (areno_amd/csrc/item_units.hpp): the least share that does is taken, and the units walk
+// over every item's steps once, in order, an item's units one behind the other as the merge takes them.  *share_out: steps a
+// unit, 0: equal shares; -1: not such a launch.
+extern "C" int item_units_check(const int* n_new, const int* ctx, int seqs, int tq, int window_left, int units, float cut_cost,
+                                int* share_out, char* msg, int msg_len) {
+  std::vector<uint32_t> steps;
+  uint32_t total = 0;
+  for (int s = 0; s < seqs; ++s) {
+    for (int j = 0; j < query_blocks(n_new[s], tq); ++j) {
+      steps.push_back(static_cast<uint32_t>(block_tiles(n_new[s], ctx[s], j, tq, window_left).count()));
+      total += steps.back();
+    }
+  }
+  const int items = static_cast<int>(steps.size());
+  *share_out = -1;
+  if (items == 0 || items >= units) return 0;
+  auto units_at = [&](uint32_t share) {
+    uint32_t n = 0;
+    for (uint32_t x : steps) n += (x + share - 1) / share;
+    return n;
+  };
+  const float least = sqrtf(cut_cost * static_cast<float>(total) / static_cast<float>(items));
+  const uint32_t share = share_of_items(total, static_cast<uint32_t>(items), static_cast<uint32_t>(units), least, units_at);
+  uint32_t lo = (total + static_cast<uint32_t>(units) - 1) / static_cast<uint32_t>(units);
+  while (lo < kMostLeastSteps && static_cast<float>(lo + 1) <= least) ++lo;
+  *share_out = static_cast<int>(share);
+  for (uint32_t x = lo; x < lo + kSegmentSteps; ++x) {  // the first of these that does, or none
+    if (units_at(x) > static_cast<uint32_t>(units)) continue;
+    if (share != x) {
+      snprintf(msg, msg_len, "share %u, the least that does is %u", share, x);
+      return 1;
+    }
+    break;
+  }
+  if (share == 0) {
+    if (units_at(lo + kSegmentSteps - 1) > static_cast<uint32_t>(units)) return 0;
+    snprintf(msg, msg_len, "equal shares, but %u steps a unit do", lo + kSegmentSteps - 1);
+    return 1;
+  }
+  int item = 0, nth = 0;
+  for (int u = 0; u < units; ++u) {
+    const ItemUnit at = item_of_unit(u, items, [&](int i) { return static_cast<int>((steps[i] + share - 1) / share); });
+    if (at.item != (item < items ? item : -1) || (item < items && at.nth != nth)) {
+      snprintf(msg, msg_len, "unit %d: item %d, its unit %d, the walk is at item %d, unit %d", u, at.item, at.nth, item, nth);
+      return 1;
+    }
+    if (item < items && ++nth * share >= steps[item]) ++item, nth = 0;
+  }
+  if (item < items) {
+    snprintf(msg, msg_len, "item %d of %d has steps that no unit takes", item, items);
+    return 1;
+  }
   return 0;
 }

@@ -640,3 +640,14 @@ def test_paged_prefill_of_few_items(hq, hkv, window_left, new, ctx):
                                                   v_scale=w.v_scale)  # fmt: skip
     assert_close(out[:t], _expected_prefill(w, window_left), *tolerances("int8"), what="prefill of few items")
     assert not out[t:].any()
+
+
+@pytest.mark.parametrize("kv,d,page", [("bf16", 64, 16), ("fp8", 128, 64), ("int8", 192, 16), ("bf16", 256, 24), ("int8", 64, 256), ("bf16", 512, 16)])
+@pytest.mark.parametrize("hq,hkv", [(14, 2), (16, 16)])
+@pytest.mark.parametrize("new,ctx", [([9], [3000]), ([3] * 8, [3000, 2500, 2000, 1500, 1000, 600, 300, 100]), ([40, 0, 3, 0], [700, 50, 2, 0])])
+def test_paged_prefill_of_few_items_in_every_type(kv, d, page, hq, hkv, new, ctx):
+    """The same over the caches' types, head dims and page sizes; the second pack, at 16 heads, is one that looks for units of one
+    item in vain and takes equal shares."""
+    w = workloads.make_prefill_workload("few", seed=d + page, new_lens=torch.tensor(new), ctx_lens=torch.tensor(ctx), hq=hq, hkv=hkv, d=d, bs=page,
+                                        kv=kv, device=DEV, quantize_fn=gpu_quantize)  # fmt: skip
+    assert_close(_run_prefill(w), _expected_prefill(w, None), *tolerances(kv), what="prefill of few items")

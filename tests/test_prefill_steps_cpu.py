@@ -58,3 +58,24 @@ def test_closed_forms_on_large_and_random_shapes(lib):
     # a known total: 4 096 new tokens without context in blocks of 64 see 2 j + 2 tiles each
     lib.prefill_steps_check(4096, 0, 64, -1, 0, ctypes.byref(steps), msg, 256)
     assert steps.value == sum(2 * j + 2 for j in range(64))
+
+
+def test_units_of_few_items_take_every_step_once(lib):
+    """Launches with fewer items than units, of one step and of thousands, empty sequences, windows: the least share, every
+    step once, in the merge's order; both outcomes of the search."""
+    rng = random.Random(11)
+    msg = ctypes.create_string_buffer(256)
+    share = ctypes.c_int(0)
+    lib.item_units_check.argtypes = [ctypes.POINTER(ctypes.c_int)] * 2 + [ctypes.c_int] * 4 + [ctypes.c_float, ctypes.POINTER(ctypes.c_int), ctypes.c_char_p, ctypes.c_int]  # fmt: skip
+    packs = [([1], [0]), ([1], [100000]), ([0, 0, 3], [5, 7, 9]), ([1] * 63, [0] * 63), ([3] * 8, [3000, 2500, 2000, 1500, 1000, 600, 300, 100])]
+    for _ in range(4000):
+        seqs, new, ctx = rng.choice([1, 2, 4, 8, 16, 40]), rng.choice([1, 8, 64, 512]), rng.choice([0, 64, 600, 4000, 16000])
+        packs.append(([rng.randint(0 if rng.random() < 0.1 else 1, new) for _ in range(seqs)], [rng.randint(0, ctx) for _ in range(seqs)]))
+    outcomes = {}
+    for new, ctx in packs:
+        tq, units, window = rng.choice(BLOCK_TOKENS), rng.choice([2, 8, 16, 32, 64, 128, 256, 512]), rng.choice([-1, -1, 0, 40, 1000])
+        ints = ctypes.c_int * len(new)
+        rc = lib.item_units_check(ints(*new), ints(*ctx), len(new), tq, window, units, rng.choice([1.0, 1.3, 4.0, 20.0]), ctypes.byref(share), msg, 256)
+        assert rc == 0, (msg.value.decode(), new, ctx, tq, units, window)
+        outcomes[min(share.value, 9)] = outcomes.get(min(share.value, 9), 0) + 1
+    assert all(outcomes.get(x, 0) > 50 for x in (-1, 0, 1, 2, 8, 9)), outcomes
