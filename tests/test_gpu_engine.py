@@ -172,7 +172,7 @@ def test_loop_driven_by_device_block_tables():
 @pytest.mark.parametrize("kv", ["auto", "int8"])
 def test_a_pass_is_the_same_through_the_extension_and_the_ops(kv):
     """The backend hands most calls to the extension as a whole; a call that wants a gradient, or whose values need padding,
-    goes through the ops.  Same output and pages either way, and the refusals are the ops'."""
+    goes through the ops.  Same output and pages either way; what is refused there is refused here (in which words: below)."""
     gen = torch.Generator().manual_seed(9)
     hq, hkv, d, t = 8, 2, 64, 45
     backend = build_infer_attention_backend()

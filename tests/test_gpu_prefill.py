@@ -562,7 +562,7 @@ def test_prefill_with_its_cache_write(kv, act, hq, hkv, d, lens):
 
 
 def test_prefill_whose_keys_lie_in_the_pages_it_writes():
-    """Keys that are read while pages are written must not be those pages: such a call stores first and attends then."""
+    """Keys that lie in the pages, every one in its own place: the store leaves them as they are."""
     t, bs = 64, 16
     g = torch.Generator().manual_seed(3)
     q, v = (torch.randn(t, h, 128, generator=g).to(torch.bfloat16).to(DEV) for h in (8, 2))
@@ -575,6 +575,25 @@ def test_prefill_whose_keys_lie_in_the_pages_it_writes():
     want = ops.areno_varlen_causal_attention(q, want_pool.view(t, 2, 128), v, cu)
     out = ops.areno_varlen_causal_attention_cache_write(q, pool.view(t, 2, 128), v, cu, pool, other, ids, offs)
     assert torch.equal(out, want) and torch.equal(pool, want_pool) and torch.equal(other.view(t, 2, 128), v)
+
+
+@pytest.mark.parametrize("kv", ["same", "int8"])
+@pytest.mark.parametrize("first_row", [0, 40, 63])
+def test_prefill_whose_queries_lie_in_the_pages_it_writes(kv, first_row):
+    """What the attention reads must not be pages that its launch writes: such a call stores first and attends then, with the stored
+    rows as queries.  Queries that are the pages of K, or share their last row (8-bit pages: the last bytes) with them."""
+    t, bs, h, d = 64, 16, 2, 128
+    _, k, v, cu = (x.to(DEV) for x in _packed([40, 24], h, h, d, torch.bfloat16))
+    slots = torch.arange(t, device=DEV)
+    dtype, per_row = (torch.bfloat16, h * d) if kv == "same" else (torch.int8, 2 * h * d)  # (elements of a row of queries)
+    memory = torch.randint(0, 60, (2 * t * per_row,), device=DEV, dtype=torch.int32).to(dtype)  # K's pool, and queries from first_row on
+    pools = [memory[: t * h * d].view(t // bs, bs, h, d), torch.zeros(t // bs, bs, h, d, device=DEV, dtype=dtype)]
+    q = memory[first_row * h * d :][: t * per_row].view(torch.bfloat16).view(t, h, d)
+    scales = {} if kv == "same" else {n: torch.zeros(t // bs, bs, h, device=DEV) for n in ("k_scale", "v_scale")}
+    out = ops.areno_varlen_causal_attention_cache_write(q, k, v, cu, *pools, slots // bs, slots % bs, **scales)
+    want = ops.areno_varlen_causal_attention(q.clone(), k, v, cu)  # (the pages are stored: q is what it became)
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))  # (codes read as 16-bit numbers may be NaN)
+    assert kv != "same" or torch.equal(pools[0].view(t, h, d), k)
 
 
 @pytest.mark.parametrize("first_row", [0, 40, 63])
