@@ -222,15 +222,17 @@ __device__ __forceinline__ int unit_start_step(int total, int u, int units) {
 }
 
 // Few items for many units: units that belong to one item each, instead of equal shares of all steps.  A unit that an item's
-// border cuts has two segments, and a segment costs ~10 us besides its steps (a fill, a query block, an end), as much as eight
-// steps: with six items over 64 units, six or seven steps each, the launch is those few units.  Here an item has as many
-// units as it needs at `share` steps each, the least share that does with the launch's units.  Every wave finds its place
-// by itself, a lane per sequence and then per item, with nothing to wait for but the lengths.  Where shares would become
-// a segment's cost larger than equal ones they stay equal, and what the lanes hold becomes the table that those are looked up in.  The attention with equal shares and with this, us: 28 / 4 heads
-// of 128, 4 x 64 tokens on 4 k int8 ones: 33 -> 30; 8 x 512 on 4 k 101 -> 65; 2 x 512 on 64, 16 bits, 48.7 -> 30.8; 8 / 2,
-// 1 x 12 on 600 20.0 -> 11.8; of 411 launches of 1 .. 16 sequences of 1 .. 512 tokens on up to 16 k, by how many steps a share
-// is larger: none 0.82 of the time, 1 .. 3 0.82, 4 .. 7 0.89.  The look that finds it eight or more, and in vain, costs up
-// to 1 us, which the table gives back in part (48 such launches 0.993 of the time with a table of the lengths read again).
+// border cuts has two segments, and a segment costs ~10 us besides its steps (a fill, a query block, an end; the kernel over
+// one item, 28 / 4 heads of 128, 8 .. 64 steps a unit: 15 us, five of them a launch's start, and 1.18 us a step with int8 pages, 1.11
+// with 16-bit ones), as much as eight steps: with six items over 64 units, six or seven steps each, the launch is those few units.
+// Here an item has as many units as it needs at `share` steps each, the least share that does with the launch's units
+// (item_units.hpp).  Every wave finds its place by itself, a lane per sequence and then per item, with nothing to wait for but the
+// lengths.  Where shares would become a segment's cost larger than equal ones they stay equal, and what the lanes hold becomes the
+// table that those are looked up in.  The attention with equal shares and with this, us: 28 / 4 heads of 128, 2 x 512 tokens on 64,
+// 16 bits, 46 -> 32; 8 / 2, 1 x 12 on 600 23 -> 13; of 411 launches of 1 .. 16 sequences of 1 .. 512 tokens on up to 16 k the 319 that it
+// serves take 0.80 of the time.  The look that finds a share eight steps larger or more, and is in vain, costs up to 1 us (24 / 8 heads of
+// 64, int8, 16 x 8 on up to 4 k: 38.9 -> 39.5), which the table gives back in part (48 such launches 0.993 of the time with a table of
+// the lengths read again); the host, which knows no contexts, cannot tell those launches.
 struct UnitPlace {
   StepPos pos;     // (item_x0 = 0: steps count from the item's first)
   int x_begin, x_end;
@@ -241,9 +243,9 @@ struct UnitPlace {
 // A unit of a cut item leaves a partial, 128 KB of a whole block at head dim 128, to be written, found and read again.  So a unit
 // has no fewer steps than makes the sum least of its own, of the partials' traffic and of the merge's chain over an
 // item's partials, which both fall as the steps grow: share + steps of an item * cut_cost / share is least at the root of the
-// product.  Above eight steps the rest of the launch hides that.  With one step a unit where the units allow it, and with
-// these, us: 8 / 2 heads of 128, 1 x 2 tokens on 8 k 45.1 -> 21.1, 2 x 5 on 4 k 33.1 -> 16.2; 28 / 4, 1 x 31 on 2 k 33.9 -> 21.5, 8 x 60 on
-// 64 30.8 -> 21.7; the 411 launches above 0.955 of the time (least 2: 0.953 and up to 1.07; without the longest item's chain 0.96).
+// product.  Above eight steps (kMostLeastSteps) the rest of the launch hides that.  With one step a unit where the units allow it, and with
+// these, us: 8 / 2 heads of 128, 1 x 2 tokens on 8 k 45 -> 23, 2 x 5 on 4 k 33 -> 19; 28 / 4, 1 x 31 on 2 k 34 -> 25, 8 x 60 on
+// 64 31 -> 24; the 411 launches above 0.955 of the time (least 2: 0.953 and up to 1.07; without the longest item's chain 0.96).
 enum class Placed { kUnit, kTable, kNothing };  // the unit's place; where sequences begin and end on the line of steps (s_cum)
 __device__ __forceinline__ Placed place_of_unit(const PrefillParams& p, int tq, int unit, int* s_cum, UnitPlace& at) {
   const int lane = threadIdx.x & (kWave - 1), s = min(lane, p.num_seqs - 1);
@@ -1392,7 +1394,7 @@ int launch_prefill_mfma(const areno_paged_cache* cache, const void* q, void* out
   p.units = prefill_units(vheads);
   p.rows_per_wg = rows_per_wg;
   p.few_items = num_seqs <= kWave && tokens / block_tokens + num_seqs <= std::min(kWave, p.units - 1) ? 1 : 0;
-  // (all rows, 32 bits, written and read, at 6.7 MB a step: 0.65 us at twice what a large copy takes from memory, and one step)
+  // (all rows, 32 bits, written and read, at 6.7 MB a step -- 1.15 us at 5.8 TB/s -- and one step of the merge's chain)
   p.cut_cost = 1.0f + static_cast<float>(vheads) * static_cast<float>(tokens) * static_cast<float>(fold * cache->head_dim) * (8.0f / 6.7e6f);
   p.scale_log2e = softmax_scale * kLog2e;
   p.cuts = static_cast<CutItem*>(workspace);
