@@ -137,8 +137,8 @@ class HipInferBackend(nn.Module):
     def _native(q, k, v, k_cache, v_cache, meta, window_size, softmax_scale, update_cache, k_scale, v_scale):
         """The pass as one call of the extension: small ones last as long as the host needs for them.  Through the ops and as one
         call, us: decode of one row with 4 k cached tokens 16.8, 13.7, of short rows 17.1, 11.7; prompts of a few tokens
-        (two ops) 21.3, 11.5.  None: whatever it does not take as a matter of course, and every call that the checks of the
-        ops refuse."""
+        (two ops) 21.3, 11.5.  None: whatever it does not take as a matter of course, and every call that the ops refuse by
+        themselves; the extension's own checks raise here what they raise there."""
         if not q.is_cuda or not update_cache or (window_size is not None and window_size[1] != 0 and tuple(window_size) != (-1, -1)):
             return None
         window_left = -1 if window_size is None else int(window_size[0])
