@@ -892,8 +892,8 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
       // the exponent's multiply-add -----------------------------------------------------------------------------------
       // The reference value m of a row only has to be the same for all its keys and to bound the scores well enough
       // for the exponentials to fit the operand type; it need not be the exact maximum.  So it is raised (and the
-      // accumulators rescaled) only when a tile's scores exceed it by more than kLazy in the log2 domain (a factor
-      // 2^kLazy in the probabilities, far inside fp16's range); each lane checks its own eight scores and one ballot
+      // accumulators rescaled) only when a tile's scores exceed it by more than `lazy` in the log2 domain (8: a factor
+      // 2^8 in the probabilities, far inside fp16's range); each lane checks its own eight scores and one ballot
       // decides for the wave, which skips the cross-lane maximum and the rescale on most tiles.
       // In units of one item (place_of_unit), which have more steps than equal shares had, more keys would share a reference, and
       // the probability that is exactly one, the largest, would be rounded in more rows.  There it is raised by a factor of
@@ -911,7 +911,7 @@ __global__ __launch_bounds__(kPrefillThreads, RT <= 2 ? 8 / kPrefillWaves : 1) v
         mt_lane[nq] = max3_f32(max3_f32(s_cur[nq][0][0], s_cur[nq][0][1], s_cur[nq][0][2]),
                                max3_f32(s_cur[nq][0][3], s_cur[nq][1][0], s_cur[nq][1][1]),
                                max3_f32(s_cur[nq][1][2], s_cur[nq][1][3], s_cur[nq][1][3]));
-        // (-inf > -inf + kLazy is false: a fully masked row stays at -inf; anything finite beats -inf)
+        // (-inf > -inf + lazy is false: a fully masked row stays at -inf; anything finite beats -inf)
         raise = raise | (mt_lane[nq] * p.scale_log2e > m_run[nq] + lazy);  // no short circuit: straight-line code
       }
       if (__builtin_amdgcn_ballot_w64(raise) != 0) {
